@@ -12,7 +12,8 @@ namespace qsv {
 
 constexpr int kBlock = 256;          // threads per workgroup (4 waves of 64)
 constexpr int kReduceBlocks = 1024;  // fixed grid for FP64 reductions
-constexpr int kMaxPauliPerPass = 8;  // Pauli terms evaluated per pass over the state
+constexpr int kPartials = 128 * kReduceBlocks;   // doubles of reduction scratch per state
+constexpr int kReduceOut = 4096;     // doubles of reduction results per state
 constexpr int kSampleChunkLog = 10;  // amplitudes per chunk in the sampling prefix
 
 // Zero-bit insertion plan: enumerate `count` indices j and map each to the
@@ -82,10 +83,40 @@ void launch_c64_to_f64(const void* src, double* dst, uint64_t count, hipStream_t
 void launch_norm2(int prec, const void* psi, uint64_t S, double* partials, double* out, hipStream_t st);
 void launch_inner(int prec, const void* a, const void* b, uint64_t S, double* partials, double* out,
                   hipStream_t st);
-void launch_pauli(int prec, const void* psi, uint64_t S, int nterms, const uint64_t* xmask, const uint64_t* smask,
-                  double* partials, double* out, hipStream_t st);
 void launch_expect1q(int prec, const void* psi, uint64_t S, uint64_t tbit, const double m[8], double* partials,
                      double* out, hipStream_t st);
+// Pauli-string sums (qsv_pauli.hip). One sweep over tiles of 12 index bits
+// `pos` (ascending): nz Z strings (basis-index masks) and nu units, a multiple
+// of four, of two strings each that share the X part x (tile-local, top = its
+// highest bit). A string's sign part is split into tile-local bits s and the
+// bits outside the tile g; im picks Im instead of Re. Results: out[0..nz) the
+// Z sums, out[nz + 2 u + j] the sum over half the pairs of string j of unit u.
+constexpr int kPauliZ = 128;
+constexpr int kPauliUnits = 48;
+constexpr int kPauliXBlocks = 512;
+struct PauliUnit {
+  uint32_t x, top;
+  uint32_t s0, s1;
+  uint64_t g0, g1;
+  int32_t im0, im1;
+};
+struct PauliSweep {
+  int32_t nz, nu;
+  int32_t pos[12];
+  uint64_t zmask[kPauliZ];
+  PauliUnit u[kPauliUnits];
+};
+hipError_t launch_pauli_sweep(int prec, const void* psi, uint64_t S, const PauliSweep& sw, double* partials,
+                              double* out, hipStream_t st);
+// n <= kPauliRows strings, each over the state on its own: x == 0 the whole
+// sum, else half the pairs (bit r of im: Im instead of Re of string r).
+constexpr int kPauliRows = 64;
+struct PauliRows {
+  uint64_t x[kPauliRows], s[kPauliRows];
+  uint64_t im;
+};
+hipError_t launch_pauli_rows(int prec, const void* psi, uint64_t S, const PauliRows& rows, int n, double* partials,
+                             double* out, hipStream_t st);
 void launch_probs(int prec, const void* psi, uint64_t offset, uint64_t count, double* out, hipStream_t st);
 
 // Sampling: chunk sums -> inclusive prefix -> one wave per shot.

@@ -1,5 +1,5 @@
 // qsv_kernels.hip — state initialisation, conversions, FP64 reductions
-// (norm, overlaps, Pauli expectations), sampling and measurement of libqsv.
+// (norm, overlaps, one-qubit expectations), sampling and measurement of libqsv.
 //
 // State layout: 2^n amplitudes, interleaved (re, im); c128 = double2 (16 B),
 // c64 = float2 (8 B). Reference qubit q is index bit b = n-1-q.
@@ -227,52 +227,6 @@ __global__ __launch_bounds__(kBlock) void k_inner(const typename VT<R>::T* __res
   if (threadIdx.x == 0) {
     partials[blockIdx.x] = r0;
     partials[kReduceBlocks + blockIdx.x] = r1;
-  }
-}
-
-struct PauliArgs {
-  int32_t nterms;
-  uint64_t xmask[kMaxPauliPerPass];
-  uint64_t smask[kMaxPauliPerPass];
-};
-
-// For each term t: sum_i (-1)^popc(i & s_t) conj(a_i) a_{i ^ x_t}.
-template <typename R>
-__global__ __launch_bounds__(kBlock) void k_pauli(const typename VT<R>::T* __restrict__ psi, uint64_t S,
-                                                   PauliArgs pa, double* __restrict__ partials)
-{
-  __shared__ double sh[kBlock / 64];
-  double re[kMaxPauliPerPass], im[kMaxPauliPerPass];
-#pragma unroll
-  for (int t = 0; t < kMaxPauliPerPass; ++t) { re[t] = 0.0; im[t] = 0.0; }
-  const uint64_t stride = (uint64_t)gridDim.x * kBlock;
-  for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < S; i += stride) {
-    const auto a = psi[i];
-    const double ar = a.x, ai = a.y;
-#pragma unroll
-    for (int t = 0; t < kMaxPauliPerPass; ++t) {
-      if (t < pa.nterms) {
-        const double sgn = (__popcll(i & pa.smask[t]) & 1) ? -1.0 : 1.0;
-        if (pa.xmask[t] == 0) {
-          re[t] += sgn * (ar * ar + ai * ai);
-        } else {
-          const auto b = psi[i ^ pa.xmask[t]];
-          re[t] += sgn * (ar * (double)b.x + ai * (double)b.y);
-          im[t] += sgn * (ar * (double)b.y - ai * (double)b.x);
-        }
-      }
-    }
-  }
-#pragma unroll
-  for (int t = 0; t < kMaxPauliPerPass; ++t) {
-    if (t < pa.nterms) {
-      const double r0 = block_sum(re[t], sh);
-      const double r1 = block_sum(im[t], sh);
-      if (threadIdx.x == 0) {
-        partials[(uint64_t)(2 * t) * kReduceBlocks + blockIdx.x] = r0;
-        partials[(uint64_t)(2 * t + 1) * kReduceBlocks + blockIdx.x] = r1;
-      }
-    }
   }
 }
 
@@ -574,24 +528,6 @@ void launch_inner(int prec, const void* a, const void* b, uint64_t S, double* pa
     hipLaunchKernelGGL((k_inner<float>), dim3(kReduceBlocks), dim3(kBlock), 0, st, (const float2*)a,
                        (const float2*)b, S, partials);
   hipLaunchKernelGGL(k_final_sum, dim3(2), dim3(kBlock), 0, st, partials, out);
-}
-
-void launch_pauli(int prec, const void* psi, uint64_t S, int nterms, const uint64_t* xmask, const uint64_t* smask,
-                  double* partials, double* out, hipStream_t st)
-{
-  PauliArgs pa{};
-  pa.nterms = nterms;
-  for (int t = 0; t < nterms; ++t) {
-    pa.xmask[t] = xmask[t];
-    pa.smask[t] = smask[t];
-  }
-  if (prec == QSV_C128)
-    hipLaunchKernelGGL((k_pauli<double>), dim3(kReduceBlocks), dim3(kBlock), 0, st, (const double2*)psi, S, pa,
-                       partials);
-  else
-    hipLaunchKernelGGL((k_pauli<float>), dim3(kReduceBlocks), dim3(kBlock), 0, st, (const float2*)psi, S, pa,
-                       partials);
-  hipLaunchKernelGGL(k_final_sum, dim3(2 * nterms), dim3(kBlock), 0, st, partials, out);
 }
 
 void launch_expect1q(int prec, const void* psi, uint64_t S, uint64_t tbit, const double m[8], double* partials,
