@@ -85,6 +85,8 @@ struct qsv_state {
   uint64_t passes_launched = 0;
   int tile_low = -1;            // tile low-run width forced by the tuner (-1: none)
   double* norm_buf = nullptr;   // complex64 FP32 passes: per-tile norms (2 x ntiles) + control (2)
+  uint64_t* shot_dev = nullptr;   // qsv_sample's outcomes (lazy, at most kShotsKept)
+  uint64_t shot_cap = 0;
   uint64_t* samp_dev = nullptr;   // serving: reusable shot buffers (grow only)
   uint64_t* samp_host = nullptr;  // pinned
   uint64_t samp_cap = 0;
@@ -1577,6 +1579,7 @@ int check_state(const qsv_state* s)
 }
 
 constexpr uint64_t kXferChunk = 1ull << 24;  // amplitudes per staged transfer
+constexpr uint64_t kShotsKept = 1ull << 16;  // outcomes of qsv_sample that a state keeps room for
 
 }  // namespace
 
@@ -1708,6 +1711,7 @@ int qsv_state_destroy(qsv_state* s)
   if (s->prefix) hipFree(s->prefix);
   if (s->hist) hipFree(s->hist);
   if (s->norm_buf) hipFree(s->norm_buf);
+  if (s->shot_dev) hipFree(s->shot_dev);
   if (s->samp_dev) hipFree(s->samp_dev);
   if (s->samp_host) hipHostFree(s->samp_host);
   if (s->stream) hipStreamDestroy(s->stream);
@@ -1903,14 +1907,29 @@ int qsv_sample(const qsv_state* cs, uint64_t shots, uint64_t seed, uint64_t* out
     const uint64_t nch = std::max<uint64_t>(1, s->S >> kSampleChunkLog);
     HIPCHK(hipMalloc(&s->prefix, nch * sizeof(double)));
   }
+  // outcomes: up to kShotsKept in a device buffer that the state keeps (a
+  // hipMalloc and the device-wide wait of a hipFree per call otherwise)
   uint64_t* dout = nullptr;
-  if (shots) HIPCHK(hipMalloc(&dout, shots * sizeof(uint64_t)));
+  const bool keep = shots <= kShotsKept;
+  if (keep) {
+    if (shots > s->shot_cap) {
+      if (s->shot_dev) HIPCHK(hipFree(s->shot_dev));
+      s->shot_dev = nullptr;
+      s->shot_cap = 0;
+      const uint64_t cap = std::max<uint64_t>(shots, 1024);
+      HIPCHK(hipMalloc((void**)&s->shot_dev, cap * sizeof(uint64_t)));
+      s->shot_cap = cap;
+    }
+    dout = s->shot_dev;
+  } else {
+    HIPCHK(hipMalloc(&dout, shots * sizeof(uint64_t)));
+  }
   launch_sample(s->prec, s->amps, s->S, s->prefix, shots, seed, dout, s->stream);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess && shots)
     e = hipMemcpyAsync(outcomes, dout, shots * sizeof(uint64_t), hipMemcpyDeviceToHost, s->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
-  if (dout) hipFree(dout);
+  if (!keep) hipFree(dout);
   if (e != hipSuccess) return fail(QSV_E_DEVICE, std::string("sample: ") + hipGetErrorString(e));
   return QSV_OK;
 }

@@ -272,8 +272,10 @@ __global__ __launch_bounds__(kBlock) void k_probs(const typename VT<R>::T* __res
 
 // ---------------------------------------------------------------------------
 // Shot sampling (measure-state, inverse CDF): chunk sums, inclusive scan of
-// chunk sums, then one wave per shot: binary search over chunks and a wave
-// scan inside the chunk.
+// chunk sums, then one wave per shot: a search over chunks and a wave scan
+// inside the chunk. Bound by the one read of the state (chunk sums 350 us for
+// 2 GiB); 1000 shots take 7 to 10 us, a chain of loads per shot (15 to 20 us
+// with binary searches and 64 amplitudes a step).
 // ---------------------------------------------------------------------------
 template <typename R>
 __global__ __launch_bounds__(kBlock) void k_chunk_sums(const typename VT<R>::T* __restrict__ psi, int chunk_log,
@@ -290,14 +292,57 @@ __global__ __launch_bounds__(kBlock) void k_chunk_sums(const typename VT<R>::T* 
   if (threadIdx.x == 0) sums[blockIdx.x] = r;
 }
 
-// Inclusive scan of n doubles with one block of 1024 threads.
-__global__ __launch_bounds__(1024) void k_scan_inclusive(double* __restrict__ v, uint64_t n)
+// The prefix over chunk sums is kept in groups of 1024 chunks: entry c of group
+// g holds the sum of the group's chunks up to c, except the group's last entry,
+// which holds the sum of everything up to it. A state of 2^20 amplitudes or
+// fewer is one group and its entries are the plain inclusive prefix. Groups are
+// scanned by one workgroup each (k_scan_groups), their totals by one more
+// (k_scan_totals); the serial walk of one workgroup over all chunk sums that
+// these replace took 347 us on 27 qubits (2^17 sums), as long as reading the
+// 2 GiB state; they take 5 us each.
+constexpr int kGroupLog = 10;
+
+__device__ __forceinline__ double wave_scan(double v, int lane)
+{
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const double t = __shfl_up(v, off, 64);
+    if (lane >= off) v += t;
+  }
+  return v;
+}
+
+__global__ __launch_bounds__(kBlock) void k_scan_groups(double* __restrict__ v, uint64_t n)
+{
+  __shared__ double tot[kBlock / 64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const uint64_t b = ((uint64_t)blockIdx.x << kGroupLog) + 4 * threadIdx.x;
+  double x[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) x[k] = b + k < n ? v[b + k] : 0.0;
+#pragma unroll
+  for (int k = 1; k < 4; ++k) x[k] += x[k - 1];
+  const double inc = wave_scan(x[3], lane);
+  if (lane == 63) tot[w] = inc;
+  __syncthreads();
+  double off = 0.0;
+  for (int k = 0; k < w; ++k) off += tot[k];
+  const double before = __shfl_up(inc, 1, 64);
+  if (lane) off += before;
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    if (b + k < n) v[b + k] = off + x[k];
+}
+
+// Running totals of the groups, in place at each group's last entry.
+__global__ __launch_bounds__(1024) void k_scan_totals(double* __restrict__ v, uint64_t groups)
 {
   __shared__ double tot[1024];
-  const uint64_t seg = (n + 1023) / 1024;
-  const uint64_t b = threadIdx.x * seg, e = (b + seg < n) ? b + seg : n;
+  auto at = [&](uint64_t g) -> double& { return v[(g << kGroupLog) + (1u << kGroupLog) - 1]; };
+  const uint64_t seg = (groups + 1023) / 1024;
+  const uint64_t b = threadIdx.x * seg, e = (b + seg < groups) ? b + seg : groups;
   double run = 0.0;
-  for (uint64_t k = b; k < e; ++k) { run += v[k]; v[k] = run; }
+  for (uint64_t k = b; k < e; ++k) run += at(k);
   tot[threadIdx.x] = run;
   __syncthreads();
   for (int off = 1; off < 1024; off <<= 1) {
@@ -306,8 +351,11 @@ __global__ __launch_bounds__(1024) void k_scan_inclusive(double* __restrict__ v,
     tot[threadIdx.x] += t;
     __syncthreads();
   }
-  const double offset = threadIdx.x ? tot[threadIdx.x - 1] : 0.0;
-  for (uint64_t k = b; k < e; ++k) v[k] += offset;
+  run = threadIdx.x ? tot[threadIdx.x - 1] : 0.0;
+  for (uint64_t k = b; k < e; ++k) {
+    run += at(k);
+    at(k) = run;
+  }
 }
 
 __device__ __forceinline__ double uniform01(uint64_t seed, uint64_t k)
@@ -319,6 +367,28 @@ __device__ __forceinline__ double uniform01(uint64_t seed, uint64_t k)
   return (double)(z >> 11) * (1.0 / 9007199254740992.0);
 }
 
+// The first k in [0, n) with !(val(k) < r), n if there is none: the wave probes
+// 64 places at a time (a binary search is a chain of 10 to 17 dependent loads).
+template <typename F>
+__device__ __forceinline__ uint64_t wave_search(uint64_t n, double r, int lane, F&& val)
+{
+  uint64_t lo = 0, len = n;
+  while (len) {
+    const uint64_t step = (len + 63) >> 6;
+    const uint64_t first = (uint64_t)lane * step, last = first + step < len ? first + step : len;
+    const uint64_t hit = __ballot(first < len && !(val(lo + last - 1) < r));
+    if (!hit) return n;
+    const uint64_t at = (uint64_t)(__ffsll((unsigned long long)hit) - 1) * step;
+    if (step == 1) return lo + at;
+    lo += at;
+    len = at + step < len ? step : len - at;
+  }
+  return n;
+}
+
+// One wave per shot. The shot's chunk is read in one round of loads, sixteen
+// neighbouring amplitudes a lane, and scanned over the wave once; the lane that
+// holds the outcome walks its own sixteen.
 template <typename R>
 __global__ __launch_bounds__(kBlock) void k_sample(const typename VT<R>::T* __restrict__ psi, uint64_t S,
                                                     int chunk_log, const double* __restrict__ prefix,
@@ -328,42 +398,60 @@ __global__ __launch_bounds__(kBlock) void k_sample(const typename VT<R>::T* __re
   const int lane = threadIdx.x & 63;
   const uint64_t shot = (uint64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
   if (shot >= shots) return;
+  constexpr uint64_t G = 1ull << kGroupLog;
   const double total = prefix[nchunks - 1];
   const double r = uniform01(seed, shot) * total;
-  // first chunk whose inclusive prefix is >= r
-  uint64_t lo = 0, hi = nchunks;
-  while (lo < hi) {
-    const uint64_t mid = (lo + hi) >> 1;
-    if (prefix[mid] < r) lo = mid + 1; else hi = mid;
+  // first chunk whose inclusive prefix is >= r: its group, then the chunk in it
+  uint64_t g = 0;
+  const uint64_t ng = nchunks > G ? nchunks / G : 1;
+  if (ng > 1) g = wave_search(ng, r, lane, [&](uint64_t k) { return prefix[k * G + G - 1]; });
+  const double off = g && g < ng ? prefix[g * G - 1] : 0.0;
+  uint64_t c = nchunks;
+  if (g < ng) {
+    const uint64_t len = nchunks < G ? nchunks : G;
+    c = g * G + wave_search(len, r, lane, [&](uint64_t k) {
+      const double v = prefix[g * G + k];
+      return ng > 1 && k == G - 1 ? v : off + v;
+    });
   }
-  if (lo >= nchunks) {
+  if (c >= nchunks) {
     if (lane == 0) out[shot] = S - 1;
     return;
   }
-  const uint64_t c = lo;
-  double run = c ? prefix[c - 1] : 0.0;
-  const uint64_t len = 1ull << chunk_log, c0 = c << chunk_log;
-  uint64_t result = c0 + len - 1;
-  for (uint64_t piece = 0; piece < len; piece += 64) {
-    double v = 0.0;
-    if (piece + lane < len) {
-      const auto a = psi[c0 + piece + lane];
-      v = (double)a.x * a.x + (double)a.y * a.y;
-    }
+  const double run = (c & (G - 1)) ? off + prefix[c - 1] : off;
+  const uint32_t len = 1u << chunk_log, per = len < 64 ? 1u : len >> 6;
+  const uint64_t c0 = c << chunk_log;
+  double v[1 << (kSampleChunkLog - 6)], sum = 0.0;
 #pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const double t = __shfl_up(v, off, 64);
-      if (lane >= off) v += t;
+  for (uint32_t j = 0; j < (1u << (kSampleChunkLog - 6)); ++j) {
+    v[j] = 0.0;
+    if (j < per && lane * per + j < len) {
+      const auto a = psi[c0 + lane * per + j];
+      v[j] = (double)a.x * a.x + (double)a.y * a.y;
     }
-    const double cum = run + v;
-    const uint64_t hit = __ballot(cum >= r && piece + lane < len);
-    if (hit) {
-      result = c0 + piece + (uint64_t)(__ffsll((unsigned long long)hit) - 1);
-      break;
-    }
-    run += __shfl(v, 63, 64);
   }
-  if (lane == 0) out[shot] = result;
+#pragma unroll
+  for (uint32_t j = 0; j < (1u << (kSampleChunkLog - 6)); ++j) sum += v[j];
+  const double inc = wave_scan(sum, lane);
+  double cum = __shfl_up(inc, 1, 64);
+  cum = run + (lane ? cum : 0.0);
+  const uint64_t hit = __ballot(run + inc >= r && lane * per < len);
+  if (!hit) {
+    if (lane == 0) out[shot] = c0 + len - 1;
+    return;
+  }
+  if (lane != __ffsll((unsigned long long)hit) - 1) return;
+  uint32_t pick = per - 1;
+  bool found = false;
+#pragma unroll
+  for (uint32_t j = 0; j < (1u << (kSampleChunkLog - 6)); ++j) {
+    cum += v[j];
+    if (!found && j < per && cum >= r) {
+      pick = j;
+      found = true;
+    }
+  }
+  out[shot] = c0 + lane * per + pick;
 }
 
 // ---------------------------------------------------------------------------
@@ -566,7 +654,9 @@ void launch_sample(int prec, const void* psi, uint64_t S, double* chunk_prefix, 
   else
     hipLaunchKernelGGL((k_chunk_sums<float>), dim3((unsigned)nchunks), dim3(kBlock), 0, st, (const float2*)psi,
                        chunk_log, chunk_prefix);
-  hipLaunchKernelGGL(k_scan_inclusive, dim3(1), dim3(1024), 0, st, chunk_prefix, nchunks);
+  const uint64_t groups = (nchunks + (1ull << kGroupLog) - 1) >> kGroupLog;
+  hipLaunchKernelGGL(k_scan_groups, dim3((unsigned)groups), dim3(kBlock), 0, st, chunk_prefix, nchunks);
+  if (groups > 1) hipLaunchKernelGGL(k_scan_totals, dim3(1), dim3(1024), 0, st, chunk_prefix, groups);
   if (shots == 0) return;
   const unsigned g = (unsigned)((shots + (kBlock / 64) - 1) / (kBlock / 64));
   if (prec == QSV_C128)
