@@ -73,9 +73,9 @@ struct qsv_state {
   qsv_kernel_stat stats[QSV_KCLASS_COUNT] = {};
   // fused-pass descriptor ring (pinned host staging + device copy per slot)
   struct PassSlot {
-    qsv::PProg* host = nullptr;
-    qsv::PProg* dev = nullptr;
-    size_t cap = 0;
+    char* host = nullptr;
+    char* dev = nullptr;
+    size_t cap = 0;   // bytes
     hipEvent_t event = nullptr;
   };
   static constexpr int kRing = 4;
@@ -572,340 +572,59 @@ int run_direct(qsv_state* s, const BGate& g)
 // Pass descriptors travel through a small ring of pinned host + device
 // buffers; a slot is reused only after the event recorded behind its last
 // pass has completed.
-// ---- compiling a planned pass into the micro-op program of k_pass ---------
-// Local bit b's rank among the set bits of mask (b must be in mask).
-inline uint32_t rank_in(uint32_t mask, int b) { return __builtin_popcount(mask & ((1u << b) - 1u)); }
-
-// The two tile bits that thread-id bits 6 and 7 (the wave index) map to in
-// layout reg: the two highest bits outside the register mask.
-inline uint32_t wave_bits(uint32_t reg)
-{
-  uint32_t nonreg = ((1u << kPassTileBits) - 1u) & ~reg;
-  uint32_t out = 0;
-  for (int k = 0; k < 2; ++k) {
-    const uint32_t top = 1u << (31 - __builtin_clz(nonreg));
-    out |= top;
-    nonreg &= ~top;
-  }
-  return out;
-}
-
-// Resolve every gate of p against the register layout it runs in: register
-// bits become slot indices, thread bits thread-id bits (thread t holds local
-// bits pdep(t, ~reg)). Returns the byte length of the program.
-// The kernel's LDS swizzle of a tile-local index (k_pass): XOR-linear.
-inline uint32_t pass_swz(uint32_t l) { return l ^ (((l >> 4) ^ (l >> 8)) & 15u); }
-
-// Offsets of layout `reg` for the kernel: LDS bytes of 8-byte elements and
-// global index bits (pos: global bit of each tile-local bit).
-void make_layout(uint32_t reg, const int32_t pos[16], PLayout& L)
-{
-  constexpr uint32_t FULL = (1u << kPassTileBits) - 1u;
-  std::memset(&L, 0, sizeof(L));
-  int j = 0;
-  for (int b = 0; b < kPassTileBits; ++b)
-    if (((FULL & ~reg) >> b) & 1u) {
-      L.lt[j] = pass_swz(1u << b) * 8u;
-      L.gt[j] = 1ull << pos[b];
-      ++j;
-    }
-  int rb[4], nr = 0;
-  for (int b = 0; b < kPassTileBits; ++b)
-    if ((reg >> b) & 1u) rb[nr++] = b;
-  for (int k = 0; k < 16; ++k) {
-    uint32_t l = 0;
-    uint64_t g = 0;
-    for (int i = 0; i < 4; ++i)
-      if ((k >> i) & 1) {
-        l |= 1u << rb[i];
-        g |= 1ull << pos[rb[i]];
-      }
-    L.ls[k] = pass_swz(l) * 8u;
-    L.gs[k] = g;
-  }
-}
-
-// A PO_BLOCK costs a wave 48 v_mfma_f32_16x16x4f32 (three real 16 x 16 x 16
-// products per column block of 16 lanes: 0.66 ms per 2^30 amplitudes at the
-// FP32 matrix peak) plus an LDS round trip, whatever it absorbs, so it pays
-// only for long runs of expensive ops. Vector instructions per wave of each
-// register-bit op in an FP32 pass (dense real, dense general and two-sided
-// diagonal measured with one op kind per pass; the exchange and the one-sided
-// diagonal estimated), and the least total a block must replace
-// (QSV_PASS_BLOCKS; 0 keeps every op on the vector units). On complex64
-// 30-qubit passes a threshold of 650 ran U3/CZ layers 3.7 % and random
-// layers 0.8 % faster than the vector units alone; 450 broke even, and 300
-// (blocks of about three ops) ran 6-14 % slower.
-int reg_op_cost(const POp& op)
-{
-  const int c = op.code;
-  if (c < PO_PHASE) {
-    const int dm = c & 3;
-    return dm == PM_GENERAL ? 147 : dm == PM_EXCHANGE ? 40 : 83;
-  }
-  if (c < PO_PHASE_T) return ((c - PO_PHASE) & 4) ? 60 : 101;
-  return 101;   // PO_BLOCKADE
-}
-
 int pass_block_cost()
 {
-  const char* e = std::getenv("QSV_PASS_BLOCKS");   // read per pass: a test may lower it
+  const char* e = std::getenv("QSV_PASS_BLOCKS");   // read per launch: a test may lower it
   return e ? std::max(0, std::atoi(e)) : 650;
 }
 
-// Slot bits an op of a stage reads or writes; `reg_only`: it has no
-// thread-bit part, so it is the same 16 x 16 map on every thread's slots.
-uint32_t op_slot_bits(const POp& op, bool* reg_only)
-{
-  const int c = op.code;
-  if (c < PO_PHASE) {
-    *reg_only = op.tmask == 0;
-    return (1u << (c >> 2)) | op.kc;
-  }
-  if (c < PO_PHASE_T) {
-    *reg_only = op.tmask == 0;
-    return (1u << ((c - PO_PHASE) & 3)) | op.kc;
-  }
-  *reg_only = c == PO_BLOCKADE && op.aux == 0;
-  return op.kc;   // PO_PHASE_T, PO_BLOCKADE
-}
-
-// v = (map of a register-bit op) v on one thread's 16 slots, as k_pass applies it.
-void apply_reg_op(const POp& op, std::complex<double> v[16])
-{
-  using C = std::complex<double>;
-  const int c = op.code;
-  const uint32_t kc = op.kc;
-  if (c < PO_PHASE) {
-    const int d = 1 << (c >> 2);
-    const C m00(op.m[0], op.m[1]), m01(op.m[2], op.m[3]), m10(op.m[4], op.m[5]), m11(op.m[6], op.m[7]);
-    for (int k = 0; k < 16; ++k) {
-      if ((k & d) || (k & kc) != kc) continue;
-      const C a = v[k], b = v[k | d];
-      v[k] = m00 * a + m01 * b;
-      v[k | d] = m10 * a + m11 * b;
-    }
-  } else if (c < PO_PHASE_T) {
-    const int d = 1 << ((c - PO_PHASE) & 3);
-    const bool only1 = ((c - PO_PHASE) & 4) != 0;
-    const C d0(op.m[0], op.m[1]), d1(op.m[6], op.m[7]);
-    for (int k = 0; k < 16; ++k) {
-      if ((k & kc) != kc) continue;
-      if (k & d) v[k] *= d1;
-      else if (!only1) v[k] *= d0;
-    }
-  } else {   // PO_BLOCKADE without a thread part
-    const C ph(op.m[0], op.m[1]);
-    for (int k = 0; k < 16; ++k)
-      if (__builtin_popcount((uint32_t)k & kc) == 1) v[k] *= ph;
-  }
-}
-
-// Fold the register-bit ops of one stage (ops [n0, n) of `out`) into dense
-// 16 x 16 blocks for the matrix cores. Scanning in order, an op without a
-// thread-bit part joins the open block if its slot bits miss those of every
-// op set aside since the block opened; an op with a thread-bit part is set
-// aside and runs after the block (ops on disjoint bits commute). A block
-// whose ops cost the vector units less than min_cost keeps its ops in
-// program order. Returns the new op count.
-int form_blocks(PProg& out, int n0, int n, int& nblk, int min_cost)
-{
-  const std::vector<POp> src(out.ops + n0, out.ops + n);
-  std::vector<int> blk, aside;
-  uint32_t aside_bits = 0;
-  int w = n0, cost = 0;
-  auto flush = [&]() {
-    if (cost >= min_cost && nblk < kMaxPassBlocks) {
-      std::complex<double> U[16][16];
-      for (int col = 0; col < 16; ++col) {
-        std::complex<double> v[16];
-        for (int k = 0; k < 16; ++k) v[k] = k == col ? 1.0 : 0.0;
-        for (int i : blk) apply_reg_op(src[i], v);
-        for (int k = 0; k < 16; ++k) U[k][col] = v[k];
-      }
-      float* tab = out.blk[nblk];
-      for (int kk = 0; kk < 4; ++kk)
-        for (int l = 0; l < 64; ++l) {
-          const std::complex<double> u = U[l & 15][4 * kk + (l >> 4)];
-          tab[2 * (kk * 64 + l)] = (float)u.real();
-          tab[2 * (kk * 64 + l) + 1] = (float)u.imag();
-        }
-      POp& b = out.ops[w++];
-      std::memset(&b, 0, sizeof(b));
-      b.code = PO_BLOCK;
-      b.aux = (uint32_t)(offsetof(PProg, blk) + (size_t)nblk * sizeof(out.blk[0]));
-      ++nblk;
-      for (int i : aside) out.ops[w++] = src[i];
-    } else {
-      std::vector<int> all(blk);
-      all.insert(all.end(), aside.begin(), aside.end());
-      std::sort(all.begin(), all.end());
-      for (int i : all) out.ops[w++] = src[i];
-    }
-    blk.clear();
-    aside.clear();
-    aside_bits = 0;
-    cost = 0;
-  };
-  for (int i = 0; i < (int)src.size(); ++i) {
-    const POp& op = src[i];
-    if (op.code == PO_SWAP || op.code == PO_RELAYOUT) {
-      flush();
-      out.ops[w++] = op;
-      continue;
-    }
-    bool reg_only = false;
-    const uint32_t sb = op_slot_bits(op, &reg_only);
-    if (reg_only) {
-      if (sb & aside_bits) flush();
-      blk.push_back(i);
-      cost += reg_op_cost(op);
-    } else {
-      aside.push_back(i);
-      aside_bits |= sb;
-    }
-  }
-  flush();
-  return w;
-}
-
-size_t compile_pass(const FPass& p, PProg& out, bool blocks)
-{
-  constexpr uint32_t FULL = (1u << kPassTileBits) - 1u;
-  std::memset(&out.h, 0, sizeof(out.h));
-  out.h.renorm = p.renorm;
-  out.h.load_mask = p.load_mask;
-  out.h.store_mask = p.store_mask;
-  std::memcpy(out.h.sorted_pos, p.sorted_pos, sizeof(out.h.sorted_pos));
-  int nl = 0;
-  make_layout(p.load_mask, p.pos, out.lay[nl]);
-  out.h.load_lay = nl++;
-  int cur = out.h.load_lay;
-  int n = 0, nblk = 0;
-  const int block_cost = blocks ? pass_block_cost() : 0;
-  uint32_t reg = p.load_mask;
-  auto emit = [&]() -> POp& {
-    POp& op = out.ops[n++];
-    std::memset(&op, 0, sizeof(op));
-    return op;
-  };
-  for (int s = 0; s < p.nstages; ++s) {
-    const FStage& st = p.stages[s];
-    if (st.regmask != reg) {
-      make_layout(st.regmask, p.pos, out.lay[nl]);
-      POp& op = emit();
-      op.code = PO_RELAYOUT;
-      op.tmask = (uint32_t)cur;
-      op.kc = (uint32_t)nl;
-      op.aux = st.regmask;
-      op.only1 = wave_bits(reg) == wave_bits(st.regmask) ? 1 : 0;
-      reg = st.regmask;
-      cur = nl++;
-    }
-    const uint32_t nonreg = FULL & ~reg;
-    auto slot_mask = [&](uint32_t local) {
-      uint32_t m = 0;
-      for (int b = 0; b < kPassTileBits; ++b)
-        if (((local & reg) >> b) & 1u) m |= 1u << rank_in(reg, b);
-      return m;
-    };
-    auto tid_mask = [&](uint32_t local) {
-      uint32_t m = 0;
-      for (int b = 0; b < kPassTileBits; ++b)
-        if (((local & nonreg) >> b) & 1u) m |= 1u << rank_in(nonreg, b);
-      return m;
-    };
-    const int n0 = n;
-    for (int gi = st.g0; gi < st.g1; ++gi) {
-      const FGate& g = p.gates[gi];
-      POp& op = emit();
-      std::memcpy(op.m, g.m, sizeof(op.m));
-      for (int k = 0; k < 8; ++k) op.f[k] = (float)g.m[k];
-      switch (g.kind) {
-      case FG_DENSE:
-        op.code = PO_DENSE + 4 * (int)rank_in(reg, g.a) + g.sub;
-        op.kc = slot_mask(g.cmask);
-        op.tmask = tid_mask(g.cmask);
-        break;
-      case FG_PHASE:
-        if ((reg >> g.a) & 1u) {
-          op.code = PO_PHASE + 4 * (g.sub ? 1 : 0) + (int)rank_in(reg, g.a);
-        } else {
-          op.code = PO_PHASE_T;
-          op.aux = 1u << rank_in(nonreg, g.a);
-          op.only1 = g.sub ? 1 : 0;
-        }
-        op.kc = slot_mask(g.cmask);
-        op.tmask = tid_mask(g.cmask);
-        break;
-      case FG_BLOCKADE:
-        op.code = PO_BLOCKADE;
-        op.kc = slot_mask(g.bmask);
-        op.aux = tid_mask(g.bmask);
-        break;
-      default:   // FG_SWAP: local bits and local controls
-        op.code = PO_SWAP;
-        op.kc = (uint32_t)g.a;
-        op.aux = (uint32_t)g.b;
-        op.tmask = g.cmask;
-        break;
-      }
-    }
-    if (block_cost > 0) n = form_blocks(out, n0, n, nblk, block_cost);
-  }
-  out.h.nops = n;
-  if (reg == p.store_mask) {
-    out.h.store_lay = cur;
-  } else {
-    make_layout(p.store_mask, p.pos, out.lay[nl]);
-    out.h.store_lay = nl++;
-    out.h.store_local = wave_bits(reg) == wave_bits(p.store_mask) ? 1 : 0;
-  }
-  out.h.nlay = nl;
-  out.h.lay_off = (int32_t)offsetof(PProg, lay);
-  return offsetof(PProg, ops) + (size_t)n * sizeof(POp);
-}
-
-int upload_passes(qsv_state* s, const std::vector<FPass>& passes, bool blocks, PProg** dev)
+int upload_passes(qsv_state* s, const std::vector<char>& progs, const char** dev)
 {
   auto& slot = s->ring[s->ring_next];
   s->ring_next = (s->ring_next + 1) % qsv_state::kRing;
   if (slot.event) HIPCHK(hipEventSynchronize(slot.event));
-  const size_t need = passes.size();
+  const size_t need = progs.size();
   if (slot.cap < need) {
     if (slot.host) HIPCHK(hipHostFree(slot.host));
     if (slot.dev) HIPCHK(hipFree(slot.dev));
     slot.host = nullptr;
     slot.dev = nullptr;
-    const size_t cap = std::max<size_t>(need, 64);
-    HIPCHK(hipHostMalloc((void**)&slot.host, cap * sizeof(PProg), hipHostMallocDefault));
-    HIPCHK(hipMalloc((void**)&slot.dev, cap * sizeof(PProg)));
+    slot.cap = 0;
+    const size_t cap = std::max<size_t>(need + need / 2, 256 << 10);
+    HIPCHK(hipHostMalloc((void**)&slot.host, cap, hipHostMallocDefault));
+    HIPCHK(hipMalloc((void**)&slot.dev, cap));
     slot.cap = cap;
   }
   if (!slot.event) HIPCHK(hipEventCreateWithFlags(&slot.event, hipEventDisableTiming));
-  for (size_t i = 0; i < need; ++i) compile_pass(passes[i], slot.host[i], blocks);
-  HIPCHK(hipMemcpyAsync(slot.dev, slot.host, need * sizeof(PProg), hipMemcpyHostToDevice, s->stream));
+  std::memcpy(slot.host, progs.data(), need);
+  HIPCHK(hipMemcpyAsync(slot.dev, slot.host, need, hipMemcpyHostToDevice, s->stream));
   *dev = slot.dev;
   s->ring_pending = &slot;
   return QSV_OK;
 }
 
-// blocks: FP32 passes fold register-bit runs into PO_BLOCK ops
+// blocks: FP32 passes fold register-bit runs into PO_BLOCK ops. The factors
+// common to the whole state are applied by the last of the passes.
 int launch_passes(qsv_state* s, std::vector<FPass>& passes, bool f32, bool blocks)
 {
   if (passes.empty()) return QSV_OK;
-  const int TB = s->prec == QSV_C128 ? kTileBitsC128 : kTileBitsC64;
-  const uint64_t ntiles = s->S >> TB;
+  const uint64_t ntiles = s->S >> kPassTileBits;
   TileNorm nb{nullptr, nullptr, nullptr};
   if (f32) {
     if (!s->norm_buf) HIPCHK(hipMalloc((void**)&s->norm_buf, (2 * ntiles + 2) * sizeof(double)));
     nb = TileNorm{s->norm_buf, s->norm_buf + ntiles, s->norm_buf + 2 * ntiles};
   }
-  PProg* dev = nullptr;
-  int rc = upload_passes(s, passes, f32 && blocks, &dev);
+  const int block_cost = f32 && blocks ? pass_block_cost() : 0;
+  std::vector<char> progs;
+  std::vector<size_t> at(passes.size());
+  std::complex<double> scalar(1.0, 0.0);
+  for (size_t i = 0; i < passes.size(); ++i)
+    at[i] = compile_pass(passes[i], f32, block_cost, scalar, i + 1 == passes.size(), progs);
+  const char* dev = nullptr;
+  int rc = upload_passes(s, progs, &dev);
   if (rc) return rc;
   for (size_t i = 0; i < passes.size(); ++i) {
-    const PProg* p = dev + i;
+    const char* p = dev + at[i];
     rc = timed(s, QSV_KCLASS_BLOCK, 2.0 * s->S * s->bytes_per_amp(),
                [&] { launch_pass(s->prec, f32, s->amps, p, ntiles, nb, s->stream); });
     if (rc) return rc;
@@ -935,7 +654,7 @@ int tile_low_bits(const qsv_state* s)
     const char* v = std::getenv("QSV_TILE_LOWBITS");
     return v ? std::atoi(v) : -1;
   }();
-  const int TB = s->prec == QSV_C128 ? kTileBitsC128 : kTileBitsC64;
+  const int TB = kPassTileBits;
   const int tuned = g_tuned_low[s->prec == QSV_C128 ? 0 : 1].load();
   int L = s->tile_low >= 0 ? s->tile_low : env >= 0 ? env : tuned >= 0 ? tuned : 4;
   return std::max(low_bit_threshold(s), std::min(L, TB - 2));
@@ -951,16 +670,29 @@ int dense_structure(const double m[8])
   return DM_GENERAL;
 }
 
-// Build one pass from the chosen gates (program order) and the tile bit set.
-// Returns the number of chosen gates the pass holds (a suffix may be cut to
-// respect the stage limit).
-size_t build_pass(const qsv_state* s, const std::vector<BGate>& gs, const std::vector<size_t>& chosen,
-                  uint64_t set, FPass& p)
+// A gate on tile-local bits (loc: local bit of each global bit).
+FGate local_gate(const BGate& g, const int loc[64])
 {
-  const int TB = s->prec == QSV_C128 ? kTileBitsC128 : kTileBitsC64;
-  const int RB = 4;   // register bits per thread in the tile kernel
-  const int L = tile_low_bits(s);
-  std::memset(&p, 0, sizeof(p));
+  FGate fg{};
+  fg.kind = g.kind;
+  fg.a = g.a >= 0 ? loc[g.a] : -1;
+  fg.b = g.b >= 0 ? loc[g.b] : -1;
+  for (int c : g.cbits) fg.cmask |= 1u << loc[c];
+  if (g.kind == FG_BLOCKADE)
+    for (uint64_t m = g.bmask; m; m &= m - 1) fg.bmask |= 1u << loc[__builtin_ctzll(m)];
+  fg.sub = g.kind == FG_DENSE ? dense_structure(g.m) : (g.phase_only ? 1 : 0);
+  std::memcpy(fg.m, g.m, sizeof(fg.m));
+  return fg;
+}
+
+// Build one pass from the chosen gates (program order) and the tile bit set.
+void build_pass(const qsv_state* s, const std::vector<BGate>& gs, const std::vector<size_t>& chosen, uint64_t set,
+                FPass& p)
+{
+  const int TB = kPassTileBits;
+  const int L = std::min(tile_low_bits(s), TB - 4);
+  p.tb = TB;
+  p.low = L;
   uint64_t tile = set;
   for (int b = 0; __builtin_popcountll(tile) < TB; ++b) tile |= 1ull << b;
   // Local bit order: the low run first (coalesced lanes), then the other tile
@@ -971,7 +703,7 @@ size_t build_pass(const qsv_state* s, const std::vector<BGate>& gs, const std::v
   int ntarget[64] = {};
   for (size_t i = 0; i < chosen.size(); ++i) {
     const BGate& g = gs[chosen[i]];
-    if (g.kind == FG_DENSE && g.a >= 0) ntarget[g.a]++;
+    if (g.kind == FG_DENSE && g.a >= 0 && !(g.cbits.size() == 1 && dense_structure(g.m) == DM_EXCHANGE)) ntarget[g.a]++;
   }
   int w1 = -1, w2 = -1;   // the two least-targeted non-low tile bits
   for (int b = s->n - 1; b >= L; --b) {
@@ -990,55 +722,8 @@ size_t build_pass(const qsv_state* s, const std::vector<BGate>& gs, const std::v
   int ns = 0;
   for (int b = 0; b < s->n; ++b)
     if ((tile >> b) & 1ull) p.sorted_pos[ns++] = b;
-  const uint32_t lowmask = (1u << L) - 1u;
-  uint32_t cur = 0;
-  int g0 = 0, nst = 0;
-  size_t taken = 0;
-  for (size_t i = 0; i < chosen.size(); ++i) {
-    const BGate& g = gs[chosen[i]];
-    FGate fg{};
-    fg.kind = g.kind;
-    fg.a = g.a >= 0 ? loc[g.a] : -1;
-    fg.b = g.b >= 0 ? loc[g.b] : -1;
-    for (int c : g.cbits) fg.cmask |= 1u << loc[c];
-    if (g.kind == FG_BLOCKADE)
-      for (int b = 0; b < s->n; ++b)
-        if ((g.bmask >> b) & 1ull) fg.bmask |= 1u << loc[b];
-    fg.sub = g.kind == FG_DENSE ? dense_structure(g.m) : (g.phase_only ? 1 : 0);
-    std::memcpy(fg.m, g.m, sizeof(fg.m));
-    // only dense targets must be register bits (swaps go through LDS)
-    const uint32_t need = (g.kind == FG_DENSE) ? (1u << fg.a) : 0u;
-    if (__builtin_popcount(cur | need) > RB) {
-      if (nst == kMaxPassStages - 1) break;   // stage limit: cut the pass here
-      p.stages[nst++] = FStage{cur, g0, (int32_t)i};
-      cur = need;
-      g0 = (int)i;
-    } else {
-      cur |= need;
-    }
-    p.gates[i] = fg;
-    taken = i + 1;
-  }
-  p.stages[nst++] = FStage{cur, g0, (int32_t)taken};
-  p.nstages = nst;
-  p.ngates = (int)taken;
-  // fill every register mask to RB bits: non-low bits below the wave pair
-  // (highest first, so consecutive stages tend to share them), then the wave
-  // pair, then low bits
-  for (int k = 0; k < nst; ++k) {
-    uint32_t r = p.stages[k].regmask;
-    for (int b = TB - 3; b >= L && __builtin_popcount(r) < RB; --b) r |= 1u << b;
-    for (int b = TB - 1; b >= TB - 2 && __builtin_popcount(r) < RB; --b) r |= 1u << b;
-    for (int b = 0; b < TB && __builtin_popcount(r) < RB; ++b) r |= 1u << b;
-    p.stages[k].regmask = r;
-  }
-  // load/store layout when a stage's own would split the low run: registers
-  // just below the wave pair, so the lanes cover the low run
-  const uint32_t natural = (L <= TB - 2 - RB) ? (((1u << RB) - 1u) << (TB - 2 - RB))
-                                              : (((1u << TB) - 1u) & ~((1u << (TB - RB)) - 1u));
-  p.load_mask = (p.stages[0].regmask & lowmask) ? natural : p.stages[0].regmask;
-  p.store_mask = (p.stages[nst - 1].regmask & lowmask) ? natural : p.stages[nst - 1].regmask;
-  return taken;
+  p.gates.resize(chosen.size());
+  for (size_t i = 0; i < chosen.size(); ++i) p.gates[i] = local_gate(gs[chosen[i]], loc);
 }
 
 // The last pass of a run of passes needs no scale for a successor.
@@ -1063,10 +748,11 @@ template <class Emit, class Barrier>
 int fuse_walk(const qsv_state* s, const std::vector<BGate>& gs, bool f32, Emit&& emit, Barrier&& barrier,
               PassShape* record = nullptr)
 {
-  const int TB = s->prec == QSV_C128 ? kTileBitsC128 : kTileBitsC64;
+  const int TB = kPassTileBits;
   const int L = tile_low_bits(s);
   const uint64_t lowmask = (1ull << L) - 1ull;
   const uint64_t all = (s->n >= 64) ? ~0ull : ((1ull << s->n) - 1ull);
+  const int max_gates = f32 ? kMaxPassGatesF32 : kMaxPassGates;
   const size_t N = gs.size();
   std::vector<char> done(N, 0);
   std::vector<uint64_t> gbits(N);
@@ -1082,7 +768,7 @@ int fuse_walk(const qsv_state* s, const std::vector<BGate>& gs, bool f32, Emit&&
     int cnt = 0;
     for (const uint64_t gb : wbits) {
       if (!(gb & blocked) && !(gb & ~set)) {
-        if (++cnt >= kMaxPassGates) break;
+        if (++cnt >= max_gates) break;
       } else {
         blocked |= gb;
         if ((blocked & all) == all) break;
@@ -1147,7 +833,7 @@ int fuse_walk(const qsv_state* s, const std::vector<BGate>& gs, bool f32, Emit&&
       const uint64_t gb = gbits[i];
       if (!(gb & blocked)) {
         const uint64_t nu = set | gb;
-        if (__builtin_popcountll(nu) <= TB && chosen.size() < (size_t)kMaxPassGates) {
+        if (__builtin_popcountll(nu) <= TB && chosen.size() < (size_t)max_gates) {
           set = nu;
           chosen.push_back(i);
           continue;
@@ -1157,12 +843,12 @@ int fuse_walk(const qsv_state* s, const std::vector<BGate>& gs, bool f32, Emit&&
       if ((blocked & all) == all) break;
     }
     FPass p;
-    const size_t taken = build_pass(s, gs, chosen, set, p);
-    for (size_t i = 0; i < taken; ++i) done[chosen[i]] = 1;
-    if (record) record->emplace_back(std::vector<uint32_t>(chosen.begin(), chosen.begin() + taken), set);
+    build_pass(s, gs, chosen, set, p);
+    for (size_t i : chosen) done[i] = 1;
+    if (record) record->emplace_back(std::vector<uint32_t>(chosen.begin(), chosen.end()), set);
     p.renorm = f32 ? (FP_RENORM_OUT | (run_first ? FP_RENORM_IN : FP_RENORM_APPLY)) : 0;
     run_first = false;
-    if ((rc = emit(p))) return rc;
+    if ((rc = emit(std::move(p)))) return rc;
   }
   return QSV_OK;
 }
@@ -1320,7 +1006,7 @@ std::vector<BGate> fold_gates(const std::vector<BGate>& in)
 int run_fused(qsv_state* s, const std::vector<BGate>& gs_in, uint32_t flags)
 {
   const std::vector<BGate> gs = fold_gates(gs_in);
-  const int TB = s->prec == QSV_C128 ? kTileBitsC128 : kTileBitsC64;
+  const int TB = kPassTileBits;
   if (s->n < TB) {
     for (const auto& g : gs) {
       int rc = run_direct(s, g);
@@ -1333,8 +1019,8 @@ int run_fused(qsv_state* s, const std::vector<BGate>& gs_in, uint32_t flags)
   std::vector<FPass> passes;
   int rc = fuse_walk(
       s, gs, f32,
-      [&](const FPass& p) {
-        passes.push_back(p);
+      [&](FPass&& p) {
+        passes.push_back(std::move(p));
         return passes.size() >= 512 ? launch_passes(s, passes, f32, blocks) : QSV_OK;
       },
       [&](size_t i) {
@@ -1506,22 +1192,7 @@ bool plan_group_passes(int n, int prec, const std::vector<BGate>& gs, std::vecto
   view.n = n;
   view.prec = prec;
   view.S = 1ull << n;
-  PProg prog;
-  auto append = [&](const FPass& p) {
-    // header and ops, then the layout table right after the last op; the
-    // instance's first pass writes |0..0> itself
-    const size_t ops_end = compile_pass(p, prog, false);
-    if (offsets.empty()) prog.h.renorm |= FP_INIT_ZERO;
-    const size_t lay_bytes = (size_t)prog.h.nlay * sizeof(PLayout);
-    const size_t lay_at = (ops_end + 15) & ~(size_t)15;
-    prog.h.lay_off = (int32_t)lay_at;
-    const size_t len = (lay_at + lay_bytes + 255) & ~(size_t)255;
-    const size_t off = bytes.size();
-    bytes.resize(off + len, 0);
-    std::memcpy(bytes.data() + off, &prog, ops_end);
-    std::memcpy(bytes.data() + off + lay_at, prog.lay, lay_bytes);
-    offsets.push_back((int64_t)off);
-  };
+  std::vector<FPass> passes;
   std::vector<uint64_t> key = structure_key(n, prec, tile_low_bits(&view), gs);
   const uint64_t h = key_hash(key);
   PassShape shape;
@@ -1541,25 +1212,24 @@ bool plan_group_passes(int n, int prec, const std::vector<BGate>& gs, std::vecto
     std::vector<size_t> chosen;
     for (const auto& ps : shape) {
       chosen.assign(ps.first.begin(), ps.first.end());
-      FPass p;
-      if (build_pass(&view, gs, chosen, ps.second, p) != chosen.size()) return false;   // cannot happen: same structure
-      append(p);
+      passes.emplace_back();
+      build_pass(&view, gs, chosen, ps.second, passes.back());
     }
-    return true;
   }
   bool ok = true;
-  fuse_walk(
-      &view, gs, false,
-      [&](const FPass& p) {
-        append(p);
-        return QSV_OK;
-      },
-      [&](size_t) {
-        ok = false;
-        return QSV_E_UNSUPPORTED;
-      },
-      &shape);
-  if (ok) {
+  if (!hit)
+    fuse_walk(
+        &view, gs, false,
+        [&](FPass&& p) {
+          passes.push_back(std::move(p));
+          return QSV_OK;
+        },
+        [&](size_t) {
+          ok = false;
+          return QSV_E_UNSUPPORTED;
+        },
+        &shape);
+  if (!hit && ok) {
     std::lock_guard<std::mutex> lk(g_shape_mu);
     if (g_shape_count >= kMaxShapes) {
       g_shapes.clear();
@@ -1567,6 +1237,12 @@ bool plan_group_passes(int n, int prec, const std::vector<BGate>& gs, std::vecto
     }
     g_shapes[h].push_back(ShapeEntry{std::move(key), std::move(shape)});
     ++g_shape_count;
+  }
+  // the instance's first pass writes |0..0> itself
+  std::complex<double> scalar(1.0, 0.0);
+  for (size_t i = 0; ok && i < passes.size(); ++i) {
+    if (i == 0) passes[i].renorm |= FP_INIT_ZERO;
+    offsets.push_back((int64_t)compile_pass(passes[i], false, 0, scalar, i + 1 == passes.size(), bytes));
   }
   return ok;
 }
@@ -3484,7 +3160,7 @@ int qsv_tune_fused(int precision, int num_qubits, qsv_tune_result* out)
   }
   // each candidate's time: the device time of its kernels (per-launch events),
   // not the host's fusion and compilation before them
-  const int TB = precision == QSV_C128 ? kTileBitsC128 : kTileBitsC64;
+  const int TB = kPassTileBits;
   const int lo = low_bit_threshold(s), hi = std::min(TB - 4, lo + QSV_TUNE_MAX - 1);
   double best = 1e300;
   int bestL = 4;

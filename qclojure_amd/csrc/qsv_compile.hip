@@ -1,0 +1,671 @@
+// qsv_compile.hip — fused passes compiled into the micro-op programs of k_pass
+// (host code).
+//
+// Only dense 2x2s need their target among the four register bits of the layout
+// they run in. The rest costs little or nothing:
+//   * CNOTs and swaps permute the tile's indices linearly over GF(2), and so
+//     does a layout: they are applied to the columns of the current layout and
+//     take effect in the addresses of the next round trip through LDS (or of
+//     the store). On 30-qubit random layers they were 40 % of a pass's ops, 105
+//     vector instructions each on complex128.
+//   * Diagonal gates become factors of the amplitudes whose bits are all set,
+//     kept with their bit mask and multiplied together until a dense gate, a
+//     CNOT target or the end of the pass needs them applied: thread bits cost
+//     one complex product per lane and factor, not one per amplitude. Factors
+//     common to the whole state are collected over a run of passes.
+//   * A unitary 2x2 without structure is diag * real * diag in FP64 passes.
+// Gates are taken from per-bit queues: everything that can run in the current
+// layout runs, then the next layout takes the register bits of the dense gates
+// that wait.
+#include <algorithm>
+#include <cmath>
+#include <cstring>
+
+#include "qsv_internal.h"
+
+namespace qsv {
+
+namespace {
+
+using C = std::complex<double>;
+
+inline uint32_t pass_swz(uint32_t l) { return l ^ (((l >> 4) ^ (l >> 8)) & 15u); }
+
+// A PO_BLOCK costs a wave 48 v_mfma_f32_16x16x4f32 (three real 16 x 16 x 16
+// products per column block of 16 lanes: 0.66 ms per 2^30 amplitudes at the
+// FP32 matrix peak) plus an LDS round trip, whatever it absorbs, so it pays
+// only for long runs of expensive ops: vector instructions per wave of each
+// register-bit op in an FP32 pass.
+int reg_op_cost(const POp& op)
+{
+  if (op.code < PO_DENSE_K) {
+    const int dm = op.code & 3;
+    return dm == PM_GENERAL ? 147 : dm == PM_EXCHANGE ? 40 : 83;
+  }
+  if (op.code < PO_PHASE) return 147;
+  if (op.code < PO_BLOCKADE) return op.code == PO_PHASE && op.kc ? 60 : 101;
+  return 101;   // PO_BLOCKADE
+}
+
+// Slot bits an op of a stage reads or writes; `reg_only`: it has no
+// thread-bit part, so it is the same 16 x 16 map on every thread's slots.
+uint32_t op_slot_bits(const POp& op, bool* reg_only)
+{
+  if (op.code < PO_DENSE_K) {
+    *reg_only = op.tmask == 0;
+    return 1u << (op.code >> 2);
+  }
+  if (op.code < PO_PHASE) {
+    *reg_only = op.tmask == 0;
+    return (1u << (op.code - PO_DENSE_K)) | op.kc;
+  }
+  *reg_only = op.code < PO_BLOCKADE ? op.cnt == 0 : op.code == PO_BLOCKADE && op.aux == 0;
+  return op.kc | (op.code > PO_PHASE && op.code < PO_BLOCKADE ? 1u << (op.code - PO_PHASE2) : 0u);
+}
+
+// v = (map of a register-bit op) v on one thread's 16 slots, as k_pass applies it.
+void apply_reg_op(const POp& op, C v[16])
+{
+  const uint32_t kc = op.kc;
+  if (op.code < PO_PHASE) {
+    const int rb = op.code < PO_DENSE_K ? op.code >> 2 : op.code - PO_DENSE_K;
+    const int d = 1 << rb;
+    const C m00(op.m[0], op.m[1]), m01(op.m[2], op.m[3]), m10(op.m[4], op.m[5]), m11(op.m[6], op.m[7]);
+    for (int k = 0; k < 16; ++k) {
+      if ((k & d) || ((uint32_t)k & kc) != kc) continue;
+      const C a = v[k], b = v[k | d];
+      v[k] = m00 * a + m01 * b;
+      v[k | d] = m10 * a + m11 * b;
+    }
+  } else if (op.code == PO_PHASE) {
+    for (int k = 0; k < 16; ++k)
+      if (((uint32_t)k & kc) == kc) v[k] *= C(op.m[0], op.m[1]);
+  } else if (op.code < PO_BLOCKADE) {
+    const int rb = op.code - PO_PHASE2;
+    for (int k = 0; k < 16; ++k)
+      if (((uint32_t)k & kc) == kc) v[k] *= (k >> rb) & 1 ? C(op.m[6], op.m[7]) : C(op.m[0], op.m[1]);
+  } else {   // PO_BLOCKADE without a thread part
+    for (int k = 0; k < 16; ++k)
+      if (__builtin_popcount((uint32_t)k & kc) == 1) v[k] *= C(op.m[0], op.m[1]);
+  }
+}
+
+struct Compiler {
+  const FPass& p;
+  const bool f32;
+  const int block_cost;
+  const int TB, NT;        // tile bits, thread bits
+  const uint32_t FULL;
+  std::vector<POp> ops;
+  std::vector<PTerm> terms;
+  std::vector<float> blk;
+  int nblk = 0;
+  size_t stage0 = 0;       // first op of the current stage
+  uint16_t stage_col[kCols] = {};
+  uint32_t stage_wr[4] = {};
+
+  // current layout: logical index columns of thread bits and slots, and the
+  // clean layout they started from
+  uint32_t ct[kColT] = {}, cr[4] = {};
+  uint32_t reg = 0;
+  uint32_t wr[4] = {};     // wave-index bits as functionals of the logical index
+  uint32_t row_dirty = 0;  // bits whose value is not one physical bit's
+  uint32_t col_dirty = 0;  // bits whose flip is not one physical bit's
+  uint16_t last_to[kCols] = {};
+  bool have_last = false;
+  uint32_t own[4] = {};    // wave functionals after the last LDS round trip
+  bool have_own = false;
+  uint32_t load_wr[4] = {};
+  bool synced = false;     // every wave's tile has crossed a workgroup barrier
+
+  // diagonal factors not applied yet: where the bits `mask` are set, `on` and
+  // `off` by the value of bit t (t < 0: `on`)
+  struct Factor {
+    uint32_t mask;
+    int t;
+    C on, off;
+    uint32_t bits() const { return mask | (t >= 0 ? 1u << t : 0u); }
+  };
+  std::vector<Factor> pend;
+  C& scalar;
+
+  Compiler(const FPass& p_, bool f32_, int bc, C& sc)
+      : p(p_), f32(f32_), block_cost(bc), TB(p_.tb), NT(p_.tb - 4), FULL((1u << p_.tb) - 1u), scalar(sc)
+  {
+  }
+
+  uint32_t rank_in(uint32_t mask, int b) const { return __builtin_popcount(mask & ((1u << b) - 1u)); }
+  uint32_t slot_mask(uint32_t local) const
+  {
+    uint32_t m = 0;
+    for (uint32_t l = local & reg; l; l &= l - 1) m |= 1u << rank_in(reg, __builtin_ctz(l));
+    return m;
+  }
+  uint32_t tid_mask(uint32_t local) const
+  {
+    const uint32_t nonreg = FULL & ~reg;
+    uint32_t m = 0;
+    for (uint32_t l = local & nonreg; l; l &= l - 1) m |= 1u << rank_in(nonreg, __builtin_ctz(l));
+    return m;
+  }
+  POp& emit(int code)
+  {
+    ops.emplace_back();
+    POp& op = ops.back();
+    std::memset(&op, 0, sizeof(op));
+    op.code = code;
+    return op;
+  }
+
+  void set_clean(uint32_t r)
+  {
+    reg = r;
+    row_dirty = col_dirty = 0;
+    int j = 0, i = 0;
+    for (int b = 0; b < TB; ++b) {
+      if ((r >> b) & 1u) cr[i++] = 1u << b;
+      else ct[j++] = 1u << b;
+    }
+    for (int k = 0; k + 6 < NT; ++k) wr[k] = ct[6 + k];
+  }
+  void lds_columns(uint16_t col[kCols]) const
+  {
+    std::memset(col, 0, kCols * sizeof(uint16_t));
+    for (int j = 0; j < NT; ++j) col[j] = (uint16_t)pass_swz(ct[j]);
+    for (int i = 0; i < 4; ++i) col[kColT + i] = (uint16_t)pass_swz(cr[i]);
+  }
+  void begin_stage()
+  {
+    stage0 = ops.size();
+    lds_columns(stage_col);
+    std::memcpy(stage_wr, wr, sizeof(wr));
+  }
+  bool same_waves(const uint32_t a[4], const uint32_t b[4]) const
+  {
+    for (int k = 0; k + 6 < NT; ++k)
+      if (a[k] != b[k]) return false;
+    return true;
+  }
+  void relayout(uint32_t r)
+  {
+    if (block_cost > 0) form_blocks();
+    POp& op = emit(PO_RELAYOUT);
+    lds_columns(op.col);
+    uint32_t from[4];
+    std::memcpy(from, wr, sizeof(from));
+    if (have_last && !std::memcmp(last_to, op.col, sizeof(last_to))) op.flag |= PR_SAME;
+    if (have_own && !same_waves(own, from)) op.flag |= PR_WAIT;
+    set_clean(r);
+    lds_columns(op.col + kCols);
+    std::memcpy(last_to, op.col + kCols, sizeof(last_to));
+    have_last = true;
+    if (same_waves(from, wr)) op.flag |= PR_LOCAL;
+    else synced = true;
+    std::memcpy(own, wr, sizeof(own));
+    have_own = true;
+    begin_stage();
+  }
+
+  // ---- diagonal factors -----------------------------------------------------
+  void add_term(uint32_t mask, C f)
+  {
+    if (f == C(1.0, 0.0)) return;
+    if (mask == 0) {
+      scalar *= f;
+      return;
+    }
+    add_two(mask, -1, f, f);
+  }
+  void add_two(uint32_t mask, int t, C on, C off)
+  {
+    for (auto& f : pend)
+      if (f.mask == mask && f.t == t) {
+        f.on *= on;
+        f.off *= off;
+        return;
+      }
+    pend.push_back(Factor{mask, t, on, off});
+  }
+  // Can every pending factor with one of the bits `touch` be applied here?
+  bool can_flush(uint32_t touch) const
+  {
+    for (const auto& f : pend)
+      if ((f.bits() & touch) && (f.bits() & row_dirty)) return false;
+    return true;
+  }
+  // Applies the pending factors with one of the bits `touch`, one op per set of
+  // slot bits; `with`: a factor of every amplitude joins the group without slot bits.
+  void flush(uint32_t touch, C with = C(1.0, 0.0))
+  {
+    struct Group { uint32_t kc; int rb; C on, off; std::vector<PTerm> t; };
+    std::vector<Group> groups;
+    auto group = [&](uint32_t kc, int rb) -> Group& {
+      for (auto& g : groups)
+        if (g.kc == kc && g.rb == rb) return g;
+      groups.push_back(Group{kc, rb, C(1.0, 0.0), C(1.0, 0.0), {}});
+      return groups.back();
+    };
+    size_t w = 0;
+    for (size_t i = 0; i < pend.size(); ++i) {
+      const Factor f = pend[i];
+      if (!(f.bits() & touch)) {
+        pend[w++] = f;
+        continue;
+      }
+      const bool on_slot = f.t >= 0 && ((reg >> f.t) & 1u);
+      Group& g = group(slot_mask(f.mask), on_slot ? (int)rank_in(reg, f.t) : -1);
+      const uint32_t tm = tid_mask(f.mask), tb = f.t >= 0 && !on_slot ? tid_mask(1u << f.t) : 0u;
+      if (!tm && !tb) {
+        g.on *= f.on;
+        g.off *= f.off;
+        continue;
+      }
+      PTerm q;
+      std::memset(&q, 0, sizeof(q));
+      q.tmask = tm;
+      q.tbit = tb;
+      if (f32) {
+        q.f[0] = (float)f.on.real();
+        q.f[1] = (float)f.on.imag();
+        q.f[2] = (float)f.off.real();
+        q.f[3] = (float)f.off.imag();
+      } else {
+        q.d[0] = f.on.real();
+        q.d[1] = f.on.imag();
+      }
+      g.t.push_back(q);
+    }
+    pend.resize(w);
+    if (with != C(1.0, 0.0)) group(0, -1).on *= with;
+    for (auto& g : groups) {
+      if (g.t.empty() && g.on == C(1.0, 0.0) && (g.rb < 0 || g.off == g.on)) continue;
+      POp& op = emit(g.rb < 0 ? PO_PHASE : PO_PHASE2 + g.rb);
+      const C first = g.rb < 0 ? g.on : g.off;
+      op.kc = g.kc;
+      op.m[0] = first.real();
+      op.m[1] = first.imag();
+      op.m[6] = g.on.real();
+      op.m[7] = g.on.imag();
+      op.aux = (uint32_t)terms.size();   // index now, byte offset when the program is laid out
+      op.cnt = (int32_t)g.t.size();
+      terms.insert(terms.end(), g.t.begin(), g.t.end());
+    }
+  }
+
+  // ---- matrix-core blocks -----------------------------------------------------
+  // Fold the register-bit ops of the stage just ended into dense 16 x 16
+  // blocks. Scanning in order, an op without a thread-bit part joins the open
+  // block if its slot bits miss those of every op set aside since the block
+  // opened; an op with a thread-bit part is set aside and runs after the block
+  // (ops on disjoint bits commute). A block whose ops cost the vector units
+  // less than block_cost keeps its ops in program order.
+  void form_blocks()
+  {
+    const std::vector<POp> src(ops.begin() + stage0, ops.end());
+    ops.resize(stage0);
+    std::vector<int> in, aside;
+    uint32_t aside_bits = 0;
+    int cost = 0;
+    auto close = [&]() {
+      if (cost >= block_cost && nblk < kMaxPassBlocks) {
+        C U[16][16];
+        for (int col = 0; col < 16; ++col) {
+          C v[16];
+          for (int k = 0; k < 16; ++k) v[k] = k == col ? 1.0 : 0.0;
+          for (int i : in) apply_reg_op(src[i], v);
+          for (int k = 0; k < 16; ++k) U[k][col] = v[k];
+        }
+        for (int kk = 0; kk < 4; ++kk)
+          for (int l = 0; l < 64; ++l) {
+            const C u = U[l & 15][4 * kk + (l >> 4)];
+            blk.push_back((float)u.real());
+            blk.push_back((float)u.imag());
+          }
+        POp& b = emit(PO_BLOCK);
+        b.aux = (uint32_t)nblk++;   // index now, byte offset when the program is laid out
+        std::memcpy(b.col, stage_col, sizeof(stage_col));
+        std::memcpy(own, stage_wr, sizeof(own));
+        have_own = true;
+        for (int i : aside) ops.push_back(src[i]);
+      } else {
+        std::vector<int> all(in);
+        all.insert(all.end(), aside.begin(), aside.end());
+        std::sort(all.begin(), all.end());
+        for (int i : all) ops.push_back(src[i]);
+      }
+      in.clear();
+      aside.clear();
+      aside_bits = 0;
+      cost = 0;
+    };
+    for (int i = 0; i < (int)src.size(); ++i) {
+      if (src[i].code == PO_SWAP) {
+        close();
+        ops.push_back(src[i]);
+        continue;
+      }
+      bool reg_only = false;
+      const uint32_t sb = op_slot_bits(src[i], &reg_only);
+      if (reg_only) {
+        if (sb & aside_bits) close();
+        in.push_back(i);
+        cost += reg_op_cost(src[i]);
+      } else {
+        aside.push_back(i);
+        aside_bits |= sb;
+      }
+    }
+    close();
+  }
+
+  // ---- gates --------------------------------------------------------------------
+  // a phase, which can be divided out and applied later without moving the norm
+  static bool usable(C d) { return std::fabs(std::abs(d) - 1.0) < 1e-9; }
+  static uint32_t gate_bits(const FGate& g)
+  {
+    uint32_t m = g.cmask | (g.kind == FG_BLOCKADE ? g.bmask : 0u);
+    if (g.a >= 0) m |= 1u << g.a;
+    if (g.b >= 0) m |= 1u << g.b;
+    return m;
+  }
+  // CNOTs and plain (phased) swaps
+  static bool is_linear(const FGate& g)
+  {
+    if (g.kind == FG_DENSE) return g.sub == DM_EXCHANGE && __builtin_popcount(g.cmask) == 1;
+    return g.kind == FG_SWAP && g.cmask == 0 && usable(C(g.m[0], g.m[1]));
+  }
+  // A diagonal gate as factors on bit masks; false when its first entry is no
+  // phase and cannot be divided out.
+  bool take_phase(const FGate& g)
+  {
+    const C d0(g.m[0], g.m[1]), d1(g.m[6], g.m[7]);
+    const uint32_t t = 1u << g.a;
+    if (g.sub) {   // d0 == 1
+      add_term(g.cmask | t, d1);
+      return true;
+    }
+    // FP32 passes keep both entries: rounded alike (a Z rotation's are
+    // conjugates) they leave the weights of the two halves as they are, where
+    // one rounded factor on one half moves them against each other
+    if (f32) {
+      add_two(g.cmask, g.a, d1, d0);
+      return true;
+    }
+    if (!usable(d0)) return false;
+    add_term(g.cmask, d0);
+    add_term(g.cmask | t, d1 / d0);
+    return true;
+  }
+
+  bool run_linear(const FGate& g)
+  {
+    if (g.kind == FG_SWAP) {
+      const int a = g.a, b = g.b;
+      auto sw = [&](uint32_t m) {
+        const uint32_t x = ((m >> a) ^ (m >> b)) & 1u;
+        return m ^ (x << a) ^ (x << b);
+      };
+      for (auto& f : pend) {
+        f.mask = sw(f.mask);
+        if (f.t == a || f.t == b) f.t = a + b - f.t;
+      }
+      for (int j = 0; j < NT; ++j) ct[j] = sw(ct[j]);
+      for (auto& c : cr) c = sw(c);
+      for (auto& w : wr) w = sw(w);
+      const uint32_t ab = (1u << a) | (1u << b);
+      row_dirty |= ab;
+      col_dirty |= ab;
+      const C ph(g.m[0], g.m[1]);
+      if (ph != C(1.0, 0.0)) {
+        add_term(1u << a, ph);
+        add_term(1u << b, ph);
+        add_term(ab, 1.0 / (ph * ph));
+      }
+      return true;
+    }
+    const uint32_t t = 1u << g.a, c = g.cmask;
+    if (!can_flush(t)) return false;
+    flush(t);
+    for (int j = 0; j < NT; ++j)
+      if (ct[j] & c) ct[j] ^= t;
+    for (auto& x : cr)
+      if (x & c) x ^= t;
+    for (auto& w : wr)
+      if (w & t) w ^= c;
+    row_dirty |= t;
+    col_dirty |= t | c;
+    return true;
+  }
+
+  // Runs a gate that is neither diagonal nor linear if the layout allows it.
+  bool run_gate(const FGate& g)
+  {
+    if (g.kind == FG_BLOCKADE) {
+      if (g.bmask & row_dirty) return false;
+      POp& op = emit(PO_BLOCKADE);
+      op.kc = slot_mask(g.bmask);
+      op.aux = tid_mask(g.bmask);
+      op.m[0] = g.m[0];
+      op.m[1] = g.m[1];
+      return true;
+    }
+    if (g.kind == FG_SWAP) {
+      if (row_dirty | col_dirty) return false;
+      const uint32_t ab = (1u << g.a) | (1u << g.b);
+      flush(ab);
+      POp& op = emit(PO_SWAP);
+      op.kc = (uint32_t)g.a;
+      op.aux = (uint32_t)g.b;
+      op.tmask = g.cmask;
+      op.sc[0] = g.m[0];
+      op.sc[1] = g.m[1];
+      lds_columns(op.col);
+      std::memcpy(own, wr, sizeof(own));
+      have_own = true;
+      synced = true;
+      return true;
+    }
+    const uint32_t t = 1u << g.a;
+    if (!(reg & t) || ((row_dirty | col_dirty) & t) || (g.cmask & row_dirty) || !can_flush(t)) return false;
+    const int rb = (int)rank_in(reg, g.a);
+    double m[8];
+    std::memcpy(m, g.m, sizeof(m));
+    int sub = g.kind == FG_DENSE ? g.sub : DM_GENERAL;
+    if (g.kind == FG_PHASE) m[2] = m[3] = m[4] = m[5] = 0.0;
+    // a unitary without structure: e^{ia} diag(1, f1) [[c, -s], [s, c]] diag(1, f0)
+    C f0(1.0, 0.0), f1(1.0, 0.0);
+    if (!f32 && sub == DM_GENERAL && g.cmask == 0 && g.kind == FG_DENSE) {
+      const C m00(m[0], m[1]), m01(m[2], m[3]), m10(m[4], m[5]), m11(m[6], m[7]);
+      const double c = std::abs(m00), s = std::abs(m10), s1 = std::abs(m01);
+      if (c > 1e-8 && s > 1e-8 && s1 > 1e-8) {
+        const C u = m00 / c;
+        f1 = m10 / (s * u);
+        f0 = -m01 / (s1 * u);
+        const double n = std::sqrt(c * c + s * s);
+        // equal to the matrix to the last places, or taken as it is
+        const double e = std::max({std::fabs(n - 1.0), std::abs(m01 + u * f0 * s), std::abs(m11 - u * f0 * f1 * c)});
+        if (e < 1e-15) {
+          scalar *= u;
+          sub = DM_REAL;
+          const double r[8] = {c, 0, -s, 0, s, 0, c, 0};
+          std::memcpy(m, r, sizeof(m));
+          add_term(t, f0);
+        } else {
+          f0 = f1 = C(1.0, 0.0);
+        }
+      }
+    }
+    flush(t);
+    const uint32_t kc = slot_mask(g.cmask);
+    POp& op = emit(kc ? PO_DENSE_K + rb : PO_DENSE + 4 * rb + sub);
+    op.kc = kc;
+    op.tmask = tid_mask(g.cmask);
+    std::memcpy(op.m, m, sizeof(m));
+    add_term(t, f1);
+    return true;
+  }
+
+  // Fill a register mask to four bits: bits above the low run, highest first
+  // (consecutive layouts then tend to share them) without the two that name
+  // the wave, then those two, then low bits.
+  uint32_t fill(uint32_t r) const
+  {
+    const int L = p.low;
+    for (int b = TB - 3; b >= L && __builtin_popcount(r) < 4; --b) r |= 1u << b;
+    for (int b = TB - 1; b >= std::max(0, TB - 2) && __builtin_popcount(r) < 4; --b) r |= 1u << b;
+    for (int b = 0; b < TB && __builtin_popcount(r) < 4; ++b) r |= 1u << b;
+    return r;
+  }
+  bool coalesced() const
+  {
+    for (int j = 0; j < p.low; ++j)
+      if (ct[j] >> p.low) return false;
+    return true;
+  }
+  void global_columns(uint64_t out[kCols]) const
+  {
+    auto g = [&](uint32_t l) {
+      uint64_t v = 0;
+      for (; l; l &= l - 1) v |= 1ull << p.pos[__builtin_ctz(l)];
+      return v;
+    };
+    for (int j = 0; j < kColT; ++j) out[j] = j < NT ? g(ct[j]) : 0;
+    for (int i = 0; i < 4; ++i) out[kColT + i] = g(cr[i]);
+  }
+
+  void run(PHead& h, bool last)
+  {
+    const int N = (int)p.gates.size();
+    // per-bit queues of the gates in program order
+    std::vector<int> queue[16];
+    std::vector<uint32_t> bits(N);
+    std::vector<char> done(N, 0);
+    for (int i = 0; i < N; ++i) {
+      bits[i] = gate_bits(p.gates[i]);
+      for (uint32_t m = bits[i]; m; m &= m - 1) queue[__builtin_ctz(m)].push_back(i);
+    }
+    size_t head[16] = {};
+    int left = N;
+    auto front = [&](int b) -> int { return head[b] < queue[b].size() ? queue[b][head[b]] : -1; };
+    auto ready = [&](int i) {
+      for (uint32_t m = bits[i]; m; m &= m - 1)
+        if (front(__builtin_ctz(m)) != i) return false;
+      return true;
+    };
+    auto consume = [&](int i) {
+      done[i] = 1;
+      --left;
+      for (uint32_t m = bits[i]; m; m &= m - 1) ++head[__builtin_ctz(m)];
+    };
+    // the next layout: the targets of waiting dense gates. `first`: the load
+    // layout, whose lanes must cover the low run; later ones take low bits as
+    // soon as they are wanted, so that the last layout can store.
+    auto next_regs = [&](bool first) {
+      std::vector<std::pair<int, int>> want;   // (order, bit)
+      for (int b = 0; b < TB; ++b) {
+        const int i = front(b);
+        if (i < 0 || !ready(i)) continue;
+        const FGate& g = p.gates[i];
+        if (g.a != b || is_linear(g) || (g.kind != FG_DENSE && g.kind != FG_PHASE)) continue;
+        if (first && b < p.low) continue;
+        want.emplace_back(b < p.low ? i - N : i, b);
+      }
+      std::sort(want.begin(), want.end());
+      uint32_t r = 0;
+      for (const auto& w : want)
+        if (__builtin_popcount(r) < 4) r |= 1u << w.second;
+      return r;
+    };
+    // gates that wait for nothing: diagonal ones leave the queues at once
+    auto drain_phases = [&]() {
+      bool any = false;
+      for (int b = 0; b < TB; ++b)
+        for (int i = front(b); i >= 0; i = front(b)) {
+          const FGate& g = p.gates[i];
+          if (g.kind != FG_PHASE || !ready(i) || !take_phase(g)) break;
+          consume(i);
+          any = true;
+        }
+      return any;
+    };
+    while (drain_phases()) {
+    }
+    set_clean(fill(next_regs(true)));
+    if (!coalesced()) set_clean(fill(0));
+    global_columns(h.gload);
+    std::memcpy(load_wr, wr, sizeof(load_wr));
+    begin_stage();
+    while (left) {
+      bool any = true, moved = false;
+      while (any) {   // everything this layout can run
+        any = drain_phases();
+        for (int b = 0; b < TB; ++b) {
+          const int i = front(b);
+          if (i < 0 || is_linear(p.gates[i]) || !ready(i) || !run_gate(p.gates[i])) continue;
+          consume(i);
+          any = true;
+        }
+        moved |= any;
+      }
+      for (int b = 0; b < TB; ++b) {
+        const int i = front(b);
+        if (i < 0 || !is_linear(p.gates[i]) || !ready(i) || !run_linear(p.gates[i])) continue;
+        consume(i);
+        moved = true;
+      }
+      if (moved || !left) continue;
+      relayout(fill(next_regs(false)));
+    }
+    C g(1.0, 0.0);
+    if (last) {
+      g = scalar;
+      scalar = C(1.0, 0.0);
+    }
+    if (!can_flush(FULL)) relayout(fill(0));
+    flush(FULL, g);
+    if (!coalesced()) relayout(fill(0));
+    else if (block_cost > 0) form_blocks();
+    global_columns(h.gstore);
+    // the tile is updated in place: a wave may overwrite amplitudes that another
+    // one has not loaded yet when the layouts name the waves differently
+    h.store_wait = !synced && !same_waves(load_wr, wr) ? 1 : 0;
+  }
+};
+
+}  // namespace
+
+size_t compile_pass(const FPass& p, bool f32, int block_cost, std::complex<double>& scalar, bool last,
+                    std::vector<char>& out)
+{
+  PHead h;
+  std::memset(&h, 0, sizeof(h));
+  h.renorm = p.renorm;
+  std::memcpy(h.sorted_pos, p.sorted_pos, sizeof(h.sorted_pos));
+  Compiler c(p, f32, block_cost, scalar);
+  c.run(h, last);
+  h.nops = (int32_t)c.ops.size();
+  const size_t terms_at = (sizeof(PHead) + (c.ops.size() + 1) * sizeof(POp) + 31) & ~(size_t)31;
+  const size_t blk_at = terms_at + c.terms.size() * sizeof(PTerm);
+  for (POp& op : c.ops) {
+    if (op.code >= PO_PHASE && op.code < PO_BLOCKADE) op.aux = (uint32_t)(terms_at + op.aux * sizeof(PTerm));
+    else if (op.code == PO_BLOCK) op.aux = (uint32_t)(blk_at + op.aux * kBlockTable);
+    if (f32 && (op.code <= PO_BLOCKADE)) {
+      float f[8];
+      for (int k = 0; k < 8; ++k) f[k] = (float)op.m[k];
+      std::memset(op.m, 0, sizeof(op.m));
+      std::memcpy(op.f, f, sizeof(f));
+    }
+  }
+  const size_t bytes = (blk_at + c.blk.size() * sizeof(float) + 255) & ~(size_t)255;
+  h.bytes = (int32_t)bytes;
+  const size_t at = (out.size() + 255) & ~(size_t)255;
+  out.resize(at + bytes, 0);
+  char* d = out.data() + at;
+  std::memcpy(d, &h, sizeof(h));
+  if (!c.ops.empty()) std::memcpy(d + sizeof(PHead), c.ops.data(), c.ops.size() * sizeof(POp));
+  if (!c.terms.empty()) std::memcpy(d + terms_at, c.terms.data(), c.terms.size() * sizeof(PTerm));
+  if (!c.blk.empty()) std::memcpy(d + blk_at, c.blk.data(), c.blk.size() * sizeof(float));
+  return at;
+}
+
+}  // namespace qsv

@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <complex>
 #include <string>
 #include <vector>
 #include "../../include/qsv.h"
@@ -131,10 +132,9 @@ void launch_collapse(int prec, void* psi, uint64_t S, int m, const int* pos, uin
                      hipStream_t st);
 
 // ---- fused tiled passes: planning (qsv_api.hip) ------------------------------
-constexpr int kTileBitsC128 = 12;   // 4096 x 16 B = 64 KiB of LDS per tile
-constexpr int kTileBitsC64 = 12;    // 4096 x  8 B = 32 KiB: three workgroups per CU
-constexpr int kMaxPassGates = 96;
-constexpr int kMaxPassStages = 32;
+// Gates per pass. FP32 passes are renormalised between passes, which bounds
+// the norm drift a pass may gather.
+constexpr int kMaxPassGates = 1024, kMaxPassGatesF32 = 96;
 
 // FG_RENORM: divide the state by its FP64 norm when that exceeds 1e-12, as
 // normalize-state does after a Kraus operator (a record of batched LDS
@@ -155,11 +155,6 @@ struct FGate {
   double m[8];         // dense: row-major 2x2; phase: d0 = m[0..1], d1 = m[6..7]; swap/blockade: phase m[0..1]
 };
 
-struct FStage {
-  uint32_t regmask;    // tile-local bits held in registers during this stage
-  int32_t g0, g1;      // gates [g0, g1)
-};
-
 // Complex64 passes compute in FP32 by default. The rounded 2x2 matrices are
 // unitary only to ~1e-7, so the norm would drift by that much per gate; it is
 // removed pass by pass instead: a pass sums |amplitude|^2 per tile in FP64
@@ -177,81 +172,90 @@ struct TileNorm {
   double* ctl;        // [0] target norm^2, [1] scale for the next pass
 };
 
+// The gates of one pass in program order, on tile-local bits.
 struct FPass {
-  int32_t nstages;
-  int32_t ngates;
-  uint32_t load_mask, store_mask;   // register masks used for the global load / store
-  int32_t renorm;                   // FP_RENORM_* bits
-  int32_t pad;
-  int32_t pos[16];                  // global index bit of tile-local bit i
-  int32_t sorted_pos[16];           // the same bits in ascending order
-  FStage stages[kMaxPassStages];
-  FGate gates[kMaxPassGates];
+  int32_t tb = 12;                  // tile bits
+  int32_t low = 0;                  // the low run: local bits 0..low-1 are global bits 0..low-1
+  int32_t renorm = 0;               // FP_RENORM_* bits
+  int32_t pos[16] = {};             // global index bit of tile-local bit i
+  int32_t sorted_pos[16] = {};      // the same bits in ascending order
+  std::vector<FGate> gates;
 };
 
-// ---- fused passes as micro-op programs (qsv_pass.hip) ------------------------
+// ---- fused passes as micro-op programs (qsv_compile.hip, qsv_pass.hip) -------
 // A pass compiled against the layouts it runs in: every op names the register
-// bit, slot mask and thread-id mask it acts on (compile_pass, qsv_api.hip).
+// bit, slot mask and thread-id mask it acts on.
 constexpr int kPassTileBits = 12;
-constexpr int kMaxPassOps = kMaxPassGates + kMaxPassStages + 1;
 // Dense structures share the DM_* numbering.
 enum { PM_GENERAL = DM_GENERAL, PM_REAL = DM_REAL, PM_RX = DM_RX, PM_EXCHANGE = DM_EXCHANGE };
 enum {
-  PO_DENSE = 0,       // + 4 * register bit + structure (PM_*): 0..15
-  PO_PHASE = 16,      // + 4 * only1 + register bit: diag(d0, d1) on a register bit, 16..23
-  PO_PHASE_T = 24,    // diag(d0, d1) on a thread bit (aux = its thread-id bit)
+  PO_DENSE = 0,       // + 4 * register bit + structure (PM_*): 0..15, no slot controls
+  PO_DENSE_K = 16,    // + register bit: any 2x2 on the slot pairs whose bits kc are set, 16..19
+  PO_PHASE = 20,      // one factor per lane on the slots whose bits kc are set (0, one or more)
+  PO_PHASE2 = 21,     // + register bit, 21..24: one factor per lane for that bit set, one for it clear, on the slots kc
   PO_BLOCKADE = 25,   // phase where exactly one of the bits aux (thread) / kc (slot) is set
-  PO_RELAYOUT = 26,   // layouts tmask -> kc (PProg::lay), new register mask aux; only1: wave-local
-  PO_SWAP = 27,       // exchange local bits kc and aux where the local bits tmask are set
+  PO_RELAYOUT = 26,   // layout col[0..13] -> layout col[14..27]; flag: PR_*
+  PO_SWAP = 27,       // exchange local bits kc and aux where the local bits tmask are set (layout col[0..13])
   PO_BLOCK = 28,      // dense 16x16 on the four register bits (FP32 passes only): table at byte offset aux
 };
+// PO_RELAYOUT: the round trip stays inside each wave; the old layout is the one
+// the previous relayout ended in; the workgroup must wait before writing.
+enum { PR_LOCAL = 1, PR_SAME = 2, PR_WAIT = 4 };
+// A register layout is a linear map over GF(2): thread t, slot k holds the
+// tile-local index XOR_j t_j c_j XOR XOR_i k_i r_i. col[] lists the LDS element
+// indices of the columns (the bank swizzle is linear too): c_0..c_9, r_0..r_3.
+constexpr int kColT = 10, kCols = 14;
 struct POp {
   int32_t code;
   uint32_t tmask;     // thread-id bits that must be set (thread-bit controls)
   uint32_t kc;        // slot bits that must be set (register-bit controls)
-  uint32_t aux;
-  int32_t only1;      // PO_PHASE_T: d0 == 1; PO_RELAYOUT: wave-local
-  int32_t pad;
-  double m[8];        // as FGate
-  float f[8];         // m rounded to FP32, for FP32-arithmetic passes
+  uint32_t aux;       // PO_PHASE, PO_PHASE2: byte offset of the terms
+  int32_t cnt;        // PO_PHASE, PO_PHASE2: number of terms
+  int32_t flag;
+  double sc[2];       // PO_SWAP: the exchanged amplitudes' phase
+  union {
+    double m[8];      // row-major 2x2; PO_PHASE, PO_BLOCKADE: a factor in m[0..1]; PO_PHASE2: clear m[0..1], set m[6..7]
+    float f[8];       // the same rounded, in the programs of FP32 passes
+    uint16_t col[32]; // PO_RELAYOUT, PO_SWAP and PO_BLOCK (float programs keep no m there)
+  };
 };
-// A register layout of a tile resolved on the host. Thread t, slot k holds
-// tile-local index pdep(t, ~reg) | pdep(k, reg); with t_j the bits of t, its
-// LDS byte offset is XOR_j (t_j ? lt[j] : 0) XOR ls[k] (the swizzle is
-// XOR-linear) and its global element offset is
-// tile base | OR_j (t_j ? gt[j] : 0) | gs[k].
-struct PLayout {
-  uint32_t lt[8];
-  uint32_t ls[16];
-  uint64_t gt[8];
-  uint64_t gs[16];
+static_assert(sizeof(POp) == 104, "the kernel reads ops as 26 dwords");
+// A factor of PO_PHASE or PO_PHASE2 on the lanes with all bits of tmask set. In
+// FP32 programs it has two values: PO_PHASE takes `on` where the thread bit
+// tbit is set and `off` where it is clear (tbit 0: always `on`), PO_PHASE2 `on`
+// for the set and `off` for the clear register bit.
+struct PTerm {
+  uint32_t tmask, tbit;
+  union {
+    double d[2];      // FP64 programs
+    float f[4];       // FP32 programs: on, off
+  };
 };
-constexpr int kMaxPassLayouts = kMaxPassStages + 2;
+static_assert(sizeof(PTerm) == 24, "terms are 24 bytes");
 // PO_BLOCK tables per pass: 4 steps x 64 lanes of (re, im) FP32, lane l of
 // step kk holding U[l % 16][4 kk + l / 16] (the A operand of
 // v_mfma_f32_16x16x4f32), U indexed by slot.
 constexpr int kMaxPassBlocks = 8;
+constexpr size_t kBlockTable = 4 * 64 * 2 * sizeof(float);
 struct PHead {
   int32_t nops;
   int32_t renorm;                   // FP_RENORM_* bits
-  uint32_t load_mask, store_mask;   // register masks of the global load / store
-  int32_t store_local;              // the layout change before the store is wave-local
-  int32_t load_lay, store_lay;      // their entries in the layout table
-  int32_t nlay;
-  int32_t lay_off;                  // byte offset of the layout table from the program start
-  int32_t pad;
+  int32_t bytes;                    // of the whole program
+  int32_t store_wait;               // waves store where others load, with no barrier between: wait first
   int32_t sorted_pos[16];           // the tile's global bits in ascending order
+  uint64_t gload[kCols], gstore[kCols];   // global index columns of the load and store layouts
 };
-// Ops come right after the header; the layout table sits at h.lay_off, at
-// `lay` here or packed right after the last op (grouped batches).
-struct PProg {
-  PHead h;
-  POp ops[kMaxPassOps];
-  PLayout lay[kMaxPassLayouts];
-  float blk[kMaxPassBlocks][4 * 64 * 2];
-};
+// In memory: the header, the ops and one unread op (the kernel fetches an op
+// ahead), the terms, the block tables.
+// A program appended to `out` (at a multiple of 256 bytes); returns its offset.
+// f32: an FP32 pass; block_cost > 0: runs of register-bit ops that cost the
+// vector units at least that become PO_BLOCK ops. `scalar` collects factors
+// common to the whole state: multiplied into it, applied (and reset) by this
+// pass when `last`.
+size_t compile_pass(const FPass& p, bool f32, int block_cost, std::complex<double>& scalar, bool last,
+                    std::vector<char>& out);
 // f32: complex64 arithmetic in FP32 (ignored for complex128, always FP64)
-void launch_pass(int prec, bool f32, void* psi, const PProg* dprog, uint64_t ntiles, const TileNorm& nb,
+void launch_pass(int prec, bool f32, void* psi, const char* dprog, uint64_t ntiles, const TileNorm& nb,
                  hipStream_t st);
 // A group of `count` states of S amplitudes (S >= one tile) back to back: one
 // pass round (offs[y] = byte offset of instance y's program in `progs`, or -1).

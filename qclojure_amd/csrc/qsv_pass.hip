@@ -1,28 +1,36 @@
-// qsv_pass.hip — fused tiled passes as host-compiled micro-op programs.
+// qsv_pass.hip — fused tiled passes: the micro-op programs of qsv_compile.hip.
 //
 // A pass owns TB = 12 tile bits of the index. Each workgroup of 256 threads
 // loads one tile of 2^12 amplitudes (16 per thread, in registers), runs the
 // pass's micro-ops and stores the tile back, so the state crosses HBM once per
 // pass however many gates the pass holds.
 //
-// The layout of a tile in registers is a register mask `reg` of 4 tile-local
-// bits: thread t, slot k holds local index pdep(t, ~reg) | pdep(k, reg). The
-// host resolves every gate against the layout it will run in (qsv_api.hip,
-// compile_pass), so a micro-op carries the register bit of its target, the
-// slot mask of its register-bit controls and the thread-id mask of its
-// thread-bit controls: the kernel decodes nothing, takes only uniform
-// branches, and a lane whose controls are not set applies the identity by
-// selects instead of a divergent skip.
+// The layout of a tile in registers is linear over GF(2): thread t, slot k
+// holds the local index XOR_j t_j c_j XOR XOR_i k_i r_i. A micro-op names the
+// register bit of its target, the slot mask of its register-bit controls and
+// the thread-id mask of its thread-bit controls: the kernel decodes nothing and
+// takes only uniform branches; a lane whose controls are not set applies the
+// identity through its coefficients.
 //
-// Changing the layout is one LDS round trip (a RELAYOUT op). When the two
-// wave-id bits of the thread index map to the same tile bits before and after,
-// every wave keeps its own amplitudes and the round trip needs no workgroup
-// barrier; the host marks those. complex128 tiles cross LDS one plane (real,
-// then imaginary) at a time, so a workgroup needs 32 KiB of LDS.
+// Changing the layout is one LDS round trip (PO_RELAYOUT). When the wave-id
+// bits of the thread index name the same tile bits before and after, every wave
+// keeps its own amplitudes and the round trip needs no workgroup barrier; the
+// host marks those. A wave only ever reads the addresses of the layout it
+// enters and writes those of the layout it leaves, so one barrier per exchanged
+// plane is enough. FP64 tiles cross LDS one plane (real, then imaginary) at a
+// time, so a workgroup needs 32 KiB of LDS.
 //
-// Arithmetic type A: FP64 for complex128; FP32 or FP64 for complex64. With FP32
-// the pass also reports per-tile norms and applies the previous pass's
-// renormalisation scale at load (TileNorm in qsv_internal.h).
+// Arithmetic type A: FP64 for complex128 and for complex64 states whose passes
+// are asked for in FP64 (held in FP64 registers, rounded at the store); FP32
+// for other complex64 passes, which also report per-tile norms and apply the
+// previous pass's renormalisation scale at load (TileNorm in qsv_internal.h).
+// What bounds it: the tile's access pattern (loads and stores alone stream at
+// 5.3 TB/s) with the gates' instructions partly on top; on few tiles the chain
+// of ops, whose fetch from memory is hidden behind the op before. Against the
+// interpreter that ran every gate as an op and kept two copies of the tile
+// (three waves per SIMD), per launch: 27-qubit complex128 layers 1257 -> 925 us,
+// 19-qubit ones 47 -> 22 us, 540 gates on one 12-qubit tile 524 -> 177 us,
+// 26-qubit complex64 QAOA 372 -> 352 us.
 #include "qsv_internal.h"
 
 namespace qsv {
@@ -32,155 +40,51 @@ namespace {
 template <typename R> struct PV;
 template <> struct PV<double> { typedef double T __attribute__((ext_vector_type(2))); };
 template <> struct PV<float> { typedef float T __attribute__((ext_vector_type(2))); };
-// One plane (real or imaginary parts) of a thread's 16 slots: a single vector
-// value indexed by constants only, so it never leaves registers.
-template <typename R> struct SV;
-template <> struct SV<double> { typedef double T __attribute__((ext_vector_type(16))); };
-template <> struct SV<float> { typedef float T __attribute__((ext_vector_type(16))); };
 
 constexpr int kSlots = 16;
 constexpr int kThreads = 256;
 
-// f(k) for k = K .. kSlots-1 with k a compile-time constant: the slot
-// arrays must only ever be indexed by constants, or they leave registers.
-template <int K = 0, typename F>
-__device__ __forceinline__ void each_slot(F&& f)
+__device__ __forceinline__ double mad(double a, double b, double c) { return __builtin_fma(a, b, c); }
+__device__ __forceinline__ float mad(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+
+template <int V> using Int = std::integral_constant<int, V>;
+
+// f(k) for k = K .. N-1 with k a compile-time constant: slots must only ever
+// be indexed by constants, or they leave registers.
+template <int K, int N, typename F>
+__device__ __forceinline__ void each(F&& f)
 {
-  if constexpr (K < kSlots) {
+  if constexpr (K < N) {
     f(std::integral_constant<int, K>{});
-    each_slot<K + 1>(f);
+    each<K + 1, N>(f);
   }
 }
 
-__device__ __forceinline__ uint32_t pdep32(uint32_t src, uint32_t mask)
-{
-  uint32_t out = 0;
-  for (uint32_t m = mask; m; m &= m - 1) {
-    if (src & 1u) out |= m & (~m + 1u);
-    src >>= 1;
+// One op's fields and coefficients in scalar registers, fetched one op ahead.
+template <typename A> struct OpRegs {
+  int32_t code;
+  uint32_t tmask, kc, aux;
+  int32_t cnt, flag;
+  uint32_t w[16];   // the union: coefficients or packed columns
+  __device__ __forceinline__ A m(int i) const
+  {
+    if constexpr (sizeof(A) == 8) return __hiloint2double((int)w[2 * i + 1], (int)w[2 * i]);
+    else return __uint_as_float(w[i]);
   }
-  return out;
-}
-
-// Bank-spreading swizzle of a tile-local index: a bijection that only
-// rewrites the low 4 bits, XOR-linear in the index.
-__device__ __forceinline__ uint32_t swz(uint32_t l) { return l ^ (((l >> 4) ^ (l >> 8)) & 15u); }
-
-template <typename A>
-struct Mat {
-  A m0, m1, m2, m3, m4, m5, m6, m7;
+  __device__ __forceinline__ uint32_t col(int i) const { return (w[i >> 1] >> (16 * (i & 1))) & 0xffffu; }
 };
-
-// slot K of (xr, xi) *= (re, im)
-template <int K, typename A, typename V>
-__device__ __forceinline__ void cmul_slot(A re, A im, V& xr, V& xi)
+template <typename A>
+__device__ __forceinline__ void fetch(OpRegs<A>& o, const POp* p)
 {
-  const A ax = xr[K], ay = xi[K];
-  xr[K] = re * ax - im * ay;
-  xi[K] = re * ay + im * ax;
-}
-
-// (a, b) = M (a, b) for the structure DM.
-template <int DM, typename A, typename R>
-__device__ __forceinline__ void pair_op(const Mat<A>& m, R& ar, R& ai, R& br, R& bi)
-{
-  const A ax = ar, ay = ai, bx = br, by = bi;
-  if constexpr (DM == PM_EXCHANGE) {
-    ar = (R)bx; ai = (R)by;
-    br = (R)ax; bi = (R)ay;
-  } else if constexpr (DM == PM_REAL) {
-    ar = (R)(m.m0 * ax + m.m2 * bx);
-    ai = (R)(m.m0 * ay + m.m2 * by);
-    br = (R)(m.m4 * ax + m.m6 * bx);
-    bi = (R)(m.m4 * ay + m.m6 * by);
-  } else if constexpr (DM == PM_RX) {
-    // real diagonal, imaginary off-diagonal: m01 = i m3, m10 = i m5
-    ar = (R)(m.m0 * ax - m.m3 * by);
-    ai = (R)(m.m0 * ay + m.m3 * bx);
-    br = (R)(m.m6 * bx - m.m5 * ay);
-    bi = (R)(m.m6 * by + m.m5 * ax);
-  } else {
-    ar = (R)(m.m0 * ax - m.m1 * ay + m.m2 * bx - m.m3 * by);
-    ai = (R)(m.m0 * ay + m.m1 * ax + m.m2 * by + m.m3 * bx);
-    br = (R)(m.m4 * ax - m.m5 * ay + m.m6 * bx - m.m7 * by);
-    bi = (R)(m.m4 * ay + m.m5 * ax + m.m6 * by + m.m7 * bx);
-  }
-}
-
-// Dense 2x2 on register bit RB. KC: only slot pairs whose register-bit
-// controls kc are set (a uniform test per pair); without KC every pair acts
-// and no per-pair branch is generated (a skipped pair would make the compiler
-// copy its inputs into the outputs' registers). With LS, lanes where `act` is
-// false keep their values (selects).
-template <int RB, int DM, bool LS, bool KC, typename A, typename R>
-__device__ __forceinline__ void op_dense(typename SV<R>::T& xr, typename SV<R>::T& xi, const Mat<A>& m, uint32_t kc, bool act)
-{
-  each_slot([&](auto kk) __attribute__((always_inline)) {
-    constexpr int k = decltype(kk)::value;
-    constexpr int d = 1 << RB;
-    if constexpr (!(k & d)) {
-      if (KC && (k & kc) != kc) return;
-      R ar = xr[k], ai = xi[k], br = xr[k | d], bi = xi[k | d];
-      pair_op<DM, A, R>(m, ar, ai, br, bi);
-      if constexpr (LS) {
-        ar = act ? ar : xr[k];
-        ai = act ? ai : xi[k];
-        br = act ? br : xr[k | d];
-        bi = act ? bi : xi[k | d];
-      }
-      xr[k] = ar;
-      xi[k] = ai;
-      xr[k | d] = br;
-      xi[k | d] = bi;
-    }
-  });
-}
-
-template <int RB, bool LS, bool KC, typename A, typename R>
-__device__ __forceinline__ void dense_dm(typename SV<R>::T& xr, typename SV<R>::T& xi, int dm, const Mat<A>& m, uint32_t kc,
-                                         bool act)
-{
-  if (dm == PM_GENERAL) op_dense<RB, PM_GENERAL, LS, KC, A, R>(xr, xi, m, kc, act);
-  else if (dm == PM_REAL) op_dense<RB, PM_REAL, LS, KC, A, R>(xr, xi, m, kc, act);
-  else if (dm == PM_RX) op_dense<RB, PM_RX, LS, KC, A, R>(xr, xi, m, kc, act);
-  else op_dense<RB, PM_EXCHANGE, LS, KC, A, R>(xr, xi, m, kc, act);
-}
-
-template <int RB, typename A, typename R>
-__device__ __forceinline__ void dense_rb(typename SV<R>::T& xr, typename SV<R>::T& xi, int dm, bool ls, const Mat<A>& m,
-                                         uint32_t kc, bool act)
-{
-  if (kc == 0) {
-    if (ls) dense_dm<RB, true, false, A, R>(xr, xi, dm, m, kc, act);
-    else dense_dm<RB, false, false, A, R>(xr, xi, dm, m, kc, act);
-  } else {
-    if (ls) dense_dm<RB, true, true, A, R>(xr, xi, dm, m, kc, act);
-    else dense_dm<RB, false, true, A, R>(xr, xi, dm, m, kc, act);
-  }
-}
-
-// Diagonal diag(d0, d1) on register bit RB (ONLY1: d0 == 1, slots with the bit
-// clear are left alone); KC: slots need their register-bit controls kc.
-template <int RB, bool ONLY1, bool KC, typename A, typename R>
-__device__ __forceinline__ void op_phase_reg(typename SV<R>::T& xr, typename SV<R>::T& xi, uint32_t kc, A d0r, A d0i, A d1r,
-                                             A d1i)
-{
-  each_slot([&](auto kk) __attribute__((always_inline)) {
-    constexpr int k = decltype(kk)::value;
-    if (KC && (k & kc) != kc) return;
-    if constexpr ((k >> RB) & 1) cmul_slot<k>(d1r, d1i, xr, xi);
-    else if constexpr (!ONLY1) cmul_slot<k>(d0r, d0i, xr, xi);
-  });
-}
-
-template <bool ONLY1, bool KC, typename A, typename R>
-__device__ __forceinline__ void phase_rb(typename SV<R>::T& xr, typename SV<R>::T& xi, int rb, uint32_t kc, A d0r, A d0i,
-                                         A d1r, A d1i)
-{
-  if (rb == 0) op_phase_reg<0, ONLY1, KC, A, R>(xr, xi, kc, d0r, d0i, d1r, d1i);
-  else if (rb == 1) op_phase_reg<1, ONLY1, KC, A, R>(xr, xi, kc, d0r, d0i, d1r, d1i);
-  else if (rb == 2) op_phase_reg<2, ONLY1, KC, A, R>(xr, xi, kc, d0r, d0i, d1r, d1i);
-  else op_phase_reg<3, ONLY1, KC, A, R>(xr, xi, kc, d0r, d0i, d1r, d1i);
+  o.code = p->code;
+  o.tmask = p->tmask;
+  o.kc = p->kc;
+  o.aux = p->aux;
+  o.cnt = p->cnt;
+  o.flag = p->flag;
+  const uint32_t* w = reinterpret_cast<const uint32_t*>(p->m);
+#pragma unroll
+  for (int i = 0; i < 16; ++i) o.w[i] = w[i];
 }
 
 // Fixed-order sum of v over the workgroup (valid in thread 0); red[] must
@@ -197,18 +101,6 @@ __device__ __forceinline__ double block_sum(double v, double* red)
   return s;
 }
 
-template <typename V>
-__device__ __forceinline__ double norm2_slots(const V& xr, const V& xi)
-{
-  double s = 0.0;
-  each_slot([&](auto kk) __attribute__((always_inline)) {
-    constexpr int k = decltype(kk)::value;
-    const double re = xr[k], im = xi[k];
-    s += re * re + im * im;
-  });
-  return s;
-}
-
 // Workgroup-scope LDS ordering, or wave-scope when only the wave's own
 // addresses are involved.
 __device__ __forceinline__ void lds_sync(bool wave_local)
@@ -221,48 +113,497 @@ __device__ __forceinline__ void lds_sync(bool wave_local)
   }
 }
 
-// A wave-uniform value pinned to scalar registers: a per-lane choice between
-// two uniform loads would otherwise become a per-lane (vector) load.
-__device__ __forceinline__ double uniform(double v)
-{
-  const int lo = __builtin_amdgcn_readfirstlane(__double2loint(v));
-  const int hi = __builtin_amdgcn_readfirstlane(__double2hiint(v));
-  return __hiloint2double(hi, lo);
-}
-__device__ __forceinline__ float uniform(float v) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v))); }
+// A thread's 16 slots: A re[16], im[16], indexed by constants only.
+template <typename A>
+struct Slots {
+  A re[kSlots], im[kSlots];
+};
 
-// Coefficient i of an op in the arithmetic type.
-template <typename A> __device__ __forceinline__ A coef(const POp& op, int i);
-template <> __device__ __forceinline__ double coef<double>(const POp& op, int i) { return op.m[i]; }
-template <> __device__ __forceinline__ float coef<float>(const POp& op, int i) { return op.f[i]; }
+// A uniform value as a per-lane one: conditions on it become selects. As uniform
+// branches around every slot they would cost the tile a second set of registers.
+__device__ __forceinline__ uint32_t per_lane(uint32_t v)
+{
+  uint32_t r;
+  asm("v_mov_b32 %0, %1" : "=v"(r) : "s"(v));
+  return r;
+}
+
+// A real 2x2 applied to (a, b) in place: one temporary, no moves.
+template <typename A>
+__device__ __forceinline__ void real2(A m0, A m1, A m2, A m3, A& a, A& b)
+{
+  const A t = m2 * a;
+  a = m0 * a;
+  a = mad(m1, b, a);
+  b = mad(m3, b, t);
+}
+
+// (re, im) *= (dr, di) in place.
+template <typename A>
+__device__ __forceinline__ void cmul(A dr, A di, A& re, A& im)
+{
+  const A t = di * re;
+  re = dr * re;
+  re = mad(-di, im, re);
+  im = mad(dr, im, t);
+}
+
+// A general 2x2 applied to (a, b) in place, in the order that lets each value
+// be overwritten as soon as its last use is done.
+template <typename A>
+__device__ __forceinline__ void general2(const A (&m)[8], A& ar, A& ai, A& br, A& bi)
+{
+  const A xr = mad(-m[5], ai, m[4] * ar), xi = mad(m[5], ar, m[4] * ai);
+  const A u = m[1] * ar;
+  ar = m[0] * ar;
+  ar = mad(-m[1], ai, ar);
+  ai = mad(m[0], ai, u);
+  ar = mad(m[2], br, ar);
+  ar = mad(-m[3], bi, ar);
+  ai = mad(m[2], bi, ai);
+  ai = mad(m[3], br, ai);
+  const A w = mad(m[7], br, xi);
+  br = mad(m[6], br, xr);
+  br = mad(-m[7], bi, br);
+  bi = mad(m[6], bi, w);
+  __builtin_amdgcn_sched_barrier(0);   // one pair at a time: the scheduler would keep the temporaries of all eight
+}
+
+// XOR of the columns of t's set bits; cols(j) for j < NT.
+template <int NT, typename F>
+__device__ __forceinline__ uint32_t thread_part(uint32_t t, F&& cols)
+{
+  uint32_t b = 0;
+  each<0, NT>([&](auto jj) __attribute__((always_inline)) {
+    constexpr int j = decltype(jj)::value;
+    b ^= (uint32_t)((int32_t)(t << (31 - j)) >> 31) & cols(j);
+  });
+  return b;
+}
+
+// XOR of the slot columns of k's set bits: uniform, by scalar instructions.
+template <int K, typename F>
+__device__ __forceinline__ uint32_t slot_part(F&& cols)
+{
+  uint32_t b = 0;
+  if constexpr (K & 1) b ^= cols(0);
+  if constexpr (K & 2) b ^= cols(1);
+  if constexpr (K & 4) b ^= cols(2);
+  if constexpr (K & 8) b ^= cols(3);
+  return b;
+}
+
+// Runs the ops of a program on a workgroup's tile of 2^(NT + 4) amplitudes.
+// smem: 8 bytes per amplitude.
+template <typename A, int NT>
+__device__ __forceinline__ void run_ops(const char* __restrict__ prog, char* smem, Slots<A>& x)
+{
+  constexpr bool SPLIT = sizeof(A) == 8;
+  typedef A P2 __attribute__((ext_vector_type(2)));
+  const uint32_t t = threadIdx.x;
+  const PHead& h = *reinterpret_cast<const PHead*>(prog);
+  const POp* ops = reinterpret_cast<const POp*>(prog + sizeof(PHead));
+  const int nops = h.nops;
+  auto at = [&](uint32_t e) __attribute__((always_inline)) -> A* { return reinterpret_cast<A*>(smem + e); };
+  auto at2 = [&](uint32_t e) __attribute__((always_inline)) -> P2* { return reinterpret_cast<P2*>(smem + e); };
+  uint32_t lb = 0;   // byte offset of this thread's part in the layout of the last relayout
+  OpRegs<A> nx;
+  fetch(nx, ops);   // (there is at least the unread one)
+  // no fetch is pending when the loop starts: the wait for the next op then
+  // stands at the end of the loop, behind the current op's work
+  asm volatile("" ::"s"(nx.code), "s"(nx.cnt), "s"(nx.w[0]), "s"(nx.w[15]));
+  for (int i = 0; i < nops; ++i) {
+    const OpRegs<A> op = nx;
+    fetch(nx, ops + i + 1);   // the program ends with one unread op
+    const int code = op.code;
+    // One flat dispatch whose cases share no code: a case that is merged with
+    // another in part makes the compiler keep a second copy of the tile.
+    auto dense = [&](auto rbc, auto dmc) __attribute__((always_inline)) {
+      constexpr int rb = decltype(rbc)::value, dm = decltype(dmc)::value, d = 1 << rb;
+      asm volatile("; dense %0 %1" ::"i"(rb), "i"(dm));
+      const bool act = (t & op.tmask) == op.tmask;
+      if constexpr (dm == PM_EXCHANGE) {
+        each<0, kSlots>([&](auto kk) __attribute__((always_inline)) {
+          constexpr int k = decltype(kk)::value;
+          if constexpr (!(k & d)) {
+            const A ar = x.re[k], ai = x.im[k], br = x.re[k | d], bi = x.im[k | d];
+            x.re[k] = act ? br : ar;
+            x.im[k] = act ? bi : ai;
+            x.re[k | d] = act ? ar : br;
+            x.im[k | d] = act ? ai : bi;
+          }
+        });
+      } else if constexpr (dm == PM_REAL) {
+        const A m0 = act ? op.m(0) : (A)1, m1 = act ? op.m(2) : (A)0;
+        const A m2 = act ? op.m(4) : (A)0, m3 = act ? op.m(6) : (A)1;
+        each<0, kSlots>([&](auto kk) __attribute__((always_inline)) {
+          constexpr int k = decltype(kk)::value;
+          if constexpr (!(k & d)) {
+            real2(m0, m1, m2, m3, x.re[k], x.re[k | d]);
+            real2(m0, m1, m2, m3, x.im[k], x.im[k | d]);
+          }
+        });
+      } else if constexpr (dm == PM_RX) {
+        // real diagonal, imaginary off-diagonal i m3, i m5: a real 2x2 on
+        // (a.re, b.im) and one of the other signs on (a.im, b.re)
+        const A m0 = act ? op.m(0) : (A)1, m3 = act ? op.m(3) : (A)0;
+        const A m5 = act ? op.m(5) : (A)0, m6 = act ? op.m(6) : (A)1;
+        each<0, kSlots>([&](auto kk) __attribute__((always_inline)) {
+          constexpr int k = decltype(kk)::value;
+          if constexpr (!(k & d)) {
+            real2(m0, -m3, m5, m6, x.re[k], x.im[k | d]);
+            real2(m0, m3, -m5, m6, x.im[k], x.re[k | d]);
+          }
+        });
+      } else {
+        const uint32_t kc = per_lane(op.kc);
+        A m[8];
+        each<0, 8>([&](auto ii) __attribute__((always_inline)) {
+          constexpr int e = decltype(ii)::value;
+          m[e] = act ? op.m(e) : (A)(e == 0 || e == 6 ? 1 : 0);
+        });
+        each<0, kSlots>([&](auto kk) __attribute__((always_inline)) {
+          constexpr int k = decltype(kk)::value;
+          if constexpr (!(k & d)) {
+            if constexpr (dm == PM_GENERAL) {
+              general2(m, x.re[k], x.im[k], x.re[k | d], x.im[k | d]);
+            } else {   // PO_DENSE_K: only the pairs whose slot controls are set
+              A ar = x.re[k], ai = x.im[k], br = x.re[k | d], bi = x.im[k | d];
+              general2(m, ar, ai, br, bi);
+              const bool in = ((uint32_t)k & kc) == kc;
+              x.re[k] = in ? ar : x.re[k];
+              x.im[k] = in ? ai : x.im[k];
+              x.re[k | d] = in ? br : x.re[k | d];
+              x.im[k | d] = in ? bi : x.im[k | d];
+            }
+          }
+        });
+      }
+      asm volatile("; end %0 %1" ::"i"(rb), "i"(dm));
+    };
+    // diagonal on a register bit of an FP32 pass: one factor per lane for the
+    // clear bit, one for the set bit
+    auto phase2 = [&](auto rbc) __attribute__((always_inline)) {
+      if constexpr (!SPLIT) {
+        constexpr int rb = decltype(rbc)::value;
+        A gr = op.m(0), gi = op.m(1), fr = op.m(6), fi = op.m(7);
+        const PTerm* tm = reinterpret_cast<const PTerm*>(prog + op.aux);
+        for (int j = 0; j < op.cnt; ++j) {
+          const PTerm& q = tm[j];
+          const bool on = (t & q.tmask) == q.tmask;
+          cmul(on ? q.f[0] : (A)1, on ? q.f[1] : (A)0, fr, fi);
+          cmul(on ? q.f[2] : (A)1, on ? q.f[3] : (A)0, gr, gi);
+        }
+        asm volatile("; phase2 %0" ::"i"(rb));
+        const uint32_t kc = per_lane(op.kc);
+        each<0, kSlots>([&](auto kk) __attribute__((always_inline)) {
+          constexpr int k = decltype(kk)::value;
+          const bool in = ((uint32_t)k & kc) == kc;
+          cmul(in ? ((k >> rb) & 1 ? fr : gr) : (A)1, in ? ((k >> rb) & 1 ? fi : gi) : (A)0, x.re[k], x.im[k]);
+        });
+        asm volatile("; end %0" ::"i"(rb));
+      }
+    };
+#define QSV_DENSE(RB)                                                                            \
+  case PO_DENSE + 4 * RB + PM_GENERAL: dense(Int<RB>{}, Int<PM_GENERAL>{}); break;               \
+  case PO_DENSE + 4 * RB + PM_REAL: dense(Int<RB>{}, Int<PM_REAL>{}); break;                     \
+  case PO_DENSE + 4 * RB + PM_RX: dense(Int<RB>{}, Int<PM_RX>{}); break;                         \
+  case PO_DENSE + 4 * RB + PM_EXCHANGE: dense(Int<RB>{}, Int<PM_EXCHANGE>{}); break;             \
+  case PO_DENSE_K + RB: dense(Int<RB>{}, Int<4>{}); break
+    switch (code) {
+    QSV_DENSE(0);
+    QSV_DENSE(1);
+    QSV_DENSE(2);
+    QSV_DENSE(3);
+#undef QSV_DENSE
+    case PO_PHASE: {
+      // one factor per lane: the uniform part times the terms of the lane's set bits
+      A fr = op.m(0), fi = op.m(1);
+      const PTerm* tm = reinterpret_cast<const PTerm*>(prog + op.aux);
+      for (int j = 0; j < op.cnt; ++j) {
+        const PTerm& q = tm[j];
+        const bool on = (t & q.tmask) == q.tmask;
+        if constexpr (SPLIT) {
+          cmul(on ? (A)q.d[0] : (A)1, on ? (A)q.d[1] : (A)0, fr, fi);
+        } else {
+          const bool set = (t & q.tbit) == q.tbit;
+          const A qr = set ? q.f[0] : q.f[2], qi = set ? q.f[1] : q.f[3];
+          cmul(on ? qr : (A)1, on ? qi : (A)0, fr, fi);
+        }
+      }
+      auto all_with = [&](auto mask) __attribute__((always_inline)) {
+        each<0, kSlots>([&](auto kk) __attribute__((always_inline)) {
+          constexpr int k = decltype(kk)::value;
+          if constexpr ((k & decltype(mask)::value) == decltype(mask)::value) cmul(fr, fi, x.re[k], x.im[k]);
+        });
+      };
+      const uint32_t kc = op.kc;
+      if (kc == 0) all_with(std::integral_constant<int, 0>{});
+      else if (kc == 1) all_with(std::integral_constant<int, 1>{});
+      else if (kc == 2) all_with(std::integral_constant<int, 2>{});
+      else if (kc == 4) all_with(std::integral_constant<int, 4>{});
+      else if (kc == 8) all_with(std::integral_constant<int, 8>{});
+      else {
+        const uint32_t kv = per_lane(kc);
+        each<0, kSlots>([&](auto kk) __attribute__((always_inline)) {
+          constexpr int k = decltype(kk)::value;
+          const bool in = ((uint32_t)k & kv) == kv;
+          cmul(in ? fr : (A)1, in ? fi : (A)0, x.re[k], x.im[k]);
+        });
+      }
+      break;
+    }
+#define QSV_PHASE2(RB)                                                                           \
+  case PO_PHASE2 + RB: phase2(Int<RB>{}); break
+    QSV_PHASE2(0);
+    QSV_PHASE2(1);
+    QSV_PHASE2(2);
+    QSV_PHASE2(3);
+#undef QSV_PHASE2
+    case PO_RELAYOUT: {
+      const bool local = (op.flag & PR_LOCAL) != 0;
+      if (op.flag & PR_WAIT) __syncthreads();
+      const uint32_t fb = (op.flag & PR_SAME)
+                              ? lb
+                              : thread_part<NT>(t, [&](int j) __attribute__((always_inline)) { return op.col(j); }) << 3;
+      lb = thread_part<NT>(t, [&](int j) __attribute__((always_inline)) { return op.col(kCols + j); }) << 3;
+      auto from = [&](auto kk) __attribute__((always_inline)) {
+        return slot_part<decltype(kk)::value>(
+            [&](int j) __attribute__((always_inline)) { return op.col(kColT + j) << 3; });
+      };
+      auto to = [&](auto kk) __attribute__((always_inline)) {
+        return slot_part<decltype(kk)::value>(
+            [&](int j) __attribute__((always_inline)) { return op.col(kCols + kColT + j) << 3; });
+      };
+      if constexpr (SPLIT) {
+        each<0, kSlots>([&](auto kk) __attribute__((always_inline)) { *at(fb ^ from(kk)) = x.re[decltype(kk)::value]; });
+        lds_sync(local);
+        each<0, kSlots>([&](auto kk) __attribute__((always_inline)) { x.re[decltype(kk)::value] = *at(lb ^ to(kk)); });
+        lds_sync(local);
+        each<0, kSlots>([&](auto kk) __attribute__((always_inline)) { *at(fb ^ from(kk)) = x.im[decltype(kk)::value]; });
+        lds_sync(local);
+        each<0, kSlots>([&](auto kk) __attribute__((always_inline)) { x.im[decltype(kk)::value] = *at(lb ^ to(kk)); });
+      } else {
+        each<0, kSlots>([&](auto kk) __attribute__((always_inline)) {
+          constexpr int k = decltype(kk)::value;
+          P2 v;
+          v.x = x.re[k];
+          v.y = x.im[k];
+          *at2(fb ^ from(kk)) = v;
+        });
+        lds_sync(local);
+        each<0, kSlots>([&](auto kk) __attribute__((always_inline)) {
+          constexpr int k = decltype(kk)::value;
+          const P2 v = *at2(lb ^ to(kk));
+          x.re[k] = v.x;
+          x.im[k] = v.y;
+        });
+      }
+      // nothing may move above the reads of this wave's next writes
+      lds_sync(true);
+      break;
+    }
+    case PO_BLOCKADE: {
+      // phase where exactly one blockade bit is set: thread part popcount(t &
+      // aux), register part popcount(k & kc)
+      const uint32_t pt = __popc(t & op.aux);
+      const A pr = op.m(0), pi = op.m(1);
+      each<0, kSlots>([&](auto kk) __attribute__((always_inline)) {
+        constexpr int k = decltype(kk)::value;
+        const bool on = pt + (uint32_t)__builtin_popcount((uint32_t)k & op.kc) == 1u;
+        cmul(on ? pr : (A)1, on ? pi : (A)0, x.re[k], x.im[k]);
+      });
+      break;
+    }
+    case PO_SWAP: {
+      // exchange local bits a = kc, b = aux (times the phase) where the local
+      // control bits tmask are set: every thread writes its slots to permuted
+      // LDS addresses and reads its own back
+      __syncthreads();
+      const uint32_t tl = thread_part<NT>(t, [&](int j) __attribute__((always_inline)) { return op.col(j); });
+      const POp& full = ops[i];
+      const A pr = (A)full.sc[0], pi = (A)full.sc[1];
+      const uint32_t ba = 1u << op.kc, bb = 1u << op.aux, tmk = op.tmask;
+      auto swz = [](uint32_t l) { return l ^ (((l >> 4) ^ (l >> 8)) & 15u); };   // its own inverse
+      auto own = [&](auto kk) __attribute__((always_inline)) {
+        return tl ^ slot_part<decltype(kk)::value>(
+                        [&](int j) __attribute__((always_inline)) { return op.col(kColT + j); });
+      };
+      auto moves = [&](uint32_t e) __attribute__((always_inline)) -> bool {
+        const uint32_t l = swz(e);
+        return ((l & tmk) == tmk) && (((l & ba) != 0) != ((l & bb) != 0));
+      };
+      const uint32_t dsw = swz(ba ^ bb);
+      each<0, kSlots>([&](auto kk) __attribute__((always_inline)) {
+        constexpr int k = decltype(kk)::value;
+        const bool mv = moves(own(kk));
+        cmul(mv ? pr : (A)1, mv ? pi : (A)0, x.re[k], x.im[k]);
+      });
+      each<0, 2>([&](auto cc) __attribute__((always_inline)) {
+        constexpr int c = decltype(cc)::value;
+        if constexpr (SPLIT || c == 0) {
+          each<0, kSlots>([&](auto kk) __attribute__((always_inline)) {
+            constexpr int k = decltype(kk)::value;
+            const uint32_t e = own(kk), to = (e ^ (moves(e) ? dsw : 0u)) << 3;
+            if constexpr (SPLIT) {
+              *at(to) = c ? x.im[k] : x.re[k];
+            } else {
+              P2 v;
+              v.x = x.re[k];
+              v.y = x.im[k];
+              *at2(to) = v;
+            }
+          });
+          __syncthreads();
+          each<0, kSlots>([&](auto kk) __attribute__((always_inline)) {
+            constexpr int k = decltype(kk)::value;
+            const uint32_t e = own(kk) << 3;
+            if constexpr (SPLIT) {
+              (c ? x.im[k] : x.re[k]) = *at(e);
+            } else {
+              const P2 v = *at2(e);
+              x.re[k] = v.x;
+              x.im[k] = v.y;
+            }
+          });
+          __syncthreads();
+        }
+      });
+      break;
+    }
+    default: {
+      // PO_BLOCK (FP32 arithmetic): Y = U X for the wave's 16 x 64 matrix X
+      // (row = slot, column = lane) on the matrix cores, as four column blocks
+      // of 16 lanes, 12 v_mfma_f32_16x16x4f32 each (three real products per
+      // complex one). X crosses LDS at the addresses of the stage's layout, the
+      // wave's own, so the round trip is wave-local. The offsets are XOR-linear
+      // in the thread and slot bits: lane 16 cb + jc's slot s sits at
+      // (wave part ^ jc part ^ cb part) ^ ls[s].
+      if constexpr (!SPLIT) {
+        typedef float f4 __attribute__((ext_vector_type(4)));
+        const uint32_t l = t & 63u, kr = l >> 4, jc = l & 15u;
+        const float2* tab = reinterpret_cast<const float2*>(prog + op.aux);
+        float ur[4], ui[4], us[4];
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) {
+          const float2 u = tab[kk * 64 + l];
+          ur[kk] = u.x;
+          ui[kk] = u.y;
+          us[kk] = u.x + u.y;
+        }
+        auto tcol = [&](int j) __attribute__((always_inline)) { return op.col(j) << 3; };
+        auto scol = [&](int j) __attribute__((always_inline)) { return op.col(kColT + j) << 3; };
+        const uint32_t fb = thread_part<NT>(t, tcol);
+        each<0, kSlots>([&](auto kk) __attribute__((always_inline)) {
+          constexpr int k = decltype(kk)::value;
+          P2 v;
+          v.x = x.re[k];
+          v.y = x.im[k];
+          *at2(fb ^ slot_part<k>(scol)) = v;
+        });
+        lds_sync(true);
+        const uint32_t pj = thread_part<NT>((t & ~63u) | jc, tcol);
+        const uint32_t rin = (kr & 1u ? scol(0) : 0u) ^ (kr & 2u ? scol(1) : 0u);    // B rows 4 kk + kr
+        const uint32_t rout = (kr & 1u ? scol(2) : 0u) ^ (kr & 2u ? scol(3) : 0u);   // C rows 4 kr + e
+        each<0, 4>([&](auto cbc) __attribute__((always_inline)) {
+          constexpr int cb = decltype(cbc)::value;
+          const uint32_t pb = pj ^ (cb & 1 ? tcol(4) : 0u) ^ (cb & 2 ? tcol(5) : 0u);
+          float br[4], bi[4];
+          each<0, 4>([&](auto kc) __attribute__((always_inline)) {
+            constexpr int kk = decltype(kc)::value;
+            const P2 v = *at2(pb ^ rin ^ slot_part<4 * kk>(scol));
+            br[kk] = v.x;
+            bi[kk] = v.y;
+          });
+          // three real products (Gauss): P1 = Ur Xr, P2 = Ui Xi,
+          // P3 = (Ur + Ui)(Xr + Xi); Y = (P1 - P2) + i (P3 - P1 - P2)
+          f4 p1 = {0.f, 0.f, 0.f, 0.f}, p2 = {0.f, 0.f, 0.f, 0.f}, p3 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int kk = 0; kk < 4; ++kk) {
+            p1 = __builtin_amdgcn_mfma_f32_16x16x4f32(ur[kk], br[kk], p1, 0, 0, 0);
+            p2 = __builtin_amdgcn_mfma_f32_16x16x4f32(ui[kk], bi[kk], p2, 0, 0, 0);
+            p3 = __builtin_amdgcn_mfma_f32_16x16x4f32(us[kk], br[kk] + bi[kk], p3, 0, 0, 0);
+          }
+          // element e of lane l is row 4 (l / 16) + e, column l % 16 of the block
+          each<0, 4>([&](auto ec) __attribute__((always_inline)) {
+            constexpr int e = decltype(ec)::value;
+            P2 v;
+            v.x = p1[e] - p2[e];
+            v.y = p3[e] - p1[e] - p2[e];
+            *at2(pb ^ rout ^ slot_part<e>(scol)) = v;
+          });
+        });
+        lds_sync(true);
+        each<0, kSlots>([&](auto kk) __attribute__((always_inline)) {
+          constexpr int k = decltype(kk)::value;
+          const P2 v = *at2(fb ^ slot_part<k>(scol));
+          x.re[k] = v.x;
+          x.im[k] = v.y;
+        });
+        lds_sync(true);
+      }
+      break;
+    }
+    }
+  }
+}
+
+template <typename A>
+__device__ __forceinline__ double norm2_slots(const Slots<A>& x)
+{
+  double s = 0.0;
+  each<0, kSlots>([&](auto kk) __attribute__((always_inline)) {
+    constexpr int k = decltype(kk)::value;
+    const double re = x.re[k], im = x.im[k];
+    s += re * re + im * im;
+  });
+  return s;
+}
+
+// Global element offsets of this thread's part for the columns c[0..NT).
+template <int NT>
+__device__ __forceinline__ uint64_t global_part(uint32_t t, const uint64_t* c)
+{
+  uint64_t g = 0;
+  each<0, NT>([&](auto jj) __attribute__((always_inline)) {
+    constexpr int j = decltype(jj)::value;
+    g ^= ((t >> j) & 1u) ? c[j] : 0ull;
+  });
+  return g;
+}
+template <int K>
+__device__ __forceinline__ uint64_t global_slot(const uint64_t* c)
+{
+  uint64_t g = 0;
+  if constexpr (K & 1) g ^= c[kColT + 0];
+  if constexpr (K & 2) g ^= c[kColT + 1];
+  if constexpr (K & 4) g ^= c[kColT + 2];
+  if constexpr (K & 8) g ^= c[kColT + 3];
+  return g;
+}
 
 }  // namespace
 
 // One tile of one pass per workgroup. GROUP: many states of S amplitudes back
 // to back; instance blockIdx.y runs the program at byte offset offs[y] of
-// `prog` (negative: no pass this round); group passes do not renormalise.
+// `progs` (negative: no pass this round); group passes do not renormalise.
 template <typename R, typename A, bool GROUP>
-__global__ __launch_bounds__(kThreads, sizeof(A) == 4 ? 5 : sizeof(R) == 4 ? 4 : 3) void k_pass(typename PV<R>::T* __restrict__ psi,
-                                                                           const PProg* __restrict__ prog,
+__global__ __launch_bounds__(kThreads, sizeof(A) == 4 ? 5 : 4) void k_pass(typename PV<R>::T* __restrict__ psi,
+                                                                           const char* __restrict__ progs,
                                                                            TileNorm nb, uint64_t S,
                                                                            const int64_t* __restrict__ offs)
 {
   using T = typename PV<R>::T;
-  constexpr int TB = kPassTileBits;
-  constexpr uint32_t FULL = (1u << TB) - 1u;
-  // complex128 tiles cross LDS one FP64 plane at a time; complex64 tiles as
-  // (re, im) pairs
-  constexpr bool SPLIT = sizeof(T) == 16;
-  constexpr uint32_t E = SPLIT ? sizeof(R) : sizeof(T);
-  // the tile's LDS; also the per-wave partial sums of the norm reductions,
-  // which run when no relayout is in flight
-  __shared__ __align__(16) char smem[E << TB];
+  constexpr int TB = kPassTileBits, NT = TB - 4;
+  // the tile's LDS; also the per-wave partial sums of the norm reductions
+  __shared__ __align__(16) char smem[8u << TB];
   double* red = reinterpret_cast<double*>(smem);
+  const char* prog = progs;
   if constexpr (GROUP) {
     const int64_t off = offs[blockIdx.y];
     if (off < 0) return;
     psi += (uint64_t)blockIdx.y * S;
-    prog = reinterpret_cast<const PProg*>(reinterpret_cast<const char*>(prog) + off);
+    prog += off;
   }
   // The dispatcher hands consecutive workgroups to the 8 XCDs in turn: map
   // them so that each XCD streams one contiguous eighth of the tiles (its own
@@ -270,344 +611,75 @@ __global__ __launch_bounds__(kThreads, sizeof(A) == 4 ? 5 : sizeof(R) == 4 ? 4 :
   const uint32_t g = gridDim.x, b = blockIdx.x;
   const uint32_t tile = (g & 7u) ? b : (b & 7u) * (g >> 3) + (b >> 3);
   const uint32_t t = threadIdx.x;
-  const PHead& h = prog->h;
-  const PLayout* lays = reinterpret_cast<const PLayout*>(reinterpret_cast<const char*>(prog) + h.lay_off);
+  const PHead& h = *reinterpret_cast<const PHead*>(prog);
 
   // tile base: zeros inserted at the tile's global bits (ascending)
   uint64_t base = tile;
+#pragma unroll
   for (int i = 0; i < TB; ++i) {
     const int p = h.sorted_pos[i];
     const uint64_t lo = base & ((1ull << p) - 1ull);
     base = ((base ^ lo) << 1) | lo;
   }
 
-  static_assert(E == 8, "the host resolves LDS offsets for 8-byte elements");
-  uint32_t reg = h.load_mask;   // register mask of the current layout
-  int cur = h.load_lay;         // its descriptor
-  // per-thread parts of a layout's offsets (the slot parts are uniform)
-  auto lds_base = [&](const PLayout& L) __attribute__((always_inline)) -> uint32_t {
-    uint32_t b = 0;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) b ^= ((t >> j) & 1u) ? L.lt[j] : 0u;
-    return b;
-  };
-  auto gaddr = [&](const PLayout& L, uint64_t (&ga)[kSlots]) __attribute__((always_inline)) {
-    uint64_t g = base;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) g |= ((t >> j) & 1u) ? L.gt[j] : 0ull;
-    each_slot([&](auto kk) __attribute__((always_inline)) {
-      constexpr int k = decltype(kk)::value;
-      ga[k] = g | L.gs[k];
-    });
-  };
-  auto st_r = [&](uint32_t off, R v) __attribute__((always_inline)) { *reinterpret_cast<R*>(smem + off) = v; };
-  auto ld_r = [&](uint32_t off) __attribute__((always_inline)) -> R { return *reinterpret_cast<const R*>(smem + off); };
-  auto st_c = [&](uint32_t off, R re, R im) __attribute__((always_inline)) {
-    T v;
-    v.x = re;
-    v.y = im;
-    *reinterpret_cast<T*>(smem + off) = v;
-  };
-  auto ld_c = [&](uint32_t off) __attribute__((always_inline)) -> T { return *reinterpret_cast<const T*>(smem + off); };
-
-  typename SV<R>::T xr, xi;
-  bool local_pending = false;   // a wave-local LDS round trip may still be read by its wave
-  // Move the tile from layout lay[from] to lay[to] through LDS; wave_local:
-  // no workgroup barrier.
-  auto relayout = [&](int from, int to, bool wave_local) __attribute__((always_inline)) {
-    if (!wave_local && local_pending) __syncthreads();
-    const PLayout& F = lays[from];
-    const PLayout& G = lays[to];
-    const uint32_t fb = lds_base(F), bb = lds_base(G);
-    if constexpr (SPLIT) {
-      each_slot([&](auto kk) __attribute__((always_inline)) {
-        constexpr int k = decltype(kk)::value;
-        st_r(fb ^ F.ls[k], xr[k]);
-      });
-      lds_sync(wave_local);
-      each_slot([&](auto kk) __attribute__((always_inline)) {
-        constexpr int k = decltype(kk)::value;
-        xr[k] = ld_r(bb ^ G.ls[k]);
-      });
-      lds_sync(wave_local);
-      each_slot([&](auto kk) __attribute__((always_inline)) {
-        constexpr int k = decltype(kk)::value;
-        st_r(fb ^ F.ls[k], xi[k]);
-      });
-      lds_sync(wave_local);
-      each_slot([&](auto kk) __attribute__((always_inline)) {
-        constexpr int k = decltype(kk)::value;
-        xi[k] = ld_r(bb ^ G.ls[k]);
-      });
-      lds_sync(wave_local);
-    } else {
-      each_slot([&](auto kk) __attribute__((always_inline)) {
-        constexpr int k = decltype(kk)::value;
-        st_c(fb ^ F.ls[k], xr[k], xi[k]);
-      });
-      lds_sync(wave_local);
-      each_slot([&](auto kk) __attribute__((always_inline)) {
-        constexpr int k = decltype(kk)::value;
-        { const T v = ld_c(bb ^ G.ls[k]); xr[k] = v.x; xi[k] = v.y; }
-      });
-      lds_sync(wave_local);
-    }
-    local_pending = wave_local;
-  };
-  // PO_SWAP: exchange local bits a = kc, b = aux (times the phase m[0..1])
-  // where the local control bits tmask are set: every thread writes its slots
-  // to permuted LDS addresses and reads its own back.
-  auto swap_op = [&](const POp& op) __attribute__((always_inline)) {
-    if (local_pending) __syncthreads();
-    const uint32_t tm = op.tmask;
-    const uint32_t ba = 1u << op.kc, bb = 1u << op.aux;
-    const A pr = coef<A>(op, 0), pi = coef<A>(op, 1);
-    const PLayout& L = lays[cur];
-    const uint32_t sb = lds_base(L), dsw = swz(ba ^ bb) * E;
-    // local index of each slot, from the register mask (swaps are rare)
-    const uint32_t tl = pdep32(t, FULL & ~reg);
-    uint32_t m = reg;
-    const uint32_t q0 = m & (~m + 1u); m &= m - 1;
-    const uint32_t q1 = m & (~m + 1u); m &= m - 1;
-    const uint32_t q2 = m & (~m + 1u); m &= m - 1;
-    const uint32_t q3 = m & (~m + 1u);
-    auto moves = [&](int k) __attribute__((always_inline)) -> bool {
-      const uint32_t l = tl | ((k & 1) ? q0 : 0u) | ((k & 2) ? q1 : 0u) | ((k & 4) ? q2 : 0u) | ((k & 8) ? q3 : 0u);
-      return ((l & tm) == tm) && (((l & ba) != 0) != ((l & bb) != 0));
-    };
-    each_slot([&](auto kk) __attribute__((always_inline)) {
-      constexpr int k = decltype(kk)::value;
-      const bool mv = moves(k);
-      const A ax = xr[k], ay = xi[k];
-      const R yr = (R)(pr * ax - pi * ay), yi = (R)(pr * ay + pi * ax);
-      xr[k] = mv ? yr : xr[k];
-      xi[k] = mv ? yi : xi[k];
-    });
-    if constexpr (SPLIT) {
-      each_slot([&](auto kk) __attribute__((always_inline)) {
-        constexpr int k = decltype(kk)::value;
-        st_r(sb ^ L.ls[k] ^ (moves(k) ? dsw : 0u), xr[k]);
-      });
-      __syncthreads();
-      each_slot([&](auto kk) __attribute__((always_inline)) {
-        constexpr int k = decltype(kk)::value;
-        xr[k] = ld_r(sb ^ L.ls[k]);
-      });
-      __syncthreads();
-      each_slot([&](auto kk) __attribute__((always_inline)) {
-        constexpr int k = decltype(kk)::value;
-        st_r(sb ^ L.ls[k] ^ (moves(k) ? dsw : 0u), xi[k]);
-      });
-      __syncthreads();
-      each_slot([&](auto kk) __attribute__((always_inline)) {
-        constexpr int k = decltype(kk)::value;
-        xi[k] = ld_r(sb ^ L.ls[k]);
-      });
-      __syncthreads();
-    } else {
-      each_slot([&](auto kk) __attribute__((always_inline)) {
-        constexpr int k = decltype(kk)::value;
-        st_c(sb ^ L.ls[k] ^ (moves(k) ? dsw : 0u), xr[k], xi[k]);
-      });
-      __syncthreads();
-      each_slot([&](auto kk) __attribute__((always_inline)) {
-        constexpr int k = decltype(kk)::value;
-        { const T v = ld_c(sb ^ L.ls[k]); xr[k] = v.x; xi[k] = v.y; }
-      });
-      __syncthreads();
-    }
-    local_pending = false;
-  };
-
-  // PO_BLOCK (FP32 arithmetic, complex64 tiles): Y = U X for the wave's
-  // 16 x 64 matrix X (row = slot, column = lane) on the matrix cores, as four
-  // column blocks of 16 lanes, 12 v_mfma_f32_16x16x4f32 each (three real
-  // products per complex one). X crosses LDS at the current layout's own addresses of
-  // the wave's amplitudes, so the round trip is wave-local. The offsets are
-  // XOR-linear in the thread and slot bits: lane 16 cb + jc's slot s sits at
-  // (wave part ^ jc part ^ cb part) ^ ls[s], and ls[4 a + b] = ls[4 a] ^ ls[b].
-  auto block_op = [&](const POp& op) __attribute__((always_inline)) {
-    if constexpr (sizeof(A) == 4 && !SPLIT) {
-      typedef float f4 __attribute__((ext_vector_type(4)));
-      const uint32_t l = t & 63u, kr = l >> 4, jc = l & 15u;
-      const float2* tab = reinterpret_cast<const float2*>(reinterpret_cast<const char*>(prog) + op.aux);
-      float ur[4], ui[4], us[4];
-#pragma unroll
-      for (int kk = 0; kk < 4; ++kk) {
-        const float2 u = tab[kk * 64 + l];
-        ur[kk] = u.x;
-        ui[kk] = u.y;
-        us[kk] = u.x + u.y;
-      }
-      const PLayout& L = lays[cur];
-      const uint32_t fb = lds_base(L);
-      each_slot([&](auto kk) __attribute__((always_inline)) {
-        constexpr int k = decltype(kk)::value;
-        st_c(fb ^ L.ls[k], xr[k], xi[k]);
-      });
-      lds_sync(true);
-      uint32_t pj = ((t >> 6) & 1u ? L.lt[6] : 0u) ^ ((t >> 7) & 1u ? L.lt[7] : 0u);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) pj ^= (jc >> j) & 1u ? L.lt[j] : 0u;
-      const uint32_t rin = (kr & 1u ? L.ls[1] : 0u) ^ (kr & 2u ? L.ls[2] : 0u);    // B rows 4 kk + kr
-      const uint32_t rout = (kr & 1u ? L.ls[4] : 0u) ^ (kr & 2u ? L.ls[8] : 0u);   // C rows 4 kr + e
-#pragma unroll
-      for (int cb = 0; cb < 4; ++cb) {
-        const uint32_t pb = pj ^ (cb & 1 ? L.lt[4] : 0u) ^ (cb & 2 ? L.lt[5] : 0u);
-        float br[4], bi[4];
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk) {
-          const T v = ld_c(pb ^ rin ^ L.ls[4 * kk]);
-          br[kk] = v.x;
-          bi[kk] = v.y;
-        }
-        // three real products (Gauss): P1 = Ur Xr, P2 = Ui Xi,
-        // P3 = (Ur + Ui)(Xr + Xi); Y = (P1 - P2) + i (P3 - P1 - P2)
-        f4 p1 = {0.f, 0.f, 0.f, 0.f}, p2 = {0.f, 0.f, 0.f, 0.f}, p3 = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk) {
-          p1 = __builtin_amdgcn_mfma_f32_16x16x4f32(ur[kk], br[kk], p1, 0, 0, 0);
-          p2 = __builtin_amdgcn_mfma_f32_16x16x4f32(ui[kk], bi[kk], p2, 0, 0, 0);
-          p3 = __builtin_amdgcn_mfma_f32_16x16x4f32(us[kk], br[kk] + bi[kk], p3, 0, 0, 0);
-        }
-        // element e of lane l is row 4 (l / 16) + e, column l % 16 of the block
-#pragma unroll
-        for (int e = 0; e < 4; ++e) st_c(pb ^ rout ^ L.ls[e], p1[e] - p2[e], p3[e] - p1[e] - p2[e]);
-      }
-      lds_sync(true);
-      each_slot([&](auto kk) __attribute__((always_inline)) {
-        constexpr int k = decltype(kk)::value;
-        const T v = ld_c(fb ^ L.ls[k]);
-        xr[k] = v.x;
-        xi[k] = v.y;
-      });
-      local_pending = true;
-    }
-  };
-
+  Slots<A> x;
   const int rn = h.renorm;
   {
-    uint64_t ga[kSlots];
-    gaddr(lays[cur], ga);
+    const uint64_t ga = base ^ global_part<NT>(t, h.gload);
     if (rn & FP_INIT_ZERO) {
       // |0..0>: amplitude 1 at global index 0, nothing read
-      each_slot([&](auto kk) __attribute__((always_inline)) {
+      each<0, kSlots>([&](auto kk) __attribute__((always_inline)) {
         constexpr int k = decltype(kk)::value;
-        xr[k] = ga[k] == 0 ? (R)1 : (R)0;
-        xi[k] = (R)0;
+        x.re[k] = (ga ^ global_slot<k>(h.gload)) == 0 ? (A)1 : (A)0;
+        x.im[k] = (A)0;
       });
     } else {
-      each_slot([&](auto kk) __attribute__((always_inline)) {
+      each<0, kSlots>([&](auto kk) __attribute__((always_inline)) {
         constexpr int k = decltype(kk)::value;
-        const T v = __builtin_nontemporal_load(psi + ga[k]);
-        xr[k] = v.x;
-        xi[k] = v.y;
+        const T v = __builtin_nontemporal_load(psi + (ga ^ global_slot<k>(h.gload)));
+        x.re[k] = (A)v.x;
+        x.im[k] = (A)v.y;
       });
     }
   }
-  if (rn & FP_RENORM_APPLY) {
-    const A sc = (A)nb.ctl[1];
-    each_slot([&](auto kk) __attribute__((always_inline)) {
-      constexpr int k = decltype(kk)::value;
-      xr[k] = (R)(sc * (A)xr[k]);
-      xi[k] = (R)(sc * (A)xi[k]);
-    });
+  if constexpr (sizeof(A) == 4) {
+    if (rn & FP_RENORM_APPLY) {
+      const A sc = (A)nb.ctl[1];
+      each<0, kSlots>([&](auto kk) __attribute__((always_inline)) {
+        constexpr int k = decltype(kk)::value;
+        x.re[k] *= sc;
+        x.im[k] *= sc;
+      });
+    }
+    if (rn & FP_RENORM_IN) {
+      const double v = block_sum(norm2_slots(x), red);
+      if (t == 0) nb.part_in[tile] = v;
+      __syncthreads();
+    }
   }
-  if (rn & FP_RENORM_IN) {
-    const double v = block_sum(norm2_slots(xr, xi), red);
-    if (t == 0) nb.part_in[tile] = v;
+
+  run_ops<A, NT>(prog, smem, x);
+  if (h.store_wait) {   // every wave's loads are done before any store
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
   }
 
-  const int nops = h.nops;
-  const POp* ops = prog->ops;
-  for (int i = 0; i < nops; ++i) {
-    const POp& op = ops[i];
-    const int code = op.code;
-    const uint32_t tm = op.tmask, kc = op.kc;
-    const bool act = (t & tm) == tm;
-    if (code < PO_PHASE) {
-      // dense 2x2: code = PO_DENSE + 4 * rb + structure
-      const Mat<A> m{coef<A>(op, 0), coef<A>(op, 1), coef<A>(op, 2), coef<A>(op, 3),
-                     coef<A>(op, 4), coef<A>(op, 5), coef<A>(op, 6), coef<A>(op, 7)};
-      const int rb = code >> 2, dm = code & 3;
-      const bool ls = tm != 0;
-      if (rb == 0) dense_rb<0, A, R>(xr, xi, dm, ls, m, kc, act);
-      else if (rb == 1) dense_rb<1, A, R>(xr, xi, dm, ls, m, kc, act);
-      else if (rb == 2) dense_rb<2, A, R>(xr, xi, dm, ls, m, kc, act);
-      else dense_rb<3, A, R>(xr, xi, dm, ls, m, kc, act);
-    } else if (code < PO_PHASE_T) {
-      // diagonal on a register bit: code = PO_PHASE + 4 * only1 + rb
-      const A one = (A)1, zero = (A)0;
-      const A d0r = act ? coef<A>(op, 0) : one, d0i = act ? coef<A>(op, 1) : zero;
-      const A d1r = act ? coef<A>(op, 6) : one, d1i = act ? coef<A>(op, 7) : zero;
-      const int rb = (code - PO_PHASE) & 3;
-      const bool only1 = ((code - PO_PHASE) & 4) != 0;
-      if (kc == 0) {
-        if (only1) phase_rb<true, false, A, R>(xr, xi, rb, kc, d0r, d0i, d1r, d1i);
-        else phase_rb<false, false, A, R>(xr, xi, rb, kc, d0r, d0i, d1r, d1i);
-      } else {
-        if (only1) phase_rb<true, true, A, R>(xr, xi, rb, kc, d0r, d0i, d1r, d1i);
-        else phase_rb<false, true, A, R>(xr, xi, rb, kc, d0r, d0i, d1r, d1i);
-      }
-    } else if (code == PO_PHASE_T) {
-      // diagonal on a thread bit (aux = its thread-id bit): one factor per lane
-      const bool hi = (t & op.aux) != 0;
-      const bool on = act && (hi || op.only1 == 0);
-      const A d0r = uniform(coef<A>(op, 0)), d0i = uniform(coef<A>(op, 1));
-      const A d1r = uniform(coef<A>(op, 6)), d1i = uniform(coef<A>(op, 7));
-      const A dr = on ? (hi ? d1r : d0r) : (A)1;
-      const A di = on ? (hi ? d1i : d0i) : (A)0;
-      if (kc == 0) {
-        each_slot([&](auto kk) __attribute__((always_inline)) {
-          constexpr int k = decltype(kk)::value;
-          cmul_slot<k>(dr, di, xr, xi);
-        });
-      } else {
-        each_slot([&](auto kk) __attribute__((always_inline)) {
-          constexpr int k = decltype(kk)::value;
-          if ((k & kc) == kc) cmul_slot<k>(dr, di, xr, xi);
-        });
-      }
-    } else if (code == PO_BLOCKADE) {
-      // phase where exactly one blockade bit is set: thread part popcount(t &
-      // aux), register part popcount(k & kc)
-      const uint32_t pt = __popc(t & op.aux);
-      const A pr = coef<A>(op, 0), pi = coef<A>(op, 1);
-      each_slot([&](auto kk) __attribute__((always_inline)) {
-        constexpr int k = decltype(kk)::value;
-        const bool on = pt + (uint32_t)__builtin_popcount((uint32_t)k & kc) == 1u;
-        cmul_slot<k>(on ? pr : (A)1, on ? pi : (A)0, xr, xi);
-      });
-    } else if (code == PO_RELAYOUT) {
-      relayout((int)op.tmask, (int)op.kc, op.only1 != 0);
-      reg = op.aux;
-      cur = (int)op.kc;
-    } else if (code == PO_BLOCK) {
-      block_op(op);
-    } else {
-      swap_op(op);
-    }
-  }
-
-  if (cur != h.store_lay) relayout(cur, h.store_lay, h.store_local != 0);
   {
-    uint64_t ga[kSlots];
-    gaddr(lays[h.store_lay], ga);
-    each_slot([&](auto kk) __attribute__((always_inline)) {
+    const uint64_t ga = base ^ global_part<NT>(t, h.gstore);
+    each<0, kSlots>([&](auto kk) __attribute__((always_inline)) {
       constexpr int k = decltype(kk)::value;
       T v;
-      v.x = xr[k];
-      v.y = xi[k];
-      __builtin_nontemporal_store(v, psi + ga[k]);
+      v.x = (R)x.re[k];
+      v.y = (R)x.im[k];
+      __builtin_nontemporal_store(v, psi + (ga ^ global_slot<k>(h.gstore)));
     });
   }
-  if (rn & FP_RENORM_OUT) {
-    // red[] overlays the tile's LDS: a workgroup relayout or swap ends with a
-    // barrier after its reads; after a wave-local one, wait for every wave
-    if (local_pending) __syncthreads();
-    const double v = block_sum(norm2_slots(xr, xi), red);
-    if (t == 0) nb.part_out[tile] = v;
+  if constexpr (sizeof(A) == 4) {
+    if (rn & FP_RENORM_OUT) {
+      __syncthreads();   // red[] overlays the tile's LDS
+      const double v = block_sum(norm2_slots(x), red);
+      if (t == 0) nb.part_out[tile] = v;
+    }
   }
 }
 
@@ -654,7 +726,7 @@ __global__ __launch_bounds__(1024) void k_norm_ctl(const double* __restrict__ pa
   }
 }
 
-void launch_pass(int prec, bool f32, void* psi, const PProg* dprog, uint64_t ntiles, const TileNorm& nb,
+void launch_pass(int prec, bool f32, void* psi, const char* dprog, uint64_t ntiles, const TileNorm& nb,
                  hipStream_t st)
 {
   if (prec == QSV_C128)
@@ -675,10 +747,10 @@ void launch_pass_group(int prec, void* base, uint64_t S, unsigned count, const c
   const TileNorm none{nullptr, nullptr, nullptr};
   if (prec == QSV_C128)
     hipLaunchKernelGGL((k_pass<double, double, true>), dim3((unsigned)(S >> kPassTileBits), count), dim3(kThreads),
-                       0, st, (PV<double>::T*)base, reinterpret_cast<const PProg*>(progs), none, S, offs);
+                       0, st, (PV<double>::T*)base, progs, none, S, offs);
   else
     hipLaunchKernelGGL((k_pass<float, double, true>), dim3((unsigned)(S >> kPassTileBits), count), dim3(kThreads),
-                       0, st, (PV<float>::T*)base, reinterpret_cast<const PProg*>(progs), none, S, offs);
+                       0, st, (PV<float>::T*)base, progs, none, S, offs);
 }
 
 void launch_fill_group(int prec, void* base, uint64_t S, uint64_t count, hipStream_t st)

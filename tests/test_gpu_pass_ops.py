@@ -1,0 +1,59 @@
+"""Gates that a fused pass does not run where they stand — CNOTs and swaps that
+become index permutations, diagonal gates that wait and are multiplied together —
+against the gate-by-gate path, on one tile and on enough tiles to fill the chip."""
+from __future__ import annotations
+
+import math
+
+import numpy as np
+import pytest
+
+from qclojure_amd import circuit as qc
+from qclojure_amd import engine
+from qclojure_amd._abi import OP, QSV_FLAG_FP64_PASSES, QSV_FLAG_FUSE
+
+pytestmark = pytest.mark.gpu
+
+
+def _program(kind, n, rng, count):
+    def two():
+        return [int(x) for x in rng.choice(n, 2, replace=False)]
+
+    rows = [(OP["RY"], q, 0, 0, 0, float(rng.uniform(0, math.pi))) for q in range(n)]
+    for _ in range(count):
+        ang = float(rng.uniform(0, 2 * math.pi))
+        u = rng.uniform()
+        if kind == "permute":        # CNOT chains and swaps with few dense gates between
+            a, b = two()
+            name = "CNOT" if u < 0.7 else "SWAP" if u < 0.85 else "ISWAP" if u < 0.9 else "H"
+            rows.append((OP[name], a, 0 if name == "H" else b, 0, 0, 0.0))
+        elif kind == "diagonal":     # phases of every kind, then a dense gate that needs some of them
+            a, b = two()
+            name = ["RZ", "T", "CZ", "CRZ", "RYDBERG_CPHASE", "PHASE", "RX"][rng.integers(7)]
+            rows.append((OP[name], a, b if name[0] == "C" or name[:3] == "RYD" else 0, 0, 0, ang))
+        else:                        # both, with controlled dense gates and three-qubit ones
+            a, b = two()
+            if u < 0.1:
+                x, y, z = (int(q) for q in rng.choice(n, 3, replace=False))
+                rows.append((OP[["TOFFOLI", "FREDKIN"][rng.integers(2)]], x, y, z, 0, 0.0))
+            else:
+                name = ["CNOT", "CRX", "CRY", "CRZ", "H", "RY", "RZ", "S", "X", "SWAP", "CY"][rng.integers(11)]
+                rows.append((OP[name], a, b if name[0] == "C" or name == "SWAP" else 0, 0, 0, ang))
+    return qc.ops_from_tuples(rows)
+
+
+@pytest.mark.parametrize("kind", ["permute", "diagonal", "mixed"])
+@pytest.mark.parametrize("n,count", [(12, 200), (13, 200), (17, 300), (22, 250), (24, 150)])
+def test_deferred_gates(kind, n, count):
+    rng = np.random.default_rng(n * 7 + len(kind))
+    ops = _program(kind, n, rng, count)
+    with engine.DeviceState(n, "c128") as ref, engine.DeviceState(n, "c128") as a, \
+            engine.DeviceState(n, "c64") as f32, engine.DeviceState(n, "c64") as f64:
+        ref.apply(ops)
+        a.apply(ops, QSV_FLAG_FUSE)
+        f32.apply(ops, QSV_FLAG_FUSE)
+        f64.apply(ops, QSV_FLAG_FUSE | QSV_FLAG_FP64_PASSES)
+        # FP64: a few hundred roundings of amplitudes of at most 1
+        assert a.compare(ref)["max_abs_diff"] < 1e-12
+        for s in (f32, f64):
+            assert s.compare(ref)["max_abs_diff"] < 1e-5
