@@ -15,7 +15,7 @@ CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "libqsv.so")
 ARCH = os.environ.get("QSV_OFFLOAD_ARCH", "gfx950")
 
-SOURCES = ["qsv_api.hip", "qsv_compile.hip", "qsv_gates.hip", "qsv_pass.hip", "qsv_kernels.hip", "qsv_pauli.hip", "qsv_batch.hip", "qsv_la.hip"]
+SOURCES = ["qsv_api.hip", "qsv_compile.hip", "qsv_gates.hip", "qsv_pass.hip", "qsv_small.hip", "qsv_kernels.hip", "qsv_pauli.hip", "qsv_batch.hip", "qsv_la.hip"]
 
 HIPCC_FLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC",
@@ -23,14 +23,15 @@ HIPCC_FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wall", "-Wno-unused-result", "-Wno-unused-value",
 ]
-# Flags of single files.
-FILE_FLAGS = {
+# The files that run micro-op programs:
+_OPS_FLAGS = [
     # uniform branches stay branches: structurised, the op dispatch of a fused
     # pass keeps a second copy of the tile in registers (128 VGPRs and 2500
     # spills instead of 101 and none). No vector combining: it turns a slot's
     # scalar into a two-slot vector load, which keeps FP32 tiles in scratch.
-    "qsv_pass.hip": ["-mllvm", "-structurizecfg-skip-uniform-regions=true", "-mllvm", "-disable-vector-combine"],
-}
+    "-mllvm", "-structurizecfg-skip-uniform-regions=true", "-mllvm", "-disable-vector-combine",
+]
+FILE_FLAGS = {"qsv_pass.hip": _OPS_FLAGS, "qsv_small.hip": _OPS_FLAGS}
 
 
 def _noise(text: str) -> list[str]:

@@ -998,6 +998,61 @@ std::vector<BGate> fold_gates(const std::vector<BGate>& in)
   return out;
 }
 
+// A whole-register program (qsv_small.hip) of gates [g0, g1), none of which
+// runs alone, appended to `out`; zero: it starts from |0..0>.
+size_t compile_small(int n, const BGate* g0, const BGate* g1, bool zero, std::vector<char>& out)
+{
+  FPass p;
+  p.tb = std::max(n, 4);
+  p.renorm = zero ? FP_INIT_ZERO : 0;
+  int loc[64];
+  for (int b = 0; b < 64; ++b) loc[b] = b;
+  for (int b = 0; b < 16; ++b) p.pos[b] = p.sorted_pos[b] = b;
+  p.gates.reserve(g1 - g0);
+  for (const BGate* g = g0; g != g1; ++g) p.gates.push_back(local_gate(*g, loc));
+  std::complex<double> scalar(1.0, 0.0);
+  return compile_pass(p, false, 0, scalar, true, out);
+}
+
+// Fused programs of states smaller than a pass's tile: one launch per run of
+// gates between those that run alone (per gate, a launch each: a 5-qubit
+// program of 32 gates took 110 us).
+int run_small(qsv_state* s, const std::vector<BGate>& gs)
+{
+  constexpr size_t kMaxGates = 1 << 14;   // bounds a program
+  for (size_t i = 0; i < gs.size();) {
+    if (runs_alone(gs[i].kind)) {
+      const int rc = run_direct(s, gs[i++]);
+      if (rc) return rc;
+      continue;
+    }
+    size_t j = i;
+    while (j < gs.size() && j - i < kMaxGates && !runs_alone(gs[j].kind)) ++j;
+    std::vector<char> buf(256, 0);   // the instance, then its program
+    SmallInst in{};
+    in.n = s->n;
+    in.prog = compile_small(s->n, &gs[i], &gs[i] + (j - i), false, buf);
+    in.dest = ~0ull;
+    std::memcpy(buf.data(), &in, sizeof(in));
+    const char* dev = nullptr;
+    int rc = upload_passes(s, buf, &dev);
+    if (rc) return rc;
+    SmallRun r{};
+    r.prec = s->prec;
+    r.progs = dev;
+    r.insts = reinterpret_cast<const SmallInst*>(dev);
+    r.states = s->amps;
+    hipError_t e = hipSuccess;
+    rc = timed(s, QSV_KCLASS_BLOCK, 2.0 * s->S * s->bytes_per_amp(),
+               [&] { e = launch_small(r, small_class(s->n), 1, s->stream); });
+    if (rc) return rc;
+    HIPCHK(e);
+    HIPCHK(hipEventRecord(s->ring_pending->event, s->stream));
+    i = j;
+  }
+  return QSV_OK;
+}
+
 // flags: QSV_FLAG_FP64_PASSES keeps complex64 pass arithmetic in FP64; by
 // default it is FP32, renormalised pass by pass (15 % faster per 30-qubit
 // layer: no conversions, same register budget), and its register-bit runs
@@ -1006,14 +1061,7 @@ std::vector<BGate> fold_gates(const std::vector<BGate>& in)
 int run_fused(qsv_state* s, const std::vector<BGate>& gs_in, uint32_t flags)
 {
   const std::vector<BGate> gs = fold_gates(gs_in);
-  const int TB = kPassTileBits;
-  if (s->n < TB) {
-    for (const auto& g : gs) {
-      int rc = run_direct(s, g);
-      if (rc) return rc;
-    }
-    return QSV_OK;
-  }
+  if (s->n < kPassTileBits) return run_small(s, gs);
   const bool f32 = s->prec == QSV_C64 && !(flags & QSV_FLAG_FP64_PASSES);
   const bool blocks = !(flags & QSV_FLAG_VALU_PASSES);
   std::vector<FPass> passes;
@@ -1788,9 +1836,9 @@ struct GroupGraph {
 };
 struct BatchCache {
   hipStream_t st = nullptr, gst = nullptr;
-  GrowBuf recs_h{nullptr, 0, true};   // pinned staging of the gate records
+  GrowBuf recs_h{nullptr, 0, true};   // pinned staging of the small circuits' programs
   GrowBuf bytes_h{nullptr, 0, true};  // pinned staging of the grouped pass programs
-  GrowBuf recs, insts, tz, tc, order, energy, bytes, offs, meta, part;
+  GrowBuf recs, insts, tz, tc, energy, bytes, offs, meta, part;
   std::vector<GroupGraph> graphs;   // at most kGroupGraphs, least recently used replaced
   uint64_t tick = 0;
 };
@@ -1919,7 +1967,7 @@ void batch_cache_release()
     g_shape_count = 0;
   }
   for (GrowBuf* b : {&g_batch.recs_h, &g_batch.bytes_h, &g_batch.recs, &g_batch.insts, &g_batch.tz, &g_batch.tc,
-                     &g_batch.order, &g_batch.energy, &g_batch.bytes, &g_batch.offs, &g_batch.meta, &g_batch.part}) {
+                     &g_batch.energy, &g_batch.bytes, &g_batch.offs, &g_batch.meta, &g_batch.part}) {
     if (b->p) (void)(b->pinned ? hipHostFree(b->p) : hipFree(b->p));
     b->p = nullptr;
     b->cap = 0;
@@ -1954,24 +2002,23 @@ int qsv_batch_expect_z(const qsv_batch_desc* d, double* energies)
   if (rc) return rc;
   HIPCHK(hipSetDevice(g_device));
   const int prec = d->precision;
+  const int small_n = prec == QSV_C128 ? kSmallC128 : kSmallC64;
   const size_t B = prec == QSV_C128 ? 16 : 8;
-  const int lds_n = prec == QSV_C128 ? 13 : 14;   // 2^n * B <= 128 KiB of LDS
 
   const uint64_t T0 = d->term_offsets[0];
   const uint64_t n_terms = d->term_offsets[N] - T0;
-  std::vector<BInst> insts(N);
+  std::vector<SmallInst> insts(N);
   std::vector<uint64_t> tz(n_terms);
   std::vector<double> tc(n_terms);
   std::vector<std::vector<BGate>> big_gates;
   std::vector<uint64_t> big_idx;
-  std::vector<int32_t> small_idx;
-  int max_small_n = 0;
+  std::vector<uint64_t> small_idx;
   for (uint64_t i = 0; i < N; ++i) {
     const int n = d->num_qubits[i];
     if (n < 1 || n > 34) return fail(QSV_E_INVALID, "instance " + std::to_string(i) + ": num_qubits out of range");
   }
-  // Decode every instance, convert its Z terms and fold its gates; then write
-  // the small instances' gate records into pinned staging memory. Both phases are
+  // Decode every instance, convert its Z terms, fold its gates and compile the
+  // small ones' programs, which then go to pinned staging memory. Both phases are
   // independent per instance and run on a pool of host threads (at most 16);
   // errors are reported for the first failing instance in order, decode errors
   // before term errors, as a sequential pass would.
@@ -1984,7 +2031,7 @@ int qsv_batch_expect_z(const qsv_batch_desc* d, double* energies)
   std::vector<int> dec_rc(N, 0);
   std::vector<std::string> dec_err(N);
   std::vector<char> term_bad(N, 0);
-  std::vector<uint64_t> rec_off(N + 1, 0);
+  std::vector<std::vector<char>> small_prog(N);
   const unsigned hw = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
   const unsigned nt = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>(hw, N / 8 + 1));
   auto parallel_over = [&](uint64_t count, auto&& body) {
@@ -2025,53 +2072,44 @@ int qsv_batch_expect_z(const qsv_batch_desc* d, double* energies)
       tz[k - T0] = bm;
       tc[k - T0] = d->term_coeff[k];
     }
-    if (!dec_rc[i]) decoded[i] = fold_gates(decoded[i]);
+    if (dec_rc[i]) return;
+    decoded[i] = fold_gates(decoded[i]);
+    if (n <= small_n) compile_small(n, decoded[i].data(), decoded[i].data() + decoded[i].size(), true, small_prog[i]);
   });
   for (uint64_t i = 0; i < N; ++i)
     if (dec_rc[i]) return fail(dec_rc[i], dec_err[i]);
   for (uint64_t i = 0; i < N; ++i)
     if (term_bad[i]) return fail(QSV_E_INVALID, "instance " + std::to_string(i) + ": Z term on a missing qubit");
-  for (uint64_t i = 0; i < N; ++i)
-    rec_off[i + 1] = rec_off[i] + (d->num_qubits[i] <= lds_n ? decoded[i].size() : 0);
-  const uint64_t n_recs = rec_off[N];
-  if ((rc = grow(g_batch.recs_h, n_recs * sizeof(BRec)))) return rc;
-  BRec* const recs = static_cast<BRec*>(g_batch.recs_h.p);
-  parallel([&](uint64_t i) {
-    if (d->num_qubits[i] > lds_n) return;
-    BRec* out = recs + rec_off[i];
-    for (const BGate& g : decoded[i]) {
-      BRec r{};
-      r.kind = g.kind;
-      r.a = g.a;
-      r.b = g.b;
-      r.phase_only = g.phase_only ? 1 : 0;
-      for (int c : g.cbits) r.cmask |= 1ull << c;
-      r.bmask = g.bmask;
-      std::memcpy(r.m, g.m, sizeof(r.m));
-      *out++ = r;
-    }
-  });
+  uint64_t small_bytes = 0;
   for (uint64_t i = 0; i < N; ++i) {
     const int n = d->num_qubits[i];
-    BInst& in = insts[i];
+    SmallInst& in = insts[i];
     in.n = n;
     in.t0 = d->term_offsets[i] - T0;
     in.t1 = d->term_offsets[i + 1] - T0;
-    in.out_offset = ~0ull;
-    if (n <= lds_n) {
-      in.g0 = rec_off[i];
-      in.g1 = rec_off[i + 1];
-      small_idx.push_back((int32_t)i);
-      max_small_n = std::max(max_small_n, n);
+    in.io = ~0ull;
+    in.dest = i;
+    if (n <= small_n) {
+      in.prog = small_bytes;   // programs are multiples of 256 bytes
+      small_bytes += small_prog[i].size();
+      small_idx.push_back(i);
     } else {
-      in.g0 = in.g1 = 0;
       big_idx.push_back(i);
       big_gates.push_back(std::move(decoded[i]));
     }
   }
-  // largest circuits first, so the long workgroups start early
+  if ((rc = grow(g_batch.recs_h, small_bytes))) return rc;
+  char* const recs = static_cast<char*>(g_batch.recs_h.p);
+  parallel_over(small_idx.size(), [&](uint64_t k) {
+    const std::vector<char>& p = small_prog[small_idx[k]];
+    std::memcpy(recs + insts[small_idx[k]].prog, p.data(), p.size());
+  });
+  // one launch per size class, largest circuits first, so the long workgroups
+  // start early
   std::stable_sort(small_idx.begin(), small_idx.end(),
-                   [&](int32_t a, int32_t b) { return insts[a].n > insts[b].n; });
+                   [&](uint64_t a, uint64_t b) { return insts[a].n > insts[b].n; });
+  std::vector<SmallInst> small(small_idx.size());
+  for (size_t k = 0; k < small_idx.size(); ++k) small[k] = insts[small_idx[k]];
 
   if (!g_batch.st && hipStreamCreateWithFlags(&g_batch.st, hipStreamNonBlocking) != hipSuccess)
     return fail(QSV_E_DEVICE, "batch: stream creation failed");
@@ -2082,18 +2120,15 @@ int qsv_batch_expect_z(const qsv_batch_desc* d, double* energies)
     if (uploaded) hipEventDestroy(uploaded);
     uploaded = nullptr;
   };
-  if ((rc = upload(g_batch.recs, recs, n_recs, st)) || (rc = upload(g_batch.insts, insts.data(), N, st)) ||
+  if ((rc = upload(g_batch.recs, recs, small_bytes, st)) ||
+      (rc = upload(g_batch.insts, small.data(), small.size(), st)) ||
       (rc = upload(g_batch.tz, tz.data(), tz.size(), st)) || (rc = upload(g_batch.tc, tc.data(), tc.size(), st)) ||
-      (rc = upload(g_batch.order, small_idx.data(), small_idx.size(), st)) ||
       (rc = grow(g_batch.energy, N * sizeof(double)))) {
     cleanup();
     return rc;
   }
-  BRec* const d_recs = static_cast<BRec*>(g_batch.recs.p);
-  BInst* const d_insts = static_cast<BInst*>(g_batch.insts.p);
   uint64_t* const d_tz = static_cast<uint64_t*>(g_batch.tz.p);
   double* const d_tc = static_cast<double*>(g_batch.tc.p);
-  int32_t* const d_order = static_cast<int32_t*>(g_batch.order.p);
   double* const d_energy = static_cast<double*>(g_batch.energy.p);
   // the pooled states' streams read the uploaded terms: order them after the copies
   if (hipEventCreateWithFlags(&uploaded, hipEventDisableTiming) != hipSuccess ||
@@ -2101,20 +2136,29 @@ int qsv_batch_expect_z(const qsv_batch_desc* d, double* energies)
     cleanup();
     return fail(QSV_E_DEVICE, "batch: event creation failed");
   }
-  if (!small_idx.empty()) {
-    const size_t lds = ((size_t)1 << max_small_n) * B;
-    if (setup_lds_batch(prec, lds) != 0) {
+  for (size_t k = 0; k < small.size();) {
+    const int cls = small_class(small[k].n);
+    size_t e = k;
+    while (e < small.size() && small_class(small[e].n) == cls) ++e;
+    SmallRun r{};
+    r.prec = prec;
+    r.progs = static_cast<const char*>(g_batch.recs.p);
+    r.insts = static_cast<const SmallInst*>(g_batch.insts.p) + k;
+    r.tz = d_tz;
+    r.tc = d_tc;
+    r.energies = d_energy;
+    const hipError_t le = launch_small(r, cls, (unsigned)(e - k), st);
+    if (le != hipSuccess) {
       cleanup();
-      return fail(QSV_E_DEVICE, "batch: cannot reserve " + std::to_string(lds) + " B of LDS per workgroup");
+      return fail(QSV_E_DEVICE, std::string("batch: small circuits: ") + hipGetErrorString(le));
     }
-    launch_lds_batch(prec, (unsigned)small_idx.size(), lds, d_insts, d_recs, d_tz, d_tc, d_order, d_energy, nullptr,
-                     st);
+    k = e;
   }
-  // circuits too large for LDS, grouped by qubit count: all instances of a
+  // circuits too large for one workgroup, grouped by qubit count: all instances of a
   // group sit back to back in one arena and advance one pass round per launch
   // (k_pass group mode, FP64 arithmetic); a program that needs a gate run
   // alone takes a pooled state of its own instead. Their passes are planned
-  // here, on the host threads, while the LDS batch runs on the device.
+  // here, on the host threads, while the small circuits run on the device.
   std::vector<Plan> big_plans(big_idx.size());
   parallel_over(big_idx.size(), [&](uint64_t k) {
     Plan& pl = big_plans[k];
@@ -2336,12 +2380,11 @@ int qsv_noisy_trajectories(int num_qubits, int precision, const qsv_op* ops, uin
   };
   // one trajectory's gate list: clean gates of op i, then its sites' operators.
   // A chosen operator scaled to max |k_ij| = 1 shrinks the norm (damping
-  // operators do, site after site), so a renormalisation record follows every
-  // `renorm_every`-th site: every site in the LDS batch path, where it is one
-  // sweep of LDS; every 16th between fused passes, where it is a barrier of
-  // two state passes. Without it, deep programs with strong damping would
+  // operators do, site after site), so a renormalisation follows every 16th
+  // site (the small path's last site too): between fused passes it is a barrier
+  // of two state passes. Without it, deep programs with strong damping would
   // drive the amplitudes into the subnormal range.
-  auto trajectory_gates = [&](uint64_t t, std::vector<BGate>& out, uint64_t renorm_every) {
+  auto trajectory_gates = [&](uint64_t t, std::vector<BGate>& out) {
     out.clear();
     size_t g = 0, k = 0;
     for (uint64_t i = 0; i < n_ops; ++i) {
@@ -2349,7 +2392,7 @@ int qsv_noisy_trajectories(int num_qubits, int precision, const qsv_op* ops, uin
       for (; k < n_sites && sites[k].after_op == i; ++k) {
         const int j = choose(k, qsv_uniform(seed, t * QSV_TRAJ_SLOTS + k));
         emit_ctl(out, {}, n - 1 - sites[k].qubit, kops[k][j].data());
-        if ((k + 1) % renorm_every == 0) {
+        if ((k + 1) % 16 == 0) {
           BGate r;
           r.kind = FG_RENORM;
           out.push_back(std::move(r));
@@ -2364,7 +2407,7 @@ int qsv_noisy_trajectories(int num_qubits, int precision, const qsv_op* ops, uin
   };
   const size_t B = precision == QSV_C128 ? 16 : 8;
   const uint64_t S = 1ull << n;
-  const int lds_n = precision == QSV_C128 ? 13 : 14;
+  const int small_n = precision == QSV_C128 ? kSmallC128 : kSmallC64;
   std::vector<double> host_state;
   auto keep_state = [&](const void* dev_amps, int prec, uint64_t t, hipStream_t st) -> int {
     // copy one final state to the caller as normalised interleaved FP64
@@ -2388,83 +2431,93 @@ int qsv_noisy_trajectories(int num_qubits, int precision, const qsv_op* ops, uin
     return QSV_OK;
   };
   std::vector<BGate> gs;
-  if (n <= lds_n) {
-    // one workgroup per trajectory with the state in LDS, final states into
-    // an arena, one shot each; chunks bound the arena to 1 GiB
+  if (n <= small_n) {
+    // one workgroup per trajectory, all running one program: its noise sites
+    // draw their uniform and choose their operator on the device. Final states
+    // go to an arena (chunks bound it to 1 GiB), one shot each.
+    constexpr uint64_t kRenormEvery = 16;
+    std::vector<KrausOp> table;
+    FPass p;
+    p.tb = std::max(n, 4);
+    p.renorm = FP_INIT_ZERO;
+    int loc[64];
+    for (int b = 0; b < 64; ++b) loc[b] = b;
+    for (int b = 0; b < 16; ++b) p.pos[b] = p.sorted_pos[b] = b;
+    size_t g = 0, k = 0;
+    for (uint64_t i = 0; i < n_ops; ++i) {
+      for (; g < op_end[i]; ++g) p.gates.push_back(local_gate(clean[g], loc));
+      for (; k < n_sites && sites[k].after_op == i; ++k) {
+        FGate f{};
+        f.kind = FG_KRAUS;
+        f.a = n - 1 - sites[k].qubit;
+        f.b = (int32_t)k;
+        f.cmask = (uint32_t)table.size();
+        f.sub = sites[k].n_kraus;
+        f.bmask = (k + 1) % kRenormEvery == 0 || k + 1 == n_sites ? 1u : 0u;
+        for (int j = 0; j < sites[k].n_kraus; ++j) {
+          KrausOp o;
+          o.w = kw[k][j];
+          std::memcpy(o.m, kops[k][j].data(), sizeof(o.m));
+          table.push_back(o);
+        }
+        p.gates.push_back(f);
+      }
+    }
+    if (table.empty()) table.push_back(KrausOp{});
+    std::vector<char> prog;
+    std::complex<double> scalar(1.0, 0.0);
+    compile_pass(p, false, 0, scalar, true, prog);
     const uint64_t chunk = std::max<uint64_t>(1, std::min<uint64_t>(n_traj, (1ull << 30) / (S * B)));
     hipStream_t st = nullptr;
     HIPCHK(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
     void* arena = nullptr;
-    BRec* d_recs = nullptr;
-    BInst* d_insts = nullptr;
-    int32_t* d_order = nullptr;
+    char* d_prog = nullptr;
+    KrausOp* d_table = nullptr;
     SampleJob* d_jobs = nullptr;
     uint64_t* d_out = nullptr;
     auto cleanup = [&]() {
       hipStreamSynchronize(st);
       hipFree(arena);
-      hipFree(d_recs);
-      hipFree(d_insts);
-      hipFree(d_order);
+      hipFree(d_prog);
+      hipFree(d_table);
       hipFree(d_jobs);
       hipFree(d_out);
       hipStreamDestroy(st);
     };
-    if (hipMalloc(&arena, chunk * S * B) != hipSuccess || hipMalloc((void**)&d_out, chunk * sizeof(uint64_t)) != hipSuccess) {
+    if (hipMalloc(&arena, chunk * S * B) != hipSuccess ||
+        hipMalloc((void**)&d_out, chunk * sizeof(uint64_t)) != hipSuccess ||
+        hipMalloc((void**)&d_jobs, chunk * sizeof(SampleJob)) != hipSuccess) {
       cleanup();
       return fail(QSV_E_NOMEM, "trajectories: arena allocation failed");
     }
-    if (setup_lds_batch(precision, S * B) != 0) {
+    if ((rc = dev_upload(prog, &d_prog, st)) || (rc = dev_upload(table, &d_table, st))) {
       cleanup();
-      return fail(QSV_E_DEVICE, "trajectories: LDS reservation failed");
+      return rc;
     }
+    std::vector<SampleJob> jobs(chunk);
     for (uint64_t t0 = 0; t0 < n_traj; t0 += chunk) {
       const uint64_t c = std::min(chunk, n_traj - t0);
-      std::vector<BRec> recs;
-      std::vector<BInst> insts(c);
-      std::vector<int32_t> order(c);
-      std::vector<SampleJob> jobs(c);
-      for (uint64_t i = 0; i < c; ++i) {
-        trajectory_gates(t0 + i, gs, 1);
-        BInst& in = insts[i];
-        in.n = n;
-        in.g0 = recs.size();
-        for (const BGate& g : gs) {
-          BRec r{};
-          r.kind = g.kind;
-          r.a = g.a;
-          r.b = g.b;
-          r.phase_only = g.phase_only ? 1 : 0;
-          for (int cb : g.cbits) r.cmask |= 1ull << cb;
-          r.bmask = g.bmask;
-          std::memcpy(r.m, g.m, sizeof(r.m));
-          recs.push_back(r);
-        }
-        in.g1 = recs.size();
-        in.t0 = in.t1 = 0;
-        in.out_offset = i * S;
-        order[i] = (int32_t)i;
-        jobs[i] = SampleJob{i * S, i, 1, measure_seed(t0 + i), n, 0};
+      for (uint64_t i = 0; i < c; ++i) jobs[i] = SampleJob{i * S, i, 1, measure_seed(t0 + i), n, 0};
+      SmallRun r{};
+      r.prec = precision;
+      r.progs = d_prog;
+      r.one.n = n;
+      r.one.dest = ~0ull;
+      r.states = arena;
+      r.kraus = d_table;
+      r.seed = seed;
+      r.traj0 = t0;
+      hipError_t e = launch_small(r, small_class(n), (unsigned)c, st);
+      if (e == hipSuccess) e = hipMemcpyAsync(d_jobs, jobs.data(), c * sizeof(SampleJob), hipMemcpyHostToDevice, st);
+      if (e == hipSuccess) {
+        launch_batch_sample(precision, arena, d_jobs, (unsigned)c, d_out, nullptr, st);
+        e = hipGetLastError();
       }
-      hipFree(d_recs);
-      hipFree(d_insts);
-      hipFree(d_order);
-      hipFree(d_jobs);
-      d_recs = nullptr;
-      d_insts = nullptr;
-      d_order = nullptr;
-      d_jobs = nullptr;
-      if ((rc = dev_upload(recs, &d_recs, st)) || (rc = dev_upload(insts, &d_insts, st)) ||
-          (rc = dev_upload(order, &d_order, st)) || (rc = dev_upload(jobs, &d_jobs, st))) {
+      if (e == hipSuccess) e = hipMemcpyAsync(outcomes + t0, d_out, c * sizeof(uint64_t), hipMemcpyDeviceToHost, st);
+      if (e == hipSuccess) e = hipStreamSynchronize(st);
+      if (e != hipSuccess) {
         cleanup();
-        return rc;
-      }
-      launch_lds_batch(precision, (unsigned)c, S * B, d_insts, d_recs, nullptr, nullptr, d_order, nullptr, arena, st);
-      launch_batch_sample(precision, arena, d_jobs, (unsigned)c, d_out, nullptr, st);
-      if (hipMemcpyAsync(outcomes + t0, d_out, c * sizeof(uint64_t), hipMemcpyDeviceToHost, st) != hipSuccess ||
-          hipStreamSynchronize(st) != hipSuccess) {
-        cleanup();
-        return fail(QSV_E_DEVICE, "trajectories: batched launch failed");
+        return fail(QSV_E_DEVICE, std::string("trajectories: ") + hipGetErrorString(e));
       }
       for (uint64_t i = 0; i < c && t0 + i < n_keep; ++i) {
         if ((rc = keep_state((const char*)arena + i * S * B, precision, t0 + i, st))) {
@@ -2488,7 +2541,7 @@ int qsv_noisy_trajectories(int num_qubits, int precision, const qsv_op* ops, uin
     return fail(QSV_E_NOMEM, "trajectories: allocation failed");
   }
   for (uint64_t t = 0; t < n_traj && !rc; ++t) {
-    trajectory_gates(t, gs, 16);
+    trajectory_gates(t, gs);
     launch_fill_basis(s->prec, s->amps, s->S, 0, s->stream);
     if ((rc = run_fused(s, gs, 0))) break;
     launch_sample(s->prec, s->amps, s->S, s->prefix, 1, measure_seed(t), d_out, s->stream);
@@ -2518,6 +2571,7 @@ struct SrvReq {
   uint64_t id = 0;
   int n = 0;
   std::vector<BGate> gates;
+  std::vector<char> prog;   // small requests: the compiled program
   uint64_t shots = 0, seed = 0;
   Clock::time_point t_submit, t_admit, t_done;
   int status = QSV_REQ_QUEUED;
@@ -2537,9 +2591,8 @@ struct SrvReq {
 // Reusable device/host buffers for one batched launch of small requests.
 struct SmallSlot {
   void* arena = nullptr;       size_t arena_cap = 0;     // final states, back to back
-  BRec* recs = nullptr;        size_t recs_cap = 0;
-  BInst* insts = nullptr;      size_t insts_cap = 0;
-  int32_t* order = nullptr;    size_t order_cap = 0;
+  char* progs = nullptr;       size_t progs_cap = 0;
+  SmallInst* insts = nullptr;  size_t insts_cap = 0;
   SampleJob* jobs = nullptr;   size_t jobs_cap = 0;
   uint64_t* d_out = nullptr;   size_t out_cap = 0;
   uint64_t* h_out = nullptr;   size_t hout_cap = 0;
@@ -2674,45 +2727,29 @@ int launch_small(qsv_server* sv, std::vector<SrvReq*>& batch)
   if (!slot) return 1;  // all slots in flight; retry later
   const int prec = sv->cfg.precision;
   const size_t B = prec == QSV_C128 ? 16 : 8;
-  std::vector<BRec> recs;
-  std::vector<BInst> insts(batch.size());
-  std::vector<int32_t> order(batch.size());
+  std::vector<char> progs;
+  std::vector<SmallInst> insts(batch.size());
   std::vector<SampleJob> jobs(batch.size());
   slot->out_offsets.assign(batch.size(), 0);
   uint64_t arena_amps = 0, nout = 0;
-  int maxn = 0;
   for (size_t k = 0; k < batch.size(); ++k) {
     SrvReq* r = batch[k];
-    BInst& in = insts[k];
+    SmallInst& in = insts[k];
     in.n = r->n;
-    in.g0 = recs.size();
-    for (const BGate& g : r->gates) {
-      BRec rec{};
-      rec.kind = g.kind;
-      rec.a = g.a;
-      rec.b = g.b;
-      rec.phase_only = g.phase_only ? 1 : 0;
-      for (int c : g.cbits) rec.cmask |= 1ull << c;
-      rec.bmask = g.bmask;
-      std::memcpy(rec.m, g.m, sizeof(rec.m));
-      recs.push_back(rec);
-    }
-    in.g1 = recs.size();
-    in.t0 = in.t1 = 0;
-    in.out_offset = arena_amps;
+    in.prog = progs.size();   // programs are multiples of 256 bytes
+    progs.insert(progs.end(), r->prog.begin(), r->prog.end());
+    in.io = arena_amps;
+    in.dest = ~0ull;
     jobs[k] = SampleJob{arena_amps, nout, r->shots, r->seed, r->n, 0};
     slot->out_offsets[k] = nout;
     arena_amps += 1ull << r->n;
     nout += r->shots;
-    maxn = std::max(maxn, r->n);
-    order[k] = (int32_t)k;
   }
-  std::stable_sort(order.begin(), order.end(), [&](int32_t a, int32_t b) { return insts[a].n > insts[b].n; });
+  std::stable_sort(insts.begin(), insts.end(), [](const SmallInst& a, const SmallInst& b) { return a.n > b.n; });
   int rc;
   if ((rc = grow_arena(&slot->arena, &slot->arena_cap, std::max<uint64_t>(arena_amps, 1) * B))) return rc;
-  if ((rc = grow_dev(&slot->recs, &slot->recs_cap, std::max<size_t>(recs.size(), 1)))) return rc;
+  if ((rc = grow_dev(&slot->progs, &slot->progs_cap, std::max<size_t>(progs.size(), 1)))) return rc;
   if ((rc = grow_dev(&slot->insts, &slot->insts_cap, insts.size()))) return rc;
-  if ((rc = grow_dev(&slot->order, &slot->order_cap, order.size()))) return rc;
   if ((rc = grow_dev(&slot->jobs, &slot->jobs_cap, jobs.size()))) return rc;
   if ((rc = grow_dev(&slot->d_out, &slot->out_cap, std::max<uint64_t>(nout, 1)))) return rc;
   if ((rc = grow_dev(&slot->d_norm, &slot->norm_cap, jobs.size()))) return rc;
@@ -2732,15 +2769,21 @@ int launch_small(qsv_server* sv, std::vector<SrvReq*>& batch)
   }
   if (!slot->stream) HIPCHK(hipStreamCreateWithFlags(&slot->stream, hipStreamNonBlocking));
   if (!slot->ev) HIPCHK(hipEventCreateWithFlags(&slot->ev, hipEventDisableTiming));
-  if (!recs.empty())
-    HIPCHK(hipMemcpyAsync(slot->recs, recs.data(), recs.size() * sizeof(BRec), hipMemcpyHostToDevice, slot->stream));
-  HIPCHK(hipMemcpyAsync(slot->insts, insts.data(), insts.size() * sizeof(BInst), hipMemcpyHostToDevice, slot->stream));
-  HIPCHK(hipMemcpyAsync(slot->order, order.data(), order.size() * sizeof(int32_t), hipMemcpyHostToDevice, slot->stream));
+  HIPCHK(hipMemcpyAsync(slot->progs, progs.data(), progs.size(), hipMemcpyHostToDevice, slot->stream));
+  HIPCHK(hipMemcpyAsync(slot->insts, insts.data(), insts.size() * sizeof(SmallInst), hipMemcpyHostToDevice, slot->stream));
   HIPCHK(hipMemcpyAsync(slot->jobs, jobs.data(), jobs.size() * sizeof(SampleJob), hipMemcpyHostToDevice, slot->stream));
-  const size_t lds = ((size_t)1 << maxn) * B;
-  if (setup_lds_batch(prec, lds) != 0) return fail(QSV_E_DEVICE, "serving: LDS reservation failed");
-  launch_lds_batch(prec, (unsigned)batch.size(), lds, slot->insts, slot->recs, nullptr, nullptr, slot->order, nullptr,
-                   slot->arena, slot->stream);
+  for (size_t k = 0; k < insts.size();) {
+    const int cls = small_class(insts[k].n);
+    size_t e = k;
+    while (e < insts.size() && small_class(insts[e].n) == cls) ++e;
+    SmallRun run{};
+    run.prec = prec;
+    run.progs = slot->progs;
+    run.insts = slot->insts + k;
+    run.states = slot->arena;
+    HIPCHK(launch_small(run, cls, (unsigned)(e - k), slot->stream));
+    k = e;
+  }
   launch_batch_sample(prec, slot->arena, slot->jobs, (unsigned)jobs.size(), slot->d_out, slot->d_norm, slot->stream);
   if (nout)
     HIPCHK(hipMemcpyAsync(slot->h_out, slot->d_out, nout * sizeof(uint64_t), hipMemcpyDeviceToHost, slot->stream));
@@ -2979,9 +3022,13 @@ int qsv_server_submit(qsv_server* sv, int num_qubits, const qsv_op* ops, uint64_
   const uint64_t B = sv->cfg.precision == QSV_C128 ? 16 : 8;
   r->bytes = (1ull << num_qubits) * B;
   r->small = sv->cfg.batch_small && num_qubits <= sv->lds_n;
-  // small requests run as batched LDS programs: fold their gates here (large
-  // ones are folded by the fused runner, or run gate by gate without FUSE)
-  if (r->small && (sv->cfg.flags & QSV_FLAG_FUSE)) r->gates = fold_gates(r->gates);
+  // small requests run as batched whole-register programs, folded and compiled
+  // here (large ones are folded by the fused runner, or run gate by gate without FUSE)
+  if (r->small) {
+    if (sv->cfg.flags & QSV_FLAG_FUSE) r->gates = fold_gates(r->gates);
+    compile_small(r->n, r->gates.data(), r->gates.data() + r->gates.size(), true, r->prog);
+    r->gates.clear();
+  }
   {
     std::lock_guard<std::mutex> lk(sv->mu);
     if (r->bytes > sv->budget) {
@@ -3088,9 +3135,8 @@ int qsv_server_destroy(qsv_server* sv)
   for (auto& s : sv->slots) {
     if (s.stream) hipStreamSynchronize(s.stream);
     hipFree(s.arena);
-    hipFree(s.recs);
+    hipFree(s.progs);
     hipFree(s.insts);
-    hipFree(s.order);
     hipFree(s.jobs);
     hipFree(s.d_out);
     if (s.h_out) hipHostFree(s.h_out);

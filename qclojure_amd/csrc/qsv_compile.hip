@@ -363,6 +363,7 @@ struct Compiler {
   static bool usable(C d) { return std::fabs(std::abs(d) - 1.0) < 1e-9; }
   static uint32_t gate_bits(const FGate& g)
   {
+    if (g.kind == FG_KRAUS) return 1u << g.a;
     uint32_t m = g.cmask | (g.kind == FG_BLOCKADE ? g.bmask : 0u);
     if (g.a >= 0) m |= 1u << g.a;
     if (g.b >= 0) m |= 1u << g.b;
@@ -466,8 +467,18 @@ struct Compiler {
       return true;
     }
     const uint32_t t = 1u << g.a;
-    if (!(reg & t) || ((row_dirty | col_dirty) & t) || (g.cmask & row_dirty) || !can_flush(t)) return false;
+    if (!(reg & t) || ((row_dirty | col_dirty) & t) || !can_flush(t)) return false;
     const int rb = (int)rank_in(reg, g.a);
+    if (g.kind == FG_KRAUS) {
+      flush(t);
+      POp& op = emit(PO_KRAUS + rb);
+      op.kc = (uint32_t)g.b;
+      op.aux = g.cmask;
+      op.cnt = g.sub;
+      op.flag = (int32_t)g.bmask;
+      return true;
+    }
+    if (g.cmask & row_dirty) return false;
     double m[8];
     std::memcpy(m, g.m, sizeof(m));
     int sub = g.kind == FG_DENSE ? g.sub : DM_GENERAL;
@@ -566,7 +577,7 @@ struct Compiler {
         const int i = front(b);
         if (i < 0 || !ready(i)) continue;
         const FGate& g = p.gates[i];
-        if (g.a != b || is_linear(g) || (g.kind != FG_DENSE && g.kind != FG_PHASE)) continue;
+        if (g.a != b || is_linear(g) || (g.kind != FG_DENSE && g.kind != FG_PHASE && g.kind != FG_KRAUS)) continue;
         if (first && b < p.low) continue;
         want.emplace_back(b < p.low ? i - N : i, b);
       }

@@ -139,13 +139,16 @@ constexpr int kMaxPassGates = 1024, kMaxPassGatesF32 = 96;
 // FG_RENORM: divide the state by its FP64 norm when that exceeds 1e-12, as
 // normalize-state does after a Kraus operator (a record of batched LDS
 // circuits, a barrier between fused passes; never inside a pass).
-enum { FG_DENSE = 0, FG_PHASE = 1, FG_SWAP = 2, FG_BLOCKADE = 3, FG_RENORM = 4 };
+// FG_KRAUS: a noise site of a trajectory program (an operator chosen on the
+// device); only in FGate lists.
+enum { FG_DENSE = 0, FG_PHASE = 1, FG_SWAP = 2, FG_BLOCKADE = 3, FG_RENORM = 4, FG_KRAUS = 5 };
 // Structure of a dense 2x2, which decides the arithmetic it needs per pair:
 // general (16 real multiply-adds), real entries (8), real diagonal with
 // imaginary off-diagonal, as RX (8), or the exchange [[0,1],[1,0]] (none).
 enum { DM_GENERAL = 0, DM_REAL = 1, DM_RX = 2, DM_EXCHANGE = 3 };
 
-// A gate in tile-local bit coordinates.
+// A gate in tile-local bit coordinates. FG_KRAUS: target a, site b, operators
+// cmask .. cmask + sub - 1 of the table, bmask: renormalise afterwards.
 struct FGate {
   int32_t kind;        // FG_*
   int32_t a, b;        // dense/phase target a; swap bits a, b
@@ -196,6 +199,7 @@ enum {
   PO_BLOCKADE = 25,   // phase where exactly one of the bits aux (thread) / kc (slot) is set
   PO_RELAYOUT = 26,   // layout col[0..13] -> layout col[14..27]; flag: PR_*
   PO_SWAP = 27,       // exchange local bits kc and aux where the local bits tmask are set (layout col[0..13])
+  PO_KRAUS = 29,      // + register bit, 29..32: one of cnt noise operators from aux of site kc; flag: renormalise
   PO_BLOCK = 28,      // dense 16x16 on the four register bits (FP32 passes only): table at byte offset aux
 };
 // PO_RELAYOUT: the round trip stays inside each wave; the old layout is the one
@@ -266,31 +270,37 @@ void launch_pass_group(int prec, void* base, uint64_t S, unsigned count, const c
 void launch_norm_ctl(const TileNorm& nb, uint64_t ntiles, bool first, hipStream_t st);
 void launch_fill_group(int prec, void* base, uint64_t S, uint64_t count, hipStream_t st);
 
-// ---- batched small circuits (qsv_batch.hip) -----------------------------------
-constexpr int kBatchThreads = 256;
-
-// One decoded gate of a batched circuit, in index-bit coordinates.
-struct BRec {
-  int32_t kind;        // FG_DENSE, FG_PHASE, FG_SWAP or FG_BLOCKADE
-  int32_t a, b;        // target bit / swap bits
-  int32_t phase_only;
-  uint64_t cmask;      // control bits (all must be 1)
-  uint64_t bmask;      // blockade bits
-  double m[8];         // as FGate
-};
-
-struct BInst {
+// ---- small circuits: a whole register per workgroup (qsv_small.hip) ------------
+// Registers of up to kSmallC128 / kSmallC64 qubits run a whole program in one
+// workgroup of 2^(n - 4) threads, FP64 arithmetic, 2^n * 8 B of LDS.
+constexpr int kSmallC128 = 13, kSmallC64 = 14;
+struct SmallInst {
   int32_t n;
   int32_t pad;
-  uint64_t g0, g1;       // gate records [g0, g1)
+  uint64_t prog;         // byte offset of the program
+  uint64_t io;           // amplitude offset of the state, ~0: none (it starts at |0..0> and is not stored)
   uint64_t t0, t1;       // Z terms [t0, t1)
-  uint64_t out_offset;   // amplitude offset of the final state in the output arena, ~0 for none
+  uint64_t dest;         // energies[dest], ~0: none
 };
-
-int setup_lds_batch(int prec, size_t lds_bytes);
-void launch_lds_batch(int prec, unsigned nblocks, size_t lds_bytes, const BInst* inst, const BRec* gates,
-                      const uint64_t* tz, const double* tc, const int32_t* order, double* energies,
-                      void* out_states, hipStream_t st);
+struct KrausOp {
+  double w;              // selection weight
+  double m[8];
+};
+struct SmallRun {
+  int32_t prec;
+  const char* progs;
+  const SmallInst* insts;   // one per workgroup
+  SmallInst one;            // with PO_KRAUS ops: every workgroup's, states back to back from one.io
+  void* states;
+  const uint64_t* tz;
+  const double* tc;
+  double* energies;
+  const KrausOp* kraus;     // null: no PO_KRAUS ops; trajectory traj0 + workgroup otherwise
+  uint64_t seed, traj0;
+};
+// Launches of one size class: registers of the class of `n` qubits.
+int small_class(int n);
+hipError_t launch_small(const SmallRun& r, int cls, unsigned count, hipStream_t st);
 void launch_zexpect(int prec, const void* psi, uint64_t S, const uint64_t* tz, const double* tc, uint64_t nterms,
                     double* partials, double* out, hipStream_t st);
 // Energies of `count` states of S amplitudes back to back: trange[2y..2y+1]

@@ -1,0 +1,68 @@
+"""Whole-register programs of one workgroup (small fused states, batched
+instances, trajectories) around their size classes: below 4 qubits a thread holds
+empty slots, 10 is the last single wave, 11 leaves waves without amplitudes, 13
+and 14 are the largest."""
+from __future__ import annotations
+
+import math
+
+import numpy as np
+import pytest
+
+from qclojure_amd import circuit as qc
+from qclojure_amd import engine
+from qclojure_amd._abi import OP, QSV_FLAG_FUSE
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [1, 2, 3, 4, 5, 9, 10, 11, 12, 13, 14]
+
+
+def _program(n, rng, count, measure=False):
+    rows = []
+    names = ["H", "RX", "RY", "RZ", "T", "X"] + (["CNOT", "CZ", "CRX", "CRZ", "SWAP", "ISWAP"] if n > 1 else [])
+    names += ["TOFFOLI", "FREDKIN"] if n > 2 else []
+    for k in range(count):
+        name = names[rng.integers(len(names))]
+        q = [int(x) for x in rng.permutation(n)[:3]] + [0, 0, 0]
+        used = 3 if name in ("TOFFOLI", "FREDKIN") else 2 if name in ("CNOT", "CZ", "CRX", "CRZ", "SWAP", "ISWAP") else 1
+        q = [x if i < used else 0 for i, x in enumerate(q[:3])]
+        rows.append((OP[name], q[0], q[1], q[2], 0, float(rng.uniform(0, 2 * math.pi))))
+        if measure and k == count // 2:
+            rows.append((OP["MEASURE"], 0, 0, 0, 1, 0.0))
+    return qc.ops_from_tuples(rows)
+
+
+@pytest.mark.parametrize("n", [s for s in SIZES if s < 13])
+@pytest.mark.parametrize("measure", [False, True])
+def test_fused_state(n, measure):
+    rng = np.random.default_rng(31 * n + measure)
+    first, ops = _program(n, rng, 25), _program(n, rng, 120, measure)
+    with engine.DeviceState(n, "c128") as ref, engine.DeviceState(n, "c128") as a, engine.DeviceState(n, "c64") as b:
+        for s in (ref, a, b):
+            s.apply(first)                       # the fused program starts from a loaded state
+        ref.apply(ops, 0, 5)
+        a.apply(ops, QSV_FLAG_FUSE, 5)
+        b.apply(ops, QSV_FLAG_FUSE, 5)
+        exp = ref.download()
+        assert np.max(np.abs(a.download() - exp)) < 1e-12
+        assert np.max(np.abs(b.download() - exp)) < 1e-5
+
+
+@pytest.mark.parametrize("precision", ["c128", "c64"])
+def test_batched_energies(precision):
+    rng = np.random.default_rng(12)
+    insts, exp = [], []
+    for n in SIZES * 3:
+        ops = _program(n, rng, int(rng.integers(0, 90)))
+        masks = rng.integers(0, 2 ** n, size=int(rng.integers(1, 140)), dtype=np.uint64)
+        coeff = rng.normal(size=len(masks))
+        insts.append((n, ops, (masks, coeff)))
+        with engine.DeviceState(n, "c128") as s:
+            z = s.apply(ops).expect_pauli(["".join("Z" if (int(m) >> q) & 1 else "I" for q in range(n)) for m in masks])
+        exp.append(float(np.dot(z, coeff)))
+    got = engine.batch_expect_z(insts, precision)
+    # FP64 arithmetic for both (13 and 14 qubits of complex128 and complex64 are on either side of
+    # the one-workgroup limit, beyond which complex64 states are stored in FP32 between passes)
+    scale = np.array([np.sum(np.abs(i[2][1])) for i in insts])
+    assert np.max(np.abs(got - exp) / scale) < (1e-12 if precision == "c128" else 1e-6)
