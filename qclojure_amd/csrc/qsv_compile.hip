@@ -14,6 +14,10 @@
 //     one complex product per lane and factor, not one per amplitude. Factors
 //     common to the whole state are collected over a run of passes.
 //   * A unitary 2x2 without structure is diag * real * diag in FP64 passes.
+//   * Bits outside the tile are constants in it: controls and phases on them
+//     are conditions on the tile's base, a CNOT controlled by one is a shift of
+//     the tile's indices, so only dense targets and swapped bits have to be
+//     tile bits at all.
 // Gates are taken from per-bit queues: everything that can run in the current
 // layout runs, then the next layout takes the register bits of the dense gates
 // that wait.
@@ -52,11 +56,11 @@ int reg_op_cost(const POp& op)
 uint32_t op_slot_bits(const POp& op, bool* reg_only)
 {
   if (op.code < PO_DENSE_K) {
-    *reg_only = op.tmask == 0;
+    *reg_only = op.tmask == 0 && op.gm == 0;
     return 1u << (op.code >> 2);
   }
   if (op.code < PO_PHASE) {
-    *reg_only = op.tmask == 0;
+    *reg_only = op.tmask == 0 && op.gm == 0;
     return (1u << (op.code - PO_DENSE_K)) | op.kc;
   }
   *reg_only = op.code < PO_BLOCKADE ? op.cnt == 0 : op.code == PO_BLOCKADE && op.aux == 0;
@@ -91,6 +95,12 @@ void apply_reg_op(const POp& op, C v[16])
 }
 
 struct Compiler {
+  // wave-index bits as functionals of the logical index, and the global bits
+  // whose value in the tile's base flips them
+  struct Waves {
+    uint32_t r[4] = {};
+    uint64_t o[4] = {};
+  };
   const FPass& p;
   const bool f32;
   const int block_cost;
@@ -98,35 +108,46 @@ struct Compiler {
   const uint32_t FULL;
   std::vector<POp> ops;
   std::vector<PTerm> terms;
+  std::vector<PShift> shifts;
   std::vector<float> blk;
   int nblk = 0;
   size_t stage0 = 0;       // first op of the current stage
   uint16_t stage_col[kCols] = {};
-  uint32_t stage_wr[4] = {};
+  Waves stage_wr;
 
   // current layout: logical index columns of thread bits and slots, and the
   // clean layout they started from
   uint32_t ct[kColT] = {}, cr[4] = {};
   uint32_t reg = 0;
-  uint32_t wr[4] = {};     // wave-index bits as functionals of the logical index
+  Waves wr;
+  // shifts of the layout: global bit outside the tile -> local index
+  std::vector<std::pair<int, uint32_t>> co;
   uint32_t row_dirty = 0;  // bits whose value is not one physical bit's
   uint32_t col_dirty = 0;  // bits whose flip is not one physical bit's
   uint16_t last_to[kCols] = {};
   bool have_last = false;
-  uint32_t own[4] = {};    // wave functionals after the last LDS round trip
+  Waves own;               // after the last LDS round trip
   bool have_own = false;
-  uint32_t load_wr[4] = {};
+  Waves load_wr;
   bool synced = false;     // every wave's tile has crossed a workgroup barrier
 
-  // diagonal factors not applied yet: where the bits `mask` are set, `on` and
-  // `off` by the value of bit t (t < 0: `on`)
+  // diagonal factors not applied yet: where the tile bits `mask` and the bits
+  // `gmask` outside it are set, `on` and `off` by the value of tile bit t or
+  // outside bit gt (neither: `on`)
   struct Factor {
     uint32_t mask;
+    uint64_t gmask;
     int t;
+    uint64_t gt;
     C on, off;
     uint32_t bits() const { return mask | (t >= 0 ? 1u << t : 0u); }
   };
   std::vector<Factor> pend;
+  struct Keyed {
+    int key;
+    Factor f;
+  };
+  std::vector<Keyed> now;   // flush's own
   C& scalar;
 
   Compiler(const FPass& p_, bool f32_, int bc, C& sc)
@@ -166,7 +187,9 @@ struct Compiler {
       if ((r >> b) & 1u) cr[i++] = 1u << b;
       else ct[j++] = 1u << b;
     }
-    for (int k = 0; k + 6 < NT; ++k) wr[k] = ct[6 + k];
+    wr = Waves{};
+    for (int k = 0; k + 6 < NT; ++k) wr.r[k] = ct[6 + k];
+    co.clear();
   }
   void lds_columns(uint16_t col[kCols]) const
   {
@@ -178,12 +201,12 @@ struct Compiler {
   {
     stage0 = ops.size();
     lds_columns(stage_col);
-    std::memcpy(stage_wr, wr, sizeof(wr));
+    stage_wr = wr;
   }
-  bool same_waves(const uint32_t a[4], const uint32_t b[4]) const
+  bool same_waves(const Waves& a, const Waves& b) const
   {
     for (int k = 0; k + 6 < NT; ++k)
-      if (a[k] != b[k]) return false;
+      if (a.r[k] != b.r[k] || a.o[k] != b.o[k]) return false;
     return true;
   }
   void relayout(uint32_t r)
@@ -191,9 +214,12 @@ struct Compiler {
     if (block_cost > 0) form_blocks();
     POp& op = emit(PO_RELAYOUT);
     lds_columns(op.col);
-    uint32_t from[4];
-    std::memcpy(from, wr, sizeof(from));
-    if (have_last && !std::memcmp(last_to, op.col, sizeof(last_to))) op.flag |= PR_SAME;
+    const Waves from = wr;
+    if (have_last && co.empty() && !std::memcmp(last_to, op.col, sizeof(last_to))) op.flag |= PR_SAME;
+    op.aux = (uint32_t)shifts.size();   // index now, byte offset when the program is laid out
+    for (const auto& c : co)
+      if (c.second) shifts.push_back(PShift{(uint32_t)c.first, pass_swz(c.second), 0});
+    op.cnt = (int32_t)(shifts.size() - op.aux);
     if (have_own && !same_waves(own, from)) op.flag |= PR_WAIT;
     set_clean(r);
     lds_columns(op.col + kCols);
@@ -201,30 +227,30 @@ struct Compiler {
     have_last = true;
     if (same_waves(from, wr)) op.flag |= PR_LOCAL;
     else synced = true;
-    std::memcpy(own, wr, sizeof(own));
+    own = wr;
     have_own = true;
     begin_stage();
   }
 
   // ---- diagonal factors -----------------------------------------------------
-  void add_term(uint32_t mask, C f)
+  void add_term(uint32_t mask, uint64_t gmask, C f)
   {
     if (f == C(1.0, 0.0)) return;
-    if (mask == 0) {
+    if (mask == 0 && gmask == 0) {
       scalar *= f;
       return;
     }
-    add_two(mask, -1, f, f);
+    add_two(mask, gmask, -1, 0, f, f);
   }
-  void add_two(uint32_t mask, int t, C on, C off)
+  void add_two(uint32_t mask, uint64_t gmask, int t, uint64_t gt, C on, C off)
   {
     for (auto& f : pend)
-      if (f.mask == mask && f.t == t) {
+      if (f.mask == mask && f.gmask == gmask && f.t == t && f.gt == gt) {
         f.on *= on;
         f.off *= off;
         return;
       }
-    pend.push_back(Factor{mask, t, on, off});
+    pend.push_back(Factor{mask, gmask, t, gt, on, off});
   }
   // Can every pending factor with one of the bits `touch` be applied here?
   bool can_flush(uint32_t touch) const
@@ -235,60 +261,72 @@ struct Compiler {
   }
   // Applies the pending factors with one of the bits `touch`, one op per set of
   // slot bits; `with`: a factor of every amplitude joins the group without slot bits.
-  void flush(uint32_t touch, C with = C(1.0, 0.0))
+  void flush(uint32_t touch, C with = C(1.0, 0.0), bool all = false)
   {
-    struct Group { uint32_t kc; int rb; C on, off; std::vector<PTerm> t; };
-    std::vector<Group> groups;
-    auto group = [&](uint32_t kc, int rb) -> Group& {
-      for (auto& g : groups)
-        if (g.kc == kc && g.rb == rb) return g;
-      groups.push_back(Group{kc, rb, C(1.0, 0.0), C(1.0, 0.0), {}});
-      return groups.back();
-    };
+    bool any = all || with != C(1.0, 0.0);
+    for (size_t i = 0; i < pend.size() && !any; ++i) any = (pend[i].bits() & touch) != 0;
+    if (!any) return;
+    // the factors to apply, each with its group: slot mask and, for a target on
+    // a slot, its register bit
+    now.clear();
     size_t w = 0;
+    if (with != C(1.0, 0.0)) now.push_back({0, Factor{0, 0, -1, 0, with, with}});
     for (size_t i = 0; i < pend.size(); ++i) {
-      const Factor f = pend[i];
-      if (!(f.bits() & touch)) {
-        pend[w++] = f;
+      if (!all && !(pend[i].bits() & touch)) {
+        if (w != i) pend[w] = pend[i];
+        ++w;
         continue;
       }
+      const Factor& f = pend[i];
       const bool on_slot = f.t >= 0 && ((reg >> f.t) & 1u);
-      Group& g = group(slot_mask(f.mask), on_slot ? (int)rank_in(reg, f.t) : -1);
-      const uint32_t tm = tid_mask(f.mask), tb = f.t >= 0 && !on_slot ? tid_mask(1u << f.t) : 0u;
-      if (!tm && !tb) {
-        g.on *= f.on;
-        g.off *= f.off;
-        continue;
-      }
-      PTerm q;
-      std::memset(&q, 0, sizeof(q));
-      q.tmask = tm;
-      q.tbit = tb;
-      if (f32) {
-        q.f[0] = (float)f.on.real();
-        q.f[1] = (float)f.on.imag();
-        q.f[2] = (float)f.off.real();
-        q.f[3] = (float)f.off.imag();
-      } else {
-        q.d[0] = f.on.real();
-        q.d[1] = f.on.imag();
-      }
-      g.t.push_back(q);
+      now.push_back({(int)slot_mask(f.mask) | (on_slot ? (int)(rank_in(reg, f.t) + 1) << 4 : 0), f});
     }
     pend.resize(w);
-    if (with != C(1.0, 0.0)) group(0, -1).on *= with;
-    for (auto& g : groups) {
-      if (g.t.empty() && g.on == C(1.0, 0.0) && (g.rb < 0 || g.off == g.on)) continue;
-      POp& op = emit(g.rb < 0 ? PO_PHASE : PO_PHASE2 + g.rb);
-      const C first = g.rb < 0 ? g.on : g.off;
-      op.kc = g.kc;
-      op.m[0] = first.real();
-      op.m[1] = first.imag();
-      op.m[6] = g.on.real();
-      op.m[7] = g.on.imag();
-      op.aux = (uint32_t)terms.size();   // index now, byte offset when the program is laid out
-      op.cnt = (int32_t)g.t.size();
-      terms.insert(terms.end(), g.t.begin(), g.t.end());
+    for (size_t i = 0; i < now.size(); ++i) {
+      const int key = now[i].key;
+      if (key < 0) continue;
+      const uint32_t kc = (uint32_t)key & 15u;
+      const int rb = (key >> 4) - 1;
+      C on(1.0, 0.0), off(1.0, 0.0);
+      const size_t first_term = terms.size();
+      for (size_t j = i; j < now.size(); ++j) {
+        if (now[j].key != key) continue;
+        now[j].key = -1;
+        const Factor& f = now[j].f;
+        const uint32_t tm = tid_mask(f.mask), tb = f.t >= 0 && rb < 0 ? tid_mask(1u << f.t) : 0u;
+        if (!tm && !tb && !f.gmask && !f.gt) {
+          on *= f.on;
+          off *= f.off;
+          continue;
+        }
+        PTerm q;
+        std::memset(&q, 0, sizeof(q));
+        q.tmask = tm;
+        q.tbit = tb;
+        q.gmask = f.gmask;
+        q.gbit = f.gt;
+        if (f32) {
+          q.f[0] = (float)f.on.real();
+          q.f[1] = (float)f.on.imag();
+          q.f[2] = (float)f.off.real();
+          q.f[3] = (float)f.off.imag();
+        } else {
+          q.d[0] = f.on.real();
+          q.d[1] = f.on.imag();
+        }
+        terms.push_back(q);
+      }
+      const int cnt = (int)(terms.size() - first_term);
+      if (!cnt && on == C(1.0, 0.0) && (rb < 0 || off == on)) continue;
+      POp& op = emit(rb < 0 ? PO_PHASE : PO_PHASE2 + rb);
+      const C lead = rb < 0 ? on : off;
+      op.kc = kc;
+      op.m[0] = lead.real();
+      op.m[1] = lead.imag();
+      op.m[6] = on.real();
+      op.m[7] = on.imag();
+      op.aux = (uint32_t)first_term;   // index now, byte offset when the program is laid out
+      op.cnt = cnt;
     }
   }
 
@@ -324,7 +362,7 @@ struct Compiler {
         POp& b = emit(PO_BLOCK);
         b.aux = (uint32_t)nblk++;   // index now, byte offset when the program is laid out
         std::memcpy(b.col, stage_col, sizeof(stage_col));
-        std::memcpy(own, stage_wr, sizeof(own));
+        own = stage_wr;
         have_own = true;
         for (int i : aside) ops.push_back(src[i]);
       } else {
@@ -360,7 +398,8 @@ struct Compiler {
 
   // ---- gates --------------------------------------------------------------------
   // a phase, which can be divided out and applied later without moving the norm
-  static bool usable(C d) { return std::fabs(std::abs(d) - 1.0) < 1e-9; }
+  static bool usable(C d) { return is_phase(d.real(), d.imag()); }
+  static C over(C a, C b) { return a * std::conj(b) / std::norm(b); }
   static uint32_t gate_bits(const FGate& g)
   {
     if (g.kind == FG_KRAUS) return 1u << g.a;
@@ -372,30 +411,28 @@ struct Compiler {
   // CNOTs and plain (phased) swaps
   static bool is_linear(const FGate& g)
   {
-    if (g.kind == FG_DENSE) return g.sub == DM_EXCHANGE && __builtin_popcount(g.cmask) == 1;
-    return g.kind == FG_SWAP && g.cmask == 0 && usable(C(g.m[0], g.m[1]));
+    if (g.kind == FG_DENSE)
+      return g.sub == DM_EXCHANGE && __builtin_popcount(g.cmask) + __builtin_popcountll(g.gmask) == 1;
+    return g.kind == FG_SWAP && g.cmask == 0 && g.gmask == 0 && usable(C(g.m[0], g.m[1]));
   }
-  // A diagonal gate as factors on bit masks; false when its first entry is no
-  // phase and cannot be divided out.
-  bool take_phase(const FGate& g)
+  // A diagonal gate as factors on bit masks (its first entry is 1 or a phase).
+  void take_phase(const FGate& g)
   {
     const C d0(g.m[0], g.m[1]), d1(g.m[6], g.m[7]);
-    const uint32_t t = 1u << g.a;
+    const uint32_t t = g.a >= 0 ? 1u << g.a : 0u;
     if (g.sub) {   // d0 == 1
-      add_term(g.cmask | t, d1);
-      return true;
+      add_term(g.cmask | t, g.gmask | g.gt, d1);
+      return;
     }
     // FP32 passes keep both entries: rounded alike (a Z rotation's are
     // conjugates) they leave the weights of the two halves as they are, where
     // one rounded factor on one half moves them against each other
     if (f32) {
-      add_two(g.cmask, g.a, d1, d0);
-      return true;
+      add_two(g.cmask, g.gmask, g.a, g.gt, d1, d0);
+      return;
     }
-    if (!usable(d0)) return false;
-    add_term(g.cmask, d0);
-    add_term(g.cmask | t, d1 / d0);
-    return true;
+    add_term(g.cmask, g.gmask, d0);
+    add_term(g.cmask | t, g.gmask | g.gt, over(d1, d0));
   }
 
   bool run_linear(const FGate& g)
@@ -412,26 +449,43 @@ struct Compiler {
       }
       for (int j = 0; j < NT; ++j) ct[j] = sw(ct[j]);
       for (auto& c : cr) c = sw(c);
-      for (auto& w : wr) w = sw(w);
+      for (auto& w : wr.r) w = sw(w);
+      for (auto& c : co) c.second = sw(c.second);
       const uint32_t ab = (1u << a) | (1u << b);
       row_dirty |= ab;
       col_dirty |= ab;
       const C ph(g.m[0], g.m[1]);
       if (ph != C(1.0, 0.0)) {
-        add_term(1u << a, ph);
-        add_term(1u << b, ph);
-        add_term(ab, 1.0 / (ph * ph));
+        add_term(1u << a, 0, ph);
+        add_term(1u << b, 0, ph);
+        add_term(ab, 0, 1.0 / (ph * ph));
       }
       return true;
     }
     const uint32_t t = 1u << g.a, c = g.cmask;
     if (!can_flush(t)) return false;
     flush(t);
+    if (g.gmask) {   // the control outside the tile: a shift
+      const int b = __builtin_ctzll(g.gmask);
+      bool found = false;
+      for (auto& x : co)
+        if (x.first == b) {
+          x.second ^= t;
+          found = true;
+        }
+      if (!found) co.emplace_back(b, t);
+      for (int k = 0; k < 4; ++k)
+        if (wr.r[k] & t) wr.o[k] ^= g.gmask;
+      row_dirty |= t;
+      return true;
+    }
     for (int j = 0; j < NT; ++j)
       if (ct[j] & c) ct[j] ^= t;
     for (auto& x : cr)
       if (x & c) x ^= t;
-    for (auto& w : wr)
+    for (auto& x : co)
+      if (x.second & c) x.second ^= t;
+    for (auto& w : wr.r)
       if (w & t) w ^= c;
     row_dirty |= t;
     col_dirty |= t | c;
@@ -461,7 +515,7 @@ struct Compiler {
       op.sc[0] = g.m[0];
       op.sc[1] = g.m[1];
       lds_columns(op.col);
-      std::memcpy(own, wr, sizeof(own));
+      own = wr;
       have_own = true;
       synced = true;
       return true;
@@ -485,22 +539,22 @@ struct Compiler {
     if (g.kind == FG_PHASE) m[2] = m[3] = m[4] = m[5] = 0.0;
     // a unitary without structure: e^{ia} diag(1, f1) [[c, -s], [s, c]] diag(1, f0)
     C f0(1.0, 0.0), f1(1.0, 0.0);
-    if (!f32 && sub == DM_GENERAL && g.cmask == 0 && g.kind == FG_DENSE) {
+    if (!f32 && sub == DM_GENERAL && g.cmask == 0 && g.gmask == 0 && g.kind == FG_DENSE) {
       const C m00(m[0], m[1]), m01(m[2], m[3]), m10(m[4], m[5]), m11(m[6], m[7]);
       const double c = std::abs(m00), s = std::abs(m10), s1 = std::abs(m01);
       if (c > 1e-8 && s > 1e-8 && s1 > 1e-8) {
         const C u = m00 / c;
-        f1 = m10 / (s * u);
-        f0 = -m01 / (s1 * u);
+        f1 = over(m10, s * u);
+        f0 = over(-m01, s1 * u);
         const double n = std::sqrt(c * c + s * s);
         // equal to the matrix to the last places, or taken as it is
-        const double e = std::max({std::fabs(n - 1.0), std::abs(m01 + u * f0 * s), std::abs(m11 - u * f0 * f1 * c)});
-        if (e < 1e-15) {
+        const double e = std::max({(n - 1.0) * (n - 1.0), std::norm(m01 + u * f0 * s), std::norm(m11 - u * f0 * f1 * c)});
+        if (e < 1e-30) {
           scalar *= u;
           sub = DM_REAL;
           const double r[8] = {c, 0, -s, 0, s, 0, c, 0};
           std::memcpy(m, r, sizeof(m));
-          add_term(t, f0);
+          add_term(t, 0, f0);
         } else {
           f0 = f1 = C(1.0, 0.0);
         }
@@ -511,8 +565,9 @@ struct Compiler {
     POp& op = emit(kc ? PO_DENSE_K + rb : PO_DENSE + 4 * rb + sub);
     op.kc = kc;
     op.tmask = tid_mask(g.cmask);
+    op.gm = g.gmask;
     std::memcpy(op.m, m, sizeof(m));
-    add_term(t, f1);
+    add_term(t, 0, f1);
     return true;
   }
 
@@ -547,80 +602,95 @@ struct Compiler {
   void run(PHead& h, bool last)
   {
     const int N = (int)p.gates.size();
-    // per-bit queues of the gates in program order
+    // Per-bit queues of the gates in program order. A gate is ready when it is
+    // the front of all its bits' queues; `ready` holds, per class of gates, the
+    // lowest bits of the ready ones.
+    enum { PHASE, LINEAR, OTHER };
     std::vector<int> queue[16];
     std::vector<uint32_t> bits(N);
-    std::vector<char> done(N, 0);
+    std::vector<int8_t> cls(N), waits(N);
+    uint32_t ready[3] = {};
+    int left = N;
+    ops.reserve(2 * N + 16);
+    size_t head[16] = {};
+    auto at_front = [&](int i) {
+      if (--waits[i] == 0) ready[cls[i]] |= bits[i] & -bits[i];
+    };
     for (int i = 0; i < N; ++i) {
-      bits[i] = gate_bits(p.gates[i]);
+      const FGate& g = p.gates[i];
+      bits[i] = gate_bits(g);
+      cls[i] = (int8_t)(g.kind == FG_PHASE && (g.sub || usable(C(g.m[0], g.m[1]))) ? PHASE
+                        : is_linear(g)                                             ? LINEAR
+                                                                                   : OTHER);
+      if (!bits[i]) {   // a phase on bits outside the tile: one factor per tile
+        take_phase(g);
+        --left;
+        continue;
+      }
+      waits[i] = (int8_t)__builtin_popcount(bits[i]);
       for (uint32_t m = bits[i]; m; m &= m - 1) queue[__builtin_ctz(m)].push_back(i);
     }
-    size_t head[16] = {};
-    int left = N;
-    auto front = [&](int b) -> int { return head[b] < queue[b].size() ? queue[b][head[b]] : -1; };
-    auto ready = [&](int i) {
-      for (uint32_t m = bits[i]; m; m &= m - 1)
-        if (front(__builtin_ctz(m)) != i) return false;
-      return true;
-    };
+    for (int b = 0; b < TB; ++b)
+      if (!queue[b].empty()) at_front(queue[b][0]);
     auto consume = [&](int i) {
-      done[i] = 1;
       --left;
-      for (uint32_t m = bits[i]; m; m &= m - 1) ++head[__builtin_ctz(m)];
+      ready[cls[i]] &= ~(bits[i] & -bits[i]);
+      for (uint32_t m = bits[i]; m; m &= m - 1) {
+        const int b = __builtin_ctz(m);
+        if (++head[b] < queue[b].size()) at_front(queue[b][head[b]]);
+      }
+    };
+    auto ready_gate = [&](uint32_t m) {
+      const int b = __builtin_ctz(m);
+      return queue[b][head[b]];
     };
     // the next layout: the targets of waiting dense gates. `first`: the load
     // layout, whose lanes must cover the low run; later ones take low bits as
     // soon as they are wanted, so that the last layout can store.
     auto next_regs = [&](bool first) {
-      std::vector<std::pair<int, int>> want;   // (order, bit)
-      for (int b = 0; b < TB; ++b) {
-        const int i = front(b);
-        if (i < 0 || !ready(i)) continue;
+      int want[16], n = 0;   // gates, those on low bits before the others
+      for (uint32_t m = ready[OTHER]; m; m &= m - 1) {
+        const int i = ready_gate(m);
         const FGate& g = p.gates[i];
-        if (g.a != b || is_linear(g) || (g.kind != FG_DENSE && g.kind != FG_PHASE && g.kind != FG_KRAUS)) continue;
-        if (first && b < p.low) continue;
-        want.emplace_back(b < p.low ? i - N : i, b);
+        if (g.kind == FG_SWAP || g.kind == FG_BLOCKADE || (first && g.a < p.low)) continue;
+        want[n++] = g.a < p.low ? i - N : i;
       }
-      std::sort(want.begin(), want.end());
+      std::sort(want, want + n);
       uint32_t r = 0;
-      for (const auto& w : want)
-        if (__builtin_popcount(r) < 4) r |= 1u << w.second;
+      for (int k = 0; k < n && k < 4; ++k) r |= 1u << p.gates[want[k] < 0 ? want[k] + N : want[k]].a;
       return r;
     };
     // gates that wait for nothing: diagonal ones leave the queues at once
     auto drain_phases = [&]() {
-      bool any = false;
-      for (int b = 0; b < TB; ++b)
-        for (int i = front(b); i >= 0; i = front(b)) {
-          const FGate& g = p.gates[i];
-          if (g.kind != FG_PHASE || !ready(i) || !take_phase(g)) break;
-          consume(i);
-          any = true;
-        }
+      const bool any = ready[PHASE] != 0;
+      while (ready[PHASE]) {
+        const int i = ready_gate(ready[PHASE]);
+        take_phase(p.gates[i]);
+        consume(i);
+      }
       return any;
     };
-    while (drain_phases()) {
-    }
+    drain_phases();
     set_clean(fill(next_regs(true)));
     if (!coalesced()) set_clean(fill(0));
     global_columns(h.gload);
-    std::memcpy(load_wr, wr, sizeof(load_wr));
+    load_wr = wr;
     begin_stage();
     while (left) {
       bool any = true, moved = false;
       while (any) {   // everything this layout can run
         any = drain_phases();
-        for (int b = 0; b < TB; ++b) {
-          const int i = front(b);
-          if (i < 0 || is_linear(p.gates[i]) || !ready(i) || !run_gate(p.gates[i])) continue;
+        for (uint32_t m = ready[OTHER]; m; m &= m - 1) {
+          const int i = ready_gate(m);
+          if (!run_gate(p.gates[i])) continue;
           consume(i);
           any = true;
         }
         moved |= any;
       }
-      for (int b = 0; b < TB; ++b) {
-        const int i = front(b);
-        if (i < 0 || !is_linear(p.gates[i]) || !ready(i) || !run_linear(p.gates[i])) continue;
+      for (uint32_t m = ready[LINEAR]; m; m &= m - 1) {
+        const int i = ready_gate(m);
+        if (!run_linear(p.gates[i])) continue;
         consume(i);
         moved = true;
       }
@@ -633,10 +703,18 @@ struct Compiler {
       scalar = C(1.0, 0.0);
     }
     if (!can_flush(FULL)) relayout(fill(0));
-    flush(FULL, g);
+    flush(FULL, g, true);
     if (!coalesced()) relayout(fill(0));
     else if (block_cost > 0) form_blocks();
     global_columns(h.gstore);
+    h.shift_off = (int32_t)shifts.size();   // index now, byte offset when the program is laid out
+    for (const auto& c : co)
+      if (c.second) {
+        uint64_t v = 0;
+        for (uint32_t l = c.second; l; l &= l - 1) v |= 1ull << p.pos[__builtin_ctz(l)];
+        shifts.push_back(PShift{(uint32_t)c.first, 0, v});
+      }
+    h.nshift = (int32_t)shifts.size() - h.shift_off;
     // the tile is updated in place: a wave may overwrite amplitudes that another
     // one has not loaded yet when the layouts name the waves differently
     h.store_wait = !synced && !same_waves(load_wr, wr) ? 1 : 0;
@@ -656,9 +734,12 @@ size_t compile_pass(const FPass& p, bool f32, int block_cost, std::complex<doubl
   c.run(h, last);
   h.nops = (int32_t)c.ops.size();
   const size_t terms_at = (sizeof(PHead) + (c.ops.size() + 1) * sizeof(POp) + 31) & ~(size_t)31;
-  const size_t blk_at = terms_at + c.terms.size() * sizeof(PTerm);
+  const size_t shifts_at = terms_at + c.terms.size() * sizeof(PTerm);
+  const size_t blk_at = shifts_at + c.shifts.size() * sizeof(PShift);
+  h.shift_off = (int32_t)(shifts_at + h.shift_off * sizeof(PShift));
   for (POp& op : c.ops) {
     if (op.code >= PO_PHASE && op.code < PO_BLOCKADE) op.aux = (uint32_t)(terms_at + op.aux * sizeof(PTerm));
+    else if (op.code == PO_RELAYOUT) op.aux = (uint32_t)(shifts_at + op.aux * sizeof(PShift));
     else if (op.code == PO_BLOCK) op.aux = (uint32_t)(blk_at + op.aux * kBlockTable);
     if (f32 && (op.code <= PO_BLOCKADE)) {
       float f[8];
@@ -675,6 +756,7 @@ size_t compile_pass(const FPass& p, bool f32, int block_cost, std::complex<doubl
   std::memcpy(d, &h, sizeof(h));
   if (!c.ops.empty()) std::memcpy(d + sizeof(PHead), c.ops.data(), c.ops.size() * sizeof(POp));
   if (!c.terms.empty()) std::memcpy(d + terms_at, c.terms.data(), c.terms.size() * sizeof(PTerm));
+  if (!c.shifts.empty()) std::memcpy(d + shifts_at, c.shifts.data(), c.shifts.size() * sizeof(PShift));
   if (!c.blk.empty()) std::memcpy(d + blk_at, c.blk.data(), c.blk.size() * sizeof(float));
   return at;
 }

@@ -142,6 +142,13 @@ constexpr int kMaxPassGates = 1024, kMaxPassGatesF32 = 96;
 // FG_KRAUS: a noise site of a trajectory program (an operator chosen on the
 // device); only in FGate lists.
 enum { FG_DENSE = 0, FG_PHASE = 1, FG_SWAP = 2, FG_BLOCKADE = 3, FG_RENORM = 4, FG_KRAUS = 5 };
+// Is re + i im a phase, up to rounding? Such a first entry of a diagonal gate
+// can be divided out.
+inline bool is_phase(double re, double im)
+{
+  const double d = re * re + im * im - 1.0;
+  return d < 2e-9 && d > -2e-9;
+}
 // Structure of a dense 2x2, which decides the arithmetic it needs per pair:
 // general (16 real multiply-adds), real entries (8), real diagonal with
 // imaginary off-diagonal, as RX (8), or the exchange [[0,1],[1,0]] (none).
@@ -154,6 +161,8 @@ struct FGate {
   int32_t a, b;        // dense/phase target a; swap bits a, b
   uint32_t cmask;      // local control bits (all must be 1)
   uint32_t bmask;      // blockade bits
+  uint64_t gmask;      // control bits outside the tile (global; all must be 1)
+  uint64_t gt;         // FG_PHASE with its target outside the tile (a < 0): the global target bit
   int32_t sub;         // FG_PHASE: 1 when d0 == 1; FG_DENSE: DM_* structure of m
   double m[8];         // dense: row-major 2x2; phase: d0 = m[0..1], d1 = m[6..7]; swap/blockade: phase m[0..1]
 };
@@ -213,9 +222,10 @@ struct POp {
   int32_t code;
   uint32_t tmask;     // thread-id bits that must be set (thread-bit controls)
   uint32_t kc;        // slot bits that must be set (register-bit controls)
-  uint32_t aux;       // PO_PHASE, PO_PHASE2: byte offset of the terms
-  int32_t cnt;        // PO_PHASE, PO_PHASE2: number of terms
+  uint32_t aux;       // PO_PHASE, PO_PHASE2, PO_RELAYOUT: byte offset of the terms or shifts
+  int32_t cnt;        // ... and their number
   int32_t flag;
+  uint64_t gm;        // global bits outside the tile that must be set, else the op is skipped
   double sc[2];       // PO_SWAP: the exchanged amplitudes' phase
   union {
     double m[8];      // row-major 2x2; PO_PHASE, PO_BLOCKADE: a factor in m[0..1]; PO_PHASE2: clear m[0..1], set m[6..7]
@@ -223,19 +233,28 @@ struct POp {
     uint16_t col[32]; // PO_RELAYOUT, PO_SWAP and PO_BLOCK (float programs keep no m there)
   };
 };
-static_assert(sizeof(POp) == 104, "the kernel reads ops as 26 dwords");
-// A factor of PO_PHASE or PO_PHASE2 on the lanes with all bits of tmask set. In
-// FP32 programs it has two values: PO_PHASE takes `on` where the thread bit
-// tbit is set and `off` where it is clear (tbit 0: always `on`), PO_PHASE2 `on`
-// for the set and `off` for the clear register bit.
+static_assert(sizeof(POp) == 112, "ops are read in aligned dwords");
+// A factor of PO_PHASE or PO_PHASE2 on the lanes with all bits of tmask set, in
+// tiles with all bits of gmask set. In FP32 programs it has two values: PO_PHASE
+// takes `on` where the thread bits tbit and the tile bits gbit are set and `off`
+// otherwise (both 0: always `on`), PO_PHASE2 `on` for the set and `off` for the
+// clear register bit.
 struct PTerm {
   uint32_t tmask, tbit;
+  uint64_t gmask, gbit;
   union {
     double d[2];      // FP64 programs
     float f[4];       // FP32 programs: on, off
   };
 };
-static_assert(sizeof(PTerm) == 24, "terms are 24 bytes");
+static_assert(sizeof(PTerm) == 40, "terms are 40 bytes");
+// The indices of a tile whose base has global bit `bit` set are shifted (XOR):
+// by LDS element `col` where a relayout leaves the layout, by global offset `g`
+// at the store. CNOTs whose control lies outside the tile leave these.
+struct PShift {
+  uint32_t bit, col;
+  uint64_t g;
+};
 // PO_BLOCK tables per pass: 4 steps x 64 lanes of (re, im) FP32, lane l of
 // step kk holding U[l % 16][4 kk + l / 16] (the A operand of
 // v_mfma_f32_16x16x4f32), U indexed by slot.
@@ -246,11 +265,12 @@ struct PHead {
   int32_t renorm;                   // FP_RENORM_* bits
   int32_t bytes;                    // of the whole program
   int32_t store_wait;               // waves store where others load, with no barrier between: wait first
+  int32_t nshift, shift_off;        // shifts of the store
   int32_t sorted_pos[16];           // the tile's global bits in ascending order
   uint64_t gload[kCols], gstore[kCols];   // global index columns of the load and store layouts
 };
 // In memory: the header, the ops and one unread op (the kernel fetches an op
-// ahead), the terms, the block tables.
+// ahead), the terms, the shifts, the block tables.
 // A program appended to `out` (at a multiple of 256 bytes); returns its offset.
 // f32: an FP32 pass; block_cost > 0: runs of register-bit ops that cost the
 // vector units at least that become PO_BLOCK ops. `scalar` collects factors

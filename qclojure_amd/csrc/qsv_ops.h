@@ -35,6 +35,7 @@ template <typename A> struct OpRegs {
   int32_t code;
   uint32_t tmask, kc, aux;
   int32_t cnt, flag;
+  uint64_t gm;
   uint32_t w[16];   // the union: coefficients or packed columns
   __device__ __forceinline__ A m(int i) const
   {
@@ -52,6 +53,7 @@ __device__ __forceinline__ void fetch(OpRegs<A>& o, const POp* p)
   o.aux = p->aux;
   o.cnt = p->cnt;
   o.flag = p->flag;
+  o.gm = p->gm;
   const uint32_t* w = reinterpret_cast<const uint32_t*>(p->m);
 #pragma unroll
   for (int i = 0; i < 16; ++i) o.w[i] = w[i];
@@ -194,9 +196,10 @@ __device__ __forceinline__ double site_uniform(uint64_t seed, uint64_t k)
 
 // Runs the ops of a program on a workgroup's tile of 2^(NT + 4) amplitudes.
 // smem: 8 bytes per amplitude, and 8 per wave where there are PO_KRAUS ops.
+// base: the tile's base index (its bits outside the tile).
 // kr: the trajectory a program with PO_KRAUS ops runs (null otherwise).
 template <typename A, int NT, bool KRAUS = false>
-__device__ __forceinline__ void run_ops(const char* __restrict__ prog, char* smem, Slots<A>& x,
+__device__ __forceinline__ void run_ops(const char* __restrict__ prog, char* smem, uint64_t base, Slots<A>& x,
                                         const KrausRun* kr = nullptr)
 {
   constexpr bool SPLIT = sizeof(A) == 8;
@@ -216,6 +219,7 @@ __device__ __forceinline__ void run_ops(const char* __restrict__ prog, char* sme
   for (int i = 0; i < nops; ++i) {
     const OpRegs<A> op = nx;
     fetch(nx, ops + i + 1);   // the program ends with one unread op
+    if (op.gm & ~base) continue;   // a control outside the tile is not set
     const int code = op.code;
     // One flat dispatch whose cases share no code: a case that is merged with
     // another in part makes the compiler keep a second copy of the tile.
@@ -291,7 +295,7 @@ __device__ __forceinline__ void run_ops(const char* __restrict__ prog, char* sme
         const PTerm* tm = reinterpret_cast<const PTerm*>(prog + op.aux);
         for (int j = 0; j < op.cnt; ++j) {
           const PTerm& q = tm[j];
-          const bool on = (t & q.tmask) == q.tmask;
+          const bool on = (t & q.tmask) == q.tmask && !(q.gmask & ~base);
           cmul(on ? q.f[0] : (A)1, on ? q.f[1] : (A)0, fr, fi);
           cmul(on ? q.f[2] : (A)1, on ? q.f[3] : (A)0, gr, gi);
         }
@@ -368,11 +372,11 @@ __device__ __forceinline__ void run_ops(const char* __restrict__ prog, char* sme
       const PTerm* tm = reinterpret_cast<const PTerm*>(prog + op.aux);
       for (int j = 0; j < op.cnt; ++j) {
         const PTerm& q = tm[j];
-        const bool on = (t & q.tmask) == q.tmask;
+        const bool on = (t & q.tmask) == q.tmask && !(q.gmask & ~base);
         if constexpr (SPLIT) {
           cmul(on ? (A)q.d[0] : (A)1, on ? (A)q.d[1] : (A)0, fr, fi);
         } else {
-          const bool set = (t & q.tbit) == q.tbit;
+          const bool set = (t & q.tbit) == q.tbit && !(q.gbit & ~base);
           const A qr = set ? q.f[0] : q.f[2], qi = set ? q.f[1] : q.f[3];
           cmul(on ? qr : (A)1, on ? qi : (A)0, fr, fi);
         }
@@ -409,9 +413,11 @@ __device__ __forceinline__ void run_ops(const char* __restrict__ prog, char* sme
     case PO_RELAYOUT: {
       const bool local = (op.flag & PR_LOCAL) != 0;
       if (op.flag & PR_WAIT) __syncthreads();
-      const uint32_t fb = (op.flag & PR_SAME)
-                              ? lb
-                              : thread_part<NT>(t, [&](int j) __attribute__((always_inline)) { return op.col(j); }) << 3;
+      uint32_t fb = (op.flag & PR_SAME)
+                        ? lb
+                        : thread_part<NT>(t, [&](int j) __attribute__((always_inline)) { return op.col(j); }) << 3;
+      const PShift* sh = reinterpret_cast<const PShift*>(prog + op.aux);
+      for (int j = 0; j < op.cnt; ++j) fb ^= (base >> sh[j].bit) & 1u ? sh[j].col << 3 : 0u;
       lb = thread_part<NT>(t, [&](int j) __attribute__((always_inline)) { return op.col(kCols + j); }) << 3;
       auto from = [&](auto kk) __attribute__((always_inline)) {
         return slot_part<decltype(kk)::value>(

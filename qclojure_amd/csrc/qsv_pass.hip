@@ -121,14 +121,16 @@ __global__ __launch_bounds__(kThreads, sizeof(A) == 4 ? 5 : 4) void k_pass(typen
   }
 
   if (gridDim.x <= kTouchTiles) touch(prog, h.bytes);
-  run_ops<A, NT>(prog, smem, x);
+  run_ops<A, NT>(prog, smem, base, x);
   if (h.store_wait) {   // every wave's loads are done before any store
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
   }
 
   {
-    const uint64_t ga = base ^ global_part<NT>(t, h.gstore);
+    uint64_t ga = base ^ global_part<NT>(t, h.gstore);
+    const PShift* sh = reinterpret_cast<const PShift*>(prog + h.shift_off);
+    for (int j = 0; j < h.nshift; ++j) ga ^= (base >> sh[j].bit) & 1u ? sh[j].g : 0ull;
     each<0, kSlots>([&](auto kk) __attribute__((always_inline)) {
       constexpr int k = decltype(kk)::value;
       T v;

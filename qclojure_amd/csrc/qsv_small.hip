@@ -155,9 +155,9 @@ __global__ __launch_bounds__(1 << NT, 4) void k_small(const char* __restrict__ p
   }
   if constexpr (KRAUS) {
     const KrausRun kr{kraus, seed, traj0 + blockIdx.x, live};
-    run_ops<double, NT, true>(prog, smem, x, &kr);
+    run_ops<double, NT, true>(prog, smem, 0, x, &kr);
   } else {
-    run_ops<double, NT, false>(prog, smem, x);
+    run_ops<double, NT, false>(prog, smem, 0, x);
   }
   if (h.store_wait) {   // every wave's loads are done before any store
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");

@@ -57,3 +57,36 @@ def test_deferred_gates(kind, n, count):
         assert a.compare(ref)["max_abs_diff"] < 1e-12
         for s in (f32, f64):
             assert s.compare(ref)["max_abs_diff"] < 1e-5
+
+
+@pytest.mark.parametrize("n,targets", [(13, 1), (13, 8), (16, 4), (20, 8), (24, 11)])
+def test_bits_outside_the_tile(n, targets):
+    """Few targets, controls and phases on every qubit: most of them lie outside
+    a pass's tile, where a control is a condition and a CNOT shifts the indices."""
+    rng = np.random.default_rng(100 * n + targets)
+    pool = [int(q) for q in rng.choice(n, targets, replace=False)]
+    rows = [(OP["H"], q, 0, 0, 0, 0.0) for q in range(n)]
+    for _ in range(250):
+        ang = float(rng.uniform(0, 2 * math.pi))
+        t = pool[int(rng.integers(targets))]
+        c, d = (int(q) for q in rng.choice([q for q in range(n) if q != t], 2, replace=False))
+        name = ["CNOT", "CNOT", "CRX", "CRY", "CRZ", "CZ", "RY", "RX", "RZ", "TOFFOLI", "RYDBERG_CPHASE",
+                "FREDKIN"][rng.integers(12)]
+        if name == "TOFFOLI":
+            rows.append((OP[name], c, d, t, 0, 0.0))
+        elif name == "FREDKIN":
+            rows.append((OP[name], c, t, d, 0, 0.0) if rng.uniform() < 0.2 else (OP["T"], d, 0, 0, 0, 0.0))
+        elif name == "RZ":
+            rows.append((OP[name], d, 0, 0, 0, ang))
+        else:
+            rows.append((OP[name], c if name[0] == "C" or name[:3] == "RYD" else t,
+                         t if name[0] == "C" or name[:3] == "RYD" else 0, 0, 0, ang))
+    ops = qc.ops_from_tuples(rows)
+    with engine.DeviceState(n, "c128") as ref, engine.DeviceState(n, "c128") as a, \
+            engine.DeviceState(n, "c64") as f32:
+        ref.apply(ops)
+        a.apply(ops, QSV_FLAG_FUSE)
+        f32.apply(ops, QSV_FLAG_FUSE)
+        # as above: a few hundred roundings of amplitudes of at most 1
+        assert a.compare(ref)["max_abs_diff"] < 1e-12
+        assert f32.compare(ref)["max_abs_diff"] < 1e-5
