@@ -321,9 +321,11 @@ struct SmallRun {
 // Launches of one size class: registers of the class of `n` qubits.
 int small_class(int n);
 hipError_t launch_small(const SmallRun& r, int cls, unsigned count, hipStream_t st);
+// <H> = sum_k c_k <Z-string_k> of one state of S >= 2^12 amplitudes into out[0];
+// partials holds kReduceBlocks doubles.
 void launch_zexpect(int prec, const void* psi, uint64_t S, const uint64_t* tz, const double* tc, uint64_t nterms,
                     double* partials, double* out, hipStream_t st);
-// Energies of `count` states of S amplitudes back to back: trange[2y..2y+1]
+// The same of `count` states of S amplitudes back to back: trange[2y..2y+1]
 // = term range of state y, partials >= count * blocks_per_state doubles,
 // out[dest[y]] = <H> of state y.
 void launch_zexpect_group(int prec, const void* base, uint64_t S, unsigned count, const uint64_t* tz,
