@@ -5,6 +5,8 @@
 // c64 = float2 (8 B). Reference qubit q is index bit b = n-1-q.
 #include "qsv_internal.h"
 
+#include <algorithm>
+
 namespace qsv {
 
 template <typename R> struct VT;
@@ -469,19 +471,64 @@ __device__ __forceinline__ uint64_t gather_bits(uint64_t i, const PosArgs& p)
   return o;
 }
 
+// Weights of the outcomes of m <= 12 measured bits. A block takes `span`
+// consecutive amplitudes (a power of two), thread t those whose index is t
+// modulo kBlock. It walks them with the measured bits outermost, so a sum stays
+// in a register while the outcome does, eight loads in flight; it is then summed
+// over the lanes with the same outcome and added to the block's LDS histogram.
+// One LDS atomic per amplitude before, up to 64 lanes on one address: the three
+// measured bits of 24 qubits, complex128, 102 us; now 49 us, the time of the read.
 template <typename R>
 __global__ __launch_bounds__(kBlock) void k_outcome_hist_lds(const typename VT<R>::T* __restrict__ psi, uint64_t S,
-                                                              PosArgs p, double* __restrict__ hist)
+                                                              uint64_t span, uint64_t mask, PosArgs p,
+                                                              double* __restrict__ hist)
 {
-  __shared__ double h[4096];
+  extern __shared__ double h[];
+  constexpr int kFly = 8;
   const int no = 1 << p.m;
   for (int k = threadIdx.x; k < no; k += kBlock) h[k] = 0.0;
   __syncthreads();
-  const uint64_t stride = (uint64_t)gridDim.x * kBlock;
-  for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < S; i += stride) {
+  const uint32_t t = threadIdx.x;
+  const uint64_t first = (uint64_t)blockIdx.x * span + t;
+  const uint64_t inside = (span - 1) & ~(uint64_t)(kBlock - 1);   // the bits a thread walks
+  const uint64_t outer = inside & mask, inner = inside & ~mask;
+  const uint64_t runs = 1ull << __popcll(inner);
+  auto weight = [&](uint64_t i) {
     const auto a = psi[i];
-    atomicAdd(&h[gather_bits(i, p)], (double)a.x * a.x + (double)a.y * a.y);
-  }
+    return (double)a.x * a.x + (double)a.y * a.y;
+  };
+  uint64_t o = 0;
+  do {
+    double acc = 0.0;
+    const uint64_t at = first + o;
+    if (at < S) {
+      uint64_t k = 0;
+      if (runs >= (uint64_t)kFly) {
+        for (uint64_t l = 0; l < runs; l += kFly) {
+          double w[kFly];
+#pragma unroll
+          for (int f = 0; f < kFly; ++f) {
+            w[f] = weight(at + k);
+            k = (k - inner) & inner;   // the next subset of the inner bits
+          }
+          acc += ((w[0] + w[1]) + (w[2] + w[3])) + ((w[4] + w[5]) + (w[6] + w[7]));
+        }
+      } else {
+        for (uint64_t l = 0; l < runs; ++l) {
+          acc += weight(at + k);
+          k = (k - inner) & inner;
+        }
+      }
+    }
+    const uint32_t lane = t & 63u, same = ~(uint32_t)mask & 63u;   // lane bits the outcome does not see
+#pragma unroll
+    for (int b = 0; b < 6; ++b) {
+      const double v = __shfl_xor(acc, 1 << b, 64);
+      if ((same >> b) & 1u) acc += v;
+    }
+    if (!(lane & same) && at < S) atomicAdd(&h[gather_bits(at, p)], acc);
+    o = (o - outer) & outer;
+  } while (o);
   __syncthreads();
   for (int k = threadIdx.x; k < no; k += kBlock)
     if (h[k] != 0.0) atomicAdd(&hist[k], h[k]);
@@ -505,19 +552,21 @@ __global__ __launch_bounds__(kBlock) void k_zero_f64(double* __restrict__ v, uin
   for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += stride) v[i] = 0.0;
 }
 
+// Scales the amplitudes whose measured bits (mask) read `want`; the others are
+// set to zero unread. Three measured bits of 24 qubits, complex128: 65 us with
+// every amplitude read, now 37 us.
 template <typename R>
-__global__ __launch_bounds__(kBlock) void k_collapse(typename VT<R>::T* __restrict__ psi, uint64_t S, PosArgs p,
-                                                      uint64_t sel, R scale)
+__global__ __launch_bounds__(kBlock) void k_collapse(typename VT<R>::T* __restrict__ psi, uint64_t S, uint64_t mask,
+                                                      uint64_t want, R scale)
 {
   const uint64_t stride = (uint64_t)gridDim.x * kBlock;
   for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < S; i += stride) {
-    auto a = psi[i];
-    if (gather_bits(i, p) == sel) {
+    typename VT<R>::T a;
+    a.x = a.y = R(0);
+    if ((i & mask) == want) {
+      a = psi[i];
       a.x *= scale;
       a.y *= scale;
-    } else {
-      a.x = R(0);
-      a.y = R(0);
     }
     psi[i] = a;
   }
@@ -675,12 +724,19 @@ void launch_outcome_hist(int prec, const void* psi, uint64_t S, int m, const int
   const uint64_t no = 1ull << m;
   hipLaunchKernelGGL(k_zero_f64, dim3(stream_grid(no)), dim3(kBlock), 0, st, hist, no);
   if (m <= 12) {
+    uint64_t mask = 0;
+    for (int j = 0; j < m; ++j) mask |= 1ull << pos[j];
+    // 64 amplitudes a thread, more where that would be over kReduceBlocks blocks
+    const uint64_t least = 64ull * kBlock, share = S / kReduceBlocks;
+    const uint64_t span = std::min(S, std::max(share, least));
+    const unsigned g = (unsigned)((S + span - 1) / span);
+    const size_t lds = no * sizeof(double);
     if (prec == QSV_C128)
-      hipLaunchKernelGGL((k_outcome_hist_lds<double>), dim3(kReduceBlocks), dim3(kBlock), 0, st, (const double2*)psi,
-                         S, p, hist);
+      hipLaunchKernelGGL((k_outcome_hist_lds<double>), dim3(g), dim3(kBlock), lds, st, (const double2*)psi, S, span,
+                         mask, p, hist);
     else
-      hipLaunchKernelGGL((k_outcome_hist_lds<float>), dim3(kReduceBlocks), dim3(kBlock), 0, st, (const float2*)psi,
-                         S, p, hist);
+      hipLaunchKernelGGL((k_outcome_hist_lds<float>), dim3(g), dim3(kBlock), lds, st, (const float2*)psi, S, span,
+                         mask, p, hist);
   } else {
     if (prec == QSV_C128)
       hipLaunchKernelGGL((k_outcome_hist_global<double>), dim3(stream_grid(S)), dim3(kBlock), 0, st,
@@ -694,14 +750,16 @@ void launch_outcome_hist(int prec, const void* psi, uint64_t S, int m, const int
 void launch_collapse(int prec, void* psi, uint64_t S, int m, const int* pos, uint64_t sel, double scale,
                      hipStream_t st)
 {
-  PosArgs p{};
-  p.m = m;
-  for (int j = 0; j < m; ++j) p.pos[j] = pos[j];
+  uint64_t mask = 0, want = 0;
+  for (int j = 0; j < m; ++j) {
+    mask |= 1ull << pos[j];
+    want |= ((sel >> j) & 1ull) << pos[j];
+  }
   const unsigned g = stream_grid(S);
   if (prec == QSV_C128)
-    hipLaunchKernelGGL((k_collapse<double>), dim3(g), dim3(kBlock), 0, st, (double2*)psi, S, p, sel, scale);
+    hipLaunchKernelGGL((k_collapse<double>), dim3(g), dim3(kBlock), 0, st, (double2*)psi, S, mask, want, scale);
   else
-    hipLaunchKernelGGL((k_collapse<float>), dim3(g), dim3(kBlock), 0, st, (float2*)psi, S, p, sel, (float)scale);
+    hipLaunchKernelGGL((k_collapse<float>), dim3(g), dim3(kBlock), 0, st, (float2*)psi, S, mask, want, (float)scale);
 }
 
 }  // namespace qsv
