@@ -728,7 +728,11 @@ size_t compile_pass(const FPass& p, bool f32, int block_cost, std::complex<doubl
 {
   PHead h;
   std::memset(&h, 0, sizeof(h));
-  h.renorm = p.renorm;
+  // entries of magnitude at most 1 keep every product of a pass finite, in FP32 too
+  bool tame = std::abs(scalar.real()) <= 1.001 && std::abs(scalar.imag()) <= 1.001;
+  for (const FGate& g : p.gates)
+    for (double m : g.m) tame &= std::abs(m) <= 1.001;
+  h.renorm = p.renorm | (tame ? FP_KEEP_ZERO : 0);
   std::memcpy(h.sorted_pos, p.sorted_pos, sizeof(h.sorted_pos));
   Compiler c(p, f32, block_cost, scalar);
   c.run(h, last);

@@ -1,0 +1,47 @@
+"""States whose tiles are mostly zeros: fused passes leave zero tiles alone, the
+gate-by-gate path does not look. Basis states, few active qubits at either end,
+uncollapsed and collapsed registers, both arithmetic widths and a batch."""
+from __future__ import annotations
+
+import math
+
+import numpy as np
+import pytest
+
+from qclojure_amd import circuit as qc
+from qclojure_amd import engine
+from qclojure_amd._abi import OP, QSV_FLAG_FP64_PASSES, QSV_FLAG_FUSE
+
+pytestmark = pytest.mark.gpu
+
+
+def _program(qubits, rng, count):
+    rows = []
+    for _ in range(count):
+        a, b = (int(q) for q in rng.choice(qubits, 2, replace=False))
+        name = ["H", "RX", "RY", "RZ", "CNOT", "CNOT", "SWAP", "CZ", "X"][rng.integers(9)]
+        rows.append((OP[name], a, b if name in ("CNOT", "SWAP", "CZ") else 0, 0, 0, float(rng.uniform(0, 2 * math.pi))))
+    return rows
+
+
+@pytest.mark.parametrize("n", [12, 13, 16, 20, 23])
+@pytest.mark.parametrize("where", ["first", "last", "spread", "measured"])
+def test_sparse(n, where):
+    rng = np.random.default_rng(n)
+    some = {"first": range(5), "last": range(n - 5, n), "spread": range(0, n, 3), "measured": range(n)}[where]
+    rows = _program(list(some), rng, 60)
+    if where == "measured":   # half of the amplitudes go to zero, then more gates
+        rows += [(OP["MEASURE"], 0, 0, 0, 0b101, 0.0)] + _program(list(range(n)), rng, 30)
+    # FP32 passes end in a norm of one: a register with one tile in use has its sums in one block
+    ops = qc.ops_from_tuples(rows)
+    with engine.DeviceState(n, "c128") as ref, engine.DeviceState(n, "c128") as a, \
+            engine.DeviceState(n, "c64") as f32, engine.DeviceState(n, "c64") as f64:
+        ref.apply(ops, 0, 77)
+        a.apply(ops, QSV_FLAG_FUSE, 77)
+        f32.apply(ops, QSV_FLAG_FUSE, 77)
+        f64.apply(ops, QSV_FLAG_FUSE | QSV_FLAG_FP64_PASSES, 77)
+        # a hundred gates on amplitudes of at most 1
+        assert a.compare(ref)["max_abs_diff"] < 1e-13
+        for s in (f32, f64):
+            assert s.compare(ref)["max_abs_diff"] < 1e-5
+        assert abs(f32.norm2() - 1.0) < 2e-6
