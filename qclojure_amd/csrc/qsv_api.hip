@@ -1280,7 +1280,9 @@ std::vector<uint64_t> structure_key(int n, int prec, int L, const std::vector<BG
   k.push_back((uint64_t)n | ((uint64_t)prec << 8) | ((uint64_t)L << 16));
   for (const BGate& g : gs) {
     k.push_back((uint64_t)(uint32_t)g.kind | ((uint64_t)(uint32_t)(g.a + 1) << 16) |
-                ((uint64_t)(uint32_t)(g.b + 1) << 32) | ((uint64_t)g.cbits.size() << 48));
+                ((uint64_t)(uint32_t)(g.b + 1) << 32) | ((uint64_t)g.cbits.size() << 48) |
+                // a diagonal gate whose entries make its target a tile bit
+                ((uint64_t)(g.kind == FG_PHASE && pass_bits(g).need) << 56));
     uint64_t c = 0;
     for (int x : g.cbits) c = (c << 8) | (uint64_t)(x + 1);
     k.push_back(c);

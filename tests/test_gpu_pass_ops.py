@@ -90,3 +90,22 @@ def test_bits_outside_the_tile(n, targets):
         # as above: a few hundred roundings of amplitudes of at most 1
         assert a.compare(ref)["max_abs_diff"] < 1e-12
         assert f32.compare(ref)["max_abs_diff"] < 1e-5
+
+
+def test_diagonal_entries_change_the_plan():
+    """Two batches of one structure: the diagonal gates of the first are phases,
+    which need no tile bit, those of the second are not."""
+    n = 16
+    rng = np.random.default_rng(3)
+    angles = rng.uniform(0, math.pi, n)
+    terms = [(1.0, "".join("Z" if q == k else "I" for q in range(n))) for k in range(n)]
+    for d0 in (1j, 0.5):
+        ops = np.concatenate([qc.ops_from_tuples([(OP["RY"], q, 0, 0, 0, float(angles[q])) for q in range(n)])] +
+                             [qc.op_u(q, np.diag([d0, 1.0])) for q in range(n)] +
+                             [qc.ops_from_tuples([(OP["RX"], q, 0, 0, 0, 0.3) for q in range(n)])])
+        with engine.DeviceState(n, "c128") as ref:
+            ref.apply(ops)
+            want = sum(ref.expect_pauli([s for _, s in terms]))
+        got = engine.batch_expect_z([(n, ops, terms)] * 2, "c128")
+        # a sum of 16 values of at most 1 after 48 gates
+        assert np.max(np.abs(np.asarray(got) - want)) < 1e-12
