@@ -84,6 +84,7 @@ struct qsv_state {
   PassSlot* ring_pending = nullptr;
   uint64_t passes_launched = 0;
   int tile_low = -1;            // tile low-run width forced by the tuner (-1: none)
+  unsigned long long* reach = nullptr;   // fused passes: TileNorm::reach
   double* norm_buf = nullptr;   // complex64 FP32 passes: per-tile norms (2 x ntiles) + control (2)
   uint64_t* shot_dev = nullptr;   // qsv_sample's outcomes (lazy, at most kShotsKept)
   uint64_t shot_cap = 0;
@@ -603,27 +604,55 @@ int upload_passes(qsv_state* s, const std::vector<char>& progs, const char** dev
   return QSV_OK;
 }
 
+// A program's first passes keep track of where nonzero amplitudes can be, so
+// that the tiles elsewhere are not read (six layers of 27 qubits from |0..0>:
+// 6.13 -> 4.94 ms). States below 256 MiB are read from the memory-side cache and the
+// clearing launch would cost as much as it saves.
+constexpr int kReachPasses = 4;
+constexpr double kReachBytes = 256.0 * (1 << 20);
+
+// What the passes of one program hand on from launch to launch.
+struct PassRun {
+  std::complex<double> scalar{1.0, 0.0};   // the factors common to the whole state
+  int reach = 0;                           // passes that tracked reach; kReachPasses: no more
+};
+
 // Launches the first `count` passes and drops them from the list. blocks: FP32
-// passes fold register-bit runs into PO_BLOCK ops. The factors common to the
-// whole state collect in `scalar` and are applied by the last pass of a run (`end`).
-int launch_passes(qsv_state* s, std::vector<FPass>& passes, size_t count, bool f32, bool blocks,
-                  std::complex<double>& scalar, bool end)
+// passes fold register-bit runs into PO_BLOCK ops. The common factors are
+// applied by the last pass of a run (`end`).
+int launch_passes(qsv_state* s, std::vector<FPass>& passes, size_t count, bool f32, bool blocks, PassRun& run,
+                  bool end)
 {
   if (!count) return QSV_OK;
   const uint64_t ntiles = s->S >> kPassTileBits;
-  TileNorm nb{nullptr, nullptr, nullptr};
+  TileNorm nb{nullptr, nullptr, nullptr, nullptr};
   if (f32) {
     if (!s->norm_buf) HIPCHK(hipMalloc((void**)&s->norm_buf, (2 * ntiles + 2) * sizeof(double)));
-    nb = TileNorm{s->norm_buf, s->norm_buf + ntiles, s->norm_buf + 2 * ntiles};
+    nb = TileNorm{s->norm_buf, s->norm_buf + ntiles, s->norm_buf + 2 * ntiles, nullptr};
   }
   const int block_cost = f32 && blocks ? pass_block_cost() : 0;
   std::vector<char> progs;
   std::vector<size_t> at(count);
-  for (size_t i = 0; i < count; ++i)
-    at[i] = compile_pass(passes[i], f32, block_cost, scalar, end && i + 1 == count, progs);
+  if ((double)s->S * s->bytes_per_amp() < kReachBytes) run.reach = kReachPasses;
+  bool clear = false;
+  for (size_t i = 0; i < count; ++i) {
+    at[i] = compile_pass(passes[i], f32, block_cost, run.scalar, end && i + 1 == count, progs);
+    PHead h;
+    std::memcpy(&h, progs.data() + at[i], sizeof(h));
+    if (run.reach < kReachPasses && (h.renorm & FP_KEEP_ZERO)) {
+      clear |= run.reach == 0;
+      h.renorm |= FP_REACH | (run.reach++ ? FP_REACH_USE : 0);
+      std::memcpy(progs.data() + at[i], &h, sizeof(h));
+    } else {
+      run.reach = kReachPasses;   // a pass that does not track it ends it
+    }
+  }
   const char* dev = nullptr;
   int rc = upload_passes(s, progs, &dev);
   if (rc) return rc;
+  if (clear && !s->reach) HIPCHK(hipMalloc((void**)&s->reach, 2 * sizeof(*s->reach)));
+  nb.reach = s->reach;
+  if (clear) launch_clear_reach(s->reach, s->stream);
   for (size_t i = 0; i < count; ++i) {
     const char* p = dev + at[i];
     rc = timed(s, QSV_KCLASS_BLOCK, 2.0 * s->S * s->bytes_per_amp(),
@@ -1142,25 +1171,26 @@ int run_fused(qsv_state* s, const std::vector<BGate>& gs_in, uint32_t flags)
   // layers of 19 qubits 311 -> 303 us. A register of one tile gains nothing from
   // splitting its only pass: 12 qubits 272 us whole, 303 us in pieces of 64 gates.
   std::vector<FPass> passes;
-  std::complex<double> scalar(1.0, 0.0);
+  PassRun run;
   size_t chunk = 1;
   int rc = fuse_walk(
       s, gs, f32,
       [&](FPass&& p) {
         passes.push_back(std::move(p));
         if (passes.size() <= chunk) return (int)QSV_OK;
-        const int r = launch_passes(s, passes, chunk, f32, blocks, scalar, false);
+        const int r = launch_passes(s, passes, chunk, f32, blocks, run, false);
         chunk = std::min<size_t>(2 * chunk, 512);
         return r;
       },
       [&](size_t i) {
         end_run(passes);
-        const int r = launch_passes(s, passes, passes.size(), f32, blocks, scalar, true);
+        const int r = launch_passes(s, passes, passes.size(), f32, blocks, run, true);
+        run.reach = kReachPasses;
         return r ? r : run_direct(s, gs[i]);
       });
   if (rc) return rc;
   end_run(passes);
-  return launch_passes(s, passes, passes.size(), f32, blocks, scalar, true);
+  return launch_passes(s, passes, passes.size(), f32, blocks, run, true);
 }
 
 // ---- Pauli-string expectations ------------------------------------------------
@@ -1519,6 +1549,7 @@ int qsv_state_destroy(qsv_state* s)
   if (s->prefix) hipFree(s->prefix);
   if (s->hist) hipFree(s->hist);
   if (s->norm_buf) hipFree(s->norm_buf);
+  if (s->reach) hipFree(s->reach);
   if (s->shot_dev) hipFree(s->shot_dev);
   if (s->samp_dev) hipFree(s->samp_dev);
   if (s->samp_host) hipHostFree(s->samp_host);

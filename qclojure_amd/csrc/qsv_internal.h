@@ -178,12 +178,17 @@ enum { FP_RENORM_APPLY = 1, FP_RENORM_IN = 2, FP_RENORM_OUT = 4 };
 // instead of loading the state (the first pass round of a grouped batch).
 // FP_KEEP_ZERO (set by the compiler): every coefficient is finite, so a tile of
 // zeros stays one.
-enum { FP_INIT_ZERO = 8, FP_KEEP_ZERO = 16 };
+// FP_REACH: the pass extends `reach` (below); FP_REACH_USE: and skips the tiles
+// outside it.
+enum { FP_INIT_ZERO = 8, FP_KEEP_ZERO = 16, FP_REACH = 32, FP_REACH_USE = 64 };
 
 struct TileNorm {
   double* part_in;    // per-tile input norm^2 (first pass of a run)
   double* part_out;   // per-tile output norm^2
   double* ctl;        // [0] target norm^2, [1] scale for the next pass
+  // index bits that are set [0] and clear [1] in some amplitude that may be
+  // nonzero, from the passes so far
+  unsigned long long* reach;
 };
 
 // The gates of one pass in program order, on tile-local bits.
@@ -280,6 +285,7 @@ struct PHead {
 // pass when `last`.
 size_t compile_pass(const FPass& p, bool f32, int block_cost, std::complex<double>& scalar, bool last,
                     std::vector<char>& out);
+void launch_clear_reach(unsigned long long* reach, hipStream_t st);
 // f32: complex64 arithmetic in FP32 (ignored for complex128, always FP64)
 void launch_pass(int prec, bool f32, void* psi, const char* dprog, uint64_t ntiles, const TileNorm& nb,
                  hipStream_t st);

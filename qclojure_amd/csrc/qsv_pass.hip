@@ -48,8 +48,10 @@ constexpr uint32_t kTouchTiles = 512;
 // been set to |0..0> is nothing but zeros outside a few tiles until each of its
 // qubits has met a gate, three passes or so later. A pass is linear: such a tile
 // needs neither its ops nor a store. Two barriers and 32 ORs for the others (a
-// dense 27-qubit pass 943 us without, 948 with). The first two of seven passes
-// over 27 qubits 943 -> 325 us, of a 26-qubit complex64 ansatz 508 -> 105 us.
+// dense 27-qubit pass 943 us without, 948 with). The first of seven passes over
+// 27 qubits 943 -> 325 us and, unread where the earlier passes cannot have put
+// anything (FP_REACH), the second 40 and the third 110; a 26-qubit complex64
+// ansatz 508 -> 105 and 49 us.
 template <typename A>
 __device__ __forceinline__ bool any_nonzero(const Slots<A>& x, uint32_t* flags)
 {
@@ -114,6 +116,29 @@ __global__ __launch_bounds__(kThreads, sizeof(A) == 4 ? 5 : 4) void k_pass(typen
 
   Slots<A> x;
   const int rn = h.renorm;
+  uint64_t tmask = 0;
+  // a scale that is not finite would turn zeros into NaN
+  const bool keep = (rn & FP_KEEP_ZERO) && !(sizeof(A) == 4 && (rn & FP_RENORM_APPLY) && !(nb.ctl[1] < 1e30));
+  if constexpr (!GROUP) {
+    // A tile that no nonzero amplitude of the earlier passes can lie in is not
+    // even read: its base has a bit set, or clear, that none of those has. A
+    // launch's own tiles may extend `reach` meanwhile; that only keeps tiles.
+    if (rn & FP_REACH) {
+#pragma unroll
+      for (int i = 0; i < TB; ++i) tmask |= 1ull << h.sorted_pos[i];
+      if (rn & FP_REACH_USE) {
+        const uint64_t set = __hip_atomic_load(nb.reach, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const uint64_t clear = __hip_atomic_load(nb.reach + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const uint64_t bits = (((uint64_t)gridDim.x << TB) - 1ull) & ~tmask;
+        if (keep && (((base & ~set) | (~base & ~clear)) & bits)) {
+          if constexpr (sizeof(A) == 4) {
+            if (t == 0 && (rn & FP_RENORM_OUT)) nb.part_out[tile] = 0.0;
+          }
+          return;
+        }
+      }
+    }
+  }
   {
     const uint64_t ga = base ^ global_part<NT>(t, h.gload);
     if (rn & FP_INIT_ZERO) {
@@ -134,7 +159,7 @@ __global__ __launch_bounds__(kThreads, sizeof(A) == 4 ? 5 : 4) void k_pass(typen
   }
   if (gridDim.x <= kTouchTiles) touch(prog, h.bytes);
   if (rn & FP_INIT_ZERO) {
-    if (base != 0 && (rn & FP_KEEP_ZERO)) {
+    if (base != 0 && keep) {
       const uint64_t ga = base ^ global_part<NT>(t, h.gload);
       each<0, kSlots>([&](auto kk) __attribute__((always_inline)) {
         constexpr int k = decltype(kk)::value;
@@ -145,14 +170,20 @@ __global__ __launch_bounds__(kThreads, sizeof(A) == 4 ? 5 : 4) void k_pass(typen
       return;
     }
   } else if (rn & FP_KEEP_ZERO) {
-    // a scale that is not finite would turn zeros into NaN
-    const bool scaled = sizeof(A) == 4 && (rn & FP_RENORM_APPLY) && !(nb.ctl[1] < 1e30);
-    if (!any_nonzero(x, reinterpret_cast<uint32_t*>(smem)) && !scaled) {
+    if (!any_nonzero(x, reinterpret_cast<uint32_t*>(smem)) && keep) {
       if constexpr (sizeof(A) == 4) {
         if (t == 0 && (rn & FP_RENORM_IN)) nb.part_in[tile] = 0.0;
         if (t == 0 && (rn & FP_RENORM_OUT)) nb.part_out[tile] = 0.0;
       }
       return;
+    }
+    if constexpr (!GROUP) {
+      if ((rn & FP_REACH) && t == 0) {
+        const uint64_t set = base | tmask, clear = ~base;   // both, for the tile's own bits
+        if (set & ~__hip_atomic_load(nb.reach, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicOr(nb.reach, set);
+        if (clear & ~__hip_atomic_load(nb.reach + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+          atomicOr(nb.reach + 1, clear);
+      }
     }
   }
   if constexpr (sizeof(A) == 4) {
@@ -241,6 +272,16 @@ __global__ __launch_bounds__(1024) void k_norm_ctl(const double* __restrict__ pa
   }
 }
 
+__global__ void k_clear_reach(unsigned long long* reach)
+{
+  reach[threadIdx.x] = 0ull;
+}
+
+void launch_clear_reach(unsigned long long* reach, hipStream_t st)
+{
+  hipLaunchKernelGGL(k_clear_reach, dim3(1), dim3(2), 0, st, reach);
+}
+
 void launch_pass(int prec, bool f32, void* psi, const char* dprog, uint64_t ntiles, const TileNorm& nb,
                  hipStream_t st)
 {
@@ -259,7 +300,7 @@ void launch_pass_group(int prec, void* base, uint64_t S, unsigned count, const c
                        hipStream_t st)
 {
   // complex64 groups compute in FP64: no per-instance renormalisation needed
-  const TileNorm none{nullptr, nullptr, nullptr};
+  const TileNorm none{nullptr, nullptr, nullptr, nullptr};
   if (prec == QSV_C128)
     hipLaunchKernelGGL((k_pass<double, double, true>), dim3((unsigned)(S >> kPassTileBits), count), dim3(kThreads),
                        0, st, (PV<double>::T*)base, progs, none, S, offs);

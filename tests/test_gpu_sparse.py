@@ -45,3 +45,28 @@ def test_sparse(n, where):
         for s in (f32, f64):
             assert s.compare(ref)["max_abs_diff"] < 1e-5
         assert abs(f32.norm2() - 1.0) < 2e-6
+
+
+@pytest.mark.parametrize("prec,n", [("c128", 24), ("c64", 25)])
+@pytest.mark.parametrize("start", ["zero", "top", "two", "dense"])
+def test_reach(prec, n, start):
+    """Large states: the first passes keep track of where amplitudes can be."""
+    rng = np.random.default_rng(n + len(start))
+    rows = []
+    if start == "top":
+        rows = [(OP["X"], q, 0, 0, 0, 0.0) for q in range(n)]
+    elif start == "two":      # two far basis states
+        rows = [(OP["H"], 0, 0, 0, 0, 0.0)] + [(OP["CNOT"], 0, q, 0, 0, 0.0) for q in range(1, n)]
+    elif start == "dense":
+        rows = [(OP["H"], q, 0, 0, 0, 0.0) for q in range(n)]
+    first = qc.ops_from_tuples(rows)
+    more = [qc.ops_from_tuples(_program(list(qs), rng, 70)) for qs in (range(0, n, 2), range(n))]
+    with engine.DeviceState(n, prec) as ref, engine.DeviceState(n, prec) as a:
+        for s, flags in ((ref, 0), (a, QSV_FLAG_FUSE | (QSV_FLAG_FP64_PASSES if prec == "c64" else 0))):
+            if len(rows):
+                s.apply(first)
+            for ops in more:
+                s.apply(ops, flags)
+        # 140 gates on amplitudes of at most 1; complex64 rounds its stores
+        assert a.compare(ref)["max_abs_diff"] < (1e-13 if prec == "c128" else 1e-5)
+        assert abs(a.norm2() - 1.0) < (1e-12 if prec == "c128" else 1e-4)
