@@ -726,8 +726,10 @@ void launch_outcome_hist(int prec, const void* psi, uint64_t S, int m, const int
   if (m <= 12) {
     uint64_t mask = 0;
     for (int j = 0; j < m; ++j) mask |= 1ull << pos[j];
-    // 64 amplitudes a thread, more where that would be over kReduceBlocks blocks
-    const uint64_t least = 64ull * kBlock, share = S / kReduceBlocks;
+    // eight amplitudes a thread (its loads in flight), more where that would be
+    // over kReduceBlocks blocks; 64 at least left most CUs idle below 2^24
+    // amplitudes
+    const uint64_t least = 8ull * kBlock, share = S / kReduceBlocks;
     const uint64_t span = std::min(S, std::max(share, least));
     const unsigned g = (unsigned)((S + span - 1) / span);
     const size_t lds = no * sizeof(double);

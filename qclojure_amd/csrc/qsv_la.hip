@@ -606,19 +606,26 @@ __global__ void k_identity(double2* __restrict__ V, int64_t n)
 // round); now 1.08 ms (2.1 us), the same eigenvalues and vectors bit for bit.
 constexpr int kJacSmall = 64;
 constexpr int kJacPad = kJacSmall + 1;   // row stride: a column walk crosses LDS banks
-constexpr int kJacThreads = 1024;
 
-__global__ __launch_bounds__(kJacThreads) void k_jacobi_small(const double2* __restrict__ A,
+// P: pairs the workgroup has threads for (a power of two, n <= 2 P), one thread
+// per block of A and at least a wave beside the one that makes the rotations:
+// small matrices need no barriers of sixteen waves (matrix-exp of n = 16 and 32,
+// four waves and separate sweeps before: 482 -> 456 us, 833 -> 646 us).
+constexpr int jac_threads(int P) { return P * P < 128 ? 128 : P * P; }
+
+template <int P>
+__global__ __launch_bounds__(jac_threads(P)) void k_jacobi_small(const double2* __restrict__ A,
                                                               double2* __restrict__ Vout, double* __restrict__ w, int n,
                                                               int* __restrict__ sweeps_out)
 {
+  constexpr int kThreads = jac_threads(P);
   __shared__ double2 sM[kJacSmall][kJacPad];
   __shared__ double2 sV[kJacSmall][kJacPad];
   __shared__ Rot rot[2][kJacSmall / 2];
-  __shared__ double ra[kJacThreads / 64], rb[kJacThreads / 64];
+  __shared__ double ra[kThreads / 64], rb[kThreads / 64];
   __shared__ int stop;
   const int tid = threadIdx.x;
-  for (int e = tid; e < n * n; e += kJacThreads) {
+  for (int e = tid; e < n * n; e += kThreads) {
     const int i = e / n, j = e - i * n;
     sM[i][j] = A[e];
     sV[i][j] = make_double2(i == j ? 1.0 : 0.0, 0.0);
@@ -633,9 +640,9 @@ __global__ __launch_bounds__(kJacThreads) void k_jacobi_small(const double2* __r
     const int a = player(k, r), b = player(N - 1 - k, r);
     return a < b ? make_int2(a, b) : make_int2(b, a);
   };
-  // V <- V U of round r by half waves, one a row: rows i0, i0 + step, ...
+  // V <- V U of round r by P threads a row: rows i0, i0 + step, ...
   auto rotate_v = [&](int r, const Rot* R0, int i0, int step) {
-    const int k = tid & 31;
+    const int k = tid % P;
     if (k >= npairs) return;
     const int2 pq = pair_of(k, r);
     if (pq.y >= n) return;
@@ -646,13 +653,13 @@ __global__ __launch_bounds__(kJacThreads) void k_jacobi_small(const double2* __r
       sV[i][pq.y] = make_double2(R.s * xp.x + R.c * eq.x, R.s * xp.y + R.c * eq.y);
     }
   };
-  const int k1 = tid >> 5, k2 = tid & 31;   // this thread's block of A in every round
+  const int k1 = tid / P, k2 = tid % P;   // this thread's block of A in every round
   double prev = -1.0;
   int sweeps = 0;
   __syncthreads();
   for (; sweeps < 40; ++sweeps) {
     double off = 0.0, tot = 0.0;
-    for (int e = tid; e < n * n; e += kJacThreads) {
+    for (int e = tid; e < n * n; e += kThreads) {
       const int i = e / n, j = e - i * n;
       const double m2 = cabs2(sM[i][j]);
       tot += m2;
@@ -667,7 +674,7 @@ __global__ __launch_bounds__(kJacThreads) void k_jacobi_small(const double2* __r
     __syncthreads();
     if (tid == 0) {
       double o = 0.0, t = 0.0;
-      for (int i = 0; i < kJacThreads / 64; ++i) { o += ra[i]; t += rb[i]; }
+      for (int i = 0; i < kThreads / 64; ++i) { o += ra[i]; t += rb[i]; }
       stop = (!(o > 1e-30 * t) || o == 0.0 || (prev >= 0.0 && !(o < prev))) ? 1 : 0;
       ra[0] = o;
     }
@@ -697,7 +704,7 @@ __global__ __launch_bounds__(kJacThreads) void k_jacobi_small(const double2* __r
           rot[r & 1][tid] = R;
         }
       } else if (r > 0) {
-        rotate_v(r - 1, rot[(r - 1) & 1], (tid - 64) >> 5, (kJacThreads - 64) >> 5);
+        rotate_v(r - 1, rot[(r - 1) & 1], (tid - 64) / P, (kThreads - 64) / P);
       }
       __syncthreads();
       // block (k1, k2): rows of pair k1, columns of pair k2
@@ -737,14 +744,14 @@ __global__ __launch_bounds__(kJacThreads) void k_jacobi_small(const double2* __r
       }
       __syncthreads();
     }
-    rotate_v(nrounds - 1, rot[(nrounds - 1) & 1], tid >> 5, kJacThreads >> 5);
+    rotate_v(nrounds - 1, rot[(nrounds - 1) & 1], tid / P, kThreads / P);
     __syncthreads();
   }
-  for (int e = tid; e < n * n; e += kJacThreads) {
+  for (int e = tid; e < n * n; e += kThreads) {
     const int i = e / n, j = e - i * n;
     Vout[e] = sV[i][j];
   }
-  for (int i = tid; i < n; i += kJacThreads) w[i] = sM[i][i].x;
+  for (int i = tid; i < n; i += kThreads) w[i] = sM[i][i].x;
   if (tid == 0) *sweeps_out = sweeps;
 }
 
@@ -1527,8 +1534,13 @@ int qsv_la_eigh(const qsv_mat* A, double* eigenvalues, qsv_mat* V, int* sweeps_o
       return api_fail(QSV_E_NOMEM, "eigen-hermitian scratch allocation failed");
     int* dsw = reinterpret_cast<int*>(w + n);
     int sweeps = 0;
-    hipLaunchKernelGGL(k_jacobi_small, dim3(1), dim3(kJacThreads), 0, g_la_stream, (const double2*)A->data, V->data, w,
-                       (int)n, dsw);
+    auto run = [&](auto kernel, int threads) {
+      hipLaunchKernelGGL(kernel, dim3(1), dim3(threads), 0, g_la_stream, (const double2*)A->data, V->data, w, (int)n,
+                         dsw);
+    };
+    if (n <= 16) run(k_jacobi_small<8>, jac_threads(8));
+    else if (n <= 32) run(k_jacobi_small<16>, jac_threads(16));
+    else run(k_jacobi_small<32>, jac_threads(32));
     const bool ok = hipGetLastError() == hipSuccess &&
                     hipMemcpyAsync(eigenvalues, w, (size_t)n * sizeof(double), hipMemcpyDeviceToHost, g_la_stream) ==
                         hipSuccess &&
