@@ -224,7 +224,7 @@ int qsv_noisy_trajectories(int num_qubits, int precision, const qsv_op* ops, uin
  * A scheduler thread admits queued requests in arrival order while the sum of
  * their state bytes (2^n * 16 or 8) fits the HBM budget, keeps admitted states
  * on the device, gathers every admitted request small enough for one
- * workgroup's LDS into a single batched launch (gates + shots), runs larger
+ * workgroup into a single batched launch (gates + shots), runs larger
  * ones concurrently on their own streams through fused passes, and records
  * submit / admit / done timestamps inside the library. */
 typedef struct qsv_server qsv_server;
@@ -234,7 +234,7 @@ typedef struct qsv_server_config {
   int32_t  precision;         /* QSV_C64 or QSV_C128                               */
   int32_t  max_inflight;      /* admitted requests on the device at once (0: 32)   */
   uint32_t flags;             /* QSV_FLAG_* applied to every request               */
-  int32_t  batch_small;       /* 1: batch LDS-sized requests into one launch       */
+  int32_t  batch_small;       /* 1: batch one-workgroup requests into one launch  */
 } qsv_server_config;
 
 #define QSV_REQ_QUEUED    0

@@ -5,7 +5,7 @@ src/org/soulspace/qclojure/adapter/backend/hardware_simulator.clj:106-242:
 every shot is one trajectory (clean operation, then the gate's noise channel,
 noise.clj:53-103), measured once and passed through the readout-error model
 (noise.clj:108-202). All trajectories run in one qsv_noisy_trajectories call
-(one workgroup per trajectory with the state in LDS up to 13/14 qubits).
+(one workgroup per trajectory with the state in registers up to 13/14 qubits).
 
 Result map keys follow the reference: :measurement-results {bitstring count},
 :final-state, :trajectories (the first max-trajectories final states, when
