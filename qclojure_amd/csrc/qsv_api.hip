@@ -2435,6 +2435,30 @@ int qsv_batch_expect_z(const qsv_batch_desc* d, double* energies)
   return QSV_OK;
 }
 
+}  // extern "C"
+
+namespace {
+
+double norm2_entries(const double m[8])
+{
+  double s = 0.0;
+  for (int e = 0; e < 8; ++e) s += m[e] * m[e];
+  return s;
+}
+// Are the rows of m orthogonal and of equal length, to `tol` of that length squared?
+bool unitary_multiple(const double m[8], double tol)
+{
+  const double r0 = m[0] * m[0] + m[1] * m[1] + m[2] * m[2] + m[3] * m[3];
+  const double r1 = m[4] * m[4] + m[5] * m[5] + m[6] * m[6] + m[7] * m[7];
+  const double re = m[0] * m[4] + m[1] * m[5] + m[2] * m[6] + m[3] * m[7];
+  const double im = m[1] * m[4] - m[0] * m[5] + m[3] * m[6] - m[2] * m[7];
+  return r0 > 1e-200 && std::abs(r0 - r1) <= tol * r0 && std::abs(re) <= tol * r0 && std::abs(im) <= tol * r0;
+}
+
+}  // namespace
+
+extern "C" {
+
 int qsv_noisy_trajectories(int num_qubits, int precision, const qsv_op* ops, uint64_t n_ops,
                            const qsv_kraus_site* sites, uint64_t n_sites, uint64_t n_traj, uint64_t seed,
                            uint64_t* outcomes, uint64_t n_keep, double* final_states)
@@ -2464,11 +2488,13 @@ int qsv_noisy_trajectories(int num_qubits, int precision, const qsv_op* ops, uin
     }
     op_end[i] = clean.size();
   }
-  // each site's operators scaled to max |k_ij| = 1 (the reference renormalises
-  // after applying one, so any positive multiple gives the same state) and
-  // their selection weights max |k_ij|^2 (channel.clj:203-212)
+  // each site's operators, scaled (the reference renormalises after applying
+  // one, so any positive multiple gives the same state): to 1 where they are a
+  // multiple of a unitary, which then keeps the norm, otherwise to
+  // max |k_ij| = 1; and their selection weights max |k_ij|^2 (channel.clj:203-212)
   std::vector<std::vector<std::array<double, 8>>> kops(n_sites);
   std::vector<std::vector<double>> kw(n_sites);
+  std::vector<char> keeps_norm(n_sites, 1);
   for (uint64_t k = 0; k < n_sites; ++k) {
     const qsv_kraus_site& st = sites[k];
     if (st.after_op >= n_ops) return fail(QSV_E_INVALID, "site " + std::to_string(k) + ": after_op out of range");
@@ -2482,7 +2508,9 @@ int qsv_noisy_trajectories(int num_qubits, int precision, const qsv_op* ops, uin
       if (!(mx > 0.0) || !std::isfinite(mx))
         return fail(QSV_E_INVALID, "site " + std::to_string(k) + ": Kraus operator " + std::to_string(j) + " is zero or not finite");
       std::array<double, 8> a;
-      const double sc = 1.0 / std::sqrt(mx);
+      const bool unitary = unitary_multiple(st.m[j], 1e-14);
+      const double sc = 1.0 / std::sqrt(unitary ? 0.5 * norm2_entries(st.m[j]) : mx);
+      keeps_norm[k] &= unitary;
       for (int e = 0; e < 8; ++e) a[e] = st.m[j][e] * sc;
       kops[k].push_back(a);
       kw[k].push_back(mx);
@@ -2501,9 +2529,9 @@ int qsv_noisy_trajectories(int num_qubits, int precision, const qsv_op* ops, uin
   // one trajectory's gate list: clean gates of op i, then its sites' operators.
   // A chosen operator scaled to max |k_ij| = 1 shrinks the norm (damping
   // operators do, site after site), so a renormalisation follows every 16th
-  // site (the small path's last site too): between fused passes it is a barrier
-  // of two state passes. Without it, deep programs with strong damping would
-  // drive the amplitudes into the subnormal range.
+  // site: between fused passes it is a barrier of two state passes. Without it,
+  // deep programs with strong damping would drive the amplitudes into the
+  // subnormal range.
   auto trajectory_gates = [&](uint64_t t, std::vector<BGate>& out) {
     out.clear();
     size_t g = 0, k = 0;
@@ -2555,7 +2583,15 @@ int qsv_noisy_trajectories(int num_qubits, int precision, const qsv_op* ops, uin
     // one workgroup per trajectory, all running one program: its noise sites
     // draw their uniform and choose their operator on the device. Final states
     // go to an arena (chunks bound it to 1 GiB), one shot each.
-    constexpr uint64_t kRenormEvery = 16;
+    // The state is renormalised at every site, as the reference does, except at
+    // those whose operators keep the norm. The sites of different qubits run in
+    // no particular order, so a rule that counts them (every 16th) lets any
+    // number of others shrink the state in between. Where a gate of the program
+    // does not keep the norm, every site renormalises.
+    bool unitary = true;
+    for (const BGate& g : clean)
+      if (g.kind == FG_DENSE || g.kind == FG_PHASE)
+        unitary &= unitary_multiple(g.m, 1e-12) && std::abs(0.5 * norm2_entries(g.m) - 1.0) <= 1e-12;
     std::vector<KrausOp> table;
     FPass p;
     p.tb = std::max(n, 4);
@@ -2573,7 +2609,7 @@ int qsv_noisy_trajectories(int num_qubits, int precision, const qsv_op* ops, uin
         f.b = (int32_t)k;
         f.cmask = (uint32_t)table.size();
         f.sub = sites[k].n_kraus;
-        f.bmask = (k + 1) % kRenormEvery == 0 || k + 1 == n_sites ? 1u : 0u;
+        f.bmask = unitary && keeps_norm[k] ? 0u : 1u;
         for (int j = 0; j < sites[k].n_kraus; ++j) {
           KrausOp o;
           o.w = kw[k][j];

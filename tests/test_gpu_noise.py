@@ -102,6 +102,45 @@ def test_deep_damping_stays_normalised(eng, oracle, prec, n):
         assert np.min(ov) > 1 - 1e-5, ov
 
 
+def _damped(n, count, gamma, kind):
+    """A damping channel after every gate of a program without entanglers."""
+    if kind == "phase":      # X, then RZ on the excited qubit: K0 = diag(1, sqrt(1 - gamma)) every time
+        rows = [(qc.OP["X"], 0, 0, 0, 0, 0.0)] + [(qc.OP["RZ"], 0, 0, 0, 0, 0.3)] * count
+        kraus = nz.phase_damping_kraus_operators(gamma)
+        sites = [{"after-op": k + 1, "qubit": 0, "kraus": kraus} for k in range(count)]
+    else:                    # H and amplitude damping, qubit after qubit
+        rows = [(qc.OP["H"], k % n, 0, 0, 0, 0.0) for k in range(count)]
+        kraus = nz.amplitude_damping_kraus_operators(gamma)
+        sites = [{"after-op": k, "qubit": k % n, "kraus": kraus} for k in range(count)]
+    return qc.ops_from_tuples(rows), sites
+
+
+def _check_damped(eng, oracle, prec, n, count, gamma, kind, T):
+    ops, sites = _damped(n, count, gamma, kind)
+    note(f"damping {kind} {prec} n={n} sites={count} gamma={gamma}")
+    got, states = eng.noisy_trajectories(n, ops, sites, T, 5, prec, n_keep=T)
+    exp, fin = oracle.trajectories(n, ops, sites, T, 5, qc.op_u)
+    assert np.all(np.isfinite(states))
+    ov = np.abs(np.sum(states.conj() * fin, axis=1)) ** 2
+    if prec == "c128":
+        assert np.array_equal(got, exp)
+        assert np.max(np.abs(states - fin)) < 1e-12
+    else:
+        # a rounding of 32-bit amplitudes moves few outcomes; the excited state of the first kind has one
+        assert np.mean(got == exp) >= (1.0 if kind == "phase" else 0.75)
+        assert np.min(ov) > 1 - 1e-5, ov
+
+
+@pytest.mark.parametrize("prec", ["c64", "c128"])
+@pytest.mark.parametrize("n,count,gamma,kind", [(1, 200, 0.99, "phase"), (3, 400, 0.99, "phase"),
+                                                (8, 800, 0.9, "amplitude"), (11, 300, 0.9, "amplitude")])
+def test_strong_damping_in_registers(eng, oracle, prec, n, count, gamma, kind):
+    """Every site shrinks the norm, up to ten times, and the sites of different
+    qubits run in any order: no run of them may take the norm below the 1e-12
+    that a single renormalisation asks for, nor out of FP32's range."""
+    _check_damped(eng, oracle, prec, n, count, gamma, kind, 4)
+
+
 def test_depolarizing_statistics(eng):
     """X then depolarizing(p) on 1 qubit: P(1) = 1 - 2p/3."""
     p, T = 0.3, 20000

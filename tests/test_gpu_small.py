@@ -1,5 +1,5 @@
 """Whole-register programs of one workgroup (small fused states, batched
-instances, trajectories) around their size classes: below 4 qubits a thread holds
+instances, noisy trajectories) around their size classes: below 4 qubits a thread holds
 empty slots, 10 is the last single wave, 11 leaves waves without amplitudes, 13
 and 14 are the largest."""
 from __future__ import annotations
@@ -66,3 +66,27 @@ def test_batched_energies(precision):
     # the one-workgroup limit, beyond which complex64 states are stored in FP32 between passes)
     scale = np.array([np.sum(np.abs(i[2][1])) for i in insts])
     assert np.max(np.abs(got - exp) / scale) < (1e-12 if precision == "c128" else 1e-6)
+
+
+# (one workgroup holds 13 qubits of complex128)
+@pytest.mark.parametrize("precision,n", [(p, n) for p in ("c128", "c64") for n in SIZES if n < 14 or p == "c64"])
+def test_trajectories(oracle, n, precision):
+    """Entangling programs with operators that do not keep the norm on every
+    qubit, between ones that do; more than 16 sites in all."""
+    rng = np.random.default_rng(100 + n)
+    ops = _program(n, rng, 40 + n)
+    damp, flip, ry = 0.4, 0.3, 0.2
+    amp = [np.array([[1, 0], [0, math.sqrt(1 - damp)]]), np.array([[0, math.sqrt(damp)], [0, 0]])]
+    bit = [math.sqrt(1 - flip) * np.eye(2), math.sqrt(flip) * np.array([[0, 1], [1, 0]])]
+    turn = [np.array([[math.cos(ry), -math.sin(ry)], [math.sin(ry), math.cos(ry)]])]
+    sites = [{"after-op": k, "qubit": int(rng.integers(n)) if k >= 2 * n else k % n, "kraus": [amp, bit, turn][k % 3]}
+             for k in range(len(ops))]
+    T = 6 if n < 11 else 3
+    got, states = engine.noisy_trajectories(n, ops, sites, T, 17, precision, n_keep=T)
+    exp, fin = oracle.trajectories(n, ops, sites, T, 17, qc.op_u)
+    if precision == "c128":
+        assert np.array_equal(got, exp)
+        assert np.max(np.abs(states - fin)) < 1e-12
+    else:   # FP64 arithmetic, amplitudes stored in 32 bits: a shot moves with probability 1e-6
+        assert np.array_equal(got, exp)
+        assert np.max(np.abs(states - fin)) < 1e-6
