@@ -2445,6 +2445,14 @@ double norm2_entries(const double m[8])
   for (int e = 0; e < 8; ++e) s += m[e] * m[e];
   return s;
 }
+double least_singular(const double m[8])
+{
+  const double re = m[0] * m[6] - m[1] * m[7] - m[2] * m[4] + m[3] * m[5];
+  const double im = m[0] * m[7] + m[1] * m[6] - m[2] * m[5] - m[3] * m[4];
+  const double det = std::hypot(re, im), t = norm2_entries(m);
+  const double most = std::sqrt(0.5 * (t + std::sqrt(std::max(0.0, t * t - 4.0 * det * det))));
+  return most > 0.0 ? det / most : 0.0;
+}
 // Are the rows of m orthogonal and of equal length, to `tol` of that length squared?
 bool unitary_multiple(const double m[8], double tol)
 {
@@ -2527,24 +2535,44 @@ int qsv_noisy_trajectories(int num_qubits, int precision, const qsv_op* ops, uin
     return nk - 1;
   };
   // one trajectory's gate list: clean gates of op i, then its sites' operators.
-  // A chosen operator scaled to max |k_ij| = 1 shrinks the norm (damping
-  // operators do, site after site), so a renormalisation follows every 16th
-  // site: between fused passes it is a barrier of two state passes. Without it,
-  // deep programs with strong damping would drive the amplitudes into the
-  // subnormal range.
+  // A chosen operator scaled to max |k_ij| = 1 shrinks the norm, at most by its
+  // smaller singular value. A renormalisation is a barrier of two state passes
+  // here, so one follows every 16th site, and further ones keep the norm that the
+  // operators since the last may have left above kLeastNorm: far from the 1e-12
+  // below which a renormalisation leaves a state alone. An operator that could
+  // take it below by itself (a projector) has one on either side.
+  constexpr double kLeastNorm = 1e-8;
+  std::vector<std::vector<double>> shrink(n_sites);
+  for (uint64_t k = 0; k < n_sites; ++k)
+    for (const auto& a : kops[k]) shrink[k].push_back(std::min(1.0, least_singular(a.data())));
+  std::vector<double> clean_shrink(clean.size(), 1.0);
+  for (size_t g = 0; g < clean.size(); ++g)
+    if (clean[g].kind == FG_DENSE || clean[g].kind == FG_PHASE)
+      clean_shrink[g] = std::min(1.0, least_singular(clean[g].m));
   auto trajectory_gates = [&](uint64_t t, std::vector<BGate>& out) {
     out.clear();
     size_t g = 0, k = 0;
+    double least = 1.0;   // the norm is at least this
+    auto renorm = [&]() {
+      BGate r;
+      r.kind = FG_RENORM;
+      out.push_back(std::move(r));
+      least = 1.0;
+    };
+    auto before = [&](double s) {
+      if (!(least * s >= kLeastNorm) && least < 0.5) renorm();
+      least *= s;
+    };
     for (uint64_t i = 0; i < n_ops; ++i) {
-      for (; g < op_end[i]; ++g) out.push_back(clean[g]);
+      for (; g < op_end[i]; ++g) {
+        before(clean_shrink[g]);
+        out.push_back(clean[g]);
+      }
       for (; k < n_sites && sites[k].after_op == i; ++k) {
         const int j = choose(k, qsv_uniform(seed, t * QSV_TRAJ_SLOTS + k));
+        before(shrink[k][j]);
         emit_ctl(out, {}, n - 1 - sites[k].qubit, kops[k][j].data());
-        if ((k + 1) % 16 == 0) {
-          BGate r;
-          r.kind = FG_RENORM;
-          out.push_back(std::move(r));
-        }
+        if (least < kLeastNorm || (k + 1) % 16 == 0) renorm();
       }
     }
   };

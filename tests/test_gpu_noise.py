@@ -141,6 +141,15 @@ def test_strong_damping_in_registers(eng, oracle, prec, n, count, gamma, kind):
     _check_damped(eng, oracle, prec, n, count, gamma, kind, 4)
 
 
+@pytest.mark.parametrize("prec,n", [("c64", 15), ("c128", 14)])
+@pytest.mark.parametrize("count,gamma,kind", [(180, 0.99, "phase"), (60, 0.9999999999, "phase"),
+                                              (200, 0.97, "amplitude")])
+def test_strong_damping_in_passes(eng, oracle, prec, n, count, gamma, kind):
+    """The same above one workgroup, where a renormalisation is a barrier
+    between fused passes."""
+    _check_damped(eng, oracle, prec, n, count, gamma, kind, 2)
+
+
 def test_depolarizing_statistics(eng):
     """X then depolarizing(p) on 1 qubit: P(1) = 1 - 2p/3."""
     p, T = 0.3, 20000
