@@ -103,7 +103,10 @@ int         qsv_device_query(qsv_device_info* out);
 const char* qsv_last_error(void);
 const char* qsv_version(void);
 
-/* ---- state vectors ------------------------------------------------------ */
+/* ---- state vectors ------------------------------------------------------
+ * Calls that take a const state may come from several threads at once (those
+ * that need the state's scratch memory take turns); a call that takes it
+ * non-const must not overlap any other on that state. */
 typedef struct qsv_state qsv_state;
 
 /* zero-state / computational-basis-state (state.clj:251-284, 484-519). */

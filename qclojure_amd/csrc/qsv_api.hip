@@ -62,6 +62,10 @@ struct qsv_state {
   uint64_t S = 0;
   void* amps = nullptr;
   hipStream_t stream = nullptr;
+  // Calls that only read a state may come from several threads at once; what
+  // they share is scratch memory, held by one of them at a time from its first
+  // launch to the wait for its results.
+  mutable std::mutex scratch_mu;
   double* partials = nullptr;   // kPartials doubles
   double* dout = nullptr;       // kReduceOut doubles of reduction results
   double* prefix = nullptr;     // sampling chunk prefix (lazy)
@@ -1648,6 +1652,7 @@ int qsv_state_compare(const qsv_state* a, const qsv_state* b, double out[5])
   if (!out) return fail(QSV_E_INVALID, "null output");
   if (a->n != b->n) return fail(QSV_E_INVALID, "compare: qubit counts differ");
   HIPCHK(hipStreamSynchronize(b->stream));
+  std::lock_guard<std::mutex> lk(a->scratch_mu);
   launch_compare(a->prec, a->amps, b->prec, b->amps, a->S, a->partials, a->dout, a->stream);
   HIPCHK(hipMemcpyAsync(out, a->dout, sizeof(double) * 5, hipMemcpyDeviceToHost, a->stream));
   HIPCHK(hipStreamSynchronize(a->stream));
@@ -1695,6 +1700,7 @@ int qsv_norm2(const qsv_state* s, double* out)
   int rc = check_state(s);
   if (rc) return rc;
   if (!out) return fail(QSV_E_INVALID, "null output");
+  std::lock_guard<std::mutex> lk(s->scratch_mu);
   launch_norm2(s->prec, s->amps, s->S, s->partials, s->dout, s->stream);
   HIPCHK(hipMemcpyAsync(out, s->dout, sizeof(double), hipMemcpyDeviceToHost, s->stream));
   HIPCHK(hipStreamSynchronize(s->stream));
@@ -1741,6 +1747,7 @@ int qsv_sample(const qsv_state* cs, uint64_t shots, uint64_t seed, uint64_t* out
   int rc = check_state(cs);
   if (rc) return rc;
   if (shots && !outcomes) return fail(QSV_E_INVALID, "null outcomes");
+  std::lock_guard<std::mutex> lk(cs->scratch_mu);
   auto* s = const_cast<qsv_state*>(cs);
   if (!s->prefix) {
     const uint64_t nch = std::max<uint64_t>(1, s->S >> kSampleChunkLog);
@@ -1839,6 +1846,7 @@ int qsv_expect_pauli(const qsv_state* s, const char* strings, uint64_t n_terms, 
     }
     xm[t] = x; sm[t] = sg; ny[t] = y;
   }
+  std::lock_guard<std::mutex> lk(s->scratch_mu);
   return pauli_sums(s, xm, sm, ny, out);
 }
 
@@ -1848,6 +1856,7 @@ int qsv_expect_1q(const qsv_state* s, int qubit, const double m[8], double out[2
   if (rc) return rc;
   if (!m || !out) return fail(QSV_E_INVALID, "null argument");
   if (!qok(qubit, s->n)) return fail(QSV_E_INVALID, "qubit out of range");
+  std::lock_guard<std::mutex> lk(s->scratch_mu);
   launch_expect1q(s->prec, s->amps, s->S, 1ull << (s->n - 1 - qubit), m, s->partials, s->dout, s->stream);
   HIPCHK(hipMemcpyAsync(out, s->dout, sizeof(double) * 2, hipMemcpyDeviceToHost, s->stream));
   HIPCHK(hipStreamSynchronize(s->stream));
@@ -1863,6 +1872,7 @@ int qsv_inner(const qsv_state* a, const qsv_state* b, double out[2])
   if (!out) return fail(QSV_E_INVALID, "null output");
   if (a->n != b->n || a->prec != b->prec) return fail(QSV_E_INVALID, "inner: shape or precision mismatch");
   HIPCHK(hipStreamSynchronize(b->stream));
+  std::lock_guard<std::mutex> lk(a->scratch_mu);
   launch_inner(a->prec, a->amps, b->amps, a->S, a->partials, a->dout, a->stream);
   HIPCHK(hipMemcpyAsync(out, a->dout, sizeof(double) * 2, hipMemcpyDeviceToHost, a->stream));
   HIPCHK(hipStreamSynchronize(a->stream));

@@ -2,6 +2,8 @@
 the sampler's chunk (2^10 amplitudes) and group (2^20 amplitudes) limits."""
 from __future__ import annotations
 
+import threading
+
 import numpy as np
 import pytest
 
@@ -40,3 +42,32 @@ def test_shots(n, shots, precision):
 def test_basis_states(index):
     with engine.DeviceState(21, "c128") as st:
         assert set(st.init_basis(index).sample(64, 3).tolist()) == {index}
+
+
+def test_readers_in_threads():
+    """Several threads read one state: shots of different counts (the kept buffer
+    grows under way), expectations and norms, each as from one thread alone."""
+    n = 18
+    rng = np.random.default_rng(n)
+    psi = rng.normal(size=2 ** n) + 1j * rng.normal(size=2 ** n)
+    psi /= np.linalg.norm(psi)
+    strings = ["I" * q + p + "I" * (n - 1 - q) for q in range(n) for p in "XYZ"]
+    with engine.DeviceState(n, "c128") as st, engine.DeviceState(n, "c128") as alone:
+        st.upload(psi)
+        alone.upload(psi)
+        jobs = [(lambda s, k=k: s.sample(700 + 500 * k, k)) for k in range(4)]
+        jobs += [lambda s: s.expect_pauli(strings), lambda s: s.expect_pauli(strings[::-1]),
+                 lambda s: np.array([s.norm2(), s.expect_1q(3, [[1, 2j], [-2j, 3]]).real, s.inner(alone).real])]
+        wrong = []
+
+        def work(job, want):
+            for _ in range(40):
+                if not np.array_equal(job(st), want):
+                    wrong.append(job)
+
+        threads = [threading.Thread(target=work, args=(j, j(alone))) for j in jobs]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert not wrong
