@@ -546,10 +546,11 @@ struct Compiler {
         const C u = m00 / c;
         f1 = over(m10, s * u);
         f0 = over(-m01, s1 * u);
-        const double n = std::sqrt(c * c + s * s);
-        // equal to the matrix to the last places, or taken as it is
-        const double e = std::max({(n - 1.0) * (n - 1.0), std::norm(m01 + u * f0 * s), std::norm(m11 - u * f0 * f1 * c)});
-        if (e < 1e-30) {
+        const double n = std::sqrt(c * c + s * s) - 1.0;
+        // equal to the matrix to 1e-15 in every entry (a few roundings of the
+        // entries themselves; NaN is not), or taken as it is
+        constexpr double kSame = 1e-30;
+        if (n * n < kSame && std::norm(m01 + u * f0 * s) < kSame && std::norm(m11 - u * f0 * f1 * c) < kSame) {
           scalar *= u;
           sub = DM_REAL;
           const double r[8] = {c, 0, -s, 0, s, 0, c, 0};

@@ -109,3 +109,18 @@ def test_diagonal_entries_change_the_plan():
         got = engine.batch_expect_z([(n, ops, terms)] * 2, "c128")
         # a sum of 16 values of at most 1 after 48 gates
         assert np.max(np.abs(np.asarray(got) - want)) < 1e-12
+
+
+@pytest.mark.parametrize("n", [5, 12, 16])
+@pytest.mark.parametrize("entry", range(4))
+def test_nan_entry_is_not_dropped(n, entry):
+    """A general 2x2 with one NaN entry leaves NaN where the gate-by-gate path does."""
+    u = np.array([[0.6, 0.8j], [0.8j * np.exp(0.3j), 0.6 * np.exp(0.3j)]])
+    u[entry // 2, entry % 2] = complex(math.nan, 0.1)
+    first = qc.ops_from_tuples([(OP["RY"], q, 0, 0, 0, 0.5 + q) for q in range(n)])
+    # more than a program of a gate or two, none of them folded into the general one
+    ops = np.concatenate([qc.op_u(1, u), qc.ops_from_tuples([(OP["RY"], q, 0, 0, 0, 0.3) for q in range(2, n)])])
+    with engine.DeviceState(n, "c128") as ref, engine.DeviceState(n, "c128") as a:
+        want = np.isnan(ref.apply(first).apply(ops).download())
+        assert np.any(want)
+        assert np.array_equal(np.isnan(a.apply(first).apply(ops, QSV_FLAG_FUSE).download()), want)
