@@ -23,6 +23,8 @@
 #include <unordered_map>
 #include <vector>
 
+#include <sys/prctl.h>
+
 #include "qsv_internal.h"
 
 using namespace qsv;
@@ -706,9 +708,9 @@ int dense_structure(const double m[8])
 
 // A gate on tile-local bits (loc: local bit of each global bit, -1 outside the
 // tile, where only controls and phases may lie).
-FGate local_gate(const BGate& g, const int loc[64])
+void local_gate(const BGate& g, const int loc[64], FGate& fg)
 {
-  FGate fg{};
+  fg = FGate{};
   fg.kind = g.kind;
   fg.a = g.a >= 0 ? loc[g.a] : -1;
   fg.b = g.b >= 0 ? loc[g.b] : -1;
@@ -721,7 +723,6 @@ FGate local_gate(const BGate& g, const int loc[64])
     for (uint64_t m = g.bmask; m; m &= m - 1) fg.bmask |= 1u << loc[__builtin_ctzll(m)];
   fg.sub = g.kind == FG_DENSE ? dense_structure(g.m) : (g.phase_only ? 1 : 0);
   std::memcpy(fg.m, g.m, sizeof(fg.m));
-  return fg;
 }
 
 // Build one pass from the chosen gates (program order) and the tile bit set.
@@ -762,7 +763,7 @@ void build_pass(const qsv_state* s, const std::vector<BGate>& gs, const std::vec
   for (int b = 0; b < s->n; ++b)
     if ((tile >> b) & 1ull) p.sorted_pos[ns++] = b;
   p.gates.resize(chosen.size());
-  for (size_t i = 0; i < chosen.size(); ++i) p.gates[i] = local_gate(gs[chosen[i]], loc);
+  for (size_t i = 0; i < chosen.size(); ++i) local_gate(gs[chosen[i]], loc, p.gates[i]);
 }
 
 // The last pass of a run of passes needs no scale for a successor.
@@ -1022,8 +1023,51 @@ bool commutes_on_bit(const BGate& x, int b, const double m[8])
 // Measurements and renormalisations stay where they are and stop folding.
 std::vector<BGate> fold_gates(const std::vector<BGate>& in)
 {
-  std::vector<BGate> a;
-  a.reserve(in.size());
+  std::vector<BGate> out;
+  out.reserve(in.size());
+  // per bit: index in out of its pending one-qubit gate (-1: none), and the
+  // gates touching the bit after that one (reused across calls)
+  int last[64];
+  std::fill(last, last + 64, -1);
+  thread_local std::vector<int> since[64];
+  auto reset = [&]() {
+    std::fill(last, last + 64, -1);
+    for (auto& v : since) v.clear();
+  };
+  reset();
+  auto take = [&](const BGate& g) {
+    if (runs_alone(g.kind)) {
+      out.push_back(g);
+      reset();
+      return;
+    }
+    if (is_1q(g)) {
+      const int b = g.a;
+      if (last[b] >= 0) {
+        bool ok = true;
+        for (int j : since[b])
+          if (!commutes_on_bit(out[j], b, g.m)) { ok = false; break; }
+        if (ok) {
+          double r[8];
+          mul2(g.m, out[last[b]].m, r);
+          set_1q(out[last[b]], r);
+          return;
+        }
+      }
+      out.push_back(g);
+      last[b] = (int)out.size() - 1;
+      since[b].clear();
+      return;
+    }
+    out.push_back(g);
+    const int idx = (int)out.size() - 1;
+    uint64_t bits = gate_bits(g);
+    while (bits) {
+      const int b = __builtin_ctzll(bits);
+      bits &= bits - 1;
+      if (last[b] >= 0) since[b].push_back(idx);
+    }
+  };
   for (size_t i = 0; i < in.size(); ++i) {
     if (i + 2 < in.size()) {
       const BGate &x = in[i], &d = in[i + 1], &y = in[i + 2];
@@ -1045,75 +1089,34 @@ std::vector<BGate> fold_gates(const std::vector<BGate>& in)
           c.m[6] = (d0r * d1r + d0i * d1i) / n1;
           c.m[7] = (d0i * d1r - d0r * d1i) / n1;
           c.phase_only = is_one(c.m[0], c.m[1]);
-          a.push_back(std::move(p));
-          a.push_back(std::move(c));
+          take(p);
+          take(c);
           i += 2;
           continue;
         }
       }
     }
-    a.push_back(in[i]);
-  }
-  std::vector<BGate> out;
-  out.reserve(a.size());
-  // per bit: index in out of its pending one-qubit gate (-1: none), and the
-  // gates touching the bit after that one (reused across calls)
-  int last[64];
-  std::fill(last, last + 64, -1);
-  thread_local std::vector<int> since[64];
-  for (auto& v : since) v.clear();
-  auto reset = [&]() {
-    std::fill(last, last + 64, -1);
-    for (auto& v : since) v.clear();
-  };
-  for (BGate& g : a) {
-    if (runs_alone(g.kind)) {
-      out.push_back(std::move(g));
-      reset();
-      continue;
-    }
-    if (is_1q(g)) {
-      const int b = g.a;
-      if (last[b] >= 0) {
-        bool ok = true;
-        for (int j : since[b])
-          if (!commutes_on_bit(out[j], b, g.m)) { ok = false; break; }
-        if (ok) {
-          double r[8];
-          mul2(g.m, out[last[b]].m, r);
-          set_1q(out[last[b]], r);
-          continue;
-        }
-      }
-      out.push_back(std::move(g));
-      last[b] = (int)out.size() - 1;
-      since[b].clear();
-      continue;
-    }
-    out.push_back(std::move(g));
-    const int idx = (int)out.size() - 1;
-    uint64_t bits = gate_bits(out.back());
-    while (bits) {
-      const int b = __builtin_ctzll(bits);
-      bits &= bits - 1;
-      if (last[b] >= 0) since[b].push_back(idx);
-    }
+    take(in[i]);
   }
   return out;
 }
+
+constexpr size_t kKeepGates = 1 << 13;   // a thread's working memory, kept from program to program
 
 // A whole-register program (qsv_small.hip) of gates [g0, g1), none of which
 // runs alone, appended to `out`; zero: it starts from |0..0>.
 size_t compile_small(int n, const BGate* g0, const BGate* g1, bool zero, std::vector<char>& out)
 {
-  FPass p;
+  thread_local FPass p;   // (for the memory of its gates)
   p.tb = std::max(n, 4);
   p.renorm = zero ? FP_INIT_ZERO : 0;
   int loc[64];
   for (int b = 0; b < 64; ++b) loc[b] = b;
   for (int b = 0; b < 16; ++b) p.pos[b] = p.sorted_pos[b] = b;
-  p.gates.reserve(g1 - g0);
-  for (const BGate* g = g0; g != g1; ++g) p.gates.push_back(local_gate(*g, loc));
+  const size_t count = (size_t)(g1 - g0);
+  if (p.gates.capacity() > std::max(count, kKeepGates)) std::vector<FGate>().swap(p.gates);
+  p.gates.resize(count);
+  for (size_t i = 0; i < count; ++i) local_gate(g0[i], loc, p.gates[i]);
   std::complex<double> scalar(1.0, 0.0);
   return compile_pass(p, false, 0, scalar, true, out);
 }
@@ -2144,10 +2147,12 @@ int qsv_batch_expect_z(const qsv_batch_desc* d, double* energies)
   // Decode every instance, convert its Z terms, and plan and compile the passes
   // of the large ones; the small ones' programs follow when the device is busy
   // with those (small ones first left it idle for the larger half of the
-  // planning: 512 MaxCut instances of 8 to 20 qubits 5.87 -> 4.98 ms). Both phases are independent per instance and run on a pool of
-  // host threads (at most 16); errors are reported for the first failing
-  // instance in order, decode errors before term errors, as a sequential pass
-  // would.
+  // planning: 512 MaxCut instances of 8 to 20 qubits 5.87 -> 4.98 ms), or at once
+  // where there are no large ones: starting the host threads a second time costs
+  // as much as compiling a hundred small circuits. Both phases are independent
+  // per instance and run on a pool of host threads (at most 16); errors are
+  // reported for the first failing instance in order, decode errors before term
+  // errors, as a sequential pass would.
   std::vector<std::vector<BGate>> decoded(N);
   struct Plan {
     std::vector<char> bytes;
@@ -2159,6 +2164,8 @@ int qsv_batch_expect_z(const qsv_batch_desc* d, double* energies)
   std::vector<char> term_bad(N, 0);
   std::vector<std::vector<char>> small_prog(N);
   std::vector<Plan> plans(N);
+  bool any_large = false;
+  for (uint64_t i = 0; i < N; ++i) any_large |= d->num_qubits[i] > small_n;
   const unsigned hw = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
   const unsigned nt = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>(hw, N / 8 + 1));
   auto parallel_over = [&](uint64_t count, auto&& body) {
@@ -2171,8 +2178,21 @@ int qsv_batch_expect_z(const qsv_batch_desc* d, double* energies)
     worker();
     for (auto& t : pool) t.join();
   };
-  auto parallel = [&](auto&& body) { parallel_over(N, body); };
-  parallel([&](uint64_t i) {
+  // A small circuit's program goes straight to the pinned staging memory that
+  // earlier calls left (the stream is idle, nothing reads it), each at the next
+  // free offset; where that memory is too short, the programs are gathered
+  // again once it has grown.
+  std::atomic<uint64_t> staged{0};   // programs are multiples of 256 bytes
+  auto compile_one = [&](uint64_t i) {
+    decoded[i] = fold_gates(decoded[i]);
+    std::vector<char>& prog = small_prog[i];
+    compile_small(d->num_qubits[i], decoded[i].data(), decoded[i].data() + decoded[i].size(), true, prog);
+    const uint64_t at = staged.fetch_add(prog.size());
+    insts[i].prog = at;
+    if (at + prog.size() <= g_batch.recs_h.cap)
+      std::memcpy(static_cast<char*>(g_batch.recs_h.p) + at, prog.data(), prog.size());
+  };
+  parallel_over(N, [&](uint64_t i) {
     const int n = d->num_qubits[i];
     uint64_t mk = 0;
     decoded[i].reserve(d->op_offsets[i + 1] - d->op_offsets[i] + 8);   // about one gate per op
@@ -2199,7 +2219,11 @@ int qsv_batch_expect_z(const qsv_batch_desc* d, double* energies)
       tz[k - T0] = bm;
       tc[k - T0] = d->term_coeff[k];
     }
-    if (dec_rc[i] || n <= small_n) return;
+    if (dec_rc[i] || (n <= small_n && any_large)) return;
+    if (n <= small_n) {
+      compile_one(i);
+      return;
+    }
     decoded[i] = fold_gates(decoded[i]);
     plans[i].ok = plan_group_passes(n, prec, decoded[i], plans[i].bytes, plans[i].offs);
   });
@@ -2241,25 +2265,21 @@ int qsv_batch_expect_z(const qsv_batch_desc* d, double* energies)
     cleanup();
     return fail(QSV_E_DEVICE, "batch: event creation failed");
   }
-  // The small circuits: compile, gather the programs in pinned staging memory,
-  // copy them up, one launch per size class, largest circuits first, so the long
-  // workgroups start early.
+  // The small circuits: compile them if that is still to do, copy the programs
+  // up, one launch per size class, largest circuits first, so the long workgroups
+  // start early.
   std::vector<SmallInst> small;   // read by its copy until the stream is waited for
   auto run_small_circuits = [&]() -> int {
-    parallel_over(small_idx.size(), [&](uint64_t k) {
-      const uint64_t i = small_idx[k];
-      decoded[i] = fold_gates(decoded[i]);
-      compile_small(insts[i].n, decoded[i].data(), decoded[i].data() + decoded[i].size(), true, small_prog[i]);
-    });
-    uint64_t bytes = 0;
-    for (uint64_t i : small_idx) {
-      insts[i].prog = bytes;   // programs are multiples of 256 bytes
-      bytes += small_prog[i].size();
+    if (any_large) parallel_over(small_idx.size(), [&](uint64_t k) { compile_one(small_idx[k]); });
+    const uint64_t bytes = staged.load();
+    if (bytes > g_batch.recs_h.cap) {
+      const int rc = grow(g_batch.recs_h, bytes + bytes / 2);
+      if (rc) return rc;
+      for (uint64_t i : small_idx)
+        std::memcpy(static_cast<char*>(g_batch.recs_h.p) + insts[i].prog, small_prog[i].data(), small_prog[i].size());
     }
-    int rc = grow(g_batch.recs_h, bytes);
-    if (rc) return rc;
+    int rc = QSV_OK;
     char* const recs = static_cast<char*>(g_batch.recs_h.p);
-    for (uint64_t i : small_idx) std::memcpy(recs + insts[i].prog, small_prog[i].data(), small_prog[i].size());
     std::stable_sort(small_idx.begin(), small_idx.end(),
                      [&](uint64_t a, uint64_t b) { return insts[a].n > insts[b].n; });
     for (uint64_t i : small_idx) small.push_back(insts[i]);
@@ -2639,7 +2659,10 @@ int qsv_noisy_trajectories(int num_qubits, int precision, const qsv_op* ops, uin
     for (int b = 0; b < 16; ++b) p.pos[b] = p.sorted_pos[b] = b;
     size_t g = 0, k = 0;
     for (uint64_t i = 0; i < n_ops; ++i) {
-      for (; g < op_end[i]; ++g) p.gates.push_back(local_gate(clean[g], loc));
+      for (; g < op_end[i]; ++g) {
+        p.gates.emplace_back();
+        local_gate(clean[g], loc, p.gates.back());
+      }
       for (; k < n_sites && sites[k].after_op == i; ++k) {
         FGate f{};
         f.kind = FG_KRAUS;
@@ -2766,6 +2789,7 @@ struct SrvReq {
   int n = 0;
   std::vector<BGate> gates;
   std::vector<char> prog;   // small requests: the compiled program
+  bool raw = false;         // ... still to be compiled by the scheduler
   uint64_t shots = 0, seed = 0;
   Clock::time_point t_submit, t_admit, t_done;
   int status = QSV_REQ_QUEUED;
@@ -2836,6 +2860,13 @@ struct qsv_server {
   uint64_t next_id = 1;
   bool stop = false;
   std::thread th;
+  // Small requests are folded and compiled by whichever thread is free: a
+  // submitter leaves that to the scheduler while fewer than kRawMost wait for it,
+  // and does it itself otherwise. All by submitters, bursts of 64 and 128 tiny
+  // requests took 1.13 and 2.64 ms instead of 0.82 and 1.88 gate by gate; all by
+  // the scheduler, large requests would wait for them.
+  static constexpr int kRawMost = 4;
+  std::atomic<int> raw{0};
   // Finished requests' states are kept for reuse (a hipFree waits for the
   // whole device, which would stall every request in flight) up to
   // budget / 5 bytes; beyond that they are freed.
@@ -2912,6 +2943,15 @@ int poll_event(hipEvent_t ev, std::string* err)
   return POLL_FAILED;
 }
 
+// A small request's whole-register program (large requests are folded by the
+// fused runner, or run gate by gate without FUSE).
+void prepare_small(qsv_server* sv, SrvReq* r)
+{
+  if (sv->cfg.flags & QSV_FLAG_FUSE) r->gates = fold_gates(r->gates);
+  compile_small(r->n, r->gates.data(), r->gates.data() + r->gates.size(), true, r->prog);
+  std::vector<BGate>().swap(r->gates);
+}
+
 // Launch every pending small request as one batched launch on a free slot.
 int launch_small(qsv_server* sv, std::vector<SrvReq*>& batch)
 {
@@ -2922,6 +2962,16 @@ int launch_small(qsv_server* sv, std::vector<SrvReq*>& batch)
   const int prec = sv->cfg.precision;
   const size_t B = prec == QSV_C128 ? 16 : 8;
   std::vector<char> progs;
+  size_t prog_bytes = 0;
+  for (SrvReq* r : batch) {
+    if (r->raw) {
+      prepare_small(sv, r);
+      r->raw = false;
+      --sv->raw;
+    }
+    prog_bytes += r->prog.size();
+  }
+  progs.reserve(prog_bytes);
   std::vector<SmallInst> insts(batch.size());
   std::vector<SampleJob> jobs(batch.size());
   slot->out_offsets.assign(batch.size(), 0);
@@ -3049,6 +3099,9 @@ void release_large(qsv_server* sv, SrvReq* r, bool device_error = false)
 void server_loop(qsv_server* sv)
 {
   hipSetDevice(g_device);
+  // the waits below are of 50 us: the default slack of another 50 us would
+  // double them (a burst of four tiny requests 204 -> 146 us)
+  prctl(PR_SET_TIMERSLACK, 1000UL, 0UL, 0UL, 0UL);
   std::unique_lock<std::mutex> lk(sv->mu);
   while (true) {
     bool progressed = false;
@@ -3201,6 +3254,7 @@ int qsv_server_submit(qsv_server* sv, int num_qubits, const qsv_op* ops, uint64_
   r->shots = shots;
   r->seed = seed;
   uint64_t mk = 0;
+  r->gates.reserve(n_ops + 8);   // about one gate per op
   for (uint64_t i = 0; i < n_ops; ++i) {
     if (ops[i].kind == QSV_OP_MEASURE) {
       delete r;
@@ -3216,19 +3270,20 @@ int qsv_server_submit(qsv_server* sv, int num_qubits, const qsv_op* ops, uint64_
   const uint64_t B = sv->cfg.precision == QSV_C128 ? 16 : 8;
   r->bytes = (1ull << num_qubits) * B;
   r->small = sv->cfg.batch_small && num_qubits <= sv->lds_n;
-  // small requests run as batched whole-register programs, folded and compiled
-  // here (large ones are folded by the fused runner, or run gate by gate without FUSE)
+  if (r->bytes > sv->budget) {
+    delete r;
+    return fail(QSV_E_NOMEM, "request state exceeds the HBM budget");
+  }
   if (r->small) {
-    if (sv->cfg.flags & QSV_FLAG_FUSE) r->gates = fold_gates(r->gates);
-    compile_small(r->n, r->gates.data(), r->gates.data() + r->gates.size(), true, r->prog);
-    r->gates.clear();
+    if (sv->raw < qsv_server::kRawMost) {
+      r->raw = true;
+      ++sv->raw;
+    } else {
+      prepare_small(sv, r);
+    }
   }
   {
     std::lock_guard<std::mutex> lk(sv->mu);
-    if (r->bytes > sv->budget) {
-      delete r;
-      return fail(QSV_E_NOMEM, "request state exceeds the HBM budget");
-    }
     r->id = sv->next_id++;
     sv->reqs[r->id] = r;
     sv->queue.push_back(r);
@@ -3289,6 +3344,8 @@ int qsv_server_cancel(qsv_server* sv, uint64_t request_id, int* outcome)
       // never admitted: it holds no device memory and leaves the queue now
       auto q = std::find(sv->queue.begin(), sv->queue.end(), r);
       if (q != sv->queue.end()) sv->queue.erase(q);
+      if (r->raw) --sv->raw;
+      r->raw = false;
       r->t_admit = r->t_done = Clock::now();
       r->status = QSV_REQ_CANCELLED;
       sv->stats.cancelled++;

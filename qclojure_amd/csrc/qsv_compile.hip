@@ -94,6 +94,50 @@ void apply_reg_op(const POp& op, C v[16])
   }
 }
 
+// Diagonal factors not applied yet: where the tile bits `mask` and the bits
+// `gmask` outside it are set, `on` and `off` by the value of tile bit t or
+// outside bit gt (neither: `on`)
+struct Factor {
+  uint32_t mask;
+  uint64_t gmask;
+  int t;
+  uint64_t gt;
+  C on, off;
+  uint32_t bits() const { return mask | (t >= 0 ? 1u << t : 0u); }
+};
+struct Keyed {
+  int key;
+  Factor f;
+};
+struct GateInfo {
+  uint32_t bits;   // tile bits it acts on
+  int8_t cls;      // PHASE, LINEAR or OTHER
+  int8_t waits;    // its bits' queues that it is not the front of
+};
+
+// A thread's working memory, kept from pass to pass (up to kKeepOps ops): a
+// program of a hundred gates spends as long in malloc as on its gates otherwise.
+struct Scratch {
+  static constexpr size_t kKeepOps = 1 << 14;
+  std::vector<POp> ops;
+  std::vector<PTerm> terms;
+  std::vector<PShift> shifts;
+  std::vector<float> blk;
+  std::vector<Factor> pend;
+  std::vector<Keyed> now;
+  std::vector<GateInfo> info;
+  std::vector<int> queue;
+  void clear()
+  {
+    if (ops.capacity() > kKeepOps || queue.capacity() > 4 * kKeepOps) *this = Scratch{};
+    ops.clear();
+    terms.clear();
+    shifts.clear();
+    blk.clear();
+    pend.clear();
+  }
+};
+
 struct Compiler {
   // wave-index bits as functionals of the logical index, and the global bits
   // whose value in the tile's base flips them
@@ -106,10 +150,11 @@ struct Compiler {
   const int block_cost;
   const int TB, NT;        // tile bits, thread bits
   const uint32_t FULL;
-  std::vector<POp> ops;
-  std::vector<PTerm> terms;
-  std::vector<PShift> shifts;
-  std::vector<float> blk;
+  Scratch& mem;
+  std::vector<POp>& ops = mem.ops;
+  std::vector<PTerm>& terms = mem.terms;
+  std::vector<PShift>& shifts = mem.shifts;
+  std::vector<float>& blk = mem.blk;
   int nblk = 0;
   size_t stage0 = 0;       // first op of the current stage
   uint16_t stage_col[kCols] = {};
@@ -131,27 +176,12 @@ struct Compiler {
   Waves load_wr;
   bool synced = false;     // every wave's tile has crossed a workgroup barrier
 
-  // diagonal factors not applied yet: where the tile bits `mask` and the bits
-  // `gmask` outside it are set, `on` and `off` by the value of tile bit t or
-  // outside bit gt (neither: `on`)
-  struct Factor {
-    uint32_t mask;
-    uint64_t gmask;
-    int t;
-    uint64_t gt;
-    C on, off;
-    uint32_t bits() const { return mask | (t >= 0 ? 1u << t : 0u); }
-  };
-  std::vector<Factor> pend;
-  struct Keyed {
-    int key;
-    Factor f;
-  };
-  std::vector<Keyed> now;   // flush's own
+  std::vector<Factor>& pend = mem.pend;
+  std::vector<Keyed>& now = mem.now;   // flush's own
   C& scalar;
 
-  Compiler(const FPass& p_, bool f32_, int bc, C& sc)
-      : p(p_), f32(f32_), block_cost(bc), TB(p_.tb), NT(p_.tb - 4), FULL((1u << p_.tb) - 1u), scalar(sc)
+  Compiler(const FPass& p_, bool f32_, int bc, C& sc, Scratch& m)
+      : p(p_), f32(f32_), block_cost(bc), TB(p_.tb), NT(p_.tb - 4), FULL((1u << p_.tb) - 1u), mem(m), scalar(sc)
   {
   }
 
@@ -171,9 +201,8 @@ struct Compiler {
   }
   POp& emit(int code)
   {
-    ops.emplace_back();
+    ops.emplace_back();   // zeros
     POp& op = ops.back();
-    std::memset(&op, 0, sizeof(op));
     op.code = code;
     return op;
   }
@@ -607,44 +636,53 @@ struct Compiler {
     // the front of all its bits' queues; `ready` holds, per class of gates, the
     // lowest bits of the ready ones.
     enum { PHASE, LINEAR, OTHER };
-    std::vector<int> queue[16];
-    std::vector<uint32_t> bits(N);
-    std::vector<int8_t> cls(N), waits(N);
+    std::vector<GateInfo>& info = mem.info;
+    info.resize(N);
     uint32_t ready[3] = {};
     int left = N;
     ops.reserve(2 * N + 16);
-    size_t head[16] = {};
+    size_t head[16] = {}, end[16] = {};   // of the queues, back to back in `queue`
     auto at_front = [&](int i) {
-      if (--waits[i] == 0) ready[cls[i]] |= bits[i] & -bits[i];
+      GateInfo& f = info[i];
+      if (--f.waits == 0) ready[f.cls] |= f.bits & -f.bits;
     };
     for (int i = 0; i < N; ++i) {
       const FGate& g = p.gates[i];
-      bits[i] = gate_bits(g);
-      cls[i] = (int8_t)(g.kind == FG_PHASE && (g.sub || usable(C(g.m[0], g.m[1]))) ? PHASE
-                        : is_linear(g)                                             ? LINEAR
-                                                                                   : OTHER);
-      if (!bits[i]) {   // a phase on bits outside the tile: one factor per tile
+      GateInfo& f = info[i];
+      f.bits = gate_bits(g);
+      f.cls = (int8_t)(g.kind == FG_PHASE && (g.sub || usable(C(g.m[0], g.m[1]))) ? PHASE
+                       : is_linear(g)                                             ? LINEAR
+                                                                                  : OTHER);
+      if (!f.bits) {   // a phase on bits outside the tile: one factor per tile
         take_phase(g);
         --left;
         continue;
       }
-      waits[i] = (int8_t)__builtin_popcount(bits[i]);
-      for (uint32_t m = bits[i]; m; m &= m - 1) queue[__builtin_ctz(m)].push_back(i);
+      f.waits = (int8_t)__builtin_popcount(f.bits);
+      for (uint32_t m = f.bits; m; m &= m - 1) ++end[__builtin_ctz(m)];
     }
+    size_t total = 0;
+    for (int b = 0; b < TB; ++b) {
+      head[b] = total;
+      total += end[b];
+      end[b] = head[b];
+    }
+    std::vector<int>& queue = mem.queue;
+    queue.resize(total);
+    for (int i = 0; i < N; ++i)
+      for (uint32_t m = info[i].bits; m; m &= m - 1) queue[end[__builtin_ctz(m)]++] = i;
     for (int b = 0; b < TB; ++b)
-      if (!queue[b].empty()) at_front(queue[b][0]);
+      if (head[b] < end[b]) at_front(queue[head[b]]);
     auto consume = [&](int i) {
+      const GateInfo& f = info[i];
       --left;
-      ready[cls[i]] &= ~(bits[i] & -bits[i]);
-      for (uint32_t m = bits[i]; m; m &= m - 1) {
+      ready[f.cls] &= ~(f.bits & -f.bits);
+      for (uint32_t m = f.bits; m; m &= m - 1) {
         const int b = __builtin_ctz(m);
-        if (++head[b] < queue[b].size()) at_front(queue[b][head[b]]);
+        if (++head[b] < end[b]) at_front(queue[head[b]]);
       }
     };
-    auto ready_gate = [&](uint32_t m) {
-      const int b = __builtin_ctz(m);
-      return queue[b][head[b]];
-    };
+    auto ready_gate = [&](uint32_t m) { return queue[head[__builtin_ctz(m)]]; };
     // the next layout: the targets of waiting dense gates. `first`: the load
     // layout, whose lanes must cover the low run; later ones take low bits as
     // soon as they are wanted, so that the last layout can store.
@@ -735,7 +773,9 @@ size_t compile_pass(const FPass& p, bool f32, int block_cost, std::complex<doubl
     for (double m : g.m) tame &= std::abs(m) <= 1.001;
   h.renorm = p.renorm | (tame ? FP_KEEP_ZERO : 0);
   std::memcpy(h.sorted_pos, p.sorted_pos, sizeof(h.sorted_pos));
-  Compiler c(p, f32, block_cost, scalar);
+  thread_local Scratch mem;
+  mem.clear();
+  Compiler c(p, f32, block_cost, scalar, mem);
   c.run(h, last);
   h.nops = (int32_t)c.ops.size();
   const size_t terms_at = (sizeof(PHead) + (c.ops.size() + 1) * sizeof(POp) + 31) & ~(size_t)31;

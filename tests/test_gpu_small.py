@@ -68,6 +68,22 @@ def test_batched_energies(precision):
     assert np.max(np.abs(got - exp) / scale) < (1e-12 if precision == "c128" else 1e-6)
 
 
+def test_batches_of_any_size_in_turn():
+    """Programs are staged in memory that the last batch left and gathered anew
+    where it is too short; with and without circuits above one workgroup."""
+    rng = np.random.default_rng(8)
+    for sizes in ([4], [3, 9, 10] * 12, [5], [12] * 30, [2, 15, 7], [11] * 60 + [16], [6, 8]):
+        insts, exp = [], []
+        for n in sizes:
+            ops = _program(n, rng, int(rng.integers(1, 120)))
+            masks = rng.integers(0, 2 ** n, size=5, dtype=np.uint64)
+            insts.append((n, ops, (masks, np.ones(5))))
+            with engine.DeviceState(n, "c128") as s:
+                exp.append(sum(s.apply(ops).expect_pauli(["".join("Z" if (int(m) >> q) & 1 else "I" for q in range(n))
+                                                          for m in masks])))
+        assert np.max(np.abs(engine.batch_expect_z(insts, "c128") - exp)) < 5e-12
+
+
 # (one workgroup holds 13 qubits of complex128)
 @pytest.mark.parametrize("precision,n", [(p, n) for p in ("c128", "c64") for n in SIZES if n < 14 or p == "c64"])
 def test_trajectories(oracle, n, precision):
