@@ -473,8 +473,8 @@ __device__ __forceinline__ uint64_t gather_bits(uint64_t i, const PosArgs& p)
 
 // Weights of the outcomes of m <= 12 measured bits. A block takes `span`
 // consecutive amplitudes (a power of two), thread t those whose index is t
-// modulo kBlock. It walks them with the measured bits outermost, so a sum stays
-// in a register while the outcome does, eight loads in flight; it is then summed
+// modulo kBlock. It walks them with the measured bits outermost, eight loads in
+// flight, so a sum stays in a register while the outcome does; it is then summed
 // over the lanes with the same outcome and added to the block's LDS histogram.
 // One LDS atomic per amplitude before, up to 64 lanes on one address: the three
 // measured bits of 24 qubits, complex128, 102 us; now 49 us, the time of the read.
@@ -483,52 +483,72 @@ __global__ __launch_bounds__(kBlock) void k_outcome_hist_lds(const typename VT<R
                                                               uint64_t span, uint64_t mask, PosArgs p,
                                                               double* __restrict__ hist)
 {
+  using T = typename VT<R>::T;
   extern __shared__ double h[];
-  constexpr int kFly = 8;
+  constexpr uint32_t kFly = 8;
   const int no = 1 << p.m;
   for (int k = threadIdx.x; k < no; k += kBlock) h[k] = 0.0;
   __syncthreads();
-  const uint32_t t = threadIdx.x;
+  const uint32_t t = threadIdx.x, lane = t & 63u;
   const uint64_t first = (uint64_t)blockIdx.x * span + t;
+  const bool in = first < S;   // (a state of less than a block)
   const uint64_t inside = (span - 1) & ~(uint64_t)(kBlock - 1);   // the bits a thread walks
   const uint64_t outer = inside & mask, inner = inside & ~mask;
-  const uint64_t runs = 1ull << __popcll(inner);
-  auto weight = [&](uint64_t i) {
-    const auto a = psi[i];
-    return (double)a.x * a.x + (double)a.y * a.y;
+  const uint64_t total = 1ull << __popcll(inside), runs = 1ull << __popcll(inner);
+  const uint32_t same = ~(uint32_t)mask & 63u;   // lane bits the outcome does not see
+  uint64_t o = 0, k = 0;   // the walk: subsets of the outer and, within, of the inner bits
+  auto step = [&]() -> bool {   // true at the end of a run of one outcome
+    k = (k - inner) & inner;
+    if (k) return false;
+    o = (o - outer) & outer;
+    return true;
   };
-  uint64_t o = 0;
-  do {
-    double acc = 0.0;
-    const uint64_t at = first + o;
-    if (at < S) {
-      uint64_t k = 0;
-      if (runs >= (uint64_t)kFly) {
-        for (uint64_t l = 0; l < runs; l += kFly) {
-          double w[kFly];
+  double acc = 0.0;
+  auto add = [&](uint64_t at) {
 #pragma unroll
-          for (int f = 0; f < kFly; ++f) {
-            w[f] = weight(at + k);
-            k = (k - inner) & inner;   // the next subset of the inner bits
-          }
-          acc += ((w[0] + w[1]) + (w[2] + w[3])) + ((w[4] + w[5]) + (w[6] + w[7]));
-        }
-      } else {
-        for (uint64_t l = 0; l < runs; ++l) {
-          acc += weight(at + k);
-          k = (k - inner) & inner;
+    for (int b = 0; b < 6; ++b)
+      if ((same >> b) & 1u) acc += __shfl_xor(acc, 1 << b, 64);
+    if (!(lane & same) && in) atomicAdd(&h[gather_bits(at, p)], acc);
+    acc = 0.0;
+  };
+  for (uint64_t l = 0; l < total; l += kFly) {
+    T v[kFly];
+    double w[kFly];
+    const uint64_t o0 = o, k0 = k;
+    if (total >= kFly) {
+#pragma unroll
+      for (uint32_t f = 0; f < kFly; ++f) {
+        v[f] = psi[first + o + k];
+        step();
+      }
+    } else {
+#pragma unroll
+      for (uint32_t f = 0; f < kFly; ++f) {
+        v[f].x = v[f].y = R(0);
+        if (f < total) {
+          if (in) v[f] = psi[first + o + k];
+          step();
         }
       }
     }
-    const uint32_t lane = t & 63u, same = ~(uint32_t)mask & 63u;   // lane bits the outcome does not see
 #pragma unroll
-    for (int b = 0; b < 6; ++b) {
-      const double v = __shfl_xor(acc, 1 << b, 64);
-      if ((same >> b) & 1u) acc += v;
+    for (uint32_t f = 0; f < kFly; ++f) w[f] = (double)v[f].x * v[f].x + (double)v[f].y * v[f].y;
+    if (runs >= kFly) {   // one outcome
+      acc += ((w[0] + w[1]) + (w[2] + w[3])) + ((w[4] + w[5]) + (w[6] + w[7]));
+      if (!k) add(first + o0);
+    } else {
+      o = o0;
+      k = k0;
+#pragma unroll
+      for (uint32_t f = 0; f < kFly; ++f) {
+        if (f < total) {
+          acc += w[f];
+          const uint64_t at = first + o;
+          if (step()) add(at);
+        }
+      }
     }
-    if (!(lane & same) && at < S) atomicAdd(&h[gather_bits(at, p)], acc);
-    o = (o - outer) & outer;
-  } while (o);
+  }
   __syncthreads();
   for (int k = threadIdx.x; k < no; k += kBlock)
     if (h[k] != 0.0) atomicAdd(&hist[k], h[k]);
@@ -726,11 +746,16 @@ void launch_outcome_hist(int prec, const void* psi, uint64_t S, int m, const int
   if (m <= 12) {
     uint64_t mask = 0;
     for (int j = 0; j < m; ++j) mask |= 1ull << pos[j];
-    // eight amplitudes a thread (its loads in flight), more where that would be
-    // over kReduceBlocks blocks; 64 at least left most CUs idle below 2^24
-    // amplitudes
-    const uint64_t least = 8ull * kBlock, share = S / kReduceBlocks;
-    const uint64_t span = std::min(S, std::max(share, least));
+    // At most 512 blocks, 1024 where the read dominates: each adds its outcomes to the same few global sums (one
+    // measured bit of 20 qubits: 51 us a call with 256 blocks, 56 with 512, 63 with
+    // 1024; of 22 qubits 73 with 512, 77 with 1024). 16 amplitudes a thread, half as
+    // many for each measured bit among those that it walks: a thread of several
+    // outcomes makes as many chains of lane exchanges (8 high bits of 13 qubits 41
+    // us a call; 49 with eight outcomes a thread; 42 with one LDS atomic an
+    // amplitude, which is within 3 % of this for 10 bits or less of up to 19 qubits
+    // and up to 60 % slower above; for 12 bits of 20 or 21 qubits it is 10 % faster).
+    const uint64_t least = (uint64_t)kBlock << (4 - __builtin_popcountll(mask & (15ull * kBlock)));
+    const uint64_t span = std::min(S, std::max(S >> (S >= 1ull << 23 ? 10 : 9), least));
     const unsigned g = (unsigned)((S + span - 1) / span);
     const size_t lds = no * sizeof(double);
     if (prec == QSV_C128)
