@@ -49,6 +49,19 @@ def test_fused_state(n, measure):
         assert np.max(np.abs(b.download() - exp)) < 1e-5
 
 
+@pytest.mark.parametrize("n", [1, 4, 11])
+@pytest.mark.parametrize("count", [0, 1, 2, 3, 4, 5])
+def test_short_fused_programs(n, count):
+    """A few gates are launched one by one, on either side of a measurement too."""
+    rng = np.random.default_rng(n + 50 * count)
+    first, a, b = _program(n, rng, 25), _program(n, rng, count), _program(n, rng, count)
+    meas = qc.ops_from_tuples([(OP["MEASURE"], 0, 0, 0, 1, 0.0)])
+    for ops in (a, np.concatenate([a, meas, b])):
+        with engine.DeviceState(n, "c128") as ref, engine.DeviceState(n, "c128") as s:
+            exp = ref.apply(first).apply(ops, 0, 9).download()
+            assert np.max(np.abs(s.apply(first).apply(ops, QSV_FLAG_FUSE, 9).download() - exp)) < 1e-13
+
+
 @pytest.mark.parametrize("precision", ["c128", "c64"])
 def test_batched_energies(precision):
     rng = np.random.default_rng(12)
