@@ -90,7 +90,7 @@ struct qsv_state {
   PassSlot* ring_pending = nullptr;
   uint64_t passes_launched = 0;
   int tile_low = -1;            // tile low-run width forced by the tuner (-1: none)
-  unsigned long long* reach = nullptr;   // fused passes: TileNorm::reach
+  int reach_left = 0;           // passes that may still track where amplitudes can be
   double* norm_buf = nullptr;   // complex64 FP32 passes: per-tile norms (2 x ntiles) + control (2)
   uint64_t* shot_dev = nullptr;   // qsv_sample's outcomes (lazy, at most kShotsKept)
   uint64_t shot_cap = 0;
@@ -347,6 +347,16 @@ void transpose2(const double g[8], double t[8])
   t[6] = g[6]; t[7] = g[7];
 }
 
+// A program's first passes keep track of where nonzero amplitudes can be, so
+// that the tiles elsewhere are not read (six layers of 27 qubits from |0..0>:
+// 6.13 -> 4.94 ms). States below 256 MiB are read from the memory-side cache. A
+// dense state only pays for it (24 qubits, complex128: 15 us of the first pass's
+// 100), so a state has kReachTotal such passes from when it was last set, copied
+// or measured, and a program of a single pass, which no pass follows, has none.
+constexpr int kReachPasses = 4, kReachTotal = 2 * kReachPasses;
+constexpr double kReachBytes = 256.0 * (1 << 20);
+constexpr size_t kReachHead = 256;   // room for TileNorm::reach before the programs of a launch
+
 int measure_impl(qsv_state* s, uint64_t mask, double u, uint64_t* outcome, double* probs_out)
 {
   const int n = s->n;
@@ -385,6 +395,7 @@ int measure_impl(qsv_state* s, uint64_t mask, double u, uint64_t* outcome, doubl
   rc = timed(s, QSV_KCLASS_OTHER, 2.0 * s->S * s->bytes_per_amp(),
              [&] { launch_collapse(s->prec, s->amps, s->S, m, pos.data(), sel, f, s->stream); });
   if (rc) return rc;
+  s->reach_left = kReachTotal;
   if (outcome) *outcome = sel;
   if (probs_out) std::memcpy(probs_out, pr.data(), no * sizeof(double));
   return QSV_OK;
@@ -592,6 +603,8 @@ int upload_passes(qsv_state* s, const std::vector<char>& progs, const char** dev
   if (slot.event) HIPCHK(hipEventSynchronize(slot.event));
   const size_t need = progs.size();
   if (slot.cap < need) {
+    // (passes of later slots may use the reach words that a slot starts with)
+    HIPCHK(hipStreamSynchronize(s->stream));
     if (slot.host) HIPCHK(hipHostFree(slot.host));
     if (slot.dev) HIPCHK(hipFree(slot.dev));
     slot.host = nullptr;
@@ -610,70 +623,83 @@ int upload_passes(qsv_state* s, const std::vector<char>& progs, const char** dev
   return QSV_OK;
 }
 
-// A program's first passes keep track of where nonzero amplitudes can be, so
-// that the tiles elsewhere are not read (six layers of 27 qubits from |0..0>:
-// 6.13 -> 4.94 ms). States below 256 MiB are read from the memory-side cache and the
-// clearing launch would cost as much as it saves.
-constexpr int kReachPasses = 4;
-constexpr double kReachBytes = 256.0 * (1 << 20);
-
-// What the passes of one program hand on from launch to launch.
+// The passes of one program on their way to the device: compiled one by one,
+// launched a few at a time.
 struct PassRun {
+  bool f32 = false;
+  int block_cost = 0;                      // FP32 passes: register-bit runs of that cost become PO_BLOCK ops
   std::complex<double> scalar{1.0, 0.0};   // the factors common to the whole state
   int reach = 0;                           // passes that tracked reach; kReachPasses: no more
+  unsigned long long* reach_at = nullptr;  // in the buffer of the first launch (the ring reuses it after
+                                           // four; tracked passes are in the first three)
+  // compiled and not launched yet
+  std::vector<char> progs;
+  std::vector<size_t> at;
+  std::vector<int> renorm;                 // FP_RENORM_* of each
+  bool reach_head = false;                 // they start with room for TileNorm::reach
 };
 
-// Launches the first `count` passes and drops them from the list. blocks: FP32
-// passes fold register-bit runs into PO_BLOCK ops. The common factors are
-// applied by the last pass of a run (`end`).
-int launch_passes(qsv_state* s, std::vector<FPass>& passes, size_t count, bool f32, bool blocks, PassRun& run,
-                  bool end)
+// |index> in s.
+void fill_basis(qsv_state* s, uint64_t index)
 {
-  if (!count) return QSV_OK;
+  launch_fill_basis(s->prec, s->amps, s->S, index, s->stream);
+  s->reach_left = kReachTotal;
+}
+
+// Compiles the next pass of a run. The last one applies the factors common to the
+// whole state; `only`: it is the first one too.
+void add_pass(qsv_state* s, PassRun& run, const FPass& p, bool last, bool only)
+{
+  if ((double)s->S * s->bytes_per_amp() < kReachBytes || only) run.reach = kReachPasses;
+  if (run.reach == 0 && s->reach_left > 0) {
+    run.progs.resize(kReachHead, 0);
+    run.reach_head = true;
+  }
+  run.at.push_back(compile_pass(p, run.f32, run.block_cost, run.scalar, last, run.progs));
+  run.renorm.push_back(p.renorm);
+  PHead h;
+  std::memcpy(&h, run.progs.data() + run.at.back(), sizeof(h));
+  if (run.reach < kReachPasses && s->reach_left > 0 && (h.renorm & FP_KEEP_ZERO)) {
+    h.renorm |= FP_REACH | (run.reach++ ? FP_REACH_USE : 0);
+    --s->reach_left;
+    std::memcpy(run.progs.data() + run.at.back(), &h, sizeof(h));
+  } else {
+    run.reach = kReachPasses;   // a pass that does not track it ends it
+  }
+}
+
+int launch_passes(qsv_state* s, PassRun& run)
+{
+  if (run.at.empty()) return QSV_OK;
   const uint64_t ntiles = s->S >> kPassTileBits;
   TileNorm nb{nullptr, nullptr, nullptr, nullptr};
-  if (f32) {
+  if (run.f32) {
     if (!s->norm_buf) HIPCHK(hipMalloc((void**)&s->norm_buf, (2 * ntiles + 2) * sizeof(double)));
     nb = TileNorm{s->norm_buf, s->norm_buf + ntiles, s->norm_buf + 2 * ntiles, nullptr};
   }
-  const int block_cost = f32 && blocks ? pass_block_cost() : 0;
-  std::vector<char> progs;
-  std::vector<size_t> at(count);
-  if ((double)s->S * s->bytes_per_amp() < kReachBytes) run.reach = kReachPasses;
-  bool clear = false;
-  for (size_t i = 0; i < count; ++i) {
-    at[i] = compile_pass(passes[i], f32, block_cost, run.scalar, end && i + 1 == count, progs);
-    PHead h;
-    std::memcpy(&h, progs.data() + at[i], sizeof(h));
-    if (run.reach < kReachPasses && (h.renorm & FP_KEEP_ZERO)) {
-      clear |= run.reach == 0;
-      h.renorm |= FP_REACH | (run.reach++ ? FP_REACH_USE : 0);
-      std::memcpy(progs.data() + at[i], &h, sizeof(h));
-    } else {
-      run.reach = kReachPasses;   // a pass that does not track it ends it
-    }
-  }
   const char* dev = nullptr;
-  int rc = upload_passes(s, progs, &dev);
+  int rc = upload_passes(s, run.progs, &dev);
   if (rc) return rc;
-  if (clear && !s->reach) HIPCHK(hipMalloc((void**)&s->reach, 2 * sizeof(*s->reach)));
-  nb.reach = s->reach;
-  if (clear) launch_clear_reach(s->reach, s->stream);
-  for (size_t i = 0; i < count; ++i) {
-    const char* p = dev + at[i];
+  if (run.reach_head) run.reach_at = reinterpret_cast<unsigned long long*>(const_cast<char*>(dev));
+  nb.reach = run.reach_at;
+  for (size_t i = 0; i < run.at.size(); ++i) {
+    const char* p = dev + run.at[i];
     rc = timed(s, QSV_KCLASS_BLOCK, 2.0 * s->S * s->bytes_per_amp(),
-               [&] { launch_pass(s->prec, f32, s->amps, p, ntiles, nb, s->stream); });
+               [&] { launch_pass(s->prec, run.f32, s->amps, p, ntiles, nb, s->stream); });
     if (rc) return rc;
-    if (passes[i].renorm & FP_RENORM_OUT) {
-      const bool first = (passes[i].renorm & FP_RENORM_IN) != 0;
+    if (run.renorm[i] & FP_RENORM_OUT) {
+      const bool first = (run.renorm[i] & FP_RENORM_IN) != 0;
       rc = timed(s, QSV_KCLASS_OTHER, (first ? 2.0 : 1.0) * ntiles * sizeof(double),
                  [&] { launch_norm_ctl(nb, ntiles, first, s->stream); });
       if (rc) return rc;
     }
   }
   HIPCHK(hipEventRecord(s->ring_pending->event, s->stream));
-  s->passes_launched += count;
-  passes.erase(passes.begin(), passes.begin() + count);
+  s->passes_launched += run.at.size();
+  run.progs.clear();
+  run.at.clear();
+  run.renorm.clear();
+  run.reach_head = false;
   return QSV_OK;
 }
 
@@ -767,10 +793,9 @@ void build_pass(const qsv_state* s, const std::vector<BGate>& gs, const std::vec
 }
 
 // The last pass of a run of passes needs no scale for a successor.
-void end_run(std::vector<FPass>& passes)
+void end_run(FPass& last)
 {
-  if (passes.empty()) return;
-  int& rn = passes.back().renorm;
+  int& rn = last.renorm;
   rn &= ~FP_RENORM_OUT;
   if (!(rn & FP_RENORM_APPLY)) rn = 0;
 }
@@ -1177,33 +1202,45 @@ int run_fused(qsv_state* s, const std::vector<BGate>& gs_in, uint32_t flags)
   if (s->n < kPassTileBits) return run_small(s, gs);
   const bool f32 = s->prec == QSV_C64 && !(flags & QSV_FLAG_FP64_PASSES);
   const bool blocks = !(flags & QSV_FLAG_VALU_PASSES);
-  // Passes are launched while later ones are still planned: one, then two, four
-  // and so on, so that the device starts early and the uploads stay few. The
-  // newest pass waits until it is known whether it ends its run. Six layers of
+  // Passes are launched while later ones are still planned and compiled: one, then
+  // two, four and so on, so that the device starts early and the uploads stay few.
+  // The newest pass waits until it is known whether it ends its run. Six layers of
   // 27 qubits 6.33 -> 6.13 ms, a two-layer 26-qubit ansatz 1.74 -> 1.64 ms, ten
   // layers of 19 qubits 311 -> 303 us. A register of one tile gains nothing from
   // splitting its only pass: 12 qubits 272 us whole, 303 us in pieces of 64 gates.
-  std::vector<FPass> passes;
-  PassRun run;
   size_t chunk = 1;
-  int rc = fuse_walk(
+  PassRun run;
+  run.f32 = f32;
+  run.block_cost = f32 && blocks ? pass_block_cost() : 0;
+  FPass newest;
+  bool waiting = false, first = true;   // newest is not compiled yet; it starts its run
+  auto end = [&]() {
+    if (!waiting) return (int)QSV_OK;
+    waiting = false;
+    end_run(newest);
+    add_pass(s, run, newest, true, first && run.at.empty());
+    first = true;
+    return launch_passes(s, run);
+  };
+  const int rc = fuse_walk(
       s, gs, f32,
       [&](FPass&& p) {
-        passes.push_back(std::move(p));
-        if (passes.size() <= chunk) return (int)QSV_OK;
-        const int r = launch_passes(s, passes, chunk, f32, blocks, run, false);
+        if (waiting) {
+          add_pass(s, run, newest, false, false);
+          first = false;
+        }
+        newest = std::move(p);
+        waiting = true;
+        if (run.at.size() < chunk) return (int)QSV_OK;
         chunk = std::min<size_t>(2 * chunk, 512);
-        return r;
+        return launch_passes(s, run);
       },
       [&](size_t i) {
-        end_run(passes);
-        const int r = launch_passes(s, passes, passes.size(), f32, blocks, run, true);
+        const int r = end();
         run.reach = kReachPasses;
         return r ? r : run_direct(s, gs[i]);
       });
-  if (rc) return rc;
-  end_run(passes);
-  return launch_passes(s, passes, passes.size(), f32, blocks, run, true);
+  return rc ? rc : end();
 }
 
 // ---- Pauli-string expectations ------------------------------------------------
@@ -1535,7 +1572,7 @@ int qsv_state_create(int num_qubits, int precision, qsv_state** out)
     return cleanup(QSV_E_NOMEM, "hipMalloc of reduction output failed");
   if (hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking) != hipSuccess)
     return cleanup(QSV_E_DEVICE, "hipStreamCreate failed");
-  launch_fill_basis(s->prec, s->amps, s->S, 0, s->stream);
+  fill_basis(s, 0);
   if (hipStreamSynchronize(s->stream) != hipSuccess) return cleanup(QSV_E_DEVICE, "initialising |0..0> failed");
   *out = s;
   return QSV_OK;
@@ -1562,7 +1599,6 @@ int qsv_state_destroy(qsv_state* s)
   if (s->prefix) hipFree(s->prefix);
   if (s->hist) hipFree(s->hist);
   if (s->norm_buf) hipFree(s->norm_buf);
-  if (s->reach) hipFree(s->reach);
   if (s->shot_dev) hipFree(s->shot_dev);
   if (s->samp_dev) hipFree(s->samp_dev);
   if (s->samp_host) hipHostFree(s->samp_host);
@@ -1579,7 +1615,7 @@ int qsv_state_init_basis(qsv_state* s, uint64_t index)
   int rc = check_state(s);
   if (rc) return rc;
   if (index >= s->S) return fail(QSV_E_INVALID, "basis index out of range");
-  launch_fill_basis(s->prec, s->amps, s->S, index, s->stream);
+  fill_basis(s, index);
   HIPCHK(hipGetLastError());
   return QSV_OK;
 }
@@ -1589,6 +1625,7 @@ int qsv_state_upload(qsv_state* s, const double* amps, uint64_t offset, uint64_t
   int rc = check_state(s);
   if (rc) return rc;
   if (!amps || offset > s->S || count > s->S - offset) return fail(QSV_E_INVALID, "upload range invalid");
+  s->reach_left = kReachTotal;
   if (s->prec == QSV_C128) {
     HIPCHK(hipMemcpyAsync((char*)s->amps + offset * 16, amps, count * 16, hipMemcpyHostToDevice, s->stream));
     HIPCHK(hipStreamSynchronize(s->stream));
@@ -1647,6 +1684,7 @@ int qsv_state_copy(qsv_state* dst, const qsv_state* src)
   if (dst->n != src->n || dst->prec != src->prec) return fail(QSV_E_INVALID, "copy: shape or precision mismatch");
   HIPCHK(hipStreamSynchronize(src->stream));
   launch_copy(src->prec, src->amps, dst->amps, src->S, dst->stream);
+  dst->reach_left = kReachTotal;
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(dst->stream));
   return QSV_OK;
@@ -2452,7 +2490,7 @@ int qsv_batch_expect_z(const qsv_batch_desc* d, double* energies)
       cleanup();
       return fail(QSV_E_DEVICE, "batch: stream wait failed");
     }
-    launch_fill_basis(s->prec, s->amps, s->S, 0, s->stream);
+    fill_basis(s, 0);
     if ((rc = run_fused(s, decoded[i], 0))) {
       cleanup();
       return rc;
@@ -2765,7 +2803,7 @@ int qsv_noisy_trajectories(int num_qubits, int precision, const qsv_op* ops, uin
   }
   for (uint64_t t = 0; t < n_traj && !rc; ++t) {
     trajectory_gates(t, gs);
-    launch_fill_basis(s->prec, s->amps, s->S, 0, s->stream);
+    fill_basis(s, 0);
     if ((rc = run_fused(s, gs, 0))) break;
     launch_sample(s->prec, s->amps, s->S, s->prefix, 1, measure_seed(t), d_out, s->stream);
     if (hipMemcpyAsync(outcomes + t, d_out, sizeof(uint64_t), hipMemcpyDeviceToHost, s->stream) != hipSuccess ||
@@ -3052,7 +3090,7 @@ int launch_large(qsv_server* sv, SrvReq* r)
   int rc = take_state(sv, r->n, &r->st);
   if (rc) return rc;
   qsv_state* s = r->st;
-  launch_fill_basis(s->prec, s->amps, s->S, 0, s->stream);
+  fill_basis(s, 0);
   if (sv->cfg.flags & QSV_FLAG_FUSE) rc = run_fused(s, r->gates, sv->cfg.flags);
   else {
     for (const auto& g : r->gates)

@@ -285,7 +285,6 @@ struct PHead {
 // pass when `last`.
 size_t compile_pass(const FPass& p, bool f32, int block_cost, std::complex<double>& scalar, bool last,
                     std::vector<char>& out);
-void launch_clear_reach(unsigned long long* reach, hipStream_t st);
 // f32: complex64 arithmetic in FP32 (ignored for complex128, always FP64)
 void launch_pass(int prec, bool f32, void* psi, const char* dprog, uint64_t ntiles, const TileNorm& nb,
                  hipStream_t st);

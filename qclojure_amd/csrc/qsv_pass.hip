@@ -121,8 +121,10 @@ __global__ __launch_bounds__(kThreads, sizeof(A) == 4 ? 5 : 4) void k_pass(typen
   const bool keep = (rn & FP_KEEP_ZERO) && !(sizeof(A) == 4 && (rn & FP_RENORM_APPLY) && !(nb.ctl[1] < 1e30));
   if constexpr (!GROUP) {
     // A tile that no nonzero amplitude of the earlier passes can lie in is not
-    // even read: its base has a bit set, or clear, that none of those has. A
-    // launch's own tiles may extend `reach` meanwhile; that only keeps tiles.
+    // even read: its base has a bit set, or clear, that none of those has. The
+    // launch's own tiles extend `reach` meanwhile, but one that passed this test
+    // adds nothing but the tile's bits, which the test leaves out: every wave of a
+    // workgroup decides alike.
     if (rn & FP_REACH) {
 #pragma unroll
       for (int i = 0; i < TB; ++i) tmask |= 1ull << h.sorted_pos[i];
@@ -270,16 +272,6 @@ __global__ __launch_bounds__(1024) void k_norm_ctl(const double* __restrict__ pa
     ctl[0] = target;
     ctl[1] = (target > 0.0 && sb[0] > 0.0) ? sqrt(target / sb[0]) : 1.0;
   }
-}
-
-__global__ void k_clear_reach(unsigned long long* reach)
-{
-  reach[threadIdx.x] = 0ull;
-}
-
-void launch_clear_reach(unsigned long long* reach, hipStream_t st)
-{
-  hipLaunchKernelGGL(k_clear_reach, dim3(1), dim3(2), 0, st, reach);
 }
 
 void launch_pass(int prec, bool f32, void* psi, const char* dprog, uint64_t ntiles, const TileNorm& nb,

@@ -47,10 +47,11 @@ def test_sparse(n, where):
         assert abs(f32.norm2() - 1.0) < 2e-6
 
 
-@pytest.mark.parametrize("prec,n", [("c128", 24), ("c64", 25)])
+@pytest.mark.parametrize("prec,n,arithmetic", [("c128", 24, 64), ("c64", 25, 64), ("c64", 25, 32)])
 @pytest.mark.parametrize("start", ["zero", "top", "two", "dense"])
-def test_reach(prec, n, start):
-    """Large states: the first passes keep track of where amplitudes can be."""
+def test_reach(prec, n, arithmetic, start):
+    """Large states: the first passes keep track of where amplitudes can be, in
+    FP32 passes beside the norms that they hand on (a tile not read has none)."""
     rng = np.random.default_rng(n + len(start))
     rows = []
     if start == "top":
@@ -62,11 +63,28 @@ def test_reach(prec, n, start):
     first = qc.ops_from_tuples(rows)
     more = [qc.ops_from_tuples(_program(list(qs), rng, 70)) for qs in (range(0, n, 2), range(n))]
     with engine.DeviceState(n, prec) as ref, engine.DeviceState(n, prec) as a:
-        for s, flags in ((ref, 0), (a, QSV_FLAG_FUSE | (QSV_FLAG_FP64_PASSES if prec == "c64" else 0))):
+        for s, flags in ((ref, 0), (a, QSV_FLAG_FUSE | (QSV_FLAG_FP64_PASSES if prec == "c64" and arithmetic == 64 else 0))):
             if len(rows):
                 s.apply(first)
             for ops in more:
                 s.apply(ops, flags)
         # 140 gates on amplitudes of at most 1; complex64 rounds its stores
         assert a.compare(ref)["max_abs_diff"] < (1e-13 if prec == "c128" else 1e-5)
-        assert abs(a.norm2() - 1.0) < (1e-12 if prec == "c128" else 1e-4)
+        # FP32 passes remove their drift, stores that only round leave it
+        assert abs(a.norm2() - 1.0) < (1e-12 if prec == "c128" else 2e-6 if arithmetic == 32 else 1e-4)
+
+
+def test_reach_across_programs():
+    """Short programs on one state, as many as use up the passes that may track it
+    and more, from a basis state that is set again in between."""
+    n = 24
+    rng = np.random.default_rng(1)
+    with engine.DeviceState(n, "c128") as ref, engine.DeviceState(n, "c128") as a:
+        for k in range(8):
+            qubits = list(range(n)) if k % 3 else list(range(k, n, 2))
+            ops = qc.ops_from_tuples(_program(qubits, rng, 24))
+            for s, flags in ((ref, 0), (a, QSV_FLAG_FUSE)):
+                if k == 5:
+                    s.init_basis(3 * 2 ** 20 + 1)
+                s.apply(ops, flags)
+            assert a.compare(ref)["max_abs_diff"] < 1e-13
