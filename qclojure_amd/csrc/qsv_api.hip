@@ -2519,13 +2519,19 @@ double norm2_entries(const double m[8])
   for (int e = 0; e < 8; ++e) s += m[e] * m[e];
   return s;
 }
-double least_singular(const double m[8])
+void singular_values(const double m[8], double* least, double* most)
 {
   const double re = m[0] * m[6] - m[1] * m[7] - m[2] * m[4] + m[3] * m[5];
   const double im = m[0] * m[7] + m[1] * m[6] - m[2] * m[5] - m[3] * m[4];
   const double det = std::hypot(re, im), t = norm2_entries(m);
-  const double most = std::sqrt(0.5 * (t + std::sqrt(std::max(0.0, t * t - 4.0 * det * det))));
-  return most > 0.0 ? det / most : 0.0;
+  *most = std::sqrt(0.5 * (t + std::sqrt(std::max(0.0, t * t - 4.0 * det * det))));
+  *least = *most > 0.0 ? det / *most : 0.0;
+}
+double least_singular(const double m[8])
+{
+  double least, most;
+  singular_values(m, &least, &most);
+  return least;
 }
 // Are the rows of m orthogonal and of equal length, to `tol` of that length squared?
 bool unitary_multiple(const double m[8], double tol)
@@ -2576,7 +2582,6 @@ int qsv_noisy_trajectories(int num_qubits, int precision, const qsv_op* ops, uin
   // max |k_ij| = 1; and their selection weights max |k_ij|^2 (channel.clj:203-212)
   std::vector<std::vector<std::array<double, 8>>> kops(n_sites);
   std::vector<std::vector<double>> kw(n_sites);
-  std::vector<char> keeps_norm(n_sites, 1);
   for (uint64_t k = 0; k < n_sites; ++k) {
     const qsv_kraus_site& st = sites[k];
     if (st.after_op >= n_ops) return fail(QSV_E_INVALID, "site " + std::to_string(k) + ": after_op out of range");
@@ -2592,7 +2597,6 @@ int qsv_noisy_trajectories(int num_qubits, int precision, const qsv_op* ops, uin
       std::array<double, 8> a;
       const bool unitary = unitary_multiple(st.m[j], 1e-14);
       const double sc = 1.0 / std::sqrt(unitary ? 0.5 * norm2_entries(st.m[j]) : mx);
-      keeps_norm[k] &= unitary;
       for (int e = 0; e < 8; ++e) a[e] = st.m[j][e] * sc;
       kops[k].push_back(a);
       kw[k].push_back(mx);
@@ -2685,11 +2689,10 @@ int qsv_noisy_trajectories(int num_qubits, int precision, const qsv_op* ops, uin
     // one workgroup per trajectory, all running one program: its noise sites
     // draw their uniform and choose their operator on the device. Final states
     // go to an arena (chunks bound it to 1 GiB), one shot each.
-    // The state is renormalised at every site, as the reference does, except at
-    // those whose operators keep the norm. The sites of different qubits run in
-    // no particular order, so a rule that counts them (every 16th) lets any
-    // number of others shrink the state in between. Where a gate of the program
-    // does not keep the norm, every site renormalises.
+    // A renormalisation follows a site where the operators since the last one may
+    // have taken the norm out of range (the compiler counts: sites of different
+    // qubits run in no particular order), or every site where a gate of the program
+    // does not keep the norm itself.
     bool unitary = true;
     for (const BGate& g : clean)
       if (g.kind == FG_DENSE || g.kind == FG_PHASE)
@@ -2713,13 +2716,21 @@ int qsv_noisy_trajectories(int num_qubits, int precision, const qsv_op* ops, uin
         f.a = n - 1 - sites[k].qubit;
         f.b = (int32_t)k;
         f.cmask = (uint32_t)table.size();
-        f.sub = sites[k].n_kraus;
-        f.bmask = unitary && keeps_norm[k] ? 0u : 1u;
-        for (int j = 0; j < sites[k].n_kraus; ++j) {
+        f.bmask = unitary ? 0u : 1u;
+        f.m[0] = 1.0;   // the norm's least and most factor over the operators that a uniform below 1 reaches
+        f.m[1] = 1.0;
+        double acc = 0.0;
+        for (int j = 0; j < sites[k].n_kraus && acc < 1.0; ++j) {
           KrausOp o;
           o.w = kw[k][j];
+          acc += o.w;
           std::memcpy(o.m, kops[k][j].data(), sizeof(o.m));
           table.push_back(o);
+          ++f.sub;
+          double least, most;
+          singular_values(o.m, &least, &most);
+          f.m[0] = std::min(f.m[0], least);
+          f.m[1] = std::max(f.m[1], most);
         }
         p.gates.push_back(f);
       }

@@ -179,6 +179,8 @@ struct Compiler {
   Waves own;               // after the last LDS round trip
   bool have_own = false;
   Waves load_wr;
+  size_t last_site = SIZE_MAX;       // the last PO_KRAUS op,
+  double least = 1.0, most = 1.0;    // and the range of the norm since the last renormalisation
   bool synced = false;     // every wave's tile has crossed a workgroup barrier
 
   std::vector<Factor>& pend = mem.pend;
@@ -559,11 +561,24 @@ struct Compiler {
     const int rb = (int)rank_in(reg, g.a);
     if (g.kind == FG_KRAUS) {
       flush(t);
+      // A renormalisation after the site before this one, or after this one, where
+      // the norm could otherwise be out of range; far from the 1e-12 below which a
+      // renormalisation leaves a state alone. An operator that could take the norm
+      // there by itself (a projector) has one on either side.
+      constexpr double kLeastNorm = 1e-8, kMostNorm = 1e8;
+      if (last_site != SIZE_MAX && ((!(least * g.m[0] >= kLeastNorm) && least < 0.5) || !(most * g.m[1] <= kMostNorm))) {
+        ops[last_site].flag = 1;
+        least = most = 1.0;
+      }
       POp& op = emit(PO_KRAUS + rb);
       op.kc = (uint32_t)g.b;
       op.aux = g.cmask;
       op.cnt = g.sub;
-      op.flag = (int32_t)g.bmask;
+      least *= g.m[0];
+      most *= g.m[1];
+      op.flag = g.bmask || !(least >= kLeastNorm) ? 1 : 0;
+      if (op.flag) least = most = 1.0;
+      last_site = ops.size() - 1;
       return true;
     }
     if (g.cmask & row_dirty) return false;

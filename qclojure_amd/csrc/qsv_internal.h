@@ -155,7 +155,8 @@ inline bool is_phase(double re, double im)
 enum { DM_GENERAL = 0, DM_REAL = 1, DM_RX = 2, DM_EXCHANGE = 3 };
 
 // A gate in tile-local bit coordinates. FG_KRAUS: target a, site b, operators
-// cmask .. cmask + sub - 1 of the table, bmask: renormalise afterwards.
+// cmask .. cmask + sub - 1 of the table, which change the norm by a factor between
+// m[0] <= 1 and m[1] >= 1; bmask: renormalise afterwards in any case.
 struct FGate {
   int32_t kind;        // FG_*
   int32_t a, b;        // dense/phase target a; swap bits a, b

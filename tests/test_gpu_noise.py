@@ -103,14 +103,16 @@ def test_deep_damping_stays_normalised(eng, oracle, prec, n):
 
 
 def _damped(n, count, gamma, kind):
-    """A damping channel after every gate of a program without entanglers."""
+    """A channel that changes the norm after every gate of a program without entanglers."""
     if kind == "phase":      # X, then RZ on the excited qubit: K0 = diag(1, sqrt(1 - gamma)) every time
         rows = [(qc.OP["X"], 0, 0, 0, 0, 0.0)] + [(qc.OP["RZ"], 0, 0, 0, 0, 0.3)] * count
         kraus = nz.phase_damping_kraus_operators(gamma)
         sites = [{"after-op": k + 1, "qubit": 0, "kraus": kraus} for k in range(count)]
-    else:                    # H and amplitude damping, qubit after qubit
+    else:                    # H and amplitude damping, projectors or a shear, qubit after qubit
         rows = [(qc.OP["H"], k % n, 0, 0, 0, 0.0) for k in range(count)]
-        kraus = nz.amplitude_damping_kraus_operators(gamma)
+        kraus = {"amplitude": lambda: nz.amplitude_damping_kraus_operators(gamma),
+                 "project": lambda: [math.sqrt(0.5) * np.diag([1, 0]), math.sqrt(0.5) * np.diag([0, 1])],
+                 "shear": lambda: [np.array([[1, 1], [0, 1]])]}[kind]()
         sites = [{"after-op": k, "qubit": k % n, "kraus": kraus} for k in range(count)]
     return qc.ops_from_tuples(rows), sites
 
@@ -133,9 +135,11 @@ def _check_damped(eng, oracle, prec, n, count, gamma, kind, T):
 
 @pytest.mark.parametrize("prec", ["c64", "c128"])
 @pytest.mark.parametrize("n,count,gamma,kind", [(1, 200, 0.99, "phase"), (3, 400, 0.99, "phase"),
-                                                (8, 800, 0.9, "amplitude"), (11, 300, 0.9, "amplitude")])
+                                                (8, 800, 0.9, "amplitude"), (11, 300, 0.9, "amplitude"),
+                                                (3, 300, 0.0, "project"), (9, 200, 0.0, "project"),
+                                                (4, 900, 0.0, "shear")])
 def test_strong_damping_in_registers(eng, oracle, prec, n, count, gamma, kind):
-    """Every site shrinks the norm, up to ten times, and the sites of different
+    """Every site changes the norm, up to ten times, and the sites of different
     qubits run in any order: no run of them may take the norm below the 1e-12
     that a single renormalisation asks for, nor out of FP32's range."""
     _check_damped(eng, oracle, prec, n, count, gamma, kind, 4)
