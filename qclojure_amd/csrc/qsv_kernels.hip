@@ -746,15 +746,17 @@ void launch_outcome_hist(int prec, const void* psi, uint64_t S, int m, const int
   if (m <= 12) {
     uint64_t mask = 0;
     for (int j = 0; j < m; ++j) mask |= 1ull << pos[j];
-    // At most 512 blocks, 1024 where the read dominates: each adds its outcomes to the same few global sums (one
-    // measured bit of 20 qubits: 51 us a call with 256 blocks, 56 with 512, 63 with
-    // 1024; of 22 qubits 73 with 512, 77 with 1024). 16 amplitudes a thread, half as
-    // many for each measured bit among those that it walks: a thread of several
-    // outcomes makes as many chains of lane exchanges (8 high bits of 13 qubits 41
-    // us a call; 49 with eight outcomes a thread; 42 with one LDS atomic an
-    // amplitude, which is within 3 % of this for 10 bits or less of up to 19 qubits
-    // and up to 60 % slower above; for 12 bits of 20 or 21 qubits it is 10 % faster).
-    const uint64_t least = (uint64_t)kBlock << (4 - __builtin_popcountll(mask & (15ull * kBlock)));
+    // At most 512 blocks, 1024 where the read dominates: each adds its outcomes to
+    // the same few global sums (one measured bit of 20 qubits: 51 us a call with 256
+    // blocks, 56 with 512, 63 with 1024; of 22 qubits 73 with 512, 77 with 1024). 16
+    // amplitudes a thread, 8 below 2^20 (one round of loads), half as many for each
+    // measured bit that it would walk: a thread of several outcomes makes as many
+    // chains of lane exchanges (8 high bits of 13 qubits 41 us a call; 49 with eight
+    // outcomes a thread; 42 with one LDS atomic an amplitude, which is within 4 % of
+    // this up to 19 qubits and up to 80 % slower above; for 12 bits of 20 or 21
+    // qubits it is 10 % faster).
+    const int each = S >= 1ull << 20 ? 4 : 3;
+    const uint64_t least = (uint64_t)kBlock << (each - __builtin_popcountll(mask & (((1ull << each) - 1) * kBlock)));
     const uint64_t span = std::min(S, std::max(S >> (S >= 1ull << 23 ? 10 : 9), least));
     const unsigned g = (unsigned)((S + span - 1) / span);
     const size_t lds = no * sizeof(double);
