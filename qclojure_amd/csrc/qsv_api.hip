@@ -1353,7 +1353,8 @@ int pauli_sums(const qsv_state* s, const std::vector<uint64_t>& xm, const std::v
 
 // Pass shapes of grouped batch programs, by program structure: an optimiser
 // loop resubmits the same circuits with new angles, and the fuser's choices
-// depend only on which bits each gate touches (and the tile width), so a
+// depend only on which bits each gate touches, whether a diagonal one needs its
+// target in the tile (its first entry is no phase), and the tile width, so a
 // structure seen before skips the fuser's search. Keyed by the exact
 // structure (hash plus full comparison); cleared when it grows past a bound.
 struct ShapeEntry {
@@ -1931,7 +1932,7 @@ int qsv_inner(const qsv_state* a, const qsv_state* b, double out[2])
 namespace {
 
 // Pooled device states for batched circuits too large for one workgroup's
-// LDS, keyed by (num_qubits, precision); reused across batches.
+// registers, keyed by (num_qubits, precision); reused across batches.
 std::mutex g_pool_mu;
 std::vector<qsv_state*> g_pool[2][40];
 constexpr int kPoolPerSize = 8;
@@ -2906,7 +2907,7 @@ int grow_arena(void** p, size_t* cap, size_t need)
 struct qsv_server {
   qsv_server_config cfg{};
   uint64_t budget = 0, in_use = 0;
-  int lds_n = 14;
+  int small_n = 14;   // the largest register of one workgroup
   std::mutex mu;
   std::condition_variable cv_work, cv_done;
   std::deque<SrvReq*> queue;
@@ -3285,7 +3286,7 @@ int qsv_server_create(const qsv_server_config* cfg, qsv_server** out)
   HIPCHK(hipSetDevice(g_device));
   auto* sv = new qsv_server();
   sv->cfg = *cfg;
-  sv->lds_n = cfg->precision == QSV_C128 ? 13 : 14;
+  sv->small_n = cfg->precision == QSV_C128 ? kSmallC128 : kSmallC64;
   size_t fr = 0, tot = 0;
   if (hipMemGetInfo(&fr, &tot) != hipSuccess) {
     delete sv;
@@ -3324,7 +3325,7 @@ int qsv_server_submit(qsv_server* sv, int num_qubits, const qsv_op* ops, uint64_
   }
   const uint64_t B = sv->cfg.precision == QSV_C128 ? 16 : 8;
   r->bytes = (1ull << num_qubits) * B;
-  r->small = sv->cfg.batch_small && num_qubits <= sv->lds_n;
+  r->small = sv->cfg.batch_small && num_qubits <= sv->small_n;
   if (r->bytes > sv->budget) {
     delete r;
     return fail(QSV_E_NOMEM, "request state exceeds the HBM budget");

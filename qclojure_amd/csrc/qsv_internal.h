@@ -137,8 +137,8 @@ void launch_collapse(int prec, void* psi, uint64_t S, int m, const int* pos, uin
 constexpr int kMaxPassGates = 1024, kMaxPassGatesF32 = 96;
 
 // FG_RENORM: divide the state by its FP64 norm when that exceeds 1e-12, as
-// normalize-state does after a Kraus operator (a record of batched LDS
-// circuits, a barrier between fused passes; never inside a pass).
+// normalize-state does after a Kraus operator (in trajectories above one
+// workgroup; a barrier between fused passes, never inside one).
 // FG_KRAUS: a noise site of a trajectory program (an operator chosen on the
 // device); only in FGate lists.
 enum { FG_DENSE = 0, FG_PHASE = 1, FG_SWAP = 2, FG_BLOCKADE = 3, FG_RENORM = 4, FG_KRAUS = 5 };

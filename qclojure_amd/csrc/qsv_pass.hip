@@ -28,9 +28,8 @@
 // 5.3 TB/s) with the gates' instructions partly on top; on few tiles the chain
 // of ops, whose fetch from memory is hidden behind the op before. Against the
 // interpreter that ran every gate as an op and kept two copies of the tile
-// (three waves per SIMD), per launch: 27-qubit complex128 layers 1257 -> 925 us,
-// 19-qubit ones 47 -> 22 us, 540 gates on one 12-qubit tile 524 -> 177 us,
-// 26-qubit complex64 QAOA 372 -> 352 us.
+// (three waves per SIMD), per launch: dense 27-qubit complex128 layers 1257 ->
+// 885 us, 19-qubit ones 47 -> 23 us, 540 gates on one 12-qubit tile 524 -> 122 us.
 #include "qsv_ops.h"
 
 namespace qsv {
@@ -40,18 +39,18 @@ namespace {
 constexpr int kThreads = 256;
 // A launch of few tiles is a chain of ops whose fetches miss every cache (the
 // program was just written): its workgroups read the program into L2 first.
-// 540 gates on one tile 177 -> 138 us, 19-qubit passes (128 tiles) 21.9 -> 20.7;
+// 540 gates on one tile 146 -> 122 us, 19-qubit passes (128 tiles) 23.5 -> 22.9;
 // with thousands of tiles most find it there anyway.
 constexpr uint32_t kTouchTiles = 512;
 
 // Is some amplitude of the workgroup's tile not zero? A register that has just
 // been set to |0..0> is nothing but zeros outside a few tiles until each of its
 // qubits has met a gate, three passes or so later. A pass is linear: such a tile
-// needs neither its ops nor a store. Two barriers and 32 ORs for the others (a
-// dense 27-qubit pass 943 us without, 948 with). The first of seven passes over
-// 27 qubits 943 -> 325 us and, unread where the earlier passes cannot have put
-// anything (FP_REACH), the second 40 and the third 110; a 26-qubit complex64
-// ansatz 508 -> 105 and 49 us.
+// needs neither its ops nor a store. Two barriers and 64 ORs (32 in FP32) a thread
+// for the others (a dense 27-qubit pass 943 us without, 948 with). The first of
+// seven passes over 27 qubits 943 -> 460 us at most and, unread where the earlier
+// passes cannot have put anything (FP_REACH), the second 35 and the third 95; a
+// 26-qubit complex64 ansatz 508 -> 105 and 46 us.
 template <typename A>
 __device__ __forceinline__ bool any_nonzero(const Slots<A>& x, uint32_t* flags)
 {

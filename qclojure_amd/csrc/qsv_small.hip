@@ -11,9 +11,9 @@
 // after each; a state of fewer than 12 qubits of its own took one launch per
 // gate. Bound by the chain of ops (their fetches are hidden by a read of the
 // program up front and a fetch one op ahead). Kernel time, before and now: 280
-// batched QAOA instances of 8 to 14 qubits 1206 -> 491 us (four size classes),
-// 1000 noisy trajectories of 11 qubits 320 -> 87 us, the small requests of a
-// served burst 1780 -> 790 us, a 5-qubit program 25 launches -> one of 12 us.
+// batched QAOA instances of 8 to 14 qubits 1206 -> 535 us (four size classes),
+// 1000 noisy trajectories of 11 qubits 320 -> 85 us, the small requests of a
+// served burst 1780 -> 590 us, a 5-qubit program 25 launches -> one of 12 us.
 #include "qsv_ops.h"
 
 namespace qsv {
