@@ -19,7 +19,10 @@ def _expected(psi, shots, seed):
 
 
 @pytest.mark.parametrize("n,shots", [(1, 9), (3, 100), (6, 300), (9, 500), (10, 1000), (11, 1000), (16, 2000),
-                                     (20, 2000), (21, 2000), (22, 70000)])
+                                     (20, 2000), (21, 2000), (22, 70000),
+                                     # enough shots for the kernel that reads less and waits more
+                                     (1, 2049), (4, 3000), (7, 5000), (10, 2049), (11, 4000), (15, 9000), (20, 2048),
+                                     (20, 2049), (21, 6000)])
 @pytest.mark.parametrize("precision", ["c128", "c64"])
 def test_shots(n, shots, precision):
     rng = np.random.default_rng(n)
