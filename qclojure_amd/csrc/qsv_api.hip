@@ -1250,7 +1250,12 @@ int run_fused(qsv_state* s, const std::vector<BGate>& gs_in, uint32_t flags)
 // 30.5 / 30.3 us at 18 qubits, 33.0 / 29.8 at 19, 39 / 30 at 20; the 4n - 3
 // strings of a Heisenberg chain 44 / 59 us at 18, 53 / 58 at 19, 82 / 62 at 20
 // (complex64 within 15 % of these).
-constexpr int kPauliTileZ = 19, kPauliTileX = 20;
+// A string by itself is a row: nothing shares its sweep, whose staging then
+// only adds (a sweep / a row, one X-type string: 32 / 27 us at 20 qubits,
+// 44 / 36 at 22, 80 / 64 at 24, 830 / 774 at 28; one Z string 29 / 27, 38 / 36,
+// 67 / 63, 810 / 795). One Z string over complex64 is the exception, bound by the
+// row's instructions: 51 / 49 us at 24 qubits, 71 / 72 at 25, 124 / 173 at 26.
+constexpr int kPauliTileZ = 19, kPauliTileX = 20, kPauliLoneZ32 = 25;
 
 // out[t] = Re((-i)^ny (sum_i (-1)^popc(i & sm) conj(a_i) a_(i ^ xm))) for every
 // string t. Strings are taken 256 at a time: their launches follow one another
@@ -1269,7 +1274,8 @@ int pauli_sums(const qsv_state* s, const std::vector<uint64_t>& xm, const std::v
     int slots = 0;
     std::vector<uint64_t> zs, xs, rows;   // strings by the kernel that takes them
     for (uint64_t t = t0; t < t1; ++t) {
-      if (s->n < (xm[t] ? kPauliTileX : kPauliTileZ) || __builtin_popcountll(xm[t] | low) > TB) rows.push_back(t);
+      const bool lone = t1 - t0 == 1 && (xm[t] || s->prec == QSV_C128 || s->n < kPauliLoneZ32);
+      if (lone || s->n < (xm[t] ? kPauliTileX : kPauliTileZ) || __builtin_popcountll(xm[t] | low) > TB) rows.push_back(t);
       else (xm[t] ? xs : zs).push_back(t);
     }
     // strings with the same X part next to each other, X parts by their highest bit

@@ -77,3 +77,21 @@ def test_many_strings(n):
     exp = np.array([_expectation(psi, n, s) for s in strings])
     assert np.max(np.abs(got - exp)) < 1e-13
     assert np.array_equal(got, again)   # fixed summation order
+
+
+@pytest.mark.parametrize("precision", ["c128", "c64"])
+@pytest.mark.parametrize("n", [19, 20, 22, 25])
+def test_string_by_itself(n, precision):
+    """One string in a call, and the one left over after whole chunks of 256."""
+    rng = np.random.default_rng(200 + n)
+    psi = _random_state(n, rng)
+    if precision == "c64":
+        psi = psi.astype(np.complex64).astype(np.complex128)
+    lone = ["Z" + "I" * (n - 1), "I" * (n - 2) + "XY", "Y" + "I" * (n - 2) + "X", "".join(rng.choice(list("IXYZ"), n))]
+    with engine.DeviceState(n, precision) as st:
+        st.upload(psi)
+        got = [float(st.expect_pauli([s])[0]) for s in lone]
+        tail = st.expect_pauli([lone[0]] * 256 + [lone[1]])
+    exp = np.array([_expectation(psi, n, s) for s in lone])
+    assert np.max(np.abs(np.array(got) - exp)) < 1e-13
+    assert np.max(np.abs(tail - np.array([exp[0]] * 256 + [exp[1]]))) < 1e-13
