@@ -5,6 +5,7 @@
 from __future__ import annotations
 
 import os
+import re
 import subprocess
 import sys
 import tempfile
@@ -30,23 +31,57 @@ _OPS_FLAGS = [
     # spills instead of 101 and none). No vector combining: it turns a slot's
     # scalar into a two-slot vector load, which keeps FP32 tiles in scratch.
     "-mllvm", "-structurizecfg-skip-uniform-regions=true", "-mllvm", "-disable-vector-combine",
+    # both are the compiler's internals: what its kernels take is checked (spills)
+    "-Rpass-analysis=kernel-resource-usage",
 ]
 FILE_FLAGS = {"qsv_pass.hip": _OPS_FLAGS, "qsv_small.hip": _OPS_FLAGS}
 
 
 def _noise(text: str) -> list[str]:
-    return [l for l in text.splitlines()
-            if l.strip() and "packed-fp32-ops" not in l and "not a recognized feature" not in l]
+    out, remark = [], False
+    for l in text.splitlines():
+        if ": remark: " in l:
+            remark = True   # the source lines that it quotes follow
+        elif re.search(r": (warning|error|note): ", l):
+            remark = False
+        if l.strip() and not remark and "packed-fp32-ops" not in l and "not a recognized feature" not in l:
+            out.append(l)
+    return out
+
+
+def spills(text: str) -> dict[str, tuple[int, int]]:
+    """Scratch bytes a lane and spilled vector registers of every kernel in the compiler's resource remarks."""
+    out: dict[str, tuple[int, int]] = {}
+    name, scratch = None, 0
+    for l in text.splitlines():
+        m = re.search(r"remark: .*?(Function Name|ScratchSize \[bytes/lane\]|VGPRs Spill): (\S+)", l)
+        if not m:
+            continue
+        if m[1] == "Function Name":
+            name, scratch = m[2], 0
+        elif m[1].startswith("Scratch"):
+            scratch = int(m[2])
+        elif name:
+            out[name] = (scratch, int(m[2]))
+    return out
+
+
+def command(src: str, obj: str) -> list[str]:
+    return ["hipcc", *HIPCC_FLAGS, *FILE_FLAGS.get(os.path.basename(src), []), "-c", "-o", obj, src]
 
 
 def _compile(src: str, obj: str, verbose: bool) -> None:
-    cmd = ["hipcc", *HIPCC_FLAGS, *FILE_FLAGS.get(os.path.basename(src), []), "-c", "-o", obj, src]
+    cmd = command(src, obj)
     if verbose:
         print(" ".join(cmd), flush=True)
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         sys.stderr.write(r.stdout + r.stderr)
         raise RuntimeError(f"hipcc failed on {src}")
+    for kernel, (scratch, regs) in spills(r.stderr).items():
+        if scratch or regs:
+            sys.stderr.write(f"{os.path.basename(src)}: {kernel} keeps {scratch} bytes a lane in scratch "
+                             f"({regs} spilled registers): this compiler does not honour the flags\n")
     if verbose and _noise(r.stdout + r.stderr):
         print("\n".join(_noise(r.stdout + r.stderr)))
 
