@@ -501,6 +501,7 @@ __global__ __launch_bounds__(kBlock) void k_sample(const typename VT<R>::T* __re
 struct PosArgs {
   int32_t m;
   int32_t pos[24];
+  uint32_t out[24];   // outcome bits of the measured bits that a thread walks, lowest first
 };
 
 __device__ __forceinline__ uint64_t gather_bits(uint64_t i, const PosArgs& p)
@@ -510,16 +511,25 @@ __device__ __forceinline__ uint64_t gather_bits(uint64_t i, const PosArgs& p)
   return o;
 }
 
-// Weights of the outcomes of m <= 12 measured bits. A block takes `span`
-// consecutive amplitudes (a power of two), thread t those whose index is t
-// modulo kBlock. It walks them with the measured bits outermost, eight loads in
-// flight, so a sum stays in a register while the outcome does; it is then summed
-// over the lanes with the same outcome and added to the block's LDS histogram.
-// One LDS atomic per amplitude before, up to 64 lanes on one address: the three
-// measured bits of 24 qubits, complex128, 102 us; now 49 us, the time of the read.
+// The same for m <= 12 and places above m that say 63: no chain of loads.
+__device__ __forceinline__ uint32_t gather_bits12(uint64_t i, const PosArgs& p)
+{
+  uint32_t o = 0;
+#pragma unroll
+  for (int j = 0; j < 12; ++j) o |= (uint32_t)((i >> p.pos[j]) & 1ull) << j;
+  return o;
+}
+
+// Weights of the outcomes of m <= 12 measured bits. Thread t of a block takes the
+// amplitudes whose low bits are t; it walks the subsets of `walk`, index bits
+// above those, with the measured ones outermost and eight loads in flight, so a
+// sum stays in a register while the outcome does. It is then summed over the
+// lanes with the same outcome and added to the block's LDS histogram. One LDS
+// atomic per amplitude before, up to 64 lanes on one address: the three measured
+// bits of 24 qubits, complex128, 102 us; now 49 us, the time of the read.
 template <typename R>
 __global__ __launch_bounds__(kBlock) void k_outcome_hist_lds(const typename VT<R>::T* __restrict__ psi, uint64_t S,
-                                                              uint64_t span, uint64_t mask, PosArgs p,
+                                                              uint64_t walk, uint64_t mask, PosArgs p,
                                                               double* __restrict__ hist)
 {
   using T = typename VT<R>::T;
@@ -529,63 +539,92 @@ __global__ __launch_bounds__(kBlock) void k_outcome_hist_lds(const typename VT<R
   for (int k = threadIdx.x; k < no; k += kBlock) h[k] = 0.0;
   __syncthreads();
   const uint32_t t = threadIdx.x, lane = t & 63u;
-  const uint64_t first = (uint64_t)blockIdx.x * span + t;
-  const bool in = first < S;   // (a state of less than a block)
-  const uint64_t inside = (span - 1) & ~(uint64_t)(kBlock - 1);   // the bits a thread walks
-  const uint64_t outer = inside & mask, inner = inside & ~mask;
-  const uint64_t total = 1ull << __popcll(inside), runs = 1ull << __popcll(inner);
+  uint64_t first = (uint64_t)blockIdx.x * kBlock;
+  for (uint64_t r = walk; r; r &= r - 1) {   // the block's number in the bits that are not walked
+    const uint64_t below = (r & (0 - r)) - 1;
+    first = ((first & ~below) << 1) | (first & below);
+  }
+  const bool in = first + t < S;   // (a state of less than a block)
+  uint64_t outer = walk & mask, inner = walk & ~mask;
+  const int run_log = __popcll(inner);
+  const uint32_t total = 1u << __popcll(walk), runs = 1u << run_log;
   const uint32_t same = ~(uint32_t)mask & 63u;   // lane bits the outcome does not see
-  uint64_t o = 0, k = 0;   // the walk: subsets of the outer and, within, of the inner bits
-  auto step = [&]() -> bool {   // true at the end of a run of one outcome
-    k = (k - inner) & inner;
-    if (k) return false;
-    o = (o - outer) & outer;
-    return true;
-  };
-  double acc = 0.0;
-  auto add = [&](uint64_t at) {
+  // An outcome is that of the first amplitude and of the walk's place: E outcomes in
+  // a row differ in the lowest measured bits of the walk.
+  const uint32_t mine = gather_bits12(first + t, p);
+  uint64_t d[3];   // the walk's first three bits: the eight loads in flight
 #pragma unroll
-    for (int b = 0; b < 6; ++b)
-      if ((same >> b) & 1u) acc += __shfl_xor(acc, 1 << b, 64);
-    if (!(lane & same) && in) atomicAdd(&h[gather_bits(at, p)], acc);
-    acc = 0.0;
-  };
-  for (uint64_t l = 0; l < total; l += kFly) {
+  for (int j = 0; j < 3; ++j) {
+    uint64_t& from = inner ? inner : outer;
+    d[j] = from & (0 - from);
+    from &= ~d[j];
+  }
+  uint64_t o = 0, k = 0;   // the rest of it: subsets of the outer and, within, of the inner bits
+  double acc = 0.0;
+  for (uint32_t l = 0; l < total; l += kFly) {
     T v[kFly];
     double w[kFly];
-    const uint64_t o0 = o, k0 = k;
+    const T* at = psi + (first + o + k);
+    auto off = [&](uint32_t f) { return (f & 1 ? d[0] : 0) + (f & 2 ? d[1] : 0) + (f & 4 ? d[2] : 0); };
     if (total >= kFly) {
 #pragma unroll
-      for (uint32_t f = 0; f < kFly; ++f) {
-        v[f] = psi[first + o + k];
-        step();
-      }
+      for (uint32_t f = 0; f < kFly; ++f) v[f] = (at + off(f))[t];
     } else {
 #pragma unroll
       for (uint32_t f = 0; f < kFly; ++f) {
         v[f].x = v[f].y = R(0);
-        if (f < total) {
-          if (in) v[f] = psi[first + o + k];
-          step();
-        }
+        if (f < total && in) v[f] = (at + off(f))[t];
       }
     }
+    k = (k - inner) & inner;
+    if (!k) o = (o - outer) & outer;
 #pragma unroll
     for (uint32_t f = 0; f < kFly; ++f) w[f] = (double)v[f].x * v[f].x + (double)v[f].y * v[f].y;
+    uint32_t E = (total < kFly ? total : kFly) / (runs < kFly ? runs : kFly);
     if (runs >= kFly) {   // one outcome
       acc += ((w[0] + w[1]) + (w[2] + w[3])) + ((w[4] + w[5]) + (w[6] + w[7]));
-      if (!k) add(first + o0);
-    } else {
-      o = o0;
-      k = k0;
+      if (k) continue;
+      w[0] = acc;
+      acc = 0.0;
+    } else if (runs == 4) {
+      w[0] = (w[0] + w[1]) + (w[2] + w[3]);
+      w[1] = (w[4] + w[5]) + (w[6] + w[7]);
+    } else if (runs == 2) {
 #pragma unroll
-      for (uint32_t f = 0; f < kFly; ++f) {
-        if (f < total) {
-          acc += w[f];
-          const uint64_t at = first + o;
-          if (step()) add(at);
-        }
+      for (int e = 0; e < 4; ++e) w[e] = w[2 * e] + w[2 * e + 1];
+    }
+    // Sums over the lanes with the same outcomes: of E outcomes each lane keeps one
+    // half and hands the other to its partner, and the last one is summed as usual:
+    // eight outcomes take 10 exchanges and one atomic instead of 48 and eight.
+    uint32_t to = mine, idle = 0;
+    int q = 0;
+    for (uint32_t c = l >> run_log; c; c >>= 1, ++q) to |= c & 1 ? p.out[q] : 0;
+    for (uint32_t left = same; left; left &= left - 1) {
+      const uint32_t bit = left & (0 - left);
+      const bool up = lane & bit;
+      if (E == 8) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) w[e] = (up ? w[e + 4] : w[e]) + __shfl_xor(up ? w[e] : w[e + 4], bit, 64);
+        to |= up ? p.out[2] : 0;
+        E = 4;
+      } else if (E == 4) {
+#pragma unroll
+        for (int e = 0; e < 2; ++e) w[e] = (up ? w[e + 2] : w[e]) + __shfl_xor(up ? w[e] : w[e + 2], bit, 64);
+        to |= up ? p.out[1] : 0;
+        E = 2;
+      } else if (E == 2) {
+        w[0] = (up ? w[1] : w[0]) + __shfl_xor(up ? w[0] : w[1], bit, 64);
+        to |= up ? p.out[0] : 0;
+        E = 1;
+      } else {
+        w[0] += __shfl_xor(w[0], bit, 64);
+        idle |= bit;
       }
+    }
+    if (!(lane & idle) && in) {
+#pragma unroll
+      for (uint32_t e = 0; e < kFly; ++e)
+        if (e < E) atomicAdd(&h[to | (e & 1 ? p.out[0] : 0) | (e & 2 ? p.out[1] : 0) | (e & 4 ? p.out[2] : 0)], w[e]);
     }
   }
   __syncthreads();
@@ -787,7 +826,7 @@ void launch_outcome_hist(int prec, const void* psi, uint64_t S, int m, const int
 {
   PosArgs p{};
   p.m = m;
-  for (int j = 0; j < m; ++j) p.pos[j] = pos[j];
+  for (int j = 0; j < 24; ++j) p.pos[j] = j < m ? pos[j] : 63;
   const uint64_t no = 1ull << m;
   hipLaunchKernelGGL(k_zero_f64, dim3(stream_grid(no)), dim3(kBlock), 0, st, hist, no);
   if (m <= 12) {
@@ -796,22 +835,40 @@ void launch_outcome_hist(int prec, const void* psi, uint64_t S, int m, const int
     // At most 512 blocks, 1024 where the read dominates: each adds its outcomes to
     // the same few global sums (one measured bit of 20 qubits: 51 us a call with 256
     // blocks, 56 with 512, 63 with 1024; of 22 qubits 73 with 512, 77 with 1024). 16
-    // amplitudes a thread, 8 below 2^20 (one round of loads), half as many for each
-    // measured bit that it would walk: a thread of several outcomes makes as many
-    // chains of lane exchanges (8 high bits of 13 qubits 41 us a call; 49 with eight
-    // outcomes a thread; 42 with one LDS atomic an amplitude, which is within 4 % of
-    // this up to 19 qubits and up to 80 % slower above; for 12 bits of 20 or 21
-    // qubits it is 10 % faster).
-    const int each = S >= 1ull << 20 ? 4 : 3;
-    const uint64_t least = (uint64_t)kBlock << (each - __builtin_popcountll(mask & (((1ull << each) - 1) * kBlock)));
-    const uint64_t span = std::min(S, std::max(S >> (S >= 1ull << 23 ? 10 : 9), least));
-    const unsigned g = (unsigned)((S + span - 1) / span);
+    // amplitudes a thread, 8 below 2^20 (one round of loads). A thread walks bits
+    // that are not measured as long as there are any, so its sums are few (the nine
+    // middle qubits of 22: 98 us when it walked the next bits above its own, 63 now;
+    // one LDS atomic an amplitude 78). The highest of them up to 64 MiB, where blocks
+    // side by side then read side by side (one bit of 20 qubits 46 / 52 us, six of 22
+    // 61 / 67); the lowest above (six of 24: 129 / 119) and with 12 measured bits,
+    // whose blocks then meet fewer outcomes (of 16 qubits 59 / 47).
+    const int n = 63 - __builtin_clzll(S), block = 8;
+    int walked = 0;
+    uint64_t walk = 0;
+    if (n > block) {
+      const uint64_t above = (S - 1) & ~(uint64_t)(kBlock - 1);
+      const uint64_t from[2] = {above & ~mask, above & mask};
+      const bool high = m < 12 && S * (prec == QSV_C128 ? 16 : 8) <= 64ull << 20;
+      walked = std::max(n - block - (n >= 23 ? 10 : 9), std::min(n >= 20 ? 4 : 3, __builtin_popcountll(from[0])));
+      int left = walked;
+      for (uint64_t r : from)
+        for (; r && left; --left) {
+          const uint64_t bit = high ? 1ull << (63 - __builtin_clzll(r)) : r & (0 - r);
+          walk |= bit;
+          r &= ~bit;
+        }
+      int q = 0;
+      for (uint64_t r = walk & mask; r; r &= r - 1, ++q)
+        for (int j = 0; j < m; ++j)
+          if ((r & (0 - r)) == 1ull << pos[j]) p.out[q] = 1u << j;
+    }
+    const unsigned g = n > block ? (unsigned)(S >> (block + walked)) : 1u;
     const size_t lds = no * sizeof(double);
     if (prec == QSV_C128)
-      hipLaunchKernelGGL((k_outcome_hist_lds<double>), dim3(g), dim3(kBlock), lds, st, (const double2*)psi, S, span,
+      hipLaunchKernelGGL((k_outcome_hist_lds<double>), dim3(g), dim3(kBlock), lds, st, (const double2*)psi, S, walk,
                          mask, p, hist);
     else
-      hipLaunchKernelGGL((k_outcome_hist_lds<float>), dim3(g), dim3(kBlock), lds, st, (const float2*)psi, S, span,
+      hipLaunchKernelGGL((k_outcome_hist_lds<float>), dim3(g), dim3(kBlock), lds, st, (const float2*)psi, S, walk,
                          mask, p, hist);
   } else {
     if (prec == QSV_C128)

@@ -1,6 +1,6 @@
 """Outcome weights and collapse: which of the measured bits lie in a lane, in a
-wave, in the part a thread walks (its outcomes in runs of one amplitude and more)
-or above it; states smaller than a block."""
+wave, among the bits a thread walks (its outcomes in runs of one amplitude and more,
+up to eight in a row) or above them; states smaller than a block."""
 from __future__ import annotations
 
 import numpy as np
@@ -16,7 +16,8 @@ pytestmark = pytest.mark.gpu
     (1, [0]), (2, [0, 1]), (7, [6]), (8, [0, 7]), (9, [0]), (12, list(range(12))), (14, [0, 1]), (14, [12, 13]),
     (15, [0, 5, 6, 9, 14]), (17, [1, 2, 3, 4, 5, 6, 7, 8]), (18, list(range(6, 18))), (18, list(range(0, 14))),
     (12, [3]), (13, list(range(8))), (16, [4, 6]), (17, [5, 7, 16]), (20, list(range(12))), (21, [9, 12]),
-    (25, [0, 12, 24]),
+    (25, [0, 12, 24]), (10, [0, 1]), (10, [1]), (11, [0, 2]), (19, list(range(11)) + [17]), (21, list(range(12))),
+    (22, list(range(12))), (22, [3, 9, 13]), (22, list(range(6, 15))), (23, [2, 3, 15, 22]),
 ])
 def test_measure(prec, n, qubits):
     rng = np.random.default_rng(n * 31 + len(qubits))
