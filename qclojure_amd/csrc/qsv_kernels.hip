@@ -501,7 +501,6 @@ __global__ __launch_bounds__(kBlock) void k_sample(const typename VT<R>::T* __re
 struct PosArgs {
   int32_t m;
   int32_t pos[24];
-  uint32_t out[24];   // outcome bits of the measured bits that a thread walks, lowest first
 };
 
 __device__ __forceinline__ uint64_t gather_bits(uint64_t i, const PosArgs& p)
@@ -511,14 +510,25 @@ __device__ __forceinline__ uint64_t gather_bits(uint64_t i, const PosArgs& p)
   return o;
 }
 
-// The same for m <= 12 and places above m that say 63: no chain of loads.
-__device__ __forceinline__ uint32_t gather_bits12(uint64_t i, const PosArgs& p)
-{
-  uint32_t o = 0;
+// All that k_outcome_hist_lds is told, in one cache line: arguments come from host
+// memory (one bit of 13 qubits 40.6 -> 40.1 us a call against 240 bytes of them).
+template <typename T>
+struct HistArgs {
+  const T* psi;
+  double* hist;
+  uint64_t S, walk, mask;
+  uint8_t pos[12], m, pad[3];   // 63 from m on: no chain of loads, none set
+  uint64_t out;                 // four bits each: outcome bits of the walked measured bits, lowest first
+  __device__ __forceinline__ uint32_t gather(uint64_t i) const
+  {
+    uint32_t o = 0;
 #pragma unroll
-  for (int j = 0; j < 12; ++j) o |= (uint32_t)((i >> p.pos[j]) & 1ull) << j;
-  return o;
-}
+    for (int j = 0; j < 12; ++j) o |= (uint32_t)((i >> pos[j]) & 1ull) << j;
+    return o;
+  }
+  __device__ __forceinline__ uint32_t outer(int q) const { return 1u << ((out >> (4 * q)) & 15u); }
+};
+static_assert(sizeof(HistArgs<double>) == 64);
 
 // Weights of the outcomes of m <= 12 measured bits. Thread t of a block takes the
 // amplitudes whose low bits are t; it walks the subsets of `walk`, index bits
@@ -526,13 +536,17 @@ __device__ __forceinline__ uint32_t gather_bits12(uint64_t i, const PosArgs& p)
 // sum stays in a register while the outcome does. It is then summed over the
 // lanes with the same outcome and added to the block's LDS histogram. One LDS
 // atomic per amplitude before, up to 64 lanes on one address: the three measured
-// bits of 24 qubits, complex128, 102 us; now 49 us, the time of the read.
-template <typename R>
-__global__ __launch_bounds__(kBlock) void k_outcome_hist_lds(const typename VT<R>::T* __restrict__ psi, uint64_t S,
-                                                              uint64_t walk, uint64_t mask, PosArgs p,
-                                                              double* __restrict__ hist)
+// bits of 24 qubits, complex128, 102 us; now 49 us, the time of the read. RUNS: at
+// least eight amplitudes of an outcome in a row. A launch fetches its code cold,
+// so that case has a kernel of its own, half as long: in one body with the other
+// a call took 1 us more at 13 qubits and 3 more at 24.
+template <typename R, bool RUNS>
+__global__ __launch_bounds__(kBlock) void k_outcome_hist_lds(const HistArgs<typename VT<R>::T> p)
 {
   using T = typename VT<R>::T;
+  const T* __restrict__ psi = p.psi;
+  double* __restrict__ hist = p.hist;
+  const uint64_t S = p.S, walk = p.walk, mask = p.mask;
   extern __shared__ double h[];
   constexpr uint32_t kFly = 8;
   const int no = 1 << p.m;
@@ -551,7 +565,7 @@ __global__ __launch_bounds__(kBlock) void k_outcome_hist_lds(const typename VT<R
   const uint32_t same = ~(uint32_t)mask & 63u;   // lane bits the outcome does not see
   // An outcome is that of the first amplitude and of the walk's place: E outcomes in
   // a row differ in the lowest measured bits of the walk.
-  const uint32_t mine = gather_bits12(first + t, p);
+  const uint32_t mine = p.gather(first) | p.gather(t);
   uint64_t d[3];   // the walk's first three bits: the eight loads in flight
 #pragma unroll
   for (int j = 0; j < 3; ++j) {
@@ -560,71 +574,82 @@ __global__ __launch_bounds__(kBlock) void k_outcome_hist_lds(const typename VT<R
     from &= ~d[j];
   }
   uint64_t o = 0, k = 0;   // the rest of it: subsets of the outer and, within, of the inner bits
-  double acc = 0.0;
-  for (uint32_t l = 0; l < total; l += kFly) {
-    T v[kFly];
+  auto off = [&](uint32_t f) { return (f & 1 ? d[0] : 0) + (f & 2 ? d[1] : 0) + (f & 4 ? d[2] : 0); };
+  const uint32_t each = RUNS ? runs : kFly;   // amplitudes a round
+  for (uint32_t l = 0; l < total; l += each) {
     double w[kFly];
-    const T* at = psi + (first + o + k);
-    auto off = [&](uint32_t f) { return (f & 1 ? d[0] : 0) + (f & 2 ? d[1] : 0) + (f & 4 ? d[2] : 0); };
-    if (total >= kFly) {
+    uint32_t E = 1;
+    if constexpr (RUNS) {   // one outcome
+      double acc = 0.0;
+      do {
+        const T* at = psi + (first + o + k);
+        T v[kFly];
 #pragma unroll
-      for (uint32_t f = 0; f < kFly; ++f) v[f] = (at + off(f))[t];
-    } else {
+        for (uint32_t f = 0; f < kFly; ++f) v[f] = (at + off(f))[t];
 #pragma unroll
-      for (uint32_t f = 0; f < kFly; ++f) {
-        v[f].x = v[f].y = R(0);
-        if (f < total && in) v[f] = (at + off(f))[t];
-      }
-    }
-    k = (k - inner) & inner;
-    if (!k) o = (o - outer) & outer;
-#pragma unroll
-    for (uint32_t f = 0; f < kFly; ++f) w[f] = (double)v[f].x * v[f].x + (double)v[f].y * v[f].y;
-    uint32_t E = (total < kFly ? total : kFly) / (runs < kFly ? runs : kFly);
-    if (runs >= kFly) {   // one outcome
-      acc += ((w[0] + w[1]) + (w[2] + w[3])) + ((w[4] + w[5]) + (w[6] + w[7]));
-      if (k) continue;
+        for (uint32_t f = 0; f < kFly; ++f) w[f] = (double)v[f].x * v[f].x + (double)v[f].y * v[f].y;
+        acc += ((w[0] + w[1]) + (w[2] + w[3])) + ((w[4] + w[5]) + (w[6] + w[7]));
+        k = (k - inner) & inner;
+      } while (k);
       w[0] = acc;
-      acc = 0.0;
-    } else if (runs == 4) {
-      w[0] = (w[0] + w[1]) + (w[2] + w[3]);
-      w[1] = (w[4] + w[5]) + (w[6] + w[7]);
-    } else if (runs == 2) {
+    } else {
+      const T* at = psi + (first + o);
+      T v[kFly];
+      if (total >= kFly) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) w[e] = w[2 * e] + w[2 * e + 1];
+        for (uint32_t f = 0; f < kFly; ++f) v[f] = (at + off(f))[t];
+      } else {
+#pragma unroll
+        for (uint32_t f = 0; f < kFly; ++f) {
+          v[f].x = v[f].y = R(0);
+          if (f < total && in) v[f] = (at + off(f))[t];
+        }
+      }
+#pragma unroll
+      for (uint32_t f = 0; f < kFly; ++f) w[f] = (double)v[f].x * v[f].x + (double)v[f].y * v[f].y;
+      if (runs == 4) {
+        w[0] = (w[0] + w[1]) + (w[2] + w[3]);
+        w[1] = (w[4] + w[5]) + (w[6] + w[7]);
+      } else if (runs == 2) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) w[e] = w[2 * e] + w[2 * e + 1];
+      }
+      E = (total < kFly ? total : kFly) / runs;
     }
+    o = (o - outer) & outer;
     // Sums over the lanes with the same outcomes: of E outcomes each lane keeps one
     // half and hands the other to its partner, and the last one is summed as usual:
     // eight outcomes take 10 exchanges and one atomic instead of 48 and eight.
     uint32_t to = mine, idle = 0;
     int q = 0;
-    for (uint32_t c = l >> run_log; c; c >>= 1, ++q) to |= c & 1 ? p.out[q] : 0;
+    for (uint32_t c = l >> run_log; c; c >>= 1, ++q) to |= c & 1 ? p.outer(q) : 0;
     for (uint32_t left = same; left; left &= left - 1) {
       const uint32_t bit = left & (0 - left);
       const bool up = lane & bit;
-      if (E == 8) {
+      if (RUNS || E == 1) {
+        w[0] += __shfl_xor(w[0], bit, 64);
+        idle |= bit;
+      } else if (E == 8) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) w[e] = (up ? w[e + 4] : w[e]) + __shfl_xor(up ? w[e] : w[e + 4], bit, 64);
-        to |= up ? p.out[2] : 0;
+        to |= up ? p.outer(2) : 0;
         E = 4;
       } else if (E == 4) {
 #pragma unroll
         for (int e = 0; e < 2; ++e) w[e] = (up ? w[e + 2] : w[e]) + __shfl_xor(up ? w[e] : w[e + 2], bit, 64);
-        to |= up ? p.out[1] : 0;
+        to |= up ? p.outer(1) : 0;
         E = 2;
-      } else if (E == 2) {
-        w[0] = (up ? w[1] : w[0]) + __shfl_xor(up ? w[0] : w[1], bit, 64);
-        to |= up ? p.out[0] : 0;
-        E = 1;
       } else {
-        w[0] += __shfl_xor(w[0], bit, 64);
-        idle |= bit;
+        w[0] = (up ? w[1] : w[0]) + __shfl_xor(up ? w[0] : w[1], bit, 64);
+        to |= up ? p.outer(0) : 0;
+        E = 1;
       }
     }
     if (!(lane & idle) && in) {
 #pragma unroll
-      for (uint32_t e = 0; e < kFly; ++e)
-        if (e < E) atomicAdd(&h[to | (e & 1 ? p.out[0] : 0) | (e & 2 ? p.out[1] : 0) | (e & 4 ? p.out[2] : 0)], w[e]);
+      for (uint32_t e = 0; e < (RUNS ? 1 : kFly); ++e)
+        if (e < E)
+          atomicAdd(&h[to | (e & 1 ? p.outer(0) : 0) | (e & 2 ? p.outer(1) : 0) | (e & 4 ? p.outer(2) : 0)], w[e]);
     }
   }
   __syncthreads();
@@ -826,7 +851,7 @@ void launch_outcome_hist(int prec, const void* psi, uint64_t S, int m, const int
 {
   PosArgs p{};
   p.m = m;
-  for (int j = 0; j < 24; ++j) p.pos[j] = j < m ? pos[j] : 63;
+  for (int j = 0; j < m; ++j) p.pos[j] = pos[j];
   const uint64_t no = 1ull << m;
   hipLaunchKernelGGL(k_zero_f64, dim3(stream_grid(no)), dim3(kBlock), 0, st, hist, no);
   if (m <= 12) {
@@ -857,19 +882,26 @@ void launch_outcome_hist(int prec, const void* psi, uint64_t S, int m, const int
           walk |= bit;
           r &= ~bit;
         }
+    }
+    const unsigned g = n > block ? (unsigned)(S >> (block + walked)) : 1u;
+    auto run = [&](auto kernel, auto* amps) {
+      HistArgs<std::remove_const_t<std::remove_pointer_t<decltype(amps)>>> a{amps, hist, S, walk, mask};
+      a.m = (uint8_t)m;
+      for (int j = 0; j < 12; ++j) a.pos[j] = (uint8_t)(j < m ? pos[j] : 63);
       int q = 0;
       for (uint64_t r = walk & mask; r; r &= r - 1, ++q)
         for (int j = 0; j < m; ++j)
-          if ((r & (0 - r)) == 1ull << pos[j]) p.out[q] = 1u << j;
+          if ((r & (0 - r)) == 1ull << pos[j]) a.out |= (uint64_t)j << (4 * q);
+      hipLaunchKernelGGL(kernel, dim3(g), dim3(kBlock), no * sizeof(double), st, a);
+    };
+    const bool runs = __builtin_popcountll(walk & ~mask) >= 3;   // eight amplitudes of one outcome and more
+    if (prec == QSV_C128) {
+      if (runs) run(k_outcome_hist_lds<double, true>, (const double2*)psi);
+      else run(k_outcome_hist_lds<double, false>, (const double2*)psi);
+    } else {
+      if (runs) run(k_outcome_hist_lds<float, true>, (const float2*)psi);
+      else run(k_outcome_hist_lds<float, false>, (const float2*)psi);
     }
-    const unsigned g = n > block ? (unsigned)(S >> (block + walked)) : 1u;
-    const size_t lds = no * sizeof(double);
-    if (prec == QSV_C128)
-      hipLaunchKernelGGL((k_outcome_hist_lds<double>), dim3(g), dim3(kBlock), lds, st, (const double2*)psi, S, walk,
-                         mask, p, hist);
-    else
-      hipLaunchKernelGGL((k_outcome_hist_lds<float>), dim3(g), dim3(kBlock), lds, st, (const float2*)psi, S, walk,
-                         mask, p, hist);
   } else {
     if (prec == QSV_C128)
       hipLaunchKernelGGL((k_outcome_hist_global<double>), dim3(stream_grid(S)), dim3(kBlock), 0, st,
